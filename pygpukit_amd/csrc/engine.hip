@@ -26,6 +26,7 @@
 #include "engine_state.hip.h"
 #include "gemm_epilogues.hip.h"
 #include "pkgemm.hip.h"
+#include "wide.hip.h"
 
 namespace pgk {
 
@@ -1894,6 +1895,77 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
     return PGK_OK;
 }
 
+// Wide models, 1..7 sequences: the projections of ops_wide.hip (fp32 activations throughout, one pass over the weights for all sequences).
+// Attention leaves fp32 rows; o_proj and down_proj add to the residual stream themselves: 5 launches per layer, one more where split-KV
+// records are merged.
+static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStream_t st, int* launches, bool short_ctx) {
+    const auto& c = e->cfg;
+    const bool fp8 = c.weight_format != 0;
+    const int H = c.hidden_size, I = c.intermediate_size, D = c.head_dim, QD = c.num_heads * D, NQKV = e->qkv_dim();
+    float* h = e->h + (size_t)b0 * H;
+    const bool direct = short_ctx && !(fp8 && M == 1);   // (one sequence on e4m3 weights has always merged split-KV records, whose error is a fifth smaller)
+    for (int l = 0; l < c.num_layers; ++l) {
+        const auto& L = e->layers[l];
+        FusedArgs a{};
+        mark(KC_NORM_QKV);
+        a.w = L.w_qkv; a.wscale = (const bf16*)L.s_qkv; a.N = NQKV; a.K = H;
+        a.h = h; a.gamma = (const bf16*)L.attn_norm; a.eps = c.norm_eps;
+        a.out = e->qkv + (size_t)b0 * NQKV; a.ld_out = NQKV;
+        if (pgk_status r = wide_proj(fp8, WIDE_NORM, EPI_STORE, a, nullptr, M, e->cu_count, nullptr, st)) return r;
+        mark(KC_ATTN);
+        if (D == 128) { if (pgk_status r = launch_attn<128>(e, l, b0, M, false, direct, st)) return r; }
+        else { if (pgk_status r = launch_attn<64>(e, l, b0, M, false, direct, st)) return r; }
+        mark(KC_OPROJ);
+        a = FusedArgs{};
+        a.w = L.w_o; a.wscale = (const bf16*)L.s_o; a.N = H; a.K = QD;
+        a.xin = e->attnv + (size_t)b0 * QD;
+        a.out = h; a.ld_out = H;
+        if (pgk_status r = wide_proj(fp8, WIDE_PLAIN, EPI_RESID, a, nullptr, M, e->cu_count, nullptr, st)) return r;
+        mark(KC_GATEUP);
+        a = FusedArgs{};
+        a.w = L.w_gate_up; a.wscale = (const bf16*)L.s_gate_up; a.N = I; a.K = H;
+        a.h = h; a.gamma = (const bf16*)L.mlp_norm; a.eps = c.norm_eps;
+        if (pgk_status r = wide_proj(fp8, WIDE_NORM, EPI_SWIGLU, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
+        mark(KC_DOWN);
+        a = FusedArgs{};
+        a.w = L.w_down; a.wscale = (const bf16*)L.s_down; a.N = H; a.K = I;
+        a.out = h; a.ld_out = H;
+        if (pgk_status r = wide_proj(fp8, WIDE_PIECES, EPI_RESID, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
+        *launches += 4 + (direct ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads);
+    }
+    mark(KC_LMHEAD);
+    FusedArgs a{};
+    a.w = e->lm_head; a.N = c.vocab_size; a.K = H;
+    a.h = h; a.gamma = e->final_norm; a.eps = c.norm_eps;
+    a.out = e->logits + (size_t)b0 * c.vocab_size; a.ld_out = c.vocab_size;
+    a.amax_val = e->amax_val + (size_t)b0 * e->lm_cap; a.amax_idx = e->amax_idx + (size_t)b0 * e->lm_cap;
+    int nblk = 0;
+    if (pgk_status r = wide_proj(false, WIDE_NORM, EPI_LOGITS, a, nullptr, M, e->cu_count, &nblk, st)) return r;
+    mark(KC_ARGMAX);
+    const int32_t* sampled = nullptr;
+    if (e->sample_temperature > 0.f) {
+        if (pgk_status r = engine_sample(e, b0, M, st)) return r;
+        sampled = e->sampled + b0;
+        *launches += 1;
+    }
+    PGK_CHECK_HIP(launch_k(finalize_kernel<bf16>, dim3(M), dim3(256), 0, st, a.amax_val, a.amax_idx, nblk, e->tokens + b0, e->positions + b0, e->token_log + b0, e->step_counter,
+                                       e->cfg.max_batch, e->log_cap, e->embed, h, H, last ? 1 : 0, b0 == 0 ? e->clk_log : nullptr,
+                                       e->rope_cos, e->rope_sin, e->cur_cos + (size_t)b0 * (D / 2), e->cur_sin + (size_t)b0 * (D / 2),
+                                       D / 2, c.max_seq_len, M, sampled, (const bf16*)nullptr, H));
+    *launches += 2;
+    return PGK_OK;
+}
+
+// Rows in 16-byte loads, gammas in 8-byte ones, two block scales per word.
+static bool wide_aligned(const Engine* e) {
+    auto at = [](const void* p, uintptr_t n) { return ((uintptr_t)p & (n - 1)) == 0; };
+    bool ok = at(e->lm_head, 16) && at(e->final_norm, 8);
+    for (const auto& L : e->layers)
+        ok = ok && at(L.w_qkv, 16) && at(L.w_o, 16) && at(L.w_gate_up, 16) && at(L.w_down, 16) && at(L.attn_norm, 8) && at(L.mlp_norm, 8) && at(L.s_qkv, 4) && at(L.s_o, 4) &&
+             at(L.s_gate_up, 4) && at(L.s_down, 4);
+    return ok;
+}
+
 template <class WT>
 static pgk_status decode_step_impl(Engine* e, int batch, hipStream_t st, int* launches, bool short_ctx) {
     int b0 = 0;
@@ -1910,6 +1982,7 @@ static pgk_status decode_step_impl(Engine* e, int batch, hipStream_t st, int* la
             else r = decode_chunk_batched<WT>(e, b0, m, rem == m, st, launches, short_ctx);
             b0 += m;
         }
+        else if (rem < 8 && (e->wide >> rem & 1)) { r = decode_chunk_wide(e, b0, rem, true, st, launches, short_ctx); b0 += rem; }
         else if (rem >= 8) { r = decode_chunk<WT, bf16, 8>(e, b0, rem == 8, st, launches, short_ctx); b0 += 8; }
         else if (rem >= 4) { r = decode_chunk<WT, bf16, 4>(e, b0, rem == 4, st, launches, short_ctx); b0 += 4; }
         else if (rem >= 2) { r = decode_chunk<WT, float, 2>(e, b0, rem == 2, st, launches, short_ctx); b0 += 2; }
@@ -2299,6 +2372,23 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
         e->batched_max = (k_tiled(c.hidden_size) && k_tiled(c.intermediate_size) && k_tiled(c.num_heads * c.head_dim)) ? 64 : 16;
         if (const char* em = getenv("PGK_BATCHED_MAX")) { const int v = atoi(em); if (v >= 16 && v < e->batched_max) e->batched_max = v; }
     }
+    {
+        // How many sequences decode on ops_wide.hip, one pass over the weights (us per step before -> after, 8 layers, bf16 unless said):
+        //   * 3, 5, 6, 7, where the batch kernels of engine_batched.hip do not take the model: the GEMV kernels pass over the weights two or
+        //     three times (width 2048, 7 sequences: 2012 -> 409; Llama-3-8B shape, 6: 15300 -> 3430);
+        //   * 4 from width 1536 on, or where a row is not among the GEMV kernels' compile-time lengths (width 2048 e4m3 405 -> 355, 1536 691 ->
+        //     455, 1024 with such a row 362 -> 318; but Qwen3-0.6B, all lengths fixed: 771 against 980 here);
+        //   * 1 and 2 where both hold (Llama-3-8B shape 5340 -> 3080; 1536: 416 -> 411; 1024: 254 against 277 here).
+        // Left out: feed-forwards of which two rows do not fit LDS, which the GEMV kernels refuse for more than one sequence.
+        const bool f8 = c.weight_format != 0;
+        const int I = c.intermediate_size, QD = c.num_heads * D, NQ = e->qkv_dim(), nw = f8 ? 16 : 8;
+        auto fixed = [&](int N, int K) { return K % (64 * nw) == 0 && K / (64 * nw) <= (N >= 4096 ? 3 : 6); };
+        const bool ok = wide_proj_ok(NQ, H, false) && wide_proj_ok(H, QD, false) && wide_proj_ok(I, H, false) && wide_proj_ok(H, I, true) && wide_proj_ok(c.vocab_size, H, false) &&
+                        (size_t)I * 8 <= 156 * 1024 && wide_aligned(e);
+        const bool all_fixed = fixed(NQ, H) && fixed(H, QD) && fixed(I, H) && fixed(H, I);
+        if (ok) e->wide = 0xE8 | (H >= 1536 || !all_fixed ? 0x10 : 0) | (H >= 1536 && !all_fixed ? 0x06 : 0);
+    }
+    if (e->wide) A((void**)&e->wide_act, wide_pieces_elems(c.intermediate_size, 7) * 2, &e->ws_bytes);
     A((void**)&e->amax_val, (size_t)B * e->lm_cap * 4, &e->ws_bytes);
     A((void**)&e->amax_idx, (size_t)B * e->lm_cap * 4, &e->ws_bytes);
     A((void**)&e->clk_log, (size_t)e->log_cap * 16, &e->ws_bytes);

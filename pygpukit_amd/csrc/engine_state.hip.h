@@ -132,6 +132,8 @@ struct Engine {
     bool batched_mfma = true;   // chunks of 3 and 5..16 sequences use engine_batched.hip.h (PGK_BATCHED_MFMA=0: GEMV kernels only, =2: from 3 up)
     int batched_min = 5, batched_max = 64;   // PGK_BATCHED_MAX=16: chunks of at most 16 sequences (one weight pass per chunk), the A/B switch of the tiled kernels
     int cu_count = 256;
+    int wide = 0;               // bit M: M sequences decode on ops_wide.hip
+    bf16* wide_act = nullptr;   // ... and the SwiGLU output between its two projections (split pieces)
     bool short_path = true;     // contexts <= SHORT_CTX take the whole-context attention kernels (PGK_FUSED_ATTN=0: the split-KV sequence at every context)
     int pos_hi = -1;            // host-side upper bound of the largest position the next step sees (-1: unknown); selects the sequence, see step_is_short
     // in-graph stochastic sampling (pgk_engine_set_sampling): temperature <= 0 keeps greedy argmax
