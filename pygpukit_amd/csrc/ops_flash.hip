@@ -7,19 +7,24 @@
 //   * the probabilities are already laid out as the B operand of the second product O^T[d][q] += V^T[d][kv] . P^T[kv][q]:
 //     registers 8s..8s+7 of a sub-tile, packed pairwise to 16-bit, ARE the k-step-s fragment (k order permuted:
 //     element j of lane half h is kv = 16s + 8(j>>2) + 4h + (j&3)); the V^T operand is read in the same permuted
-//     order (two 8-byte LDS reads per fragment), so P never touches LDS;
+//     order out of V's row-major image by gfx950's transposing LDS read (two ds_read_b64_tr_b16 per fragment), so P
+//     never touches LDS;
+//   * the scores are scaled in fp32 under the exponential, exp2(s * scale - m): one fma where a subtraction would do (q used to
+//     be multiplied by the scale before, which rounded it to 16 bits once more and was no faster);
 //   * alpha (the running-max rescale) and 1/l are per-lane scalars for the O^T accumulators (q is again the lane).
-// V arrives transposed: a small pre-pass writes V^T [Hkv][D][kv_pad] (zero padded to a multiple of 64 positions) so
-// that both LDS images are filled with 16-byte row-contiguous chunks.
-// Workgroup = 4 waves = 128 query rows of one head; KV tiles of 64 positions, K [64][D] and V^T [D][64] double
+// (V used to be transposed by a pass of its own over the whole context: 5.3 us of a 1531-token prompt's 42 us of
+// attention per layer, 5.8 of 42 for 384 tokens at position 3201.)
+// Workgroup = 4 waves = 128 query rows of one head; KV tiles of 64 positions, K and V [64][D] double
 // buffered in LDS (64 KiB at D = 128: two workgroups per CU); the global loads of tile t+1 are issued before the
 // MFMAs of tile t and written to the other buffer after them: one barrier per tile.
 // Workgroups are ordered heavy-first (causal: late query tiles see more keys) and all query heads of a kv head
 // share id % Hkv, i.e. an XCD when Hkv is a multiple of 8, so the K/V stream of a head is served by one L2.
 // Mask: kv_pos <= (kv_len - q_len) + q_pos  (reference: native/ops/nn/attention_kernels.cuh:32-148).
 
+#include <algorithm>
 #include <type_traits>
 
+#include "flash.hip.h"
 #include "latent.hip.h"
 #include "pgk_device.hip.h"
 #include "pgk_internal.h"
@@ -45,13 +50,21 @@ template <> __device__ __forceinline__ uint32_t pack16x2<f16>(float lo, float hi
 
 struct FlashStrides { long long qh, qs, kh, ks, oh, os; };
 
-constexpr int FL_BQ = 128, FL_BKV = 64, FL_THREADS = 256;
+constexpr int FL_BQ = FLASH_ITEM_ROWS, FL_BKV = 64, FL_THREADS = 256;
 
 // K image: [64 kv][D] 16-bit, 16-byte chunk c (0..D/8-1) of row r at r*2D + ((c ^ (r & (D/8-1))) << 4)
 template <int D> __device__ __forceinline__ int fl_k_off(int r, int c) { return r * (2 * D) + ((c ^ (r & (D / 8 - 1))) << 4); }
-// V^T image: [D][64 kv] 16-bit = 128-byte rows, 8-byte chunk c8 (0..15) of row d at d*128 + ((c8 ^ ((d>>1) & 15)) << 3):
-// the 32 rows a half-wave reads at one c8 then fall on 32 different bank pairs
-__device__ __forceinline__ int fl_v_off(int d, int c8) { return d * 128 + ((c8 ^ ((d >> 1) & 15)) << 3); }
+// V image: [64 kv][D] 16-bit, chunk c of row r at r*2D + ((c ^ x(r)) << 4).  A transposing read takes rows 4n .. 4n+3 (two n, by
+// lane half), 64 contiguous bytes of each: x moves the four rows of an n into different 64-byte parts of the 256 bytes of banks.
+template <int D> __device__ __forceinline__ int fl_v_sw(int r) { return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
+template <int D> __device__ __forceinline__ int fl_v_off(int r, int c) { return r * (2 * D) + ((c ^ fl_v_sw<D>(r)) << 4); }
+
+// Several sequences in one launch (flash.hip.h): a workgroup takes one query tile of one of them instead of what its id says.
+struct FlashMany {
+    const FlashItem* items;
+    int n_items, rows;             // rows: query rows of all sequences
+    long long slot_stride;         // elements between the caches of two slots
+};
 
 // KV split (short prompts): nsplit > 1 cuts a query tile's KV tiles into nsplit contiguous runs, one workgroup each; every
 // workgroup leaves a NORMALISED partial output (type T) and its (m, l) per row, and flash_merge_kernel combines them.
@@ -61,7 +74,8 @@ __device__ __forceinline__ int fl_v_off(int d, int c8) { return d * 128 + ((c8 ^
 struct FlashSplit {
     int nsplit;
     float* ml;      // [nsplit][Hq][q_len][2]  (m in the exp2 domain, l)
-    void* o;        // [nsplit][q_len][Hq][D] of T
+    void* o;        // [nsplit][q_len][Hq][D] of T, or of fp32 (`wide`: up to 128 query rows, and several sequences in one launch)
+    bool wide;
     // fp8 x fp8 prefill (D = 128, bf16): instead of out, e4m3 codes [q_len][Hq * D] and one scale per (row, head) [q_len][Hq]
     // - a head's 128 output dims ARE one 128-wide scale block of the o_proj's A operand (quantize_fp8_rows' contract:
     // scale = absmax / 448 of the bf16-rounded values, 1 for an all-zero block), written by whichever kernel holds the final
@@ -71,8 +85,7 @@ struct FlashSplit {
 };
 
 // Sliding window (WIN instantiations): query i sees keys i - window + 1 .. i, tiles left of a workgroup's first window are never
-// loaded.  `gate`: OutGate, one value per (query row, head) or per element.  The scores are scaled in fp32 after the product
-// (scale > 0: the running maximum is kept on unscaled scores).
+// loaded.  `gate`: OutGate, one value per (query row, head) or per element.
 // BIAS instantiations: slopes[head] * (query - key) is taken off the scaled score - the accumulators of S = K . Q^T start at
 // -slope / scale * (query - key) instead of zero.
 struct FlashWindow {
@@ -100,57 +113,61 @@ template <class T, int N> __device__ __forceinline__ void flash_gate_cols(const 
 }
 
 template <class T, int D, bool WIN = false, bool BIAS = false>
-__global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* vt, T* out, int hq, int hkv,
-                                                              int q_len, int kv_len, int kv_pad, float scale_log2e, FlashStrides sd,
-                                                              FlashSplit sp, FlashWindow win) {
+__global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
+                                                              int q_len, int kv_len, float scale_log2e, FlashStrides sd,
+                                                              FlashSplit sp, FlashWindow win, FlashMany many) {
     constexpr int NC = D / 8;            // 16-byte chunks per K row
     constexpr int KS = D / 16;           // k-steps of Q.K^T
     constexpr int DT = D / 32;           // 32-row tiles of O^T
     constexpr int KCH = 64 * NC / FL_THREADS;   // K chunks staged per thread
-    constexpr int VCH = D * 8 / FL_THREADS;     // V^T chunks staged per thread
-    constexpr int K_BYTES = 64 * D * 2, V_BYTES = D * 128;
-    extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // K[2] | V^T[2]
+    constexpr int K_BYTES = 64 * D * 2, V_BYTES = K_BYTES;
+    extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // K[2] | V[2]
     auto Ks = [&](int buf) -> char* { return fl_smem + buf * K_BYTES; };
     auto Vs = [&](int buf) -> char* { return fl_smem + 2 * K_BYTES + buf * V_BYTES; };
 
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, ql = lane & 31, h = lane >> 5;
     // workgroup id -> (kv head, query head in its group, query tile, KV run), heavy tiles first
-    const int rep = hq / hkv, nqt = (q_len + FL_BQ - 1) / FL_BQ;
+    const int rep = hq / hkv;
     const int id = blockIdx.x;
     const int kvh = id % hkv, rest = id / hkv;
     const int head = kvh * rep + rest % rep;
     const int rest2 = rest / rep;
-    // heavy tiles first - and, when the launch is one round of two workgroups per CU (KV split), the second half of the ids in
-    // ASCENDING weight: a CU's two residents are then a heavy and a light run (ids i and i + grid / 2 sit on the same CU when
-    // the dispatcher deals one workgroup to every CU before the second)
-    int order = rest2;
-    const int nord = nqt * sp.nsplit;
-    if (sp.nsplit > 1 && order >= nord / 2) order = nord / 2 + (nord - 1 - order);
-    const int split = order % sp.nsplit;
-    const int qt = nqt - 1 - order / sp.nsplit;
+    int split, qt, row0 = 0, rows = q_len;
+    if (many.items) {
+        const FlashItem it = many.items[rest2 / sp.nsplit];
+        split = rest2 % sp.nsplit;
+        row0 = __builtin_amdgcn_readfirstlane(it.row0);
+        q_len = __builtin_amdgcn_readfirstlane(it.q_len);
+        kv_len = __builtin_amdgcn_readfirstlane(it.kv_len);
+        const int st = __builtin_amdgcn_readfirstlane(it.slot_tile);
+        qt = st & 0xFFFF;
+        rows = many.rows;
+        q += (long long)row0 * sd.qs;
+        out += (long long)row0 * sd.os;
+        k += (st >> 16) * many.slot_stride;
+        v += (st >> 16) * many.slot_stride;
+    } else {
+        // heavy tiles first - and, when the launch is one round of two workgroups per CU (KV split), the second half of the ids in
+        // ASCENDING weight: a CU's two residents are then a heavy and a light run (ids i and i + grid / 2 sit on the same CU when
+        // the dispatcher deals one workgroup to every CU before the second)
+        const int nqt = (q_len + FL_BQ - 1) / FL_BQ, nord = nqt * sp.nsplit;
+        int order = rest2;
+        if (sp.nsplit > 1 && order >= nord / 2) order = nord / 2 + (nord - 1 - order);
+        split = order % sp.nsplit;
+        qt = nqt - 1 - order / sp.nsplit;
+    }
     const int qw0 = qt * FL_BQ + wid * 32;          // first query row of this wave
     const int causal_off = kv_len - q_len;
     const T* qh = q + (size_t)head * sd.qh;
     const T* kh = k + (size_t)kvh * sd.kh;
-    const T* vh = vt + (size_t)kvh * D * kv_pad;
+    const T* vh = v + (size_t)kvh * sd.kh;
 
     // Q^T fragments (B operand): lane = query column, k = d
     uint4 qf[KS];
     {
-        // Q is pre-multiplied by scale * log2(e) here (one rounding to 16 bits more, inside the 1e-2 bar): the scores come
-        // out of the MFMA already in the exp2 domain and the per-tile scaling pass (32 multiplies per lane) disappears
         const T* qrow = qh + (size_t)min(qw0 + ql, q_len - 1) * sd.qs + 8 * h;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            Vec<T> v;
-            v.load(qrow + ks * 16);
-            float f[8];
-            v.to_float(f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) f[j] *= WIN ? 1.f : scale_log2e;
-            v.from_float(f);
-            qf[ks] = v.raw;
-        }
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const uint4*>(qrow + ks * 16);
     }
     f32x16_fl o[DT];
 #pragma unroll
@@ -169,50 +186,37 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
 
     // staging in NAMED registers (an array here ends up in scratch memory at this register pressure, see
     // ops_fp8_gemm.hip): chunk i of this thread is c = tid + 256 i; KCH = VCH = D / 32 chunks each
-    static_assert(KCH == VCH && (KCH == 2 || KCH == 4), "staging is written for D = 64 / 128");
+    static_assert(KCH == 2 || KCH == 4, "staging is written for D = 64 / 128");
     uint4 rk0, rk1, rk2, rk3, rv0, rv1, rv2, rv3;
-    const int kr = tid / NC, kc16 = tid % NC;               // K: row kr + (256/NC) i, chunk kc16
+    const int kr = tid / NC, kc16 = tid % NC;               // row kr + (256/NC) i, chunk kc16
     constexpr int KR_STEP = FL_THREADS / NC;
-    const int vd = tid >> 3, vc = tid & 7;                  // V^T: row vd + 32 i, chunk vc
-    auto k_src = [&](int kv0, int i) { return kh + (size_t)min(kv0 + kr + KR_STEP * i, kv_len - 1) * sd.ks + kc16 * 8; };
     // Whole tiles address their rows as (wave-uniform tile base) + (per-lane element offset fixed for the kernel): the
     // per-tile address arithmetic is scalar.  (Recomputing min(row, kv_len - 1) * stride per chunk cost 48 vector
     // instructions per tile - 64-bit multiplies included - in a loop that is bound by vector issue.)  Only the ragged
-    // last tile clamps its rows.
+    // last tile clamps its rows (their probabilities are zero).
     const uint32_t ko0 = (uint32_t)(kr * sd.ks + kc16 * 8), ko_step = (uint32_t)(KR_STEP * sd.ks);
-    const uint32_t vo0 = (uint32_t)(vd * kv_pad + vc * 8), vo_step = (uint32_t)(32 * kv_pad);
-    auto load_k = [&](int t) {
+    auto load_rows = [&](const T* base, int t, uint4& r0, uint4& r1, uint4& r2, uint4& r3) {
         const int kv0 = t * FL_BKV;
         if (kv0 + FL_BKV <= kv_len) {      // wave-uniform
-            const T* kt = kh + (size_t)kv0 * sd.ks;
-            rk0 = *reinterpret_cast<const uint4*>(kt + ko0);
-            rk1 = *reinterpret_cast<const uint4*>(kt + ko0 + ko_step);
+            const T* tile = base + (size_t)kv0 * sd.ks;
+            r0 = *reinterpret_cast<const uint4*>(tile + ko0);
+            r1 = *reinterpret_cast<const uint4*>(tile + ko0 + ko_step);
             if constexpr (KCH == 4) {
-                rk2 = *reinterpret_cast<const uint4*>(kt + ko0 + 2 * ko_step);
-                rk3 = *reinterpret_cast<const uint4*>(kt + ko0 + 3 * ko_step);
+                r2 = *reinterpret_cast<const uint4*>(tile + ko0 + 2 * ko_step);
+                r3 = *reinterpret_cast<const uint4*>(tile + ko0 + 3 * ko_step);
             }
         } else {
-            rk0 = *reinterpret_cast<const uint4*>(k_src(kv0, 0));
-            rk1 = *reinterpret_cast<const uint4*>(k_src(kv0, 1));
+            auto src = [&](int i) { return base + (size_t)min(kv0 + kr + KR_STEP * i, kv_len - 1) * sd.ks + kc16 * 8; };
+            r0 = *reinterpret_cast<const uint4*>(src(0));
+            r1 = *reinterpret_cast<const uint4*>(src(1));
             if constexpr (KCH == 4) {
-                rk2 = *reinterpret_cast<const uint4*>(k_src(kv0, 2));
-                rk3 = *reinterpret_cast<const uint4*>(k_src(kv0, 3));
+                r2 = *reinterpret_cast<const uint4*>(src(2));
+                r3 = *reinterpret_cast<const uint4*>(src(3));
             }
         }
     };
-    auto load_v = [&](int t) {
-        const T* vtile = vh + t * FL_BKV;
-        rv0 = *reinterpret_cast<const uint4*>(vtile + vo0);
-        rv1 = *reinterpret_cast<const uint4*>(vtile + vo0 + vo_step);
-        if constexpr (VCH == 4) {
-            rv2 = *reinterpret_cast<const uint4*>(vtile + vo0 + 2 * vo_step);
-            rv3 = *reinterpret_cast<const uint4*>(vtile + vo0 + 3 * vo_step);
-        }
-    };
-    auto put_v = [&](char* base, int d, const uint4& x) {
-        *reinterpret_cast<uint2*>(base + fl_v_off(d, 2 * vc)) = make_uint2(x.x, x.y);
-        *reinterpret_cast<uint2*>(base + fl_v_off(d, 2 * vc + 1)) = make_uint2(x.z, x.w);
-    };
+    auto load_k = [&](int t) { load_rows(kh, t, rk0, rk1, rk2, rk3); };
+    auto load_v = [&](int t) { load_rows(vh, t, rv0, rv1, rv2, rv3); };
     auto store_k = [&](int buf) {
         char* kb = Ks(buf);
         *reinterpret_cast<uint4*>(kb + fl_k_off<D>(kr, kc16)) = rk0;
@@ -224,11 +228,11 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     };
     auto store_v = [&](int buf) {
         char* vb = Vs(buf);
-        put_v(vb, vd, rv0);
-        put_v(vb, vd + 32, rv1);
-        if constexpr (VCH == 4) {
-            put_v(vb, vd + 64, rv2);
-            put_v(vb, vd + 96, rv3);
+        *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr, kc16)) = rv0;
+        *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + KR_STEP, kc16)) = rv1;
+        if constexpr (KCH == 4) {
+            *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + 2 * KR_STEP, kc16)) = rv2;
+            *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + 3 * KR_STEP, kc16)) = rv3;
         }
     };
     // S^T = K . Q^T of one tile: two 32-kv sub-tiles (rows = positions, column = this lane's query)
@@ -275,8 +279,12 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
     __syncthreads();
-    typedef uint32_t fl_u32x2 __attribute__((ext_vector_type(2)));
-    typedef __attribute__((address_space(3))) const volatile fl_u32x2* fl_lds_cv64;     // volatile drops the inferred address space: say it
+    // V^T fragments: lane l gets dim 32 i + (l & 31) of rows 16 s + 8 u + 4 h .. + 3.  A 16-lane group's transposing read covers 4 rows x 16
+    // dims: lane l15 of it supplies the address of row l15 >> 2, dims 4 (l15 & 3) .. + 3.  The swizzle of such a row depends on l15 >> 2, h and
+    // u only, so the addresses of (i, u) serve every s with an immediate offset of 16 rows.
+    typedef short fl_v4s __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) fl_v4s* fl_lds_v4;
+    const int tr = (lane & 15) >> 2, tc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), t8 = 8 * (lane & 1);
     for (int t = t0; t < t1; ++t) {
         const int buf = t & 1, kv0 = t * FL_BKV;
         if (t + 1 < t1) { load_k(t + 1); load_v(t + 1); }
@@ -302,7 +310,7 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
 #pragma unroll
             for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(fmaxf(sc0[r], sc1[r]), fmaxf(sc0[r + 1], sc1[r + 1])), mx);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            if constexpr (WIN) mx *= scale_log2e;                        // -inf stays -inf (scale > 0)
+            mx *= scale_log2e;                                           // -inf stays -inf (scale > 0)
             // Deferred rescale: the reference point of a row only moves when its maximum grew by more than 6 (log2
             // domain), so probabilities stay <= 64 (exact in fp32 sums, fine in 16-bit P) and on most tiles - for the whole
             // wave - alpha is exactly 1 and the 64-multiply rescale of O is skipped.
@@ -313,13 +321,8 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
             float ls = 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                if constexpr (WIN) {
-                    sc0[r] = __builtin_amdgcn_exp2f(fmaf(sc0[r], scale_log2e, -m_use));
-                    sc1[r] = __builtin_amdgcn_exp2f(fmaf(sc1[r], scale_log2e, -m_use));
-                } else {
-                    sc0[r] = __builtin_amdgcn_exp2f(sc0[r] - m_use);
-                    sc1[r] = __builtin_amdgcn_exp2f(sc1[r] - m_use);
-                }
+                sc0[r] = __builtin_amdgcn_exp2f(fmaf(sc0[r], scale_log2e, -m_use));
+                sc1[r] = __builtin_amdgcn_exp2f(fmaf(sc1[r], scale_log2e, -m_use));
                 ls += sc0[r] + sc1[r];
             }
             l_run = l_run * alpha + ls;
@@ -331,14 +334,12 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
                     for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
             }
             // ---- O^T += V^T . P^T : 4 k-steps of 16 kv ----
-            // V^T fragment addresses: row d = 32 i + ql, 8-byte chunk c8 = 4 s + 2 u + h at d * 128 + ((c8 ^ ((d >> 1) & 15)) << 3).
-            // 32 i is a multiple of 32, so the swizzle term depends on the lane and on c8 only: ONE address register per
-            // (s, u) for this tile's buffer and the tile row i as the instruction's immediate offset (4096 i).  The reads are
-            // VOLATILE: left ordinary, hipcc pairs those of tiles i and i + 2 into ds_read2st64_b64, which is served 16 lanes
-            // at a time on a 32-bank modulus (2-way conflicts, half the rate); the first version kept them apart by laundering
-            // every address through an empty asm - a v_mov + v_add per read, 64 vector instructions per tile.
-            const char* vrow = Vs(buf) + ql * 128;
-            const int vsw = (ql >> 1) & 15;
+            const char* vb = Vs(buf);
+            const char* va[DT][2];
+#pragma unroll
+            for (int i = 0; i < DT; ++i)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) va[i][u] = vb + fl_v_off<D>(8 * u + 4 * h + tr, 4 * i + tc) + t8;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 uint4 pb;
@@ -351,9 +352,8 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
                 }
 #pragma unroll
                 for (int i = 0; i < DT; ++i) {
-                    // each 8-byte read stays a ds_read_b64 (two 32-lane halves, 64-bank modulus: the layout is conflict-free for it)
-                    const fl_u32x2 lo = *(fl_lds_cv64)(vrow + (((4 * s + h) ^ vsw) << 3) + i * 4096);
-                    const fl_u32x2 hi = *(fl_lds_cv64)(vrow + (((4 * s + 2 + h) ^ vsw) << 3) + i * 4096);
+                    const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][0] + s * 32 * D)));
+                    const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][1] + s * 32 * D)));
                     o[i] = mfma32<T>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb, o[i]);
                 }
             }
@@ -381,20 +381,21 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
             amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
             const float sc = amax > 0.f ? amax / 448.0f : 1.0f;
             if (qrow < q_len) {
-                uint8_t* qrow8 = sp.q8 + ((size_t)qrow * hq + head) * D;
+                uint8_t* qrow8 = sp.q8 + ((size_t)(row0 + qrow) * hq + head) * D;
 #pragma unroll
                 for (int i = 0; i < DT; ++i)
 #pragma unroll
                     for (int g = 0; g < 4; ++g)
                         *reinterpret_cast<uint32_t*>(qrow8 + i * 32 + 8 * g + 4 * h) =
                             pack_fp8x4(o[i][4 * g] / sc, o[i][4 * g + 1] / sc, o[i][4 * g + 2] / sc, o[i][4 * g + 3] / sc);
-                if (h == 0) sp.q8s[(size_t)qrow * hq + head] = sc;
+                if (h == 0) sp.q8s[(size_t)(row0 + qrow) * hq + head] = sc;
             }
             return;
         }
     }
     if (qrow < q_len) {
-        T* orow = sp.nsplit > 1 ? reinterpret_cast<T*>(sp.o) + (((size_t)split * q_len + qrow) * hq + head) * D
+        float* wrow = sp.nsplit > 1 && sp.wide ? reinterpret_cast<float*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D : nullptr;
+        T* orow = sp.nsplit > 1 ? reinterpret_cast<T*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D
                                 : out + (size_t)head * sd.oh + (size_t)qrow * sd.os;
 #pragma unroll
         for (int i = 0; i < DT; ++i)
@@ -402,10 +403,11 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
             for (int g = 0; g < 4; ++g) {
                 float y[4] = {o[i][4 * g] * inv, o[i][4 * g + 1] * inv, o[i][4 * g + 2] * inv, o[i][4 * g + 3] * inv};
                 if constexpr (WIN) { if (win.gate.gc && sp.nsplit == 1) flash_gate_cols<T, 4>(win, qrow, head, i * 32 + 8 * g + 4 * h, y); }
-                *reinterpret_cast<uint2*>(orow + i * 32 + 8 * g + 4 * h) = make_uint2(pack16x2<T>(y[0], y[1]), pack16x2<T>(y[2], y[3]));
+                if (wrow) *reinterpret_cast<float4*>(wrow + i * 32 + 8 * g + 4 * h) = make_float4(y[0], y[1], y[2], y[3]);
+                else *reinterpret_cast<uint2*>(orow + i * 32 + 8 * g + 4 * h) = make_uint2(pack16x2<T>(y[0], y[1]), pack16x2<T>(y[2], y[3]));
             }
         if (sp.nsplit > 1 && h == 0) {
-            float* ml = sp.ml + (((size_t)split * hq + head) * q_len + qrow) * 2;
+            float* ml = sp.ml + (((size_t)split * hq + head) * rows + row0 + qrow) * 2;
             ml[0] = m_run;
             ml[1] = l_tot;
         }
@@ -413,8 +415,8 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
 }
 
 // out[q][head][:] = sum_s w_s o_s / sum_s w_s,  w_s = l_s 2^(m_s - max m): one thread per 8 output elements
-template <class T, int D>
-__global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const T* po, T* out, int hq, int q_len, int nsplit, long long oh, long long os,
+template <class T, class P, int D>   // P: type of the partial rows
+__global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const P* po, T* out, int hq, int q_len, int nsplit, long long oh, long long os,
                                                           uint8_t* q8 = nullptr, float* q8s = nullptr, FlashWindow win = FlashWindow{}) {
     constexpr int CPR = D / 8;
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -422,19 +424,37 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
     if (gid >= nrow * CPR) return;          // nrow * CPR is a multiple of 16: the 16 lanes of a (row, head) stay together
     const size_t rowi = gid / CPR;
     const int c = (int)(gid % CPR), qrow = (int)(rowi / hq), head = (int)(rowi % hq);
+    // (nsplit is a power of two up to 16: four runs' records and rows are requested at a time)
     float mstar = -INFINITY;
     for (int s2 = 0; s2 < nsplit; ++s2) mstar = fmaxf(mstar, ml[(((size_t)s2 * hq + head) * q_len + qrow) * 2]);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f;
-    for (int s2 = 0; s2 < nsplit; ++s2) {
-        const float* r = ml + (((size_t)s2 * hq + head) * q_len + qrow) * 2;
-        const float w = (r[1] > 0.f) ? r[1] * __builtin_amdgcn_exp2f(r[0] - mstar) : 0.f;
-        if (w > 0.f) {
-            Vec<T> v;
-            v.load(po + (((size_t)s2 * q_len + qrow) * hq + head) * D + c * 8);
-            float f[8];
-            v.to_float(f);
+    for (int s0 = 0; s0 < nsplit; s0 += 4) {
+        uint4 v[4][sizeof(P) / 2];
+        float2 r[4];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = fmaf(w, f[j], acc[j]);
+        for (int u = 0; u < 4; ++u) {
+            const int s2 = min(s0 + u, nsplit - 1);
+            r[u] = *reinterpret_cast<const float2*>(ml + (((size_t)s2 * hq + head) * q_len + qrow) * 2);
+#pragma unroll
+            for (int x = 0; x < (int)sizeof(P) / 2; ++x) v[u][x] = *reinterpret_cast<const uint4*>(po + (((size_t)s2 * q_len + qrow) * hq + head) * D + c * 8 + 4 * x);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float w = s0 + u < nsplit && r[u].y > 0.f ? r[u].y * __builtin_amdgcn_exp2f(r[u].x - mstar) : 0.f;
+            float f[8];
+            if constexpr (sizeof(P) == 4) {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    f[4 * x] = __uint_as_float(v[u][x].x); f[4 * x + 1] = __uint_as_float(v[u][x].y);
+                    f[4 * x + 2] = __uint_as_float(v[u][x].z); f[4 * x + 3] = __uint_as_float(v[u][x].w);
+                }
+            } else {
+                Vec<P> t;
+                t.raw = v[u][0];
+                t.to_float(f);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = w > 0.f ? fmaf(w, f[j], acc[j]) : acc[j];
             den += w;
         }
     }
@@ -463,81 +483,61 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
     v.store(out + (size_t)head * oh + (size_t)qrow * os + c * 8);
 }
 
-// V [Hkv][kv][D] (element strides kh, ks) -> V^T [Hkv][D][kv_pad], zero beyond kv_len.  One workgroup per
-// (64-position tile, kv head); the tile goes through LDS so both sides move 16-byte chunks.
-template <class T, int D>
-__global__ __launch_bounds__(256) void transpose_v_kernel(const T* v, T* vt, int kv_len, int kv_pad, long long kh, long long ks) {
-    __shared__ uint16_t tile[64][D + 2];
-    const int kv0 = blockIdx.x * 64, head = blockIdx.y;
-    const T* vh = v + (size_t)head * kh;
-    constexpr int NC = D / 8;
-    for (int c = threadIdx.x; c < 64 * NC; c += 256) {
-        const int r = c / NC, kc = c % NC;
-        uint4 x = make_uint4(0, 0, 0, 0);
-        if (kv0 + r < kv_len) x = *reinterpret_cast<const uint4*>(vh + (size_t)(kv0 + r) * ks + kc * 8);
-        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tile[r][kc * 8 + 2 * j] = (uint16_t)(w[j] & 0xFFFFu);
-            tile[r][kc * 8 + 2 * j + 1] = (uint16_t)(w[j] >> 16);
-        }
-    }
-    __syncthreads();
-    T* oh = vt + (size_t)head * D * kv_pad;
-    for (int c = threadIdx.x; c < D * 8; c += 256) {
-        const int d = c >> 3, kc = c & 7;
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = (uint32_t)tile[kc * 8 + 2 * j][d] | ((uint32_t)tile[kc * 8 + 2 * j + 1][d] << 16);
-        *reinterpret_cast<uint4*>(oh + (size_t)d * kv_pad + kv0 + kc * 8) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
+static int flash_cus() {
+    int dev = 0, cus = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
+// KV runs per query tile: enough workgroups for two per CU (the kernel's occupancy), at least four KV tiles to a run
+static int flash_runs(long long wgs, int span, int most) {
+    const int cus = flash_cus();
+    int n = 1;
+    while (n < most && wgs * n < 2LL * cus && ceil_div(span, FL_BKV) >= 4 * (n * 2)) n *= 2;
+    return n;
+}
+
+// q_len: query rows of all sequences where `many` lists several (kv_len: the longest context among them)
 template <class T, int D, bool WIN = false, bool BIAS = false>
 static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int hq, int hkv, int q_len, int kv_len, float scale,
-                               const FlashStrides& sd, hipStream_t st, uint8_t* q8 = nullptr, float* q8s = nullptr, const FlashWindow& win = FlashWindow{}) {
-    const int kv_pad = ceil_div(kv_len, 64) * 64;
-    const int nqt = ceil_div(q_len, FL_BQ);
-    // KV runs per query tile: enough workgroups for two per CU (the kernel's occupancy), never more runs than the
-    // shortest useful run of two KV tiles allows for the heaviest query tile
-    int nsplit = 1;
-    {
-        int dev = 0, cus = 256;
-        hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) cus = prop.multiProcessorCount;
-        const long long wgs = (long long)nqt * hq;
-        const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-        while (nsplit < 4 && wgs * nsplit < 2LL * cus && ceil_div(span, FL_BKV) >= 4 * (nsplit * 2)) nsplit *= 2;
+                               const FlashStrides& sd, hipStream_t st, uint8_t* q8 = nullptr, float* q8s = nullptr, const FlashWindow& win = FlashWindow{},
+                               const FlashMany& many = FlashMany{}) {
+    const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
+    const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
+    int nsplit = flash_runs((long long)tiles * hq, span, WIN ? 4 : 16);
+    const bool wide = many.items || q_len <= 128;
+    if (nsplit > 1 && q_len <= 128) {      // up to 128 rows need no scratch memory to be captured
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) nsplit = 1;
     }
-    const size_t vt_bytes = (size_t)hkv * D * kv_pad * sizeof(T);
-    const size_t po_bytes = nsplit > 1 ? (size_t)nsplit * q_len * hq * D * sizeof(T) : 0;
-    const size_t ml_bytes = nsplit > 1 ? (size_t)nsplit * hq * q_len * 2 * sizeof(float) : 0;
+    FlashSplit sp{nsplit, nullptr, nullptr, wide, q8, q8s};
     void* ws = nullptr;
-    if (pgk_status r = pgk_malloc(&ws, vt_bytes + po_bytes + ml_bytes + 512)) return r;
-    char* base = (char*)ws;
-    T* vt = (T*)base;
-    FlashSplit sp{nsplit, nullptr, nullptr, q8, q8s};
     if (nsplit > 1) {
-        sp.o = base + ((vt_bytes + 255) & ~(size_t)255);
-        sp.ml = (float*)((char*)sp.o + ((po_bytes + 255) & ~(size_t)255));
+        const size_t po_bytes = (size_t)nsplit * q_len * hq * D * (wide ? 4 : sizeof(T)), ml_bytes = (size_t)nsplit * hq * q_len * 2 * sizeof(float);
+        if (pgk_malloc(&ws, po_bytes + ml_bytes + 256) == PGK_OK) {
+            sp.o = ws;
+            sp.ml = (float*)((char*)ws + ((po_bytes + 255) & ~(size_t)255));
+        } else {
+            nsplit = sp.nsplit = 1;        // slower, and right
+        }
     }
-    transpose_v_kernel<T, D><<<dim3(kv_pad / 64, hkv), 256, 0, st>>>(v, vt, kv_len, kv_pad, sd.kh, sd.ks);
-    constexpr size_t LDS = 2 * (size_t)(64 * D * 2) + 2 * (size_t)(D * 128);
+    constexpr size_t LDS = 4 * (size_t)(64 * D * 2);
     static bool attr_done = false;
     if (LDS > 48 * 1024 && !attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<T, D, WIN, BIAS>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
         attr_done = true;
     }
-    flash_fwd_kernel<T, D, WIN, BIAS><<<nqt * hq * nsplit, FL_THREADS, LDS, st>>>(q, k, (const T*)vt, out, hq, hkv, q_len, kv_len, kv_pad,
-                                                                      scale * 1.4426950408889634f, sd, sp, win);
+    flash_fwd_kernel<T, D, WIN, BIAS><<<tiles * hq * nsplit, FL_THREADS, LDS, st>>>(q, k, v, out, hq, hkv, q_len, kv_len,
+                                                                      scale * 1.4426950408889634f, sd, sp, win, many);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && nsplit > 1) {
         const size_t work = (size_t)q_len * hq * (D / 8);
-        flash_merge_kernel<T, D><<<(unsigned)((work + 255) / 256), 256, 0, st>>>(sp.ml, (const T*)sp.o, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win);
+        const unsigned grid = (unsigned)((work + 255) / 256);
+        if (wide) flash_merge_kernel<T, float, D><<<grid, 256, 0, st>>>(sp.ml, (const float*)sp.o, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win);
+        else flash_merge_kernel<T, T, D><<<grid, 256, 0, st>>>(sp.ml, (const T*)sp.o, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win);
         e = hipGetLastError();
     }
-    pgk_free(ws);   // stream-ordered reuse: later work on this stream runs after the kernels above
+    if (ws) pgk_free(ws);   // stream-ordered reuse: later work on this stream runs after the kernels above
     PGK_CHECK_HIP(e);
     return PGK_OK;
 }
@@ -576,6 +576,22 @@ pgk_status flash_prefill_q8(const void* q, const void* k, const void* v, uint8_t
     PGK_REQUIRE(q8 && q8s && q_len > 128, "flash_prefill_q8: needs output buffers and q_len > 128 (got %d)", q_len);
     const FlashStrides sd{qh, qs, kh, ks, 0, 0};
     return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, nullptr, hq, hkv, q_len, kv_len, scale, sd, st, q8, q8s);
+}
+
+int flash_items(FlashItem* items, const int* lens, const int* starts, const int* slots, int n) {
+    int at = 0;
+    for (int i = 0, row0 = 0; i < n; row0 += lens[i++])
+        for (int t = ceil_div(lens[i], FL_BQ) - 1; t >= 0; --t) items[at++] = FlashItem{row0, lens[i], starts[i] + lens[i], slots[i] << 16 | t};
+    auto keys = [](const FlashItem& a) { return a.kv_len - a.q_len + std::min((a.slot_tile & 0xFFFF) * FL_BQ + FL_BQ, a.q_len); };
+    std::stable_sort(items, items + at, [&](const FlashItem& a, const FlashItem& b) { return keys(a) > keys(b); });
+    return at;
+}
+pgk_status flash_many(const void* q, const void* k, const void* v, void* out, const FlashItem* items, int n_items, int rows, int longest, long long slot_stride, int hq,
+                      int hkv, int d, float scale, long long qh, long long qs, long long kh, long long ks, long long oh, long long os, hipStream_t st) {
+    const FlashStrides sd{qh, qs, kh, ks, oh, os};
+    const FlashMany many{items, n_items, rows, slot_stride};
+    if (d == 128) return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, rows, longest, scale, sd, st, nullptr, nullptr, FlashWindow{}, many);
+    return flash_launch<bf16, 64>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, rows, longest, scale, sd, st, nullptr, nullptr, FlashWindow{}, many);
 }
 
 }  // namespace pgk

@@ -675,6 +675,36 @@ def test_sdpa_flash_prefill(dt, cfg):
     assert np.abs(o - ref).max() < 5e-2  # reference's FA2-vs-SDPA bar (benchmarks/test_flash_attention.py:169)
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(8, 2, 1, 129, 128), (4, 4, 31, 193, 64), (16, 8, 42, 142, 128), (8, 1, 77, 777, 64), (4, 2, 128, 1024, 128), (2, 2, 5, 4100, 128),
+                                 (2, 1, 384, 3585, 128), (1, 1, 129, 8200, 64)])
+def test_sdpa_few_rows_over_a_long_context(dt, cfg):
+    """Query rows that end a long context: the context is cut into up to 16 runs, some of them empty for the first rows, and merged.  What is
+    rounded to 16 bits is p, the output and above 128 rows a run's output: three independent roundings, each of relative rms u / sqrt 3 with u
+    half the spacing at 1; bar twice their sum in quadrature.  Inside a captured graph up to 128 rows take one run and no scratch memory."""
+    hq, hkv, ql, kl, d = cfg
+    rng = np.random.default_rng(ql + kl)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((hq, ql, d), (hkv, kl, d), (hkv, kl, d)))
+    qr, kr, vr = rounded(q, dt), rounded(k, dt), rounded(v, dt)
+    ref = O.sdpa_causal(qr.astype(np.float64), np.repeat(kr, hq // hkv, axis=0), np.repeat(vr, hq // hkv, axis=0))
+    qd, kd, vd = dev(q, dt), dev(k, dt), dev(v, dt)
+    bar = 2 * (2.0**-9 if dt == "bfloat16" else 2.0**-12)
+    o = host(ops.sdpa_causal(qd, kd, vd))
+    assert rel_err(o, ref) < bar, rel_err(o, ref)
+    if ql <= 128:
+        from pygpukit_amd.core.stream import CudaGraph
+
+        out = dev(np.zeros_like(q), dt)
+        g = CudaGraph()
+        g.begin_capture()
+        ops.sdpa_causal(qd, kd, vd, out=out)
+        g.end_capture()
+        for _ in range(3):
+            out.fill_zeros()
+            g.replay()
+            assert rel_err(host(out), ref) < bar
+
+
 @pytest.mark.parametrize("ql", [128, 192])   # 128: first-generation kernel, 192: transposed-score kernel
 def test_sdpa_softmax_max_jump(ql):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
