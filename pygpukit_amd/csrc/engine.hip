@@ -22,8 +22,11 @@
 //
 // Prefill runs the MFMA GEMM / flash-attention kernels on bf16 activations with an fp32 residual stream.
 
+#include <algorithm>
+
 #include "attn_core.hip.h"
 #include "engine_state.hip.h"
+#include "flash.hip.h"
 #include "gemm_epilogues.hip.h"
 #include "pkgemm.hip.h"
 #include "wide.hip.h"
@@ -701,6 +704,8 @@ __global__ void attn_merge_kernel(unsigned long long* tl, const float* part, flo
     tls.end();
 }
 
+#include "attn_stream.hip.h"
+
 // fused path: grid ((H / rows_per_block) * Hkv, 1, batch), 256 threads.  Every workgroup of a KV head recomputes
 // that head's (short-context) attention from L2-resident K/V, then multiplies it with ITS slice of W_o
 // (rows_per_block output rows x G*D columns), whose loads were issued before anything else.
@@ -1316,7 +1321,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvwrite_kernel(bf16* qkv, con
                                                                   float eps, const float* rope_cos,
                                                                   const float* rope_sin, bf16* kcache, bf16* vcache,
                                                                   int n, int hq, int hkv, int max_seq, int start_pos,
-                                                                  const float* slabs, int nslabs) {
+                                                                  const float* slabs, int nslabs, const int2* at, long long slot_stride) {   // at, slot_stride: QkvHeadArgs
     constexpr int LPR = D / 8, HALF = D / 2, VPB = 256 / LPR;
     const int nslots = hq + 2 * hkv;
     const long long vec = (long long)blockIdx.x * VPB + threadIdx.x / LPR;
@@ -1344,7 +1349,8 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvwrite_kernel(bf16* qkv, con
         raw.load(src);
     }
     raw.to_float(x);
-    const int pos = start_pos + s;
+    const int2 place = at ? at[s] : make_int2(start_pos + s, 0);
+    const int pos = place.x;
     const bool is_q = hh < hq, is_k = !is_q && hh < hq + hkv;
     if (is_q || is_k) {
         const bf16* gamma = is_q ? q_gamma : k_gamma;
@@ -1377,7 +1383,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvwrite_kernel(bf16* qkv, con
         ov.store(src);
     } else if (pos < max_seq) {
         const int kvh = is_k ? hh - hq : hh - hq - hkv;
-        bf16* dst = (is_k ? kcache : vcache) + ((size_t)kvh * max_seq + pos) * D + sub * 8;
+        bf16* dst = (is_k ? kcache : vcache) + place.y * slot_stride + ((size_t)kvh * max_seq + pos) * D + sub * 8;
         ov.store(dst);
     }
 }
@@ -1556,6 +1562,30 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         a.nsplit = 1;
         a.attn_direct = e->attnv + (size_t)b0 * c.num_heads * D;
         if (direct_bf16) a.attn_direct16 = e->attnv16 + (size_t)b0 * c.num_heads * D;
+    }
+    // Batches stream through the matrix pipe (attn_stream.hip.h), except where one workgroup per (sequence, kv head) with the whole context
+    // fits one round of the CUs.  Slices of at least 128 positions, enough of them for two workgroups per CU and none longer than 512
+    // positions: contexts of a batch differ, and its longest sequence must not be what the launch waits for.
+    const bool whole = direct && D == 128 && e->attn_mfma && (G == 1 || G == 2 || G == 4) && m * (int)c.num_kv_heads <= e->cu_count;
+    if (m >= 2 && !fused && !merged && !whole && G <= AS_HEADS) {
+        a.g_total = G;
+        int chunk = 0;
+        if (!direct) {
+            int n = 2 * e->cu_count / (c.num_kv_heads * m);
+            if (n > ceil_div(span, 128)) n = ceil_div(span, 128);
+            if (n < ceil_div(span, 512)) n = ceil_div(span, 512);
+            n = n < 1 ? 1 : (n > e->nsplit ? e->nsplit : n);
+            chunk = ceil_div(ceil_div(span, n), 128) * 128;
+            a.nsplit = ceil_div(span, chunk);
+        }
+        const dim3 g3(a.nsplit, c.num_kv_heads, m);
+        const hipError_t se = direct ? launch_k(attn_stream_kernel<D, true>, g3, dim3(256), as_lds<D>(G), st, a, chunk)
+                                     : launch_k(attn_stream_kernel<D, false>, g3, dim3(256), as_lds<D>(G), st, a, chunk);
+        PGK_CHECK_HIP(se);
+        if (!direct)
+            PGK_CHECK_HIP(launch_k(attn_merge_kernel<D>, dim3(c.num_heads, m), dim3(D), 0, st, (const float*)a.part,
+                                   e->attnv + (size_t)b0 * c.num_heads * D, (int)c.num_heads, (int)a.nsplit));
+        return PGK_OK;
     }
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
@@ -1999,12 +2029,32 @@ static pgk_status decode_step(Engine* e, int batch, hipStream_t st, int* launche
     return decode_step_impl<bf16>(e, batch, st, launches, short_ctx);
 }
 
-static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int n, int start_pos, void* all_logits,
-                                float* h_last_logits, hipStream_t st) {
+// out[i] = the rows `want` of x, as they are and in fp32
+__global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* x, const int32_t* want, bf16* out, float* out32, int H) {
+    const bf16* row = x + (size_t)want[blockIdx.x] * H;
+    for (int i = threadIdx.x; i < H; i += 256) {
+        out[(size_t)blockIdx.x * H + i] = row[i];
+        out32[(size_t)blockIdx.x * H + i] = to_f(row[i]);
+    }
+}
+
+// One pass over the weights for the prompt rows of one or several sequences (h_tokens: their rows one behind the other).  all_logits: bf16 logits
+// of every row (one sequence only).  h_want, n_want: row indices whose fp32 logits go to h_logits, the last rows of the sequences h_want_slots.
+static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slots, const int32_t* h_lens, const int32_t* h_starts, const int32_t* h_tokens, void* all_logits,
+                                     int n_want, const int32_t* h_want, const int32_t* h_want_slots, float* h_logits, hipStream_t st) {
     const auto& c = e->cfg;
-    PGK_REQUIRE(seq >= 0 && seq < c.max_batch, "pgk_engine_prefill: sequence slot %d outside [0,%d)", seq, c.max_batch);
-    PGK_REQUIRE(n >= 1 && start_pos >= 0 && start_pos + n <= c.max_seq_len, "pgk_engine_prefill: positions %d..%d outside cache of %d",
-                start_pos, start_pos + n, c.max_seq_len);
+    int n = 0, n_items = 0, longest = 0;
+    for (int i = 0; i < n_seqs; ++i) {
+        PGK_REQUIRE(h_slots[i] >= 0 && h_slots[i] < c.max_batch, "pgk_engine_prefill: sequence slot %d outside [0,%d)", h_slots[i], c.max_batch);
+        PGK_REQUIRE(h_lens[i] >= 1 && h_starts[i] >= 0 && h_starts[i] + h_lens[i] <= c.max_seq_len, "pgk_engine_prefill: positions %d..%d outside cache of %d",
+                    h_starts[i], h_starts[i] + h_lens[i], c.max_seq_len);
+        n += h_lens[i];
+        n_items += ceil_div(h_lens[i], FLASH_ITEM_ROWS);
+        longest = h_starts[i] + h_lens[i] > longest ? h_starts[i] + h_lens[i] : longest;
+    }
+    const bool many = n_seqs > 1;
+    const int seq = many ? 0 : h_slots[0], start_pos = many ? 0 : h_starts[0];
+    const long long slot_stride = (long long)c.num_kv_heads * c.max_seq_len * c.head_dim;
     // (prompts of 129..256 tokens used to run as two chunks of <= 128 through the packed-weight kernels; since the staged 128-tile
     // GEMM and the epilogue fusions the long-prompt path is faster at every such length: 144 tokens 1.94 vs 2.38 ms,
     // 256 tokens 2.27 vs 2.62)
@@ -2018,7 +2068,7 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
     // packed-weight path (ops_pkgemm.hip): bf16 layers, n <= 128; its own split counts for the N = hidden projections
     const bool pk = ws && e->packed_ok;
     const int pk_so = pk ? pkgemm_pick_splits(n, H, QD) : 1, pk_sd = pk ? pkgemm_pick_splits(n, H, I) : 1;
-    const bool pk_heads = pk && D == 128;       // QKV epilogue: per-head norm + RoPE + cache write inside the projection
+    const bool pk_heads = pk && D == 128 && !many;       // QKV epilogue: per-head norm + RoPE + cache write inside the projection
     // long prompts, bf16 weights: the N = hidden projections as split-K slabs when their 128-tiles do not cover the chip
     // (QKV / gate_up were tried too - their consumers can sum slabs - and measured slightly slower: 3.06 vs 2.99 ms at S = 512)
     // w8a16 engines, long prompts: the staged bf16 GEMMs read the DEQUANTISED fragment-major copy the engine already holds
@@ -2044,15 +2094,31 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
         if (pgk_status r = pgk_malloc(&e->pf, need)) return r;
         e->pf_bytes = need;
     }
-    if (n > e->pf_tokens_cap) {
+    // one upload: token ids | (position, slot) of every row | attention tiles | wanted rows  (the last three for several sequences)
+    const int at_off = (n + 3) & ~3, item_off = at_off + ((2 * n + 3) & ~3), want_off = item_off + 4 * n_items, meta = many ? want_off + n_want : n;
+    if (meta > e->pf_tokens_cap) {
         if (e->pf_tokens) { PGK_CHECK_HIP(hipStreamSynchronize(st)); pgk_free(e->pf_tokens); }
-        if (pgk_status r = pgk_malloc((void**)&e->pf_tokens, (size_t)n * 4)) return r;
-        e->pf_tokens_cap = n;
+        e->pf_tokens = nullptr;
+        e->pf_tokens_cap = 0;
+        if (pgk_status r = pgk_malloc((void**)&e->pf_tokens, (size_t)meta * 4)) return r;
+        e->pf_tokens_cap = meta;
     }
     for (int i = 0; i < n; ++i)
         PGK_REQUIRE(h_tokens[i] >= 0 && h_tokens[i] < c.vocab_size, "pgk_engine_prefill: token %d out of range", h_tokens[i]);
-    PGK_CHECK_HIP(hipMemcpyAsync(e->pf_tokens, h_tokens, (size_t)n * 4, hipMemcpyHostToDevice, st));
+    std::vector<int32_t> host;
+    if (many) {
+        host.resize(meta);
+        std::copy(h_tokens, h_tokens + n, host.begin());
+        int32_t* at = host.data() + at_off;
+        for (int i = 0; i < n_seqs; ++i)
+            for (int t = 0; t < h_lens[i]; ++t, at += 2) { at[0] = h_starts[i] + t; at[1] = h_slots[i]; }
+        flash_items((FlashItem*)(host.data() + item_off), h_lens, h_starts, h_slots, n_seqs);
+        std::copy(h_want, h_want + n_want, host.begin() + want_off);
+    }
+    PGK_CHECK_HIP(hipMemcpyAsync(e->pf_tokens, many ? host.data() : h_tokens, (size_t)meta * 4, hipMemcpyHostToDevice, st));
     PGK_CHECK_HIP(hipStreamSynchronize(st));  // h_tokens may be pageable: make the copy complete before returning control
+    const int2* d_at = many ? (const int2*)(e->pf_tokens + at_off) : nullptr;
+    const FlashItem* d_items = (const FlashItem*)(e->pf_tokens + item_off);
     const bool fp8 = c.weight_format != 0;
     const bool fp8act = c.weight_format == 2 && n > 128;   // fp8 x fp8 MFMA projections, activations quantised on the fly
     char* p = (char*)e->pf;
@@ -2149,6 +2215,7 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
             hd.k_gamma = c.use_qk_norm ? (const bf16*)L.k_norm : nullptr;
             hd.eps = c.norm_eps; hd.rope_cos = e->rope_cos; hd.rope_sin = e->rope_sin; hd.kcache = kc; hd.vcache = vc;
             hd.hq = c.num_heads; hd.hkv = c.num_kv_heads; hd.max_seq = c.max_seq_len; hd.start_pos = start_pos;
+            hd.at = d_at; hd.slot_stride = slot_stride;
             if (fuse_heads8) {
                 if (pgk_status r = gemm_fp8_qkv_heads_nt(q8, q8s, (const uint8_t*)L.w_qkv, (const bf16*)L.s_qkv, qkv, n, NQKV, H, hd, st)) return r;
             } else if (pgk_status r = engine_gemm_qkv_heads_nt(x, pkd ? e->packed[l].qkv : (const bf16*)L.w_qkv, qkv, n, NQKV, H, hd, st, pkd)) return r;
@@ -2163,11 +2230,11 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
             if (D == 128)
                 qknorm_rope_kvwrite_kernel<128><<<ceil_div((long long)n * nslots, 16), 256, 0, st>>>(
                     qkv, qg, kg, c.norm_eps, e->rope_cos, e->rope_sin, kc, vc, n, c.num_heads, c.num_kv_heads, c.max_seq_len, start_pos,
-                    slabs, s_qkv > 1 ? s_qkv : 0);
+                    slabs, s_qkv > 1 ? s_qkv : 0, d_at, slot_stride);
             else
                 qknorm_rope_kvwrite_kernel<64><<<ceil_div((long long)n * nslots, 32), 256, 0, st>>>(
                     qkv, qg, kg, c.norm_eps, e->rope_cos, e->rope_sin, kc, vc, n, c.num_heads, c.num_kv_heads, c.max_seq_len, start_pos,
-                    slabs, s_qkv > 1 ? s_qkv : 0);
+                    slabs, s_qkv > 1 ? s_qkv : 0, d_at, slot_stride);
             PGK_LAUNCH_CHECK();
         }
         // fp8 x fp8: a head's 128 output dims are one scale block of the o_proj operand, so the flash kernel quantises them itself
@@ -2176,9 +2243,18 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
             if (pgk_status r = flash_prefill_q8(qkv, kc, vc, q8, q8s, c.num_heads, c.num_kv_heads, n, kv_len, 1.0f / sqrtf((float)D), D, NQKV,
                                                 (long long)c.max_seq_len * D, D, st))
                 return r;
-        } else if (pgk_status r = pgk_sdpa_causal(qkv, kc, vc, attn, c.num_heads, c.num_kv_heads, n, kv_len, D, 0.f, D, NQKV,
-                                                  (int64_t)c.max_seq_len * D, D, D, QD, PGK_BF16, st))
-            return r;
+        } else if (many && sdpa_flash_enabled()) {
+            if (pgk_status r = flash_many(qkv, kc, vc, attn, d_items, n_items, n, longest, slot_stride, c.num_heads, c.num_kv_heads, D, 1.0f / sqrtf((float)D), D, NQKV,
+                                          (long long)c.max_seq_len * D, D, D, QD, st))
+                return r;
+        } else {
+            for (int i = 0, r0 = 0; i < n_seqs; r0 += h_lens[i++]) {
+                const size_t sl = many ? (size_t)h_slots[i] * slot_stride : 0;
+                if (pgk_status r = pgk_sdpa_causal(qkv + (size_t)r0 * NQKV, kc + sl, vc + sl, attn + (size_t)r0 * QD, c.num_heads, c.num_kv_heads, h_lens[i], h_starts[i] + h_lens[i],
+                                                   D, 0.f, D, NQKV, (int64_t)c.max_seq_len * D, D, D, QD, PGK_BF16, st))
+                    return r;
+            }
+        }
         // N = hidden projections of the packed path: fp32 split-K slabs summed by the next norm (or h32 += with one split)
         auto pk_accum = [&](const bf16* x_in, const bf16* wp, int K_, int splits) -> pgk_status {
             if (splits == 1) return pkgemm_nt(x_in, K_, wp, h32, H, PK_EPI_ACCUM, 1, n, H, K_, nullptr, st);
@@ -2226,34 +2302,88 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
     if (all_logits) {
         if (pgk_status r = engine_gemm_nt(x, e->lm_head, nullptr, false, all_logits, false, n, c.vocab_size, H, st)) return r;
     }
-    if (h_last_logits) {
-        // last row through the fp32-output GEMV (the decode lm_head kernel with a plain prologue)
-        float* xin = h32;  // reuse: widen the last normed row
-        bf16_rows_to_f32_kernel<<<4, 256, 0, st>>>(x + (size_t)(n - 1) * H, xin, H);
+    if (n_want == 0) return PGK_OK;
+    // Logits of the wanted rows, into the logits rows of their slots.  Several rows share passes over the vocabulary: the matrix kernels of the
+    // decode step where the model's sizes suit them (a row at a time took 50 us each on Qwen3-0.6B, 16 rows together 60 us), 8 rows a pass on
+    // ops_wide.hip otherwise, a row at a time on the fp32-output GEMV where neither fits.
+    const size_t V = c.vocab_size;
+    bool in_order = true;
+    for (int i = 1; i < n_want; ++i) in_order = in_order && h_want_slots[i] == h_want_slots[0] + i;
+    const bool mfma = n_want >= 3 && e->batched_mfma, wide = n_want > 1 && !mfma && wide_proj_ok(c.vocab_size, H, false) && wide_aligned(e);
+    if (many && in_order && (mfma || wide) && NQKV + QD + 3 * I >= H) {
+        float* lg = e->logits + h_want_slots[0] * V;
+        bf16* rows16 = qkv;                       // free by now: [n_want][H], n_want <= n
+        gather_rows_kernel<<<n_want, 256, 0, st>>>(x, e->pf_tokens + want_off, rows16, h32, H);
         PGK_LAUNCH_CHECK();
-        FusedArgs a{};
-        a.w = e->lm_head; a.N = c.vocab_size; a.K = H; a.xin = xin;
-        a.out = e->logits + (size_t)seq * c.vocab_size; a.ld_out = c.vocab_size;
-        if (pgk_status r = launch_fused<bf16, float, 1, 4, PRO_PLAIN, EPI_STORE>(a, c.vocab_size, st)) return r;
-        PGK_CHECK_HIP(hipMemcpyAsync(h_last_logits, a.out, (size_t)c.vocab_size * 4, hipMemcpyDeviceToHost, st));
-        PGK_CHECK_HIP(hipStreamSynchronize(st));
+        const int most = mfma ? e->batched_max : 8, nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
+        for (int i = 0; i < n_want; i += most) {
+            const int m = n_want - i < most ? n_want - i : most;
+            FusedArgs a{};
+            a.w = e->lm_head; a.N = c.vocab_size; a.K = H;
+            a.out = lg + i * V; a.ld_out = c.vocab_size;
+            if (mfma) {
+                a.xin = h32 + (size_t)i * H; a.xin16 = rows16 + (size_t)i * H; a.wp = e->packed_lm;
+                a.amax_val = e->amax_val; a.amax_idx = e->amax_idx;
+                if (pgk_status r = batched_proj(false, PRO_PLAIN, EPI_LOGITS, a, m, st, nblk)) return r;
+            } else {
+                a.xin = h32 + (size_t)i * H;
+                if (pgk_status r = wide_proj(false, WIDE_PLAIN, EPI_STORE, a, nullptr, m, e->cu_count, nullptr, st)) return r;
+            }
+        }
+        PGK_CHECK_HIP(hipMemcpyAsync(h_logits, lg, n_want * V * 4, hipMemcpyDeviceToHost, st));
+    } else {
+        for (int i = 0; i < n_want; ++i) {
+            float* xin = h32;  // reuse: widen the wanted normed row
+            bf16_rows_to_f32_kernel<<<4, 256, 0, st>>>(x + (size_t)h_want[i] * H, xin, H);
+            PGK_LAUNCH_CHECK();
+            FusedArgs a{};
+            a.w = e->lm_head; a.N = c.vocab_size; a.K = H; a.xin = xin;
+            a.out = e->logits + h_want_slots[i] * V; a.ld_out = c.vocab_size;
+            if (pgk_status r = launch_fused<bf16, float, 1, 4, PRO_PLAIN, EPI_STORE>(a, c.vocab_size, st)) return r;
+            PGK_CHECK_HIP(hipMemcpyAsync(h_logits + i * V, a.out, V * 4, hipMemcpyDeviceToHost, st));
+        }
     }
+    PGK_CHECK_HIP(hipStreamSynchronize(st));
     return PGK_OK;
 }
 
-// A sequence at a time: the prompt kernels below take one sequence's rows; logits only of a sequence's last row.
+static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int n, int start_pos, void* all_logits, float* h_last_logits, hipStream_t st) {
+    const int32_t last = n - 1;
+    return dense_prefill_rows(e, 1, &seq, &n, &start_pos, h_tokens, all_logits, h_last_logits ? 1 : 0, &last, &seq, h_last_logits, st);
+}
+
+// Sequences share passes over the weights, up to PREFILL_ROWS rows each (one longer prompt: a pass of its own), which is past what a pass needs to
+// be bound by its products and bounds the scratch memory; only the logits of a sequence's last row.  Sixteen prompts of 20..400 tokens on
+// Qwen3-0.6B: 31.4 -> 6.3 ms.  fp8 x fp8 engines keep a sequence to a pass: there a prompt's length decides whether its activations are rounded
+// to e4m3.
+constexpr int PREFILL_ROWS = 8192;
 static pgk_status dense_prefill_batch(Engine* e, int n_seqs, const int32_t* h_slots, const int32_t* h_lens, const int32_t* h_starts, const int32_t* h_tokens,
                                       int n_want, const int32_t* h_want, float* h_logits, hipStream_t st) {
     int row0 = 0, w = 0;
-    for (int i = 0; i < n_seqs; ++i) {
+    for (int i = 0; i < n_seqs; row0 += h_lens[i++]) {
         const int last = row0 + h_lens[i] - 1;
         PGK_REQUIRE(w >= n_want || h_want[w] >= last, "pgk_engine_prefill_batch: this model gives the logits of a sequence's last row only");
-        float* out = (w < n_want && h_want[w] == last) ? h_logits + (size_t)w * e->cfg.vocab_size : nullptr;
-        if (pgk_status r = dense_prefill(e, h_slots[i], h_tokens + row0, h_lens[i], h_starts[i], nullptr, out, st)) return r;
-        if (out) ++w;
-        row0 += h_lens[i];
+        if (w < n_want && h_want[w] == last) ++w;
     }
     PGK_REQUIRE(w == n_want, "pgk_engine_prefill_batch: wanted rows must be ascending last rows");
+    std::vector<int32_t> want, slots;
+    row0 = w = 0;
+    for (int i0 = 0; i0 < n_seqs;) {
+        int i = i0, rows = 0;
+        want.clear();
+        slots.clear();
+        do {
+            rows += h_lens[i];
+            if (w + (int)want.size() < n_want && h_want[w + want.size()] == row0 + rows - 1) { want.push_back(rows - 1); slots.push_back(h_slots[i]); }
+            ++i;
+        } while (i < n_seqs && e->cfg.weight_format != 2 && rows + h_lens[i] <= PREFILL_ROWS && e->cfg.max_batch <= FLASH_MOST_SLOTS);
+        if (pgk_status r = dense_prefill_rows(e, i - i0, h_slots + i0, h_lens + i0, h_starts + i0, h_tokens + row0, nullptr, (int)want.size(), want.data(), slots.data(),
+                                              h_logits + (size_t)w * e->cfg.vocab_size, st))
+            return r;
+        w += (int)want.size();
+        row0 += rows;
+        i0 = i;
+    }
     return PGK_OK;
 }
 

@@ -91,6 +91,9 @@ static pgk_status batched_proj_t(int pro, int epi, const FusedArgs& a, int M, hi
             case EPI_STORE: return launch_batched<WT, PRO_PLAIN, EPI_STORE>(a, M, st);
             case EPI_RESID: return launch_batched<WT, PRO_PLAIN, EPI_RESID>(a, M, st);
             case EPI_SWIGLU: return launch_batched<WT, PRO_PLAIN, EPI_SWIGLU>(a, M, st);
+            case EPI_LOGITS:                       // rows a prompt left, already normalised
+                if constexpr (!std::is_same<WT, fp8e4m3>::value) return launch_batched<WT, PRO_PLAIN, EPI_LOGITS>(a, M, st, nblk);
+                break;
         }
     }
     return set_error(PGK_ERR_INVALID, "batched_proj: prologue %d with epilogue %d is not instantiated", pro, epi);

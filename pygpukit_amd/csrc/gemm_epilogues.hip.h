@@ -13,6 +13,10 @@ struct QkvHeadArgs {
     const float *rope_cos, *rope_sin;     // [max_seq][64]
     bf16 *kcache, *vcache;                // this layer's, this sequence's: [Hkv][max_seq][128]
     int hq, hkv, max_seq, start_pos;
+    // rows of several sequences: (position, slot) of each; kcache / vcache are then slot 0's and slot_stride elements apart.  Null: position
+    // start_pos + row
+    const int2* at;
+    long long slot_stride;
 };
 struct ActArgs { float pos, neg; bool gelu; };     // pgk_device.hip.h: xielu's factors, or gelu_erf
 
@@ -20,7 +24,8 @@ struct ActArgs { float pos, neg; bool gelu; };     // pgk_device.hip.h: xielu's 
 // the arithmetic of qknorm_rope_kvwrite_kernel, operation for operation, then the store.  All 16 lanes must be active.
 __device__ __forceinline__ void qkv_head_finish(float (&x)[8], int sub, int slot, int grow, int M, const QkvHeadArgs& hd, bf16* qkv, int ldq) {
     const bool is_q = slot < hd.hq, is_k = !is_q && slot < hd.hq + hd.hkv;
-    const int pos = hd.start_pos + grow;
+    const int2 place = hd.at ? hd.at[min(grow, M - 1)] : make_int2(hd.start_pos + grow, 0);
+    const int pos = place.x;
     if (is_q || is_k) {
         const bf16* gamma = is_q ? hd.q_gamma : hd.k_gamma;
         if (gamma) {
@@ -52,7 +57,7 @@ __device__ __forceinline__ void qkv_head_finish(float (&x)[8], int sub, int slot
         ov.store(qkv + (size_t)grow * ldq + slot * 128 + sub * 8);
     } else if (pos < hd.max_seq) {
         const int kvh = is_k ? slot - hd.hq : slot - hd.hq - hd.hkv;
-        ov.store((is_k ? hd.kcache : hd.vcache) + ((size_t)kvh * hd.max_seq + pos) * 128 + sub * 8);
+        ov.store((is_k ? hd.kcache : hd.vcache) + place.y * hd.slot_stride + ((size_t)kvh * hd.max_seq + pos) * 128 + sub * 8);
     }
 }
 

@@ -365,6 +365,7 @@ pgk_status launch_wide_e(int src, int epi, const FusedArgs& a, bf16* pieces, int
     if (src == WIDE_PLAIN && epi == EPI_RESID) return launch_wide_k<WT, WIDE_PLAIN, EPI_RESID>(a, pieces, M, cu_count, n_blk, st);
     if (src == WIDE_PIECES && epi == EPI_RESID) return launch_wide_k<WT, WIDE_PIECES, EPI_RESID>(a, pieces, M, cu_count, n_blk, st);
     if constexpr (std::is_same<WT, bf16>::value) {
+        if (src == WIDE_PLAIN && epi == EPI_STORE) return launch_wide_k<WT, WIDE_PLAIN, EPI_STORE>(a, pieces, M, cu_count, n_blk, st);
         if (src == WIDE_NORM && epi == EPI_LOGITS) return launch_wide_k<WT, WIDE_NORM, EPI_LOGITS>(a, pieces, M, cu_count, n_blk, st);
     }
     return set_error(PGK_ERR_INVALID, "wide_proj: source %d with epilogue %d", src, epi);
