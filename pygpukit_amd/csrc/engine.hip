@@ -704,8 +704,6 @@ __global__ void attn_merge_kernel(unsigned long long* tl, const float* part, flo
     tls.end();
 }
 
-#include "attn_stream.hip.h"
-
 // fused path: grid ((H / rows_per_block) * Hkv, 1, batch), 256 threads.  Every workgroup of a KV head recomputes
 // that head's (short-context) attention from L2-resident K/V, then multiplies it with ITS slice of W_o
 // (rows_per_block output rows x G*D columns), whose loads were issued before anything else.
@@ -1562,30 +1560,6 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         a.nsplit = 1;
         a.attn_direct = e->attnv + (size_t)b0 * c.num_heads * D;
         if (direct_bf16) a.attn_direct16 = e->attnv16 + (size_t)b0 * c.num_heads * D;
-    }
-    // Batches stream through the matrix pipe (attn_stream.hip.h), except where one workgroup per (sequence, kv head) with the whole context
-    // fits one round of the CUs.  Slices of at least 128 positions, enough of them for two workgroups per CU and none longer than 512
-    // positions: contexts of a batch differ, and its longest sequence must not be what the launch waits for.
-    const bool whole = direct && D == 128 && e->attn_mfma && (G == 1 || G == 2 || G == 4) && m * (int)c.num_kv_heads <= e->cu_count;
-    if (m >= 2 && !fused && !merged && !whole && G <= AS_HEADS) {
-        a.g_total = G;
-        int chunk = 0;
-        if (!direct) {
-            int n = 2 * e->cu_count / (c.num_kv_heads * m);
-            if (n > ceil_div(span, 128)) n = ceil_div(span, 128);
-            if (n < ceil_div(span, 512)) n = ceil_div(span, 512);
-            n = n < 1 ? 1 : (n > e->nsplit ? e->nsplit : n);
-            chunk = ceil_div(ceil_div(span, n), 128) * 128;
-            a.nsplit = ceil_div(span, chunk);
-        }
-        const dim3 g3(a.nsplit, c.num_kv_heads, m);
-        const hipError_t se = direct ? launch_k(attn_stream_kernel<D, true>, g3, dim3(256), as_lds<D>(G), st, a, chunk)
-                                     : launch_k(attn_stream_kernel<D, false>, g3, dim3(256), as_lds<D>(G), st, a, chunk);
-        PGK_CHECK_HIP(se);
-        if (!direct)
-            PGK_CHECK_HIP(launch_k(attn_merge_kernel<D>, dim3(c.num_heads, m), dim3(D), 0, st, (const float*)a.part,
-                                   e->attnv + (size_t)b0 * c.num_heads * D, (int)c.num_heads, (int)a.nsplit));
-        return PGK_OK;
     }
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
