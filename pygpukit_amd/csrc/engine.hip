@@ -672,7 +672,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(unsigned long long* tl
 // owns record s's (m, l): one load each, a wave max and a wave sum give the weights; then every thread sums its
 // element over the records with independent loads.
 template <int D>
-__global__ void attn_merge_kernel(unsigned long long* tl, const float* part, float* attn, int hq, int nsplit) {
+__global__ void attn_merge_kernel(unsigned long long* tl, const float* part, float* attn, bf16* attn16, int hq, int nsplit) {   // attn16: bf16 rows instead of attn
     const TLStamp tls(tl);
     __shared__ float w_s[64];
     __shared__ float inv_l;
@@ -700,9 +700,13 @@ __global__ void attn_merge_kernel(unsigned long long* tl, const float* part, flo
         for (int u = 0; u < 8; ++u) o = fmaf(w_s[s + u], v[u], o);
     }
     for (; s < nsplit; ++s) o = fmaf(w_s[s], recs[(size_t)s * (D + 2) + 2 + d], o);
-    attn[((size_t)b * hq + h) * D + d] = o * inv_l;
+    const size_t at = ((size_t)b * hq + h) * D + d;
+    if (attn16) attn16[at] = from_f<bf16>(o * inv_l);
+    else attn[at] = o * inv_l;
     tls.end();
 }
+
+#include "attn_stream.hip.h"
 
 // fused path: grid ((H / rows_per_block) * Hkv, 1, batch), 256 threads.  Every workgroup of a KV head recomputes
 // that head's (short-context) attention from L2-resident K/V, then multiplies it with ITS slice of W_o
@@ -1499,9 +1503,10 @@ static pgk_status launch_fused_auto(const FusedArgs& a, int n_out, hipStream_t s
     }
 }
 
-// attention launches per layer for a GQA group of G query heads per kv head (chunks of 4 / 2 / 1 beyond the instantiated sizes)
-static int gqa_chunks(int G) {
-    if (G == 1 || G == 2 || G == 4) return 1;
+// attention launches per layer of m sequences for a GQA group of G query heads per kv head: one, or for a single sequence chunks of 4 / 2 / 1 heads
+// beyond the instantiated sizes (attn_stream_kernel takes any group up to AS_HEADS)
+static int gqa_chunks(int G, int m) {
+    if (G == 1 || G == 2 || G == 4 || (m >= 2 && G <= AS_HEADS)) return 1;
     int n = 0;
     for (int off = 0; off < G; ++n) off += (G - off >= 4) ? 4 : ((G - off >= 2) ? 2 : 1);
     return n;
@@ -1556,10 +1561,41 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
     a.nsplit = ceil_div(span, decode_chunk_len(span, ns, 4 * (64 / (D / 8))));
     a.w_o = (const bf16*)L.w_o; a.w_o_scale = (const bf16*)L.s_o; a.H = c.hidden_size; a.rows_per_block = e->oproj_rows;
     a.opart = e->opart ? e->opart + (size_t)b0 * c.num_kv_heads * c.hidden_size : nullptr;
+    // split-KV records -> attention rows, in the type that `direct` would leave
+    auto merge = [&]() {
+        return launch_k(attn_merge_kernel<D>, dim3(c.num_heads, m), dim3(D), 0, st, (const float*)a.part, e->attnv + (size_t)b0 * c.num_heads * D,
+                        direct_bf16 ? e->attnv16 + (size_t)b0 * c.num_heads * D : (bf16*)nullptr, (int)c.num_heads, (int)a.nsplit);
+    };
     if (direct) {
         a.nsplit = 1;
         a.attn_direct = e->attnv + (size_t)b0 * c.num_heads * D;
         if (direct_bf16) a.attn_direct16 = e->attnv16 + (size_t)b0 * c.num_heads * D;
+    }
+    // Batches stream through the matrix pipe (attn_stream.hip.h), except where one workgroup per (sequence, kv head) with the whole context
+    // fits one round of the CUs, and where one or two query heads share a kv head and slices of 128 positions fit two: there the first bytes'
+    // latency counts, and attn_decode_kernel requests them before it knows the position (Qwen3-0.6B, us per step, that kernel and this one:
+    // 4 sequences of 1500 positions 937 and 984, 8 of 600 828 and 855; 12 of 1000 1301 and 1250; Llama-3-8B shape, four query heads, 6 of 1100
+    // 3434 and 3338).  Slices of at least 128 positions, enough for two workgroups per CU and none longer than 512: contexts of a batch differ,
+    // and its longest sequence must not be what the launch waits for.
+    const bool whole = direct && (G == 1 || G == 2 || G == 4) && m * (int)c.num_kv_heads <= e->cu_count;
+    const bool latency = !direct && G <= 2 && (long long)m * c.num_kv_heads * ceil_div(span, 128) <= 2 * e->cu_count;
+    if (m >= 2 && !fused && !merged && !whole && !latency && G <= AS_HEADS) {
+        a.g_total = G;
+        int chunk = 0;
+        if (!direct) {
+            int n = 2 * e->cu_count / (c.num_kv_heads * m);
+            n = n > ceil_div(span, 128) ? ceil_div(span, 128) : n;
+            n = n < ceil_div(span, 512) ? ceil_div(span, 512) : n;
+            n = n < 1 ? 1 : (n > e->nsplit ? e->nsplit : n);
+            chunk = ceil_div(ceil_div(span, n), 128) * 128;
+            a.nsplit = ceil_div(span, chunk);
+        }
+        const dim3 g3(c.num_kv_heads, a.nsplit, m);
+        const hipError_t se = direct ? launch_k(attn_stream_kernel<D, true>, g3, dim3(256), as_lds<D>(G), st, a, chunk)
+                                     : launch_k(attn_stream_kernel<D, false>, g3, dim3(256), as_lds<D>(G), st, a, chunk);
+        PGK_CHECK_HIP(se);
+        if (!direct) PGK_CHECK_HIP(merge());
+        return PGK_OK;
     }
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
@@ -1610,8 +1646,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
 #undef PGK_MO
         PGK_CHECK_HIP(he);
     } else if (!fused && !direct) {
-        PGK_CHECK_HIP(launch_k(attn_merge_kernel<D>, dim3(c.num_heads, m), dim3(D), 0, st, (const float*)a.part,
-                               e->attnv + (size_t)b0 * c.num_heads * D, (int)c.num_heads, (int)a.nsplit));
+        PGK_CHECK_HIP(merge());
     }
     return PGK_OK;
 }
@@ -1658,7 +1693,7 @@ static pgk_status decode_chunk(Engine* e, int b0, bool last, hipStream_t st, int
             a.xin = e->attnv + (size_t)b0 * QD;
             a.res = h; a.out = h; a.ld_out = H;
             if (pgk_status r = launch_fused_auto<WT, XT, M, PRO_PLAIN, EPI_RESID>(a, H, st)) return r;
-            *launches += (direct ? 1 : 2) + gqa_chunks(c.num_heads / c.num_kv_heads) - 1;   // o_proj (+ the merge kernel unless attention normalised in place)
+            *launches += (direct ? 1 : 2) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;   // o_proj (+ the merge kernel unless attention normalised in place)
         }
         // 4. act = silu(Wg x) * (Wu x), x = rmsnorm(h [+ sum of o_proj partials])
         mark(KC_GATEUP);
@@ -1747,13 +1782,8 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
         a = FusedArgs{};
         a.w = L.w_o; a.wscale = (const bf16*)L.s_o; a.N = H; a.K = QD;
         a.xin = e->attnv + (size_t)b0 * QD;
-        if (direct) a.xin16 = e->attnv16 + (size_t)b0 * QD;   // the whole-context attention kernel wrote bf16
+        a.xin16 = e->attnv16 + (size_t)b0 * QD;               // attention left bf16 rows
         a.res = h; a.out = h; a.ld_out = H;
-        if (tiled && !direct) {   // long contexts: the merge kernel leaves fp32 rows; the tiled kernels read bf16 fragments
-            if (pgk_status r = norm_rows_bf16(a.xin, nullptr, e->attnv16 + (size_t)b0 * QD, M, QD, 0.f, st)) return r;
-            a.xin16 = e->attnv16 + (size_t)b0 * QD;
-            *launches += 1;
-        }
         if (pgk_status r = batched_proj(FP8, PRO_PLAIN, EPI_RESID, a, M, st)) return r;
         mark(KC_GATEUP);
         a = FusedArgs{};
@@ -1775,7 +1805,7 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
         a.xin16 = e->act16 + (size_t)b0 * I;
         a.res = h; a.out = h; a.ld_out = H;
         if (pgk_status r = batched_proj(FP8, PRO_PLAIN, EPI_RESID, a, M, st)) return r;
-        *launches += (direct ? 5 : 6) + gqa_chunks(c.num_heads / c.num_kv_heads) - 1;
+        *launches += (direct ? 5 : 6) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
     }
     const int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
     mark(KC_LMHEAD);
@@ -1844,10 +1874,6 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
         else { if (pgk_status r = launch_attn<64>(e, l, b0, M, false, direct, st, true)) return r; }
         mark(KC_OPROJ);
         bf16* attn16 = e->attnv16 + (size_t)b0 * QD;
-        if (!direct) {   // long contexts: the merge kernel leaves fp32 rows
-            if (pgk_status r = norm_rows_bf16(e->attnv + (size_t)b0 * QD, nullptr, attn16, M, QD, 0.f, st)) return r;
-            *launches += 1;
-        }
         bf16* act16 = e->act16 + (size_t)b0 * I;
         if (carried) {
             if (pgk_status r = pkgemm_resid_nt(attn16, QD, P.o, h, M, H, QD, (const bf16*)L.mlp_norm, x16, e->pk_ss, &ss_n, st)) return r;
@@ -1858,7 +1884,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
             mark(KC_DOWN);
             const bf16* gnext = l + 1 < c.num_layers ? (const bf16*)e->layers[l + 1].attn_norm : nullptr;
             if (pgk_status r = pkgemm_resid_nt(act16, I, P.down, h, M, H, I, gnext, x16, e->pk_ss, &ss_n, st)) return r;
-            *launches += (direct ? 5 : 6) + (l == 0 ? 1 : 0) + gqa_chunks(c.num_heads / c.num_kv_heads) - 1;
+            *launches += (direct ? 5 : 6) + (l == 0 ? 1 : 0) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
             continue;
         }
         if (pgk_status r = pkgemm_nt(attn16, QD, P.o, e->dec_slabs, H, PK_EPI_SLAB, s_o, M, H, QD, nullptr, st)) return r;
@@ -1869,7 +1895,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
         mark(KC_DOWN);
         if (pgk_status r = pkgemm_nt(act16, I, P.down, e->dec_slabs, H, PK_EPI_SLAB, s_d, M, H, I, nullptr, st)) return r;
         pending = s_d;
-        *launches += (direct ? 7 : 8) + gqa_chunks(c.num_heads / c.num_kv_heads) - 1;
+        *launches += (direct ? 7 : 8) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
     }
     const int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
     if (pgk_status r = norm(e->final_norm)) return r;     // also folds the last down_proj's slabs into the residual stream
@@ -1935,7 +1961,7 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
         a.w = L.w_down; a.wscale = (const bf16*)L.s_down; a.N = H; a.K = I;
         a.out = h; a.ld_out = H;
         if (pgk_status r = wide_proj(fp8, WIDE_PIECES, EPI_RESID, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
-        *launches += 4 + (direct ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads);
+        *launches += 4 + (direct ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads, M);
     }
     mark(KC_LMHEAD);
     FusedArgs a{};
