@@ -2071,11 +2071,11 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     const bool pk_heads = pk && D == 128 && !many;       // QKV epilogue: per-head norm + RoPE + cache write inside the projection
     // long prompts, bf16 weights: the N = hidden projections as split-K slabs when their 128-tiles do not cover the chip
     // (QKV / gate_up were tried too - their consumers can sum slabs - and measured slightly slower: 3.06 vs 2.99 ms at S = 512)
-    // w8a16 engines, long prompts: the staged bf16 GEMMs read the DEQUANTISED fragment-major copy the engine already holds
-    // (pack_weights_fp8: bf16(code x scale), the value the reference's w8a16 GEMM multiplies) - same kernels, epilogues and
-    // times as a bf16 engine (S = 512: 4.23 -> 2.44 ms) instead of the in-staging-dequant 128-tile kernel / a per-call
-    // dequantisation pass in front of the 256-tile kernel
-    const bool pkd = !ws && c.weight_format == 1 && e->packed_have && engine_gemm_packed_ok(n, NQKV, H) && engine_gemm_packed_ok(n, H, QD) &&
+    // long prompts: the staged bf16 GEMMs read the fragment-major copy the engine holds, whose blocks the LDS-DMA takes as they lie (Qwen3-0.6B,
+    // 1531 rows, the four projections: row-major 89 us, packed 80).  A w8a16 engine's copy is DEQUANTISED (pack_weights_fp8: bf16(code x scale), the
+    // value the reference's w8a16 GEMM multiplies): same kernels, epilogues and times as a bf16 engine (S = 512: 4.23 -> 2.44 ms) instead of the
+    // in-staging-dequant 128-tile kernel / a per-call dequantisation pass in front of the 256-tile kernel
+    const bool pkd = !ws && c.weight_format != 2 && e->packed_have && engine_gemm_packed_ok(n, NQKV, H) && engine_gemm_packed_ok(n, H, QD) &&
                      engine_gemm_packed_ok(n, 2 * I, H) && engine_gemm_packed_ok(n, H, I);
     const bool gsplit = !ws && (c.weight_format == 0 || pkd);
     const int g_so = gsplit ? engine_gemm_pick_splits(n, H, QD) : 1, g_sd = gsplit ? engine_gemm_pick_splits(n, H, I) : 1;

@@ -301,7 +301,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256_bf16_kernel(const bf16* A,
 // ---- bf16, staggered phases: the two waves of a SIMD alternate between "read + DMA issue" and "32 MFMAs" ---------
 // In the kernel above both waves of a SIMD leave each barrier together, request fragments together and want the MFMA
 // pipe together: the pipe idles while both wait (57 % busy).  Here the stage is half a K tile ([256 rows][32 k] per
-// operand, 64-byte rows; four stages in the same 128 KiB, three in flight) and a wave's work on stage s is two phases,
+// operand, 16 KiB each; three in flight) and a wave's work on stage s is two phases,
 //     A(s): request the 12 fragments of stage s, issue the DMA of stage s+3, wait for the fragments  | barrier
 //     B(s): 32 MFMAs                                                                                  | barrier
 // with waves 4-7 (the second wave of every SIMD) running ONE PHASE BEHIND waves 0-3 (one extra barrier up front, one
@@ -314,15 +314,26 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256_bf16_kernel(const bf16* A,
 // (r >> 2) & 3 was conflict-free for runs of 16 and 2-way conflicted for the real groups (SQ_LDS_BANK_CONFLICT = half of
 // SQ_LDS_IDX_ACTIVE on the round-2 kernel); (r >> 2) & 2 is conflict-free for them (exhaustive check; counter 0 in
 // profiles/r03_gemm256s_pmc.txt).
+// What the loop waits for is not latency (eight stages in flight instead of three: the same time) but the rate at which the LDS-DMA delivers, and
+// that depends on how a wave instruction's 1 KiB lies in memory.  L2-resident, all CUs: 33 TB/s for whole 128-byte lines, 31 for 64-byte halves in
+// passing pairs, 9.7 for a fragment-major block fetched in another order than memory's.  So
+//   * the packed W block goes to LDS as it lies, which is also the image a fragment read wants (lane l reads chunk l: no swizzle);
+//   * A comes two stages at a time, 8 rows x 128 B per instruction, into a ring of G2S_ARING half-stage slots of its own: image [rows][128 B], chunk
+//     c of row r at c ^ (r & 7) (g2_off), conflict-free in the groups above too.  A pair is requested at the even stages, 4 stages ahead, so between
+//     any stage and its wait lie two W stages and one A pair: the counts of the three-in-flight scheme, vmcnt(8).
+// M = 4096, packed W, us, both changes: N = 4096, K = 14336 396 -> 344; N = 14336 (SwiGLU), K = 4096 774 -> 704; N = 6144, K = 4096 198 -> 171.  Row-major
+// W keeps its 64-byte rows (ring slots for pairs of both operands would not fit): 743 -> 719 for the SwiGLU product.
 // TN = n-fragments per wave column: 4 = 256-column tiles; 3 = 192-column tiles (EPI 0 only), for shapes whose 256-tiles leave a
 // half-empty last round: Llama's QKV (4096 x 6144) is 384 tiles = 1.5 rounds of the 256 CUs, 512 tiles of 256 x 192 are two
 // full rounds of three quarters the work.  The W stage then has 192 rows = 12 DMA instructions: waves 0-3 move two (rows 0-127),
 // waves 4-7 one (rows 128-191), so the "two younger stages in flight" count is vmcnt(8) for the former, vmcnt(6) for the latter.
+constexpr int G2S_ARING = 6;      // slots of A, in stages
+constexpr size_t G2S_LDS = (G2S_ARING + 4) * (size_t)256 * 64;
 template <int EPI, int TN = 4>   // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store
 __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                                                     int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa = ActArgs{}) {
     static_assert(TN == 4 || (TN == 3 && (EPI == 0 || EPI >= 2)), "192-column tiles: bf16 store and SwiGLU only");
-    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // 4 stages x (A 16 KiB | W 16 KiB)
+    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -331,44 +342,46 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     g2_tile_of(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
     const int m0 = tm * G2_BM, n0 = tn * BN;
 
-    const int drow = wid * 32 + (lane >> 2);                 // one DMA instruction = 16 rows x 64 B
+    const int drow = wid * 32 + (lane >> 2);                 // one DMA instruction of W = 16 rows x 64 B
     const int dchunk = (lane & 3) ^ ((lane >> 4) & 2);      // = (lane & 3) ^ g2s_sw(row & 15), row & 15 = lane >> 2
-    const bf16* a_src0 = A + (size_t)min(m0 + drow, M - 1) * K + dchunk * 8;
-    const bf16* a_src1 = A + (size_t)min(m0 + drow + 16, M - 1) * K + dchunk * 8;
+    const bf16* a_src[4];                                    // of A: 8 rows x 128 B, two stages
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a_src[i] = A + (size_t)min(m0 + wid * 32 + 8 * i + (lane >> 3), M - 1) * K + ((lane & 7) ^ (lane >> 3)) * 8;
     // B-tile row r of an EPI-2 workgroup: gate row 128 tn + r for r < 128, up row N + 128 tn + (r - 128) after that (N = I)
     const int wtile_row = (TN == 4 || !late) ? drow : 128 + (wid - 4) * 16 + (lane >> 2);
     constexpr int GATE = TN * 32;     // EPI 2: gate rows per B tile (128 / 96), the matching up rows follow
     const int wrow = (EPI == 2) ? (wtile_row < GATE ? tn * GATE + wtile_row : N + tn * GATE + wtile_row - GATE) : n0 + wtile_row;
     const int wlast = (EPI == 2) ? 2 * N - 1 : N - 1;
     // W row-major [rows][K], or (packed) the fragment-major copy of ops_pkgemm.hip: block (16-row tile nt, k-step ks) = 1 KiB at
-    // ((nt K/32 + ks) 64 + chunk 16 + row) 8 elements.  One DMA instruction moves 16 rows x 32 k = exactly one such block; only
-    // the per-lane source offset inside it differs (this lane's logical chunk and row), and a stage advances 512 elements.
+    // ((nt K/32 + ks) 64 + chunk 16 + row) 8 elements.  One DMA instruction moves 16 rows x 32 k = exactly one such block, as it lies,
+    // and a stage advances 512 elements.
     const bf16 *w_src0, *w_src1;
     const int wk = packed ? 512 : 32;
     if (packed) {
         const int r_in = lane >> 2, nt_last = (wlast >> 4);
-        w_src0 = W + ((size_t)min((wrow - r_in) >> 4, nt_last) * (K >> 5) * 64 + dchunk * 16 + r_in) * 8;
-        w_src1 = W + ((size_t)min((wrow - r_in + 16) >> 4, nt_last) * (K >> 5) * 64 + dchunk * 16 + r_in) * 8;
+        w_src0 = W + ((size_t)min((wrow - r_in) >> 4, nt_last) * (K >> 5) * 64 + lane) * 8;
+        w_src1 = W + ((size_t)min((wrow - r_in + 16) >> 4, nt_last) * (K >> 5) * 64 + lane) * 8;
     } else {
         w_src0 = W + (size_t)min(wrow, wlast) * K + dchunk * 8;
         w_src1 = W + (size_t)min(wrow + 16, wlast) * K + dchunk * 8;
     }
     const uint32_t lds0 = g2_lds_addr(g2_smem);
     const int nh = K / 32;
-    auto stage = [&](int h, int buf) {
-        const int hc = min(h, nh - 1), k = hc * 32;
-        const size_t kw = (size_t)hc * wk;
-        const uint32_t a_dst = __builtin_amdgcn_readfirstlane(lds0 + buf * 2 * HALF + wid * 2048);
-        g2_dma16(a_src0 + k, a_dst);
-        g2_dma16(a_src1 + k, a_dst + 1024);
-        if constexpr (TN == 4) {
-            g2_dma16(w_src0 + kw, a_dst + HALF);
-            g2_dma16(w_src1 + kw, a_dst + HALF + 1024);
-        } else if (!late) {
-            g2_dma16(w_src0 + kw, a_dst + HALF);
-            g2_dma16(w_src1 + kw, a_dst + HALF + 1024);
+    // past the end of K the last stage is read again (never consumed): the counts below stay constant
+    auto stage_a = [&](int h, int at) {                      // `at`: byte offset of the ring's slot
+        const int k = min(h, nh - 2) * 32;
+        const uint32_t a_dst = __builtin_amdgcn_readfirstlane(lds0 + at + wid * 4096);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g2_dma16(a_src[i] + k, a_dst + i * 1024);
+    };
+    auto stage_w = [&](int h, int buf) {
+        const size_t kw = (size_t)min(h, nh - 1) * wk;
+        const uint32_t w_dst = __builtin_amdgcn_readfirstlane(lds0 + (G2S_ARING + buf) * HALF + wid * 2048);
+        if (TN == 4 || !late) {
+            g2_dma16(w_src0 + kw, w_dst);
+            g2_dma16(w_src1 + kw, w_dst + 1024);
         } else {
-            g2_dma16(w_src0 + kw, __builtin_amdgcn_readfirstlane(lds0 + buf * 2 * HALF + HALF + 128 * 64 + (wid - 4) * 1024));
+            g2_dma16(w_src0 + kw, __builtin_amdgcn_readfirstlane(lds0 + (G2S_ARING + buf) * HALF + 128 * 64 + (wid - 4) * 1024));
         }
     };
     // "this wave's share of the oldest of three stages in flight has landed"
@@ -383,24 +396,33 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
-    const int f_off = l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
-    const int a_base = wr * 128 * 64, w_base = HALF + wc * WN * 64;
+    const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
+    const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
+    const int a_base = wr * 128 * 128, w_base = G2S_ARING * HALF + wc * WN * 64;
     uint4 fa[8], fb[TN];
 
-    stage(0, 0);
-    stage(1, 1);
-    stage(2, 2);
+    stage_a(0, 0);
+    stage_w(0, 0);
+    stage_a(2, 2 * HALF);
+    stage_w(1, 1);
+    stage_w(2, 2);
+    int a_cur = 0;                                           // ring slot of A's stage s
     wait_two_younger();
     __builtin_amdgcn_s_barrier();
     if (late) __builtin_amdgcn_s_barrier();                  // waves 4-7 start one phase behind
 #define G2S_STEP(S, BUF)                                                                                     \
     {   /* phase A */                                                                                        \
-        const char* As = g2_smem + (BUF) * 2 * HALF + a_base + f_off;                                        \
-        const char* Ws = g2_smem + (BUF) * 2 * HALF + w_base + f_off;                                        \
-        _Pragma("unroll") for (int i = 0; i < 8; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 1024); \
+        const char* As = g2_smem + a_cur + a_base + (((BUF) & 1) ? a_off1 : a_off0);                           \
+        const char* Ws = g2_smem + (BUF) * HALF + w_base + w_off;                                        \
+        _Pragma("unroll") for (int i = 0; i < 8; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 2048); \
         _Pragma("unroll") for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const uint4*>(Ws + j * 1024); \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
-        stage((S) + 3, ((BUF) + 3) & 3);                                                                     \
+        if (((BUF) & 1) == 0) {                                                                              \
+            const int a_new = a_cur >= 2 * HALF ? a_cur - 2 * HALF : a_cur + 4 * HALF;                       \
+            stage_a((S) + 4, a_new);                                                                         \
+        }                                                                                                    \
+        stage_w((S) + 3, ((BUF) + 3) & 3);                                                                   \
+        if (((BUF) & 1) == 1) a_cur = a_cur == 4 * HALF ? 0 : a_cur + 2 * HALF;                              \
         if (late) wait_two_younger();                                                                        \
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                   \
         __builtin_amdgcn_s_barrier();                                                                        \
@@ -461,11 +483,13 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 // (Qwen3-0.6B at S = 2048: N = 1024 projections = 128 tiles, QKV 512 tiles with K = 1024.)  The register-staged 128-tile
 // kernel of ops_gemm.hip keeps ONE K step in flight (global -> registers -> LDS -> barrier): with one or two workgroups
 // per CU every step costs a memory round trip - 1.9 us per 64 k at M = 2048, N = 1024 (30 us for 8.6 GFLOP).  Here: 4 waves
-// (2 x 2, 64 x 64 each = 64 accumulator registers), stages of 32 k ([128 rows][64 B] per operand, 16 KiB per stage, the
-// swizzle of gemm256s), four stages of which three are in flight behind a counted vmcnt(8), ONE barrier per stage; 64 KiB
+// (2 x 2, 64 x 64 each = 64 accumulator registers), stages of 32 k (16 KiB, the images, rings and counts of gemm256s: A a pair of stages at a
+// time in whole lines, packed W as it lies), three stages in flight behind a counted vmcnt(8), ONE barrier per stage; 80 KiB
 // of LDS and < 128 registers, so two workgroups share a CU and one's MFMAs cover the other's barrier and fragment reads -
 // no stagger needed.  blockIdx.y = K split (EPI 2: fp32 slab z of [splits][M][N], summed by the consumer).
-// Epilogue through LDS: the fp32 tile (64 KiB = the four stages) is written with the lane quarters XOR-ed apart, then read
+// (Reading the next stage's fragments under this one's MFMAs, or eight stages, changes nothing: the loop waits for what the DMA delivers.  M = 1531,
+// N = 4096, K = 1024, us: row-major W, 64-byte rows of A 20.6; packed 25.6 -> 19.2.  M = 384, N = 1024, K = 3072 in four splits: 12.4; 13.7 -> 10.9.)
+// Epilogue through LDS: the fp32 tile (64 KiB of the stages) is written with the lane quarters XOR-ed apart, then read
 // back as rows - 32 lanes x 16 B = one 512-byte row segment per instruction - for coalesced stores (EPI 1: float4
 // read-modify-write of the residual stream, all loads issued before the first store).
 constexpr int G1_THREADS = 256, G1_HALF = 128 * 64;
@@ -475,7 +499,7 @@ constexpr int G1_THREADS = 256, G1_HALF = 128 * 64;
 template <int EPI, bool GRP>
 __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                               int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga) {
-    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // 4 stages x (A 8 KiB | W 8 KiB)
+    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 8 KiB | W: 4 stages of 8 KiB
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int wr = wid >> 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
     int tm, tn, m0;
@@ -500,8 +524,9 @@ __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, cons
         if constexpr (GRP) return ga.div > 0 ? ga.order[r] / ga.div : r;
         else return r;
     };
-    const bf16* a_src0 = A + (size_t)a_row(m0 + drow) * K + kbeg + dchunk * 8;
-    const bf16* a_src1 = A + (size_t)a_row(m0 + drow + 16) * K + kbeg + dchunk * 8;
+    const bf16* a_src[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a_src[i] = A + (size_t)a_row(m0 + wid * 32 + 8 * i + (lane >> 3)) * K + kbeg + ((lane & 7) ^ (lane >> 3)) * 8;
     // EPI 4: B-tile rows 0-63 = gate rows 64 tn .., rows 64-127 = the matching up rows N + 64 tn .. (N = I); a wave's 32 rows stay in one half
     const int wrow = (EPI == 4) ? (drow < 64 ? tn * 64 + drow : N + tn * 64 + drow - 64) : n0 + drow;
     const int wlast = (EPI == 4) ? 2 * N - 1 : N - 1;
@@ -510,22 +535,26 @@ __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, cons
     const int wk = packed ? 512 : 32;
     if (packed) {
         const int r_in = lane >> 2, nt_last = (wlast >> 4);
-        w_src0 = W + (((size_t)min((wrow - r_in) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + dchunk * 16 + r_in) * 8;
-        w_src1 = W + (((size_t)min((wrow - r_in + 16) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + dchunk * 16 + r_in) * 8;
+        w_src0 = W + (((size_t)min((wrow - r_in) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + lane) * 8;
+        w_src1 = W + (((size_t)min((wrow - r_in + 16) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + lane) * 8;
     } else {
         w_src0 = W + (size_t)min(wrow, wlast) * K + kbeg + dchunk * 8;
         w_src1 = W + (size_t)min(wrow + 16, wlast) * K + kbeg + dchunk * 8;
     }
     const uint32_t lds0 = g2_lds_addr(g2_smem);
     const int nh = (kend - kbeg) / 32;
-    auto stage = [&](int h, int buf) {
-        const int hc = min(h, nh - 1), k = hc * 32;          // past the end: re-read the last stage (never consumed), the count stays constant
-        const size_t kw = (size_t)hc * wk;
-        const uint32_t a_dst = __builtin_amdgcn_readfirstlane(lds0 + buf * 2 * G1_HALF + wid * 2048);
-        g2_dma16(a_src0 + k, a_dst);
-        g2_dma16(a_src1 + k, a_dst + 1024);
-        g2_dma16(w_src0 + kw, a_dst + G1_HALF);
-        g2_dma16(w_src1 + kw, a_dst + G1_HALF + 1024);
+    // past the end of K the last stage is read again (never consumed): the counts below stay constant
+    auto stage_a = [&](int h, int at) {
+        const int k = min(h, nh - 2) * 32;
+        const uint32_t a_dst = __builtin_amdgcn_readfirstlane(lds0 + at + wid * 4096);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g2_dma16(a_src[i] + k, a_dst + i * 1024);
+    };
+    auto stage_w = [&](int h, int buf) {
+        const size_t kw = (size_t)min(h, nh - 1) * wk;
+        const uint32_t w_dst = __builtin_amdgcn_readfirstlane(lds0 + (G2S_ARING + buf) * G1_HALF + wid * 2048);
+        g2_dma16(w_src0 + kw, w_dst);
+        g2_dma16(w_src1 + kw, w_dst + 1024);
     };
 
     f32x4_g acc[4][4];
@@ -533,25 +562,34 @@ __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, cons
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
-    const int f_off = l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
-    const int a_base = wr * 64 * 64, w_base = G1_HALF + wc * 64 * 64;
+    const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
+    const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
+    const int a_base = wr * 64 * 128, w_base = G2S_ARING * G1_HALF + wc * 64 * 64;
     uint4 fa[4], fb[4];
 
-    stage(0, 0);
-    stage(1, 1);
-    stage(2, 2);
+    stage_a(0, 0);
+    stage_w(0, 0);
+    stage_a(2, 2 * G1_HALF);
+    stage_w(1, 1);
+    stage_w(2, 2);
+    int a_cur = 0;                                           // ring slot of A's stage s
     // iteration s: own share of stage s landed (two younger stages may stay in flight) | barrier: everyone's share landed AND
     // everyone finished reading stage s - 1, whose buffer the DMA of stage s + 3 - issued right behind the reads - refills
 #define G1S_STEP(S, BUF)                                                                                      \
     {                                                                                                         \
         asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                                                      \
         __builtin_amdgcn_s_barrier();                                                                         \
-        const char* As = g2_smem + (BUF) * 2 * G1_HALF + a_base + f_off;                                      \
-        const char* Ws = g2_smem + (BUF) * 2 * G1_HALF + w_base + f_off;                                      \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 1024); \
+        const char* As = g2_smem + a_cur + a_base + (((BUF) & 1) ? a_off1 : a_off0);                         \
+        const char* Ws = g2_smem + (BUF) * G1_HALF + w_base + w_off;                                      \
+        _Pragma("unroll") for (int i = 0; i < 4; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 2048); \
         _Pragma("unroll") for (int j = 0; j < 4; ++j) fb[j] = *reinterpret_cast<const uint4*>(Ws + j * 1024); \
         __builtin_amdgcn_sched_barrier(0);                                                                    \
-        stage((S) + 3, ((BUF) + 3) & 3);                                                                      \
+        if (((BUF) & 1) == 0) {                                                                               \
+            const int a_new = a_cur >= 2 * G1_HALF ? a_cur - 2 * G1_HALF : a_cur + 4 * G1_HALF;               \
+            stage_a((S) + 4, a_new);                                                                          \
+        }                                                                                                     \
+        stage_w((S) + 3, ((BUF) + 3) & 3);                                                                    \
+        if (((BUF) & 1) == 1) a_cur = a_cur == 4 * G1_HALF ? 0 : a_cur + 2 * G1_HALF;                         \
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                    \
         __builtin_amdgcn_sched_barrier(0);                                                                    \
         __builtin_amdgcn_s_setprio(1);                                                                        \
@@ -986,7 +1024,7 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
                            hipStream_t st, bool packed, const ActArgs* act) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64, "gemm256: K=%d must be a multiple of 64", K);
     PGK_REQUIRE(!packed || N % 16 == 0, "gemm256: the fragment-major weight copy has whole 16-row tiles (N=%d)", N);
-    constexpr size_t LDS = 4 * (size_t)G2_TILE;
+    constexpr size_t LDS = G2S_LDS;
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256_bf16_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
@@ -1039,7 +1077,7 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
 // act[M][I] = bf16(silu(A . Wg^T) * (A . Wu^T)), W = fused [2 I, K] gate / up weight (staggered kernel, SwiGLU epilogue)
 pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64 && I % 128 == 0, "gemm256 swiglu: K=%d must be a multiple of 64 and I=%d of 128", K, I);
-    constexpr size_t LDS = 4 * (size_t)G2_TILE;
+    constexpr size_t LDS = G2S_LDS;
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
@@ -1068,7 +1106,7 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
     PGK_REQUIRE(mode != 4 || N % 64 == 0, "gemm128s: the SwiGLU epilogue needs I=%d to be a multiple of 64", N);
     PGK_REQUIRE(mode != 3 || (heads && N == (heads->hq + 2 * heads->hkv) * 128), "gemm128s: the QKV-heads epilogue needs N=%d = (Hq + 2 Hkv) x 128", N);
     const QkvHeadArgs hd = heads ? *heads : QkvHeadArgs{};
-    constexpr size_t LDS = 8 * (size_t)G1_HALF;
+    constexpr size_t LDS = (G2S_ARING + 4) * (size_t)G1_HALF;
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
@@ -1097,7 +1135,7 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
 
 pgk_status gemm128s_grouped(const bf16* A, const bf16* W, bf16* C, MoeProduct what, const GroupArgs& g, int max_tiles, int rows, int N, int K, hipStream_t st) {
     PGK_REQUIRE(K % 64 == 0 && N % 64 == 0 && max_tiles >= 1 && g.tiles && g.n_tiles && g.order && g.wts, "gemm128s_grouped: N=%d K=%d", N, K);
-    constexpr size_t LDS = 8 * (size_t)G1_HALF;
+    constexpr size_t LDS = (G2S_ARING + 4) * (size_t)G1_HALF;
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_grouped_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));

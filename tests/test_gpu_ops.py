@@ -496,6 +496,19 @@ def test_gemm256_exact_integers(N, monkeypatch):
     np.testing.assert_array_equal(c, O.bf16_round(a @ w.T))
 
 
+@pytest.mark.parametrize("tile", ["0", "1"])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
+def test_staged_gemm_rings_exact_integers(K, tile, monkeypatch):
+    """The staged kernels keep A in a ring of three 64-k pairs and W in one of four 32-k stages: every position the two can end in, from the
+    shortest K (whose prologue already reads past its end) on, at ragged M and N.  Small integers: bit for bit."""
+    rng = np.random.default_rng(K)
+    monkeypatch.setenv("PGK_GEMM256", tile)
+    for M, N in ((129, 136), (300, 384), (515, 264)):
+        a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+        w = rng.integers(-3, 4, (N, K)).astype(np.float32)
+        np.testing.assert_array_equal(host(ops.matmul_nt(dev(a, "bfloat16"), dev(w, "bfloat16"))), O.bf16_round(a @ w.T), err_msg=f"{M} {N}")
+
+
 # ----------------------------------------------------------------------------- fp8 x fp8 GEMM
 def _fp8_vals(codes):
     return O.fp8_e4m3_table()[codes]
