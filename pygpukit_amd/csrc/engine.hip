@@ -38,6 +38,10 @@ pgk_status engine_gemm_nt(const bf16* A, const void* W, const bf16* wscale, bool
 bool engine_gemm_packed_ok(int M, int N, int K);
 int wsgemm_pick_splits(int N, int K, bool allow_split);
 int engine_gemm_pick_splits(int M, int N, int K);
+int engine_gemm_qkv_splits(int M, int N, int K, bool fused);
+int engine_gemm_short_splits(int N, int K);                    // ops_gemm.hip: prompts of <= 128 rows on the staged 128-tile kernel
+bool engine_gemm_short_ok(int hidden, int qdim, int qkv, int inter, bool packed);
+pgk_status engine_gemm_short(const bf16* A, const void* W, void* C, int mode, int splits, int M, int N, int K, hipStream_t st, bool packed, const QkvHeadArgs* heads = nullptr);
 pgk_status engine_gemm_nt_slabs(const bf16* A, const void* W, float* slabs, int splits, int M, int N, int K, hipStream_t st, bool packed = false);
 pgk_status gemm_fp8_nt(const uint8_t* a, const float* sa, const uint8_t* w, const bf16* sw, void* c, bool accum_f32, int M,
                        int N, int K, hipStream_t st);
@@ -2061,7 +2065,14 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     const int H = c.hidden_size, I = c.intermediate_size, D = c.head_dim, QD = c.num_heads * D, NQKV = e->qkv_dim();
     // workspace: h32 [n,H] f32 | x [n,H] | qkv [n,NQKV] | attn [n,QD] | gu [n,2I] | act [n,I]  (bf16)
     // + split-K slabs of the N = hidden projections on the weight-streaming path (n <= 128)
-    const bool ws = n <= 128;
+    // Up to 128 rows on the staged 128-tile kernel (engine_gemm_short): from 65 on, or where the gate_up product's tiles cover most of the chip
+    // (nothing splits that one) from the first row, or the 17th with e4m3 weights, whose codes are half the bytes of the copy read here.  Streamed /
+    // staged, ms: H = 2560, I = 6912, 3 layers 40 rows 0.345 / 0.354, 100 rows 0.433 / 0.381; Llama-3-8B bf16 8 rows 4.84 / 4.44, 100 rows
+    // 7.28 / 5.00, e4m3 12 rows 3.90 / 4.01, 20 rows 4.15 / 4.03, 100 rows 7.42 / 4.61.
+    const int staged_from = I / 64 < 192 ? 65 : c.weight_format == 0 ? 1 : 17;
+    const bool staged = n <= 128 && n >= staged_from && !e->packed_ok && (c.weight_format == 0 || (c.weight_format == 1 && e->packed_have)) &&
+                        engine_gemm_short_ok(H, QD, NQKV, I, c.weight_format == 1);
+    const bool ws = n <= 128 && !staged;
     const int s_o = ws ? wsgemm_pick_splits(H, QD, true) : 1, s_d = ws ? wsgemm_pick_splits(H, I, true) : 1;
     const int s_qkv_ws = ws ? wsgemm_pick_splits(NQKV, H, true) : 1, s_qkv = s_qkv_ws, s_gu = ws ? wsgemm_pick_splits(2 * I, H, true) : 1;
     const int maxk = I > QD ? (I > H ? I : H) : (QD > H ? QD : H);
@@ -2075,15 +2086,17 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     // 1531 rows, the four projections: row-major 89 us, packed 80).  A w8a16 engine's copy is DEQUANTISED (pack_weights_fp8: bf16(code x scale), the
     // value the reference's w8a16 GEMM multiplies): same kernels, epilogues and times as a bf16 engine (S = 512: 4.23 -> 2.44 ms) instead of the
     // in-staging-dequant 128-tile kernel / a per-call dequantisation pass in front of the 256-tile kernel
-    const bool pkd = !ws && c.weight_format != 2 && e->packed_have && engine_gemm_packed_ok(n, NQKV, H) && engine_gemm_packed_ok(n, H, QD) &&
-                     engine_gemm_packed_ok(n, 2 * I, H) && engine_gemm_packed_ok(n, H, I);
+    const bool pkd = !ws && c.weight_format != 2 && e->packed_have && (staged || (engine_gemm_packed_ok(n, NQKV, H) && engine_gemm_packed_ok(n, H, QD) &&
+                     engine_gemm_packed_ok(n, 2 * I, H) && engine_gemm_packed_ok(n, H, I)));
     const bool gsplit = !ws && (c.weight_format == 0 || pkd);
-    const int g_so = gsplit ? engine_gemm_pick_splits(n, H, QD) : 1, g_sd = gsplit ? engine_gemm_pick_splits(n, H, I) : 1;
-    const bool use_slabs = ws || g_so > 1 || g_sd > 1;
+    auto hidden_splits = [&](int K_) { return !gsplit ? 1 : staged ? engine_gemm_short_splits(H, K_) : engine_gemm_pick_splits(n, H, K_); };
+    const int g_so = hidden_splits(QD), g_sd = hidden_splits(I), g_sq = gsplit ? engine_gemm_qkv_splits(n, NQKV, H, D == 128) : 1;
+    const bool use_slabs = ws || g_so > 1 || g_sd > 1 || g_sq > 1;
     size_t slab_elems = (size_t)(s_o > s_d ? s_o : s_d) * n * H;
     if ((size_t)(g_so > g_sd ? g_so : g_sd) * n * H > slab_elems) slab_elems = (size_t)(g_so > g_sd ? g_so : g_sd) * n * H;
     if (pk && (size_t)(pk_so > pk_sd ? pk_so : pk_sd) * n * H > slab_elems) slab_elems = (size_t)(pk_so > pk_sd ? pk_so : pk_sd) * n * H;
     if (s_qkv > 1 && (size_t)s_qkv * n * NQKV > slab_elems) slab_elems = (size_t)s_qkv * n * NQKV;
+    if (g_sq > 1 && (size_t)g_sq * n * NQKV > slab_elems) slab_elems = (size_t)g_sq * n * NQKV;
     if (s_gu > 1 && (size_t)s_gu * n * 2 * I > slab_elems) slab_elems = (size_t)s_gu * n * 2 * I;
     const size_t need = (size_t)n * H * 4 + ((size_t)n * H + (size_t)n * NQKV + (size_t)n * QD + (size_t)n * 2 * I + (size_t)n * I) * 2 +
                         (use_slabs ? slab_elems * 4 : 0) + 512 + (c.weight_format == 2 ? 2 * ((size_t)n * maxk + (size_t)n * (maxk / 128) * 4 + 512) : 0);
@@ -2142,10 +2155,10 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     const bool fuse_q = fp8act && H % 128 == 0 && I % 128 == 0 && H <= 4096 && fuse_epi;
     // SwiGLU in the gate / up GEMM's epilogue (256-tile kernels; fp8 x fp8: with the quantisation of its result)
     const bool fuse_sw8 = fuse_q && gemm_fp8_swiglu_ok(n, I, H);
-    const bool fuse_sw16 = !fp8act && !ws && fuse_epi && engine_gemm_swiglu_ok(n, I, H, fp8 && !pkd);
+    const bool fuse_sw16 = !fp8act && !ws && (staged || (fuse_epi && engine_gemm_swiglu_ok(n, I, H, fp8 && !pkd)));
     // per-head norm + RoPE + cache write in the QKV GEMM's epilogue (bf16 weights, head_dim 128, 128-tile kernel: tile column = head)
     const bool fuse_heads8 = fuse_q && D == 128 && gemm_fp8_qkv_heads_ok(n, NQKV, H);      // fp8 x fp8: x's codes are already in q8
-    const bool fuse_heads = fuse_heads8 || (!ws && !pk && fuse_epi && (c.weight_format == 0 || pkd) && D == 128 && engine_gemm_qkv_heads_ok(n, NQKV, H));
+    const bool fuse_heads = fuse_heads8 || (!ws && !pk && fuse_epi && gsplit && g_sq == 1 && D == 128 && (staged || engine_gemm_qkv_heads_ok(n, NQKV, H)));
     auto proj_accum = [&](const bf16* x_in, const void* w, const void* sc, int N_, int K_, int splits, const bf16* wp = nullptr) -> pgk_status {
         if (fp8act) {
             if (x_in)
@@ -2154,7 +2167,11 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         }
         if (!ws) {
             const bool usep = pkd && wp != nullptr;
-            const int gs = gsplit ? engine_gemm_pick_splits(n, N_, K_) : 1;
+            const int gs = hidden_splits(K_);
+            if (staged) {
+                pending = gs > 1 ? gs : 0;
+                return engine_gemm_short(x_in, usep ? (const void*)wp : w, gs > 1 ? (void*)slabs : h32, gs > 1 ? 2 : 1, gs, n, N_, K_, st, usep);
+            }
             if (gs > 1) { pending = gs; return engine_gemm_nt_slabs(x_in, usep ? (const void*)wp : w, slabs, gs, n, N_, K_, st, usep); }
             if (usep) return engine_gemm_nt(x_in, wp, nullptr, false, h32, true, n, N_, K_, st, true);
             return engine_gemm_nt(x_in, w, (const bf16*)sc, fp8, h32, true, n, N_, K_, st);
@@ -2218,12 +2235,16 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             hd.at = d_at; hd.slot_stride = slot_stride;
             if (fuse_heads8) {
                 if (pgk_status r = gemm_fp8_qkv_heads_nt(q8, q8s, (const uint8_t*)L.w_qkv, (const bf16*)L.s_qkv, qkv, n, NQKV, H, hd, st)) return r;
+            } else if (staged) {
+                if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].qkv : L.w_qkv, qkv, 3, 1, n, NQKV, H, st, pkd, &hd)) return r;
             } else if (pgk_status r = engine_gemm_qkv_heads_nt(x, pkd ? e->packed[l].qkv : (const bf16*)L.w_qkv, qkv, n, NQKV, H, hd, st, pkd)) return r;
+        } else if (staged || g_sq > 1) {
+            if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].qkv : L.w_qkv, g_sq > 1 ? (void*)slabs : qkv, g_sq > 1 ? 2 : 0, g_sq, n, NQKV, H, st, pkd)) return r;
         } else {
             if (pgk_status r = proj_store(fuse_q ? nullptr : x, L.w_qkv, L.s_qkv, qkv, NQKV, H, s_qkv, pkd ? e->packed[l].qkv : nullptr)) return r;
         }
         if (!pk_heads && !fuse_heads) {
-            const int s_qkv = pk ? 1 : s_qkv_ws;
+            const int s_qkv = pk ? 1 : g_sq > 1 ? g_sq : s_qkv_ws;
             const int nslots = c.num_heads + 2 * c.num_kv_heads;
             const bf16* qg = c.use_qk_norm ? (const bf16*)L.q_norm : nullptr;
             const bf16* kg = c.use_qk_norm ? (const bf16*)L.k_norm : nullptr;
@@ -2288,7 +2309,9 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             continue;
         }
         if (fuse_sw16) {
-            if (pgk_status r = engine_gemm_swiglu_nt(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, (const bf16*)L.s_gate_up, fp8 && !pkd, act, n, I, H, st, pkd)) return r;
+            if (staged) {
+                if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, act, 4, 1, n, I, H, st, pkd)) return r;
+            } else if (pgk_status r = engine_gemm_swiglu_nt(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, (const bf16*)L.s_gate_up, fp8 && !pkd, act, n, I, H, st, pkd)) return r;
             if (pgk_status r = proj_accum(act, L.w_down, L.s_down, H, I, s_d, pkd ? e->packed[l].down : nullptr)) return r;
             continue;
         }

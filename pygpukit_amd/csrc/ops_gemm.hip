@@ -25,6 +25,7 @@ pgk_status wsgemm_nt(const bf16* a, int lda, const void* w, const bf16* wscale, 
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
                            hipStream_t st, bool packed = false, const ActArgs* act = nullptr);
 pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed = false);
+bool gemm128s_shape_ok(int N, int K);
 bool gemm128s_ok(int M, int N, int K);    // ops_gemm256.hip: 128 x 128 tiles on the staged LDS-DMA pipeline (bf16, M > 128, K % 64 == 0, N % 8 == 0)
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
                             const QkvHeadArgs* heads = nullptr, bool packed = false, const ActArgs* act = nullptr);
@@ -397,6 +398,34 @@ int engine_gemm_pick_splits(int M, int N, int K) {
     if (s > 4) s = 4;
     while (s > 1 && (K / s < 512 || (gemm128s_ok(M, N, K) && K % (64 * s) != 0))) --s;
     return s < 1 ? 1 : s;
+}
+// The QKV projection of prompts whose 128-tiles leave most of the chip idle: slabs that the per-head norm / RoPE pass sums, where the shorter
+// serial chain (0.33 us per 32 k of a workgroup) pays for that pass, 5 us, which the unsplit product does as its epilogue (`fused`).
+// K = 4096, N = 6144, us: 200 rows unsplit 44, two runs 26 + 5; 100 rows 45, four runs 17 + 5.
+int engine_gemm_qkv_splits(int M, int N, int K, bool fused) {
+    const long long tiles = (long long)ceil_div(M, 128) * ceil_div(N, 128);
+    if (!gemm128s_shape_ok(N, K) || (M > 128 && use_gemm256(M, N, K))) return 1;
+    int s = (int)(256 / tiles);
+    if (s > 8) s = 8;
+    while (s > 1 && (K / s < (fused ? 1024 : 512) || K % (64 * s) != 0)) --s;
+    return s < 1 ? 1 : s;
+}
+// The products of a prompt of <= 128 rows on the staged 128-tile kernel (one row of tiles, split along K towards a workgroup per CU), for layers
+// that the packed kernels do not take.  The weight-streaming kernel (ops_wsgemm.hip) keeps one K tile in flight per wave and reads every A fragment
+// once per 16 weight rows: Llama-3-8B shape, 100 rows, us, that one / this one on row-major / on packed weights: gate_up 102 / 60 / 49,
+// down 48 / 29 / 26, QKV 29 / 17 / 15, o 16 / 12 / 11; 16 rows: 58 / 55 / 44, 31 / 25 / 23, 17 / 15 / 13, 10 / 10 / 9.
+int engine_gemm_short_splits(int N, int K) {
+    int s = 256 / ceil_div(N, 128);
+    if (s > 8) s = 8;            // (16 runs were slower: the slabs' bytes)
+    while (s > 1 && (K / s < 512 || K % (64 * s) != 0)) --s;
+    return s < 1 ? 1 : s;
+}
+bool engine_gemm_short_ok(int hidden, int qdim, int qkv, int inter, bool packed) {
+    return gemm128s_shape_ok(qkv, hidden) && gemm128s_shape_ok(hidden, qdim) && gemm128s_shape_ok(hidden, inter) && inter % 64 == 0 && (!packed || (qkv % 16 == 0 && hidden % 16 == 0));
+}
+// mode: gemm128s_bf16_nt
+pgk_status engine_gemm_short(const bf16* A, const void* W, void* C, int mode, int splits, int M, int N, int K, hipStream_t st, bool packed, const QkvHeadArgs* heads) {
+    return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, C, mode, splits, M, N, K, st, heads, packed);
 }
 pgk_status engine_gemm_nt_slabs(const bf16* A, const void* W, float* slabs, int splits, int M, int N, int K, hipStream_t st, bool packed) {
     PGK_REQUIRE(splits >= 1 && K % 8 == 0, "engine_gemm_nt_slabs: splits=%d K=%d", splits, K);
