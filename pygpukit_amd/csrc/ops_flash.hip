@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
     if (gid >= nrow * CPR) return;          // nrow * CPR is a multiple of 16: the 16 lanes of a (row, head) stay together
     const size_t rowi = gid / CPR;
     const int c = (int)(gid % CPR), qrow = (int)(rowi / hq), head = (int)(rowi % hq);
-    // (nsplit is a power of two up to 16: four runs' records and rows are requested at a time)
+    // (up to 16 runs: four runs' records and rows are requested at a time)
     float mstar = -INFINITY;
     for (int s2 = 0; s2 < nsplit; ++s2) mstar = fmaxf(mstar, ml[(((size_t)s2 * hq + head) * q_len + qrow) * 2]);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f;
@@ -488,11 +488,23 @@ static int flash_cus() {
     return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
-// KV runs per query tile: enough workgroups for two per CU (the kernel's occupancy), at least four KV tiles to a run
-static int flash_runs(long long wgs, int span, int most) {
+// KV runs per query tile, at least four KV tiles to a run, as many as one round of workgroups holds: of two per CU (the kernel's occupancy), a heavy
+// and a light one, where the causal edge makes query tiles differ; of one per CU where a long context makes all runs alike and that many still
+// cut it well.  A second round costs more than the shorter runs save, and every run costs the merge.  Launch and merge, us, runs that reached two
+// per CU / this rule: 1531 rows, 16 heads 37.4 (4) / 35.8 (2); 3500 rows 95.9 (2) / 92.3 (1); 800 rows at 1200 39.3 (8) / 33.4 (4);
+// 384 at 3201 33.8 (8) / 32.5 (5); 250 at 1750, 32 heads 29.4 (8) / 25.9 (4); 900 at 2800, 16 heads one per CU 56.0 (2), two 47.0 (4).
+static int flash_runs(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
+    long long n = cus / wgs;
+    if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
+    if (n > most) n = most;
+    if (n > ceil_div(kv_len, FL_BKV) / 4) n = ceil_div(kv_len, FL_BKV) / 4;
+    return n < 1 ? 1 : (int)n;
+}
+// with a sliding window: up to four runs over the `span` keys that the heaviest query tile walks, until two workgroups per CU are reached
+static int flash_window_runs(long long wgs, int span) {
     int n = 1;
-    while (n < most && wgs * n < 2LL * cus && ceil_div(span, FL_BKV) >= 4 * (n * 2)) n *= 2;
+    while (n < 4 && wgs * n < 2LL * flash_cus() && ceil_div(span, FL_BKV) >= 4 * (n * 2)) n *= 2;
     return n;
 }
 
@@ -503,7 +515,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
                                const FlashMany& many = FlashMany{}) {
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-    int nsplit = flash_runs((long long)tiles * hq, span, WIN ? 4 : 16);
+    int nsplit = WIN ? flash_window_runs((long long)tiles * hq, span) : flash_runs((long long)tiles * hq, q_len, kv_len, 16);
     const bool wide = many.items || q_len <= 128;
     if (nsplit > 1 && q_len <= 128) {      // up to 128 rows need no scratch memory to be captured
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

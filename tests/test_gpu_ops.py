@@ -718,6 +718,12 @@ def test_sdpa_few_rows_over_a_long_context(dt, cfg):
             assert rel_err(host(out), ref) < bar
 
 
+@pytest.mark.parametrize("cfg", [(32, 8, 600, 1500, 128), (16, 8, 384, 3585, 128), (12, 4, 300, 1900, 128), (18, 6, 257, 1300, 64), (33, 3, 100, 3000, 128)])
+def test_sdpa_runs_of_any_count(cfg):
+    """3, 5, 7, 4 and 7 runs on a card of 256 CUs: an uneven cut of the KV tiles, a merge whose last four runs are not all there."""
+    test_sdpa_few_rows_over_a_long_context("bfloat16", cfg)
+
+
 @pytest.mark.parametrize("ql", [128, 192])   # 128: first-generation kernel, 192: transposed-score kernel
 def test_sdpa_softmax_max_jump(ql):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
