@@ -25,6 +25,8 @@ pgk_status wsgemm_nt(const bf16* a, int lda, const void* w, const bf16* wscale, 
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
                            hipStream_t st, bool packed = false, const ActArgs* act = nullptr);
 pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed = false);
+bool gemm256_bf16_qkv_heads_ok(int M, int N, int K);
+pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed);
 bool gemm128s_shape_ok(int N, int K);
 bool gemm128s_ok(int M, int N, int K);    // ops_gemm256.hip: 128 x 128 tiles on the staged LDS-DMA pipeline (bf16, M > 128, K % 64 == 0, N % 8 == 0)
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
@@ -477,11 +479,14 @@ pgk_status engine_gemm_act_nt(const bf16* A, const bf16* W, bf16* act, int M, in
 }
 
 // internal (engine prefill, bf16 weights, head_dim 128): the QKV projection with per-head RMSNorm + RoPE + KV-cache write as its
-// epilogue (QkvHeadArgs) - on the 128-tile kernel, whose tile columns are whole heads; where engine_gemm_nt would pick the
-// 256-tile kernel the separate pass stays
-bool engine_gemm_qkv_heads_ok(int M, int N, int K) { return N % 128 == 0 && gemm128s_ok(M, N, K) && !use_gemm256(M, N, K); }
+// epilogue (QkvHeadArgs), on the kernels whose tile columns are whole heads: 128, or 256 for two; where engine_gemm_nt would pick
+// 192-column tiles the separate pass stays
+bool engine_gemm_qkv_heads_ok(int M, int N, int K) {
+    return use_gemm256(M, N, K) ? gemm256_bf16_qkv_heads_ok(M, N, K) : N % 128 == 0 && gemm128s_ok(M, N, K);
+}
 pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed) {
-    PGK_REQUIRE(engine_gemm_qkv_heads_ok(M, N, K), "engine_gemm_qkv_heads: M=%d N=%d K=%d outside the fused kernel's shapes", M, N, K);
+    PGK_REQUIRE(engine_gemm_qkv_heads_ok(M, N, K), "engine_gemm_qkv_heads: M=%d N=%d K=%d outside the fused kernels' shapes", M, N, K);
+    if (use_gemm256(M, N, K)) return gemm256_bf16_qkv_heads_nt(A, W, qkv, M, N, K, hd, st, packed);
     return gemm128s_bf16_nt(A, W, nullptr, qkv, 3, 1, M, N, K, st, &hd, packed);
 }
 

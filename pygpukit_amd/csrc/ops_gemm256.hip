@@ -166,9 +166,9 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
     }
 }
 
-// ---- QKV-heads epilogue (EPI 3): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
+// ---- QKV-heads epilogue (EPI 3 of the fp8 kernel, 5 of the bf16 one): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
 // g2_swiglu_epilogue), a tile = 256 token rows x two head slots, 16 consecutive lanes take one (row, head) and finish it
-// (qkv_head_finish: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
+// (qkv_heads_finish: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -183,15 +183,13 @@ __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g 
                 *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
             }
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 16; ++it) {
-        const int item = it * G2_THREADS + tid, row = item >> 5, c = item & 31, sw = ((row >> 2) & 3) << 5;
+    const int c = tid & 31;
+    qkv_heads_finish<16, 16>(c & 15, 2 * tn + (c >> 4), m0 + (tid >> 5), M, hd, qkv, N, [&](int i, float (&x)[8]) {
+        const int row = i * 16 + (tid >> 5), sw = ((row >> 2) & 3) << 5;
         Vec<bf16> raw;
         raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((c * 16) ^ sw));
-        float x[8];
         raw.to_float(x);
-        qkv_head_finish(x, c & 15, 2 * tn + (c >> 4), m0 + row, M, hd, qkv, N);
-    }
+    });
 }
 
 template <int EPI>   // 0: bf16 C store (+bias); 1: fp32 C +=
@@ -329,10 +327,12 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256_bf16_kernel(const bf16* A,
 // waves 4-7 one (rows 128-191), so the "two younger stages in flight" count is vmcnt(8) for the former, vmcnt(6) for the latter.
 constexpr int G2S_ARING = 6;      // slots of A, in stages
 constexpr size_t G2S_LDS = (G2S_ARING + 4) * (size_t)256 * 64;
-template <int EPI, int TN = 4>   // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store
+// EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store;
+// 5: QKV heads (QkvHeadArgs; a tile holds two head slots, N % 256 == 0).  Qwen3-0.6B, 3365 rows: 38 us and 14 of the separate pass -> 42.
+template <int EPI, int TN = 4>
 __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                    int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa = ActArgs{}) {
-    static_assert(TN == 4 || (TN == 3 && (EPI == 0 || EPI >= 2)), "192-column tiles: bf16 store and SwiGLU only");
+                                                                    int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa = ActArgs{}, QkvHeadArgs hd = QkvHeadArgs{}) {
+    static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -451,6 +451,10 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 
     if constexpr (EPI == 2) {
         g2_swiglu_epilogue<false, TN>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
+        return;
+    }
+    if constexpr (EPI == 5) {
+        g2_qkv_heads_epilogue(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
         return;
     }
     if constexpr (EPI == 1 && TN == 4) {
@@ -646,18 +650,16 @@ __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, cons
     } else if constexpr (EPI == 3) {
         // 16 consecutive lanes = one (token row, head): the arithmetic of qknorm_rope_kvwrite_kernel on the bf16-rounded row,
         // so the result is bit-identical to GEMM (bf16 store) + that kernel.  Tile column tn is the head slot.
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int item = it * G1_THREADS + tid, row = item >> 4, c = item & 15, sw = ((row >> 2) & 3) << 6;
+        const int c = tid & 15;
+        qkv_heads_finish<8, 16>(c, tn, m0 + (tid >> 4), M, hd, reinterpret_cast<bf16*>(Cv), N, [&](int i, float (&x)[8]) {
+            const int row = i * 16 + (tid >> 4), sw = ((row >> 2) & 3) << 6;
             const float4 v0 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32) ^ sw));
             const float4 v1 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32 + 16) ^ sw));
             const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             Vec<bf16> raw;
             raw.from_float(f);
-            float x[8];
             raw.to_float(x);
-            qkv_head_finish(x, c, tn, m0 + row, M, hd, reinterpret_cast<bf16*>(Cv), N);
-        }
+        });
     } else if constexpr (EPI == 6) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
@@ -1020,6 +1022,27 @@ pgk_status gemm256_fp8_swiglu_nt(const uint8_t* a, const float* sa, const uint8_
 }
 
 // bf16 NT on the 256^2 structure; caller guarantees K % 64 == 0 and 16-byte aligned rows
+// 192-column tiles when they fill the rounds of the chip better (cost = rounds x work per tile)
+static bool gemm256_narrow(int M, int N) {
+    const int ntm = ceil_div(M, G2_BM);
+    return N % 192 == 0 && 0.75 * ceil_div(ntm * (N / 192), 256) < (double)ceil_div(ntm * ceil_div(N, G2_BN), 256) - 0.01;
+}
+
+// QKV projection finished head by head: where whole 256-column tiles are what gemm256_bf16_nt would take
+bool gemm256_bf16_qkv_heads_ok(int M, int N, int K) { return K % 64 == 0 && K >= 64 && N % 256 == 0 && !gemm256_narrow(M, N); }
+pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed) {
+    PGK_REQUIRE(gemm256_bf16_qkv_heads_ok(M, N, K) && N == (hd.hq + 2 * hd.hkv) * 128, "gemm256 heads: N=%d K=%d (%d + 2 x %d heads)", N, K, hd.hq, hd.hkv);
+    static bool attr_done = false;
+    if (!attr_done) {
+        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<5>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)G2S_LDS));
+        attr_done = true;
+    }
+    const int ntm = ceil_div(M, G2_BM), ntn = N / G2_BN;
+    gemm256s_bf16_kernel<5><<<ntm * ntn, G2_THREADS, G2S_LDS, st>>>(A, W, nullptr, qkv, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, hd);
+    PGK_CHECK_HIP(hipGetLastError());
+    return PGK_OK;
+}
+
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
                            hipStream_t st, bool packed, const ActArgs* act) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64, "gemm256: K=%d must be a multiple of 64", K);
@@ -1040,10 +1063,8 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
             PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
             attr_s = true;
         }
-        // 192-column tiles when they fill the rounds of the chip better (cost = rounds x work per tile)
         const int ntn3 = N / 192;
-        const bool narrow = !accum_f32 && N % 192 == 0 &&
-                            0.75 * ceil_div(ntm * ntn3, 256) < (double)ceil_div(ntm * ntn, 256) - 0.01;
+        const bool narrow = !accum_f32 && gemm256_narrow(M, N);
         if (narrow) {
             static bool attr_n = false;
             if (!attr_n) {
@@ -1055,14 +1076,14 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
                 static bool attr_x[2] = {false, false};
                 if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
                 attr_x[act->gelu] = true;
-                kfn<<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn3, packed ? 1 : 0, *act);
+                kfn<<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn3, packed ? 1 : 0, *act, QkvHeadArgs{});
             } else gemm256s_bf16_kernel<0, 3><<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn3, packed ? 1 : 0, ActArgs{});
         } else if (act) {
             auto kfn = act->gelu ? &gemm256s_bf16_kernel<4> : &gemm256s_bf16_kernel<3>;
             static bool attr_x[2] = {false, false};
             if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
             attr_x[act->gelu] = true;
-            kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, *act);
+            kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, *act, QkvHeadArgs{});
         } else if (accum_f32) gemm256s_bf16_kernel<1><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{});
         else gemm256s_bf16_kernel<0><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{});
         PGK_CHECK_HIP(hipGetLastError());
