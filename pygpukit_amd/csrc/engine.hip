@@ -1528,6 +1528,27 @@ static hipError_t launch_attn_mfma(dim3 grid, hipStream_t st, const AttnArgs& a)
     return launch_k(attn_oproj_mfma_kernel<G, OPROJ>, grid, dim3(256), lds, st, a);
 }
 
+// Slices per sequence of m sequences' split attention on attn_stream_kernel, or 0 where that kernel does not take them (launch_attn says where).  At
+// least 128 positions each, enough for two workgroups per CU and none longer than 512: contexts of a batch differ, and its longest sequence must
+// not be what the launch waits for.  But one slice, and no merge, where that is one and a half workgroups per CU already and no
+// context exceeds 2048 (Qwen3-0.6B, four steps, ms, slices of 512 and one: 54 sequences of 890..1151 9.35 and 8.41, 64 of 60..1200 7.96 and 7.54,
+// 64 of 100..2000 10.15 and 9.80; 40 of 1350..1500, 1.25 workgroups per CU, 8.84 and 9.18, merged).
+static int attn_span(const Engine* e) { return (e->step_span > 0 && e->step_span < e->cfg.max_seq_len) ? e->step_span : e->cfg.max_seq_len; }
+static int stream_chunk(const Engine* e, int m) {
+    const int hkv = e->cfg.num_kv_heads, G = e->cfg.num_heads / hkv, span = attn_span(e);
+    if (m < 2 || G > AS_HEADS || (G <= 2 && (long long)m * hkv * ceil_div(span, 128) <= 2 * e->cu_count)) return 0;
+    if (2LL * m * hkv >= 3LL * e->cu_count && span <= 2048) return span;
+    int n = 2 * e->cu_count / (hkv * m);
+    n = n > ceil_div(span, 128) ? ceil_div(span, 128) : n;
+    n = n < ceil_div(span, 512) ? ceil_div(span, 512) : n;
+    n = n < 1 ? 1 : (n > e->nsplit ? e->nsplit : n);
+    return ceil_div(ceil_div(span, n), 128) * 128;
+}
+static int stream_slices(const Engine* e, int m) {
+    const int chunk = stream_chunk(e, m);
+    return chunk ? ceil_div(attn_span(e), chunk) : 0;
+}
+
 // `fused`: attention + o_proj partials in one kernel (one sequence at short context); `direct`: one workgroup per
 // (sequence, kv head) walks the whole (short) context and writes the normalised output - no merge launch; otherwise
 // split-KV slices, then `merged` (merge + o_proj partials in one launch) or the merge kernel.
@@ -1548,7 +1569,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
     a.kcache = e->kcache + lofs; a.vcache = e->vcache + lofs;
     a.positions = e->positions + b0;
     a.hq = c.num_heads; a.hkv = c.num_kv_heads; a.max_seq = c.max_seq_len;
-    const int span = (e->step_span > 0 && e->step_span < c.max_seq_len) ? e->step_span : c.max_seq_len;
+    const int span = attn_span(e);
     a.span = span;
     a.scale = 1.0f / sqrtf((float)D);
     a.part = e->part + (size_t)b0 * c.num_heads * e->nsplit * (D + 2);
@@ -1570,35 +1591,28 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         return launch_k(attn_merge_kernel<D>, dim3(c.num_heads, m), dim3(D), 0, st, (const float*)a.part, e->attnv + (size_t)b0 * c.num_heads * D,
                         direct_bf16 ? e->attnv16 + (size_t)b0 * c.num_heads * D : (bf16*)nullptr, (int)c.num_heads, (int)a.nsplit);
     };
-    if (direct) {
-        a.nsplit = 1;
-        a.attn_direct = e->attnv + (size_t)b0 * c.num_heads * D;
-        if (direct_bf16) a.attn_direct16 = e->attnv16 + (size_t)b0 * c.num_heads * D;
-    }
     // Batches stream through the matrix pipe (attn_stream.hip.h), except where one workgroup per (sequence, kv head) with the whole context
     // fits one round of the CUs, and where one or two query heads share a kv head and slices of 128 positions fit two: there the first bytes'
     // latency counts, and attn_decode_kernel requests them before it knows the position (Qwen3-0.6B, us per step, that kernel and this one:
     // 4 sequences of 1500 positions 937 and 984, 8 of 600 828 and 855; 12 of 1000 1301 and 1250; Llama-3-8B shape, four query heads, 6 of 1100
-    // 3434 and 3338).  Slices of at least 128 positions, enough for two workgroups per CU and none longer than 512: contexts of a batch differ,
-    // and its longest sequence must not be what the launch waits for.
+    // 3434 and 3338).
     const bool whole = direct && (G == 1 || G == 2 || G == 4) && m * (int)c.num_kv_heads <= e->cu_count;
-    const bool latency = !direct && G <= 2 && (long long)m * c.num_kv_heads * ceil_div(span, 128) <= 2 * e->cu_count;
-    if (m >= 2 && !fused && !merged && !whole && !latency && G <= AS_HEADS) {
+    const int chunk = direct || fused || merged ? 0 : stream_chunk(e, m);
+    const bool stream = m >= 2 && !fused && !merged && G <= AS_HEADS && (direct ? !whole : chunk > 0);
+    if (direct || chunk >= span) {
+        a.nsplit = 1;
+        a.attn_direct = e->attnv + (size_t)b0 * c.num_heads * D;
+        if (direct_bf16) a.attn_direct16 = e->attnv16 + (size_t)b0 * c.num_heads * D;
+    }
+    if (stream) {
         a.g_total = G;
-        int chunk = 0;
-        if (!direct) {
-            int n = 2 * e->cu_count / (c.num_kv_heads * m);
-            n = n > ceil_div(span, 128) ? ceil_div(span, 128) : n;
-            n = n < ceil_div(span, 512) ? ceil_div(span, 512) : n;
-            n = n < 1 ? 1 : (n > e->nsplit ? e->nsplit : n);
-            chunk = ceil_div(ceil_div(span, n), 128) * 128;
-            a.nsplit = ceil_div(span, chunk);
-        }
+        const bool one = direct || chunk >= span;
+        if (!one) a.nsplit = ceil_div(span, chunk);
         const dim3 g3(c.num_kv_heads, a.nsplit, m);
-        const hipError_t se = direct ? launch_k(attn_stream_kernel<D, true>, g3, dim3(256), as_lds<D>(G), st, a, chunk)
-                                     : launch_k(attn_stream_kernel<D, false>, g3, dim3(256), as_lds<D>(G), st, a, chunk);
+        const hipError_t se = one ? launch_k(attn_stream_kernel<D, true>, g3, dim3(256), as_lds<D>(G), st, a, chunk)
+                                  : launch_k(attn_stream_kernel<D, false>, g3, dim3(256), as_lds<D>(G), st, a, chunk);
         PGK_CHECK_HIP(se);
-        if (!direct) PGK_CHECK_HIP(merge());
+        if (!one) PGK_CHECK_HIP(merge());
         return PGK_OK;
     }
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
@@ -1697,7 +1711,7 @@ static pgk_status decode_chunk(Engine* e, int b0, bool last, hipStream_t st, int
             a.xin = e->attnv + (size_t)b0 * QD;
             a.res = h; a.out = h; a.ld_out = H;
             if (pgk_status r = launch_fused_auto<WT, XT, M, PRO_PLAIN, EPI_RESID>(a, H, st)) return r;
-            *launches += (direct ? 1 : 2) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;   // o_proj (+ the merge kernel unless attention normalised in place)
+            *launches += (direct || stream_slices(e, M) == 1 ? 1 : 2) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;   // o_proj (+ the merge kernel unless attention normalised in place)
         }
         // 4. act = silu(Wg x) * (Wu x), x = rmsnorm(h [+ sum of o_proj partials])
         mark(KC_GATEUP);
@@ -1809,7 +1823,7 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
         a.xin16 = e->act16 + (size_t)b0 * I;
         a.res = h; a.out = h; a.ld_out = H;
         if (pgk_status r = batched_proj(FP8, PRO_PLAIN, EPI_RESID, a, M, st)) return r;
-        *launches += (direct ? 5 : 6) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
+        *launches += (direct || stream_slices(e, M) == 1 ? 5 : 6) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
     }
     const int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
     mark(KC_LMHEAD);
@@ -1888,7 +1902,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
             mark(KC_DOWN);
             const bf16* gnext = l + 1 < c.num_layers ? (const bf16*)e->layers[l + 1].attn_norm : nullptr;
             if (pgk_status r = pkgemm_resid_nt(act16, I, P.down, h, M, H, I, gnext, x16, e->pk_ss, &ss_n, st)) return r;
-            *launches += (direct ? 5 : 6) + (l == 0 ? 1 : 0) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
+            *launches += (direct || stream_slices(e, M) == 1 ? 5 : 6) + (l == 0 ? 1 : 0) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
             continue;
         }
         if (pgk_status r = pkgemm_nt(attn16, QD, P.o, e->dec_slabs, H, PK_EPI_SLAB, s_o, M, H, QD, nullptr, st)) return r;
@@ -1899,7 +1913,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
         mark(KC_DOWN);
         if (pgk_status r = pkgemm_nt(act16, I, P.down, e->dec_slabs, H, PK_EPI_SLAB, s_d, M, H, I, nullptr, st)) return r;
         pending = s_d;
-        *launches += (direct ? 7 : 8) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
+        *launches += (direct || stream_slices(e, M) == 1 ? 7 : 8) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
     }
     const int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
     if (pgk_status r = norm(e->final_norm)) return r;     // also folds the last down_proj's slabs into the residual stream
@@ -1965,7 +1979,7 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
         a.w = L.w_down; a.wscale = (const bf16*)L.s_down; a.N = H; a.K = I;
         a.out = h; a.ld_out = H;
         if (pgk_status r = wide_proj(fp8, WIDE_PIECES, EPI_RESID, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
-        *launches += 4 + (direct ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads, M);
+        *launches += 4 + (direct || stream_slices(e, M) == 1 ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads, M);
     }
     mark(KC_LMHEAD);
     FusedArgs a{};
