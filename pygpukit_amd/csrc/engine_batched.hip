@@ -12,7 +12,7 @@ typedef __bf16 bf16x8_b __attribute__((ext_vector_type(8)));
 typedef float f32x4_b __attribute__((ext_vector_type(4)));
 #include "engine_batched.hip.h"
 
-// x16[m][:] = bf16(h[m][:] * rsqrt(mean(h[m]^2) + eps) * gamma)   (gamma == nullptr: plain fp32 -> bf16 rows)
+// x16[m][:] = bf16(h[m][:] * rsqrt(mean(h[m]^2) + eps) * gamma)
 // One 256-thread workgroup per row; rows up to 4096 columns stay in registers between the two passes.
 __global__ __launch_bounds__(256) void norm_rows_bf16_kernel(unsigned long long* tl, const float* h, const bf16* gamma, bf16* out, int K, float eps) {
     const TLStamp tls(tl);
@@ -35,18 +35,12 @@ __global__ __launch_bounds__(256) void norm_rows_bf16_kernel(unsigned long long*
         const float4 u = *reinterpret_cast<const float4*>(hr + i);
         ss += u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w;
     }
-    float inv = 1.0f;
-    if (gamma) {
-        ss = block_sum(ss, red);
-        inv = 1.0f / sqrtf(ss / K + eps);
-    }
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / K + eps);
     auto emit = [&](int i, const float4& u) {
-        float g0 = 1.f, g1 = 1.f, g2 = 1.f, g3 = 1.f;
-        if (gamma) {
-            const uint2 g = *reinterpret_cast<const uint2*>(gamma + i);
-            g0 = __uint_as_float(g.x << 16); g1 = __uint_as_float(g.x & 0xFFFF0000u);
-            g2 = __uint_as_float(g.y << 16); g3 = __uint_as_float(g.y & 0xFFFF0000u);
-        }
+        const uint2 g = *reinterpret_cast<const uint2*>(gamma + i);
+        const float g0 = __uint_as_float(g.x << 16), g1 = __uint_as_float(g.x & 0xFFFF0000u);
+        const float g2 = __uint_as_float(g.y << 16), g3 = __uint_as_float(g.y & 0xFFFF0000u);
         uint2 o;
         o.x = pack_bf16x2(u.x * inv * g0, u.y * inv * g1);
         o.y = pack_bf16x2(u.z * inv * g2, u.w * inv * g3);
@@ -63,7 +57,7 @@ __global__ __launch_bounds__(256) void norm_rows_bf16_kernel(unsigned long long*
 
 
 pgk_status norm_rows_bf16(const float* h, const bf16* gamma, bf16* x16, int M, int K, float eps, hipStream_t st) {
-    PGK_REQUIRE(h && x16 && M >= 1 && K >= 4 && K % 4 == 0, "norm_rows_bf16: bad arguments (M=%d, K=%d)", M, K);
+    PGK_REQUIRE(h && gamma && x16 && M >= 1 && K >= 4 && K % 4 == 0, "norm_rows_bf16: bad arguments (M=%d, K=%d)", M, K);
     PGK_CHECK_HIP(launch_k(norm_rows_bf16_kernel, dim3(M), dim3(256), 0, st, h, gamma, x16, K, eps));
     return PGK_OK;
 }
