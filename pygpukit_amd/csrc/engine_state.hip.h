@@ -161,11 +161,11 @@ struct Engine {
     int* amax_idx = nullptr;
     unsigned long long* clk_log = nullptr;
     size_t kv_bytes = 0, ws_bytes = 0;
-    // fragment-major copies of the layer weights for prompts of <= 128 tokens (ops_pkgemm.hip); PGK_PACKED_PREFILL=0: none
+    // fragment-major copies of the layer weights, for prompts (ops_pkgemm.hip, ops_gemm256.hip) and wide batches; PGK_PACKED_PREFILL=0: none
     struct PackedLayer { bf16 *qkv = nullptr, *o = nullptr, *gate_up = nullptr, *down = nullptr; };
     std::vector<PackedLayer> packed;
     bool packed_ok = false;     // the skinny-GEMM kernels of ops_pkgemm.hip can use the copy (their shape limits)
-    bool packed_have = false;   // the copy exists (w8a16 engines: also for shapes beyond those kernels - the long-prompt GEMMs read it)
+    bool packed_have = false;   // the copy exists: the staged GEMMs read it (w8a16 engines: also for shapes beyond the skinny-GEMM kernels)
     size_t packed_bytes = 0;
     bool packed_resid = false;      // o_proj / down_proj without K split, carrying the next RMSNorm (pkgemm_resid_nt); PGK_PACKED_RESID=0: split-K slabs + norm launches
     float* pk_ss = nullptr;         // its sum-of-squares table [128][PK_SS_LD]
