@@ -9,18 +9,20 @@
 //     before the activations are touched; a 16-row chunk passes through 4 KiB of the wave's own LDS (swizzled, no barrier) into the operand
 //     layout of v_mfma_f32_16x16x32_bf16.  Loading that layout directly would be 16 pieces of 64 bytes per instruction, which a CU's
 //     texture path takes three times as long for;
-//   * fp32 activations are split into bf16 pieces that take rows of the 16-row operand which few sequences leave free: three each for up to
-//     four sequences (24 bits, as the fp32 products they replace), two for up to eight; e4m3 weights are exact in bf16 and their block
-//     scales multiply fp32 sums;
+//   * fp32 activations are split into three bf16 pieces each (24 bits, as the fp32 products they replace), which take rows of the 16-row operand
+//     that few sequences leave free: all three for up to four sequences; for up to eight the first two, and the third are a second operand for
+//     the same weights (the matrix pipe has the time); e4m3 weights are exact in bf16 and their block scales multiply fp32 sums;
 //   * 1 / rms is a factor of the finished sums, so no wave waits for the row statistic.
 //
 // Measured on the Llama-3-8B shape, us per launch (before: the GEMV kernels; bf16 with 6 sequences took two launches, of 4 and of 2):
 //                 bytes (bf16)   bf16, 1 sequence   bf16, 6 sequences   e4m3, 1 sequence
-//     qkv              50 MB       19.4 -> 11.1         65.2 -> 13.0       19.1 ->  8.6
-//     o_proj           34 MB       (merged)  8.3        (merged)  9.0      (merged) 5.8
-//     gate/up         235 MB       82.7 -> 37.5        193.4 -> 38.3       67.2 -> 23.3
-//     down            117 MB       37.9 -> 20.0        107.9 -> 22.5       39.5 -> 12.9
-//     lm_head        1051 MB      171.2 -> 162.8       371.0 -> 168.6      (bf16)
+//     qkv              50 MB       19.4 -> 11.1         65.2 -> 12.3       19.1 ->  8.6
+//     o_proj           34 MB       (merged)  8.3        (merged)  8.9      (merged) 5.8
+//     gate/up         235 MB       82.7 -> 37.5        193.4 -> 38.1       67.2 -> 23.3
+//     down            117 MB       37.9 -> 20.0        107.9 -> 27.2       39.5 -> 12.9
+//     lm_head        1051 MB      171.2 -> 162.8       371.0 -> 169        (bf16)
+// (5..7 sequences: with two pieces, 16 bits, 12, 8.6, 37.7, 24.6 and 169; the pieces of down's input, read by every workgroup, are what six cost more
+// than one.)
 // i.e. 6.2 TB/s on gate/up and 6.4 on lm_head.  One step: 5.34 -> 3.05 ms, 15.3 -> 3.43 ms, 4.68 -> 2.10 ms (context 700, 1100, 700).
 
 #include "wide.hip.h"
@@ -56,10 +58,19 @@ __device__ __forceinline__ uint32_t widen2(uint32_t codes, bool hi) {
     return __builtin_bit_cast(uint32_t, r);
 }
 __device__ __forceinline__ uint4 widen8(uint32_t lo, uint32_t hi) { return make_uint4(widen2(lo, false), widen2(lo, true), widen2(hi, false), widen2(hi, true)); }
-// what a piece leaves of a value (an infinity is one piece)
+// The pieces of a value are its leading bits, cut off: three hold all 24 of them, and a value beyond the largest bf16 does not become an
+// infinity.  What the first piece leaves of a value (an infinity is one piece; what the others leave is a plain difference):
 __device__ __forceinline__ float rest(float v, float piece) { const float d = v - piece; return d == d ? d : 0.f; }
+__device__ __forceinline__ uint32_t cut2(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
 // LDS of one wave: its lanes write and read in program order, the compiler must keep that order
 __device__ __forceinline__ void wave_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
+
+// LDS bytes of a wave: 16 operand rows of `rs` bytes on their way to registers, afterwards two chunks of weights and, with eight sequence slots, the
+// third pieces of a row each (rs = 0: the operands come from memory)
+constexpr int wide_scratch(int rs, int mt) {
+    const int rows = 16 * rs, body = 8192 + (mt == 8 ? 8 * rs : 0);
+    return rows > body ? rows : body;
+}
 
 // where element k of a row lies among the pieces: 32-k block, quarter, position (e4m3: a lane's 16 codes are two steps of 8)
 template <bool FP8> __device__ __forceinline__ void piece_of(int k, int& blk, int& q, int& j) {
@@ -76,10 +87,13 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     const TLStamp tls(tl);
     constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value, REG = SRC != WIDE_PIECES;
     constexpr int KCH = 256 / sizeof(WT), STEPS = KCH / 32;      // k and matrix steps of a chunk
-    constexpr int NS = MT < 8 ? 3 : 2, SS = MT < 8 ? 4 : 8;      // pieces; operand rows s * SS + m
+    constexpr int NS = 3, SS = MT < 8 ? 4 : 8;                   // pieces; operand rows s * SS + m
+    // The third pieces of eight rows are an operand of their own: rows m those of an even step, rows 8 + m those of the step after it, and only
+    // the products with the weights of the same step count
+    constexpr bool TWO = MT == 8;
     constexpr int RD = REG || !FP8 ? 4 : 2;                              // chunks in flight per wave
     constexpr int SL = REG ? CH * KCH : 0, RS = SL * 2 + 16;     // k slice of a wave; LDS row of its pieces (16 bytes on: rows start in different banks)
-    constexpr int SCRATCH = (REG && 16 * RS > 8192) ? 16 * RS : 8192;
+    constexpr int SCRATCH = wide_scratch(REG ? RS : 0, MT);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, n16 = lane & 15;
     char* scratch = smem + wid * SCRATCH;
@@ -116,7 +130,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
 
     // ---- weight loads ----
     uint4 rb[RD][4];
-    uint4 ra[REG ? 1 : RD][REG ? 1 : STEPS];
+    uint4 ra[REG ? 1 : RD][REG ? 1 : STEPS], rc[REG || !TWO ? 1 : RD][REG || !TWO ? 1 : STEPS / 2];  // first pieces, third ones
     uint32_t sc0[FP8 ? RD : 1], sc1[FP8 ? RD : 1];
     const int am = (n16 & (SS - 1)) < MT ? (n16 & (SS - 1)) : 0, as = (n16 / SS) < NS ? n16 / SS : 0;   // this lane's operand row: sequence slot, piece
     // Rows come in groups of 8 (N and `rows` are multiples of 8): a half tile beyond the workgroup's rows reads the other half again.
@@ -126,7 +140,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
         else return r0 + t * 16 + (t * 16 + 8 * h < nr ? 8 * h : 0);
     };
     const uint32_t w_lane = (uint32_t)q * K * sizeof(WT) + n16 * 16;
-    const uint32_t p_lane = (((am * NS + as) * 4 + q) * 8) * 2;
+    const int pm = min(am, M - 1), p_step = M * NS * 64;         // (slots without a sequence read the last one's pieces again)
+    const uint32_t p_lane = (((pm * NS + as) * 4 + q) * 8) * 2, p_third = (((pm * NS + 2) * 4 + q) * 8) * 2 + (n16 >> 3) * p_step;
     int lt = 0, lj = 0;                                          // tile and chunk of the next load
     auto issue_weights = [&](int u) {
         const int ch = REG ? min(c0 + lj, nch - 1) : c0 + lj;
@@ -144,9 +159,13 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     };
     auto issue_pieces = [&](int u) {
         if constexpr (!REG) {
-            const char* base = reinterpret_cast<const char*>(a.pieces_in) + (size_t)(c0 + lj) * STEPS * MT * NS * 64;
+            const char* base = reinterpret_cast<const char*>(a.pieces_in) + (size_t)(c0 + lj) * STEPS * p_step;
 #pragma unroll
-            for (int s = 0; s < STEPS; ++s) ra[u][s] = *reinterpret_cast<const uint4*>(base + s * MT * NS * 64 + p_lane);
+            for (int s = 0; s < STEPS; ++s) ra[u][s] = *reinterpret_cast<const uint4*>(base + s * p_step + p_lane);
+            if constexpr (TWO) {
+#pragma unroll
+                for (int s = 0; s < STEPS; s += 2) rc[u][s / 2] = *reinterpret_cast<const uint4*>(base + s * p_step + p_third);
+            }
             if (++lj == ncw) { lj = 0; ++lt; }
         }
     };
@@ -157,9 +176,12 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
 
     // ---- activations -> pieces -> operands in registers ----
     uint4 A[REG ? CH * STEPS : 1];
+    char* third = scratch + 8192;                                // [8 sequences][RS], behind the weights' chunks
     if constexpr (REG) {
+        uint2 p3[TWO ? MT : 1][XI];
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
+            if (MT > 1 && m >= M) break;                         // (uniform) rows nobody reads the sums of
             float ss = 0.f;
 #pragma unroll
             for (int i = 0; i < XI; ++i) {
@@ -172,10 +194,12 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
                 }
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                    const uint32_t p0 = pack_bf16x2(v[0], v[1]), p1 = pack_bf16x2(v[2], v[3]);
+                    const uint32_t p0 = cut2(v[0], v[1]), p1 = cut2(v[2], v[3]);
+                    if (TWO && s == 2) { p3[TWO ? m : 0][i] = make_uint2(p0, p1); continue; }
                     *reinterpret_cast<uint2*>(scratch + (s * SS + m) * RS + (i * 256 + lane * 4) * 2) = make_uint2(p0, p1);
-                    v[0] = rest(v[0], __uint_as_float(p0 << 16)); v[1] = rest(v[1], __uint_as_float(p0 & 0xFFFF0000u));
-                    v[2] = rest(v[2], __uint_as_float(p1 << 16)); v[3] = rest(v[3], __uint_as_float(p1 & 0xFFFF0000u));
+                    const float p[4] = {__uint_as_float(p0 << 16), __uint_as_float(p0 & 0xFFFF0000u), __uint_as_float(p1 << 16), __uint_as_float(p1 & 0xFFFF0000u)};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = s == 0 ? rest(v[e], p[e]) : v[e] - p[e];
                 }
             }
             if constexpr (SRC == WIDE_NORM) {
@@ -193,10 +217,17 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
                 A[j * STEPS + s] = *reinterpret_cast<const uint4*>(mine + k * 2);
             }
         wave_order();
+        if constexpr (TWO) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int i = 0; i < XI; ++i) if (m < M) *reinterpret_cast<uint2*>(third + m * RS + (i * 256 + lane * 4) * 2) = p3[m][i];
+        }
     }
+    const char* third_row = third + (REG && TWO ? am * RS + (FP8 ? q * 16 + (n16 >> 3) * 8 : (n16 >> 3) * 32 + q * 8) * 2 : 0);
 
     // ---- body ----
-    f32x4_w acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4_w acc = {0.f, 0.f, 0.f, 0.f}, acc3[2] = {acc, acc};             // acc3: TWO's products, even and odd steps
     int ct = 0, cj = 0, base_t = 0;                              // tile and chunk being multiplied; first tile of the reduction group
     float best_v = -INFINITY;
     int best_i = 0x7FFFFFFF;
@@ -206,10 +237,11 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
         for (int r = 0; r < 4; ++r) {
             float v = acc[r];
             if constexpr (MT < 8) { v = q < 3 ? v : 0.f; v += __shfl_xor(v, 16, 64); }
+            if constexpr (TWO) v += q < 2 ? acc3[0][r] : acc3[1][r];
             v += __shfl_xor(v, 32, 64);
             if (MT < 8 ? (q == 0 && r < MT) : q < 2) dst[((MT < 8 ? 0 : q * 4) + r) * 16 + n16] = v;
         }
-        acc = f32x4_w{0.f, 0.f, 0.f, 0.f};
+        acc = acc3[0] = acc3[1] = f32x4_w{0.f, 0.f, 0.f, 0.f};
     };
     auto reduce = [&](int nt) {                                  // tiles [base_t, base_t + nt): sum the waves, epilogue
         __syncthreads();
@@ -232,12 +264,12 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
                     float v = y / (1.0f + __expf(-y)) * (y2 * inv);
                     int blk, pq, pj;
                     piece_of<FP8>(n, blk, pq, pj);
-                    bf16* dst = a.pieces_out + ((((size_t)blk * MT + em) * NS) * 4 + pq) * 8 + pj;
+                    bf16* dst = a.pieces_out + ((((size_t)blk * M + em) * NS) * 4 + pq) * 8 + pj;
 #pragma unroll
                     for (int s = 0; s < NS; ++s) {
-                        const uint16_t p = f_to_bf16_bits(v);
+                        const uint16_t p = (uint16_t)(__float_as_uint(v) >> 16);
                         dst[s * 32] = bf16{p};
-                        v = rest(v, bf16_bits_to_f(p));
+                        v = s == 0 ? rest(v, bf16_bits_to_f(p)) : v - bf16_bits_to_f(p);
                     }
                 } else if constexpr (EPI == EPI_RESID) {
                     float* o = a.out + (size_t)em * a.ld_out + n;
@@ -255,6 +287,10 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
 #pragma unroll
         for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(s4 + (i * 4 + q) * 256 + ((n16 ^ (i * 4 + q)) * 16)) = rb[u][i];
         auto af = [&](int s) -> const uint4& { return REG ? A[REG ? opnd * STEPS + s : 0] : ra[REG ? 0 : u][REG ? 0 : s]; };
+        auto cf = [&](int s) -> uint4 {                          // third pieces of steps s and s + 1
+            if constexpr (!REG) return rc[TWO ? u : 0][TWO ? s / 2 : 0];
+            else return *reinterpret_cast<const uint4*>(third_row + (opnd * KCH + s * 32) * 2);
+        };
         uint32_t w0 = 0, w1 = 0;
         if constexpr (FP8) { w0 = sc0[u]; w1 = sc1[u]; }
         if (more) issue_weights(u);
@@ -266,20 +302,38 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
         if constexpr (FP8) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {                        // a 128-k scale block
-                f32x4_w p = {0.f, 0.f, 0.f, 0.f};
+                f32x4_w p = {0.f, 0.f, 0.f, 0.f}, p3[2] = {p, p};
 #pragma unroll
                 for (int b = 2 * h; b < 2 * h + 2; ++b) {
-                    p = mfma_w(af(2 * b), widen8(f[b].x, f[b].y), p);
-                    p = mfma_w(af(2 * b + 1), widen8(f[b].z, f[b].w), p);
+                    const uint4 lo = widen8(f[b].x, f[b].y), hi = widen8(f[b].z, f[b].w);
+                    p = mfma_w(af(2 * b), lo, p);
+                    p = mfma_w(af(2 * b + 1), hi, p);
+                    if constexpr (TWO) {
+                        const uint4 c = cf(2 * b);
+                        p3[0] = mfma_w(c, lo, p3[0]);
+                        p3[1] = mfma_w(c, hi, p3[1]);
+                    }
                 }
                 const uint32_t w = n16 < 8 ? w0 : w1;
                 const float sc = h ? __uint_as_float(w & 0xFFFF0000u) : __uint_as_float(w << 16);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[r] = fmaf(sc, p[r], acc[r]);
+                if constexpr (TWO) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) { acc3[0][r] = fmaf(sc, p3[0][r], acc3[0][r]); acc3[1][r] = fmaf(sc, p3[1][r], acc3[1][r]); }
+                }
             }
         } else {
 #pragma unroll
-            for (int b = 0; b < 4; ++b) acc = mfma_w(af(b), f[b], acc);
+            for (int b = 0; b < 4; b += 2) {
+                acc = mfma_w(af(b), f[b], acc);
+                acc = mfma_w(af(b + 1), f[b + 1], acc);
+                if constexpr (TWO) {
+                    const uint4 c = cf(b);
+                    acc3[0] = mfma_w(c, f[b], acc3[0]);
+                    acc3[1] = mfma_w(c, f[b + 1], acc3[1]);
+                }
+            }
         }
         if (more) issue_pieces(u);
         __builtin_amdgcn_sched_barrier(0);                       // keep the next chunk's LDS traffic out of this one: registers
@@ -324,7 +378,7 @@ template <class WT, int SRC, int EPI, int CH, int MT>
 pgk_status launch_wide(const FusedArgs& a, bf16* pieces, int M, int cu_count, int* n_blk, hipStream_t st) {
     constexpr int KCH = 256 / sizeof(WT);
     constexpr int RS = CH * KCH * 2 + 16;
-    constexpr int SCRATCH = (SRC != WIDE_PIECES && 16 * RS > 8192) ? 16 * RS : 8192;
+    constexpr int SCRATCH = wide_scratch(SRC != WIDE_PIECES ? RS : 0, MT);
     constexpr int LDS = WD_WAVES * SCRATCH + WD_TILES * WD_RED * 4;
     static_assert(LDS + 512 <= 160 * 1024, "wide_kernel: LDS");
     auto kfn = &wide_kernel<WT, SRC, EPI, CH, MT>;

@@ -9,9 +9,8 @@ namespace pgk {
 // where the activations come from: fp32 rows normalised on the way in, plain fp32 rows, or the split pieces a SwiGLU epilogue left
 enum { WIDE_NORM = 0, WIDE_PLAIN, WIDE_PIECES };
 
-// Split pieces of M rows of K: [K / 32][MT][NS][4][8] bf16, MT = 1, 4 or 8 row slots, NS = 3 (MT < 8) or 2 pieces each
-inline int wide_slots(int M) { return M == 1 ? 1 : M <= 4 ? 4 : 8; }
-inline size_t wide_pieces_elems(int K, int M) { const int mt = wide_slots(M); return (size_t)(K / 32) * mt * (mt < 8 ? 3 : 2) * 32; }
+// Split pieces of M rows of K: [K / 32][M][3][4][8] bf16, three pieces each
+inline size_t wide_pieces_elems(int K, int M) { return (size_t)K * M * 3; }
 
 // x rows in registers: K <= 4096; pieces: any K; both: K % 256 == 0
 bool wide_proj_ok(int N, int K, bool pieces);
