@@ -440,7 +440,9 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const float w = s0 + u < nsplit && r[u].y > 0.f ? r[u].y * __builtin_amdgcn_exp2f(r[u].x - mstar) : 0.f;
+            // a run that saw no key has l = 0; any other counts, also one whose l is NaN (asked by its bits: no NaN is honoured in this file's comparisons)
+            const bool live = s0 + u < nsplit && __float_as_uint(r[u].y) != 0u;
+            const float w = live ? r[u].y * __builtin_amdgcn_exp2f(r[u].x - mstar) : 0.f;
             float f[8];
             if constexpr (sizeof(P) == 4) {
 #pragma unroll
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
                 t.to_float(f);
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = w > 0.f ? fmaf(w, f[j], acc[j]) : acc[j];
+            for (int j = 0; j < 8; ++j) acc[j] = live ? fmaf(w, f[j], acc[j]) : acc[j];
             den += w;
         }
     }

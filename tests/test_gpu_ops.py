@@ -718,6 +718,31 @@ def test_sdpa_few_rows_over_a_long_context(dt, cfg):
             assert rel_err(host(out), ref) < bar
 
 
+@pytest.mark.parametrize("cfg", [(8, 2, 42, 1142, 128), (4, 4, 128, 700, 64), (4, 2, 200, 2100, 128), (2, 2, 300, 306, 64)])
+def test_sdpa_nan_and_infinite_keys(cfg):
+    """A NaN in a key makes every row that sees it NaN, also where the context is cut into runs of which one holds it; a score of +infinity too
+    (inf - inf), one of -infinity takes the key out.  The other key heads are what they were.  Bar: the merge test's."""
+    hq, hkv, ql, kl, d = cfg
+    rng = np.random.default_rng(kl)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((hq, ql, d), (hkv, kl, d), (hkv, kl, d)))
+    qd, vd = dev(q, "bfloat16"), dev(v, "bfloat16")
+    qr, vr = rounded(q, "bfloat16").astype(np.float64), np.repeat(rounded(v, "bfloat16"), hq // hkv, axis=0).astype(np.float64)
+    at, rep = 5, hq // hkv                              # a position that every row sees
+    for bad in (np.nan, np.inf):
+        kb = rounded(k, "bfloat16")
+        kb[0, at, 3] = bad
+        got = host(ops.sdpa_causal(qd, dev(kb, "bfloat16"), vd))
+        with np.errstate(invalid="ignore"):
+            sc = qr @ np.repeat(kb, rep, axis=0).astype(np.float64).transpose(0, 2, 1) / np.sqrt(d)
+            sc[:, np.arange(kl)[None, :] > (kl - ql + np.arange(ql))[:, None]] = -np.inf
+            p = np.exp(sc - sc.max(axis=-1, keepdims=True))
+            ref = (p / p.sum(axis=-1, keepdims=True)) @ vr
+        lost = np.isnan(ref)
+        assert lost[:rep].any() and not lost[rep:].any() and lost[:rep].all() == np.isnan(bad)
+        np.testing.assert_array_equal(np.isnan(got), lost)
+        assert rel_err(got[~lost], ref[~lost]) < 2.0**-8
+
+
 @pytest.mark.parametrize("cfg", [(32, 8, 600, 1500, 128), (16, 8, 384, 3585, 128), (12, 4, 300, 1900, 128), (18, 6, 257, 1300, 64), (33, 3, 100, 3000, 128)])
 def test_sdpa_runs_of_any_count(cfg):
     """3, 5, 7, 4 and 7 runs on a card of 256 CUs: an uneven cut of the KV tiles, a merge whose last four runs are not all there."""
