@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256, 3) void attn_stream_kernel(unsigned long long*
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run, mx);
+        const float m_new = fmaxf(m_run, mx), m_use = m_new == -INFINITY ? 0.f : m_new;      // (a NaN is no maximum, but makes its probability NaN)
         const float alpha = m_new == -INFINITY ? 1.f : __expf(m_run - m_new);
         float ls = 0.f;
         uint32_t pk[4];
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256, 3) void attn_stream_kernel(unsigned long long*
         for (int t = 0; t < 2; ++t) {
             float p[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) p[r] = m_new == -INFINITY ? 0.f : __expf(s[t][r] - m_new);
+            for (int r = 0; r < 4; ++r) p[r] = __expf(s[t][r] - m_use);
             pk[2 * t] = pack_bf16x2(p[0], p[1]);
             pk[2 * t + 1] = pack_bf16x2(p[2], p[3]);
             // the sum runs over the rounded probabilities: numerator and denominator see the same weights
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, 3) void attn_stream_kernel(unsigned long long*
             den += wg;
         }
         if constexpr (DIRECT) {
-            const float y = den > 0.f ? num / den : 0.f;
+            const float y = den != 0.f ? num / den : 0.f;
             const size_t at = ((size_t)b * a.hq + (size_t)kvh * G) * D + e;
             if (a.attn_direct16) a.attn_direct16[at] = from_f<bf16>(y);
             else a.attn_direct[at] = y;
