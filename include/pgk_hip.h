@@ -20,7 +20,7 @@
  *     (pgk_stream_set_current; default: one library-owned stream per device).  Ops
  *     never synchronise; only D2H copies, pgk_stream_sync and pgk_device_sync do.
  *     (The reference syncs after every op, native/ops/common/error.cuh:28-37.)
- *   - ops never allocate; callers pass outputs and workspaces.  Safe to capture.
+ *   - callers pass outputs and workspaces.  Where an op needs scratch memory of its own it comes from the pool (pgk_malloc).  Safe to capture.
  */
 #ifndef PGK_HIP_H
 #define PGK_HIP_H

@@ -527,11 +527,11 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     void* ws = nullptr;
     if (nsplit > 1) {
         const size_t po_bytes = (size_t)nsplit * q_len * hq * D * (wide ? 4 : sizeof(T)), ml_bytes = (size_t)nsplit * hq * q_len * 2 * sizeof(float);
-        if (pgk_malloc(&ws, po_bytes + ml_bytes + 256) == PGK_OK) {
+        if (pool_malloc_on(&ws, po_bytes + ml_bytes + 256, st) == PGK_OK) {
             sp.o = ws;
             sp.ml = (float*)((char*)ws + ((po_bytes + 255) & ~(size_t)255));
         } else {
-            nsplit = sp.nsplit = 1;        // slower, and right
+            nsplit = sp.nsplit = 1;        // no memory, or a stream whose end the pool cannot see: slower, and right
         }
     }
     constexpr size_t LDS = 4 * (size_t)(64 * D * 2);
@@ -551,7 +551,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
         else flash_merge_kernel<T, T, D><<<grid, 256, 0, st>>>(sp.ml, (const T*)sp.o, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win);
         e = hipGetLastError();
     }
-    if (ws) pgk_free(ws);   // stream-ordered reuse: later work on this stream runs after the kernels above
+    if (ws) pgk_free(ws);   // st's again: whatever takes it runs after the kernels above
     PGK_CHECK_HIP(e);
     return PGK_OK;
 }

@@ -17,6 +17,11 @@ int set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3
 // NULL -> the calling thread's current stream (default: the device's library stream).
 hipStream_t resolve_stream(pgk_stream s);
 
+// pgk_malloc for the scratch of kernels on `st`, which need not be the current stream: the block is st's, so that pgk_free right behind the launches
+// gives it to work that runs after them.  Refused where the pool can neither tell when st has drained nor would the current stream's order do
+// (a stream this library did not create, and not the current one).
+pgk_status pool_malloc_on(void** ptr, size_t nbytes, hipStream_t st);
+
 inline size_t dtype_size(pgk_dtype dt) {
     switch (dt) {
         case PGK_F64: case PGK_I64: return 8;

@@ -108,6 +108,76 @@ static size_t size_class(size_t n) {
     return (n + g - 1) / g * g;
 }
 
+static pgk_status malloc_owned(void** ptr, size_t nbytes, hipStream_t owner) {
+    *ptr = nullptr;
+    int dev = 0;
+    PGK_CHECK_HIP(hipGetDevice(&dev));
+    const size_t cls = size_class(nbytes ? nbytes : 1);
+    Pool& P = pool();
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        P.st.n_alloc++;
+        auto take = [&](std::vector<void*>& list) {
+            void* p = list.back();
+            list.pop_back();
+            P.live[p] = Block{dev, cls, owner, g_capture_id};
+            P.st.n_pool_hit++;
+            P.st.bytes_cached -= cls;
+            P.st.bytes_in_use += cls;
+            *ptr = p;
+        };
+        auto it = P.free_lists.find({dev, cls, owner});
+        if (it != P.free_lists.end() && !it->second.empty()) { take(it->second); return PGK_OK; }
+        // another stream's cached block of this class: only once that stream has drained (never while capturing: a
+        // query on a capturing stream is an error, and the answer would say nothing about replays)
+        // key stream == nullptr: blocks whose owner was destroyed (after a sync) - free for anyone
+        if (g_capture_id == 0) {
+            for (auto lo = P.free_lists.lower_bound({dev, cls, nullptr}); lo != P.free_lists.end(); ++lo) {
+                if (std::get<0>(lo->first) != dev || std::get<1>(lo->first) != cls) break;
+                if (lo->second.empty()) continue;
+                hipStream_t os = std::get<2>(lo->first);
+                if (os != nullptr) {
+                    if (!P.streams.count(os)) continue;                     // not ours to query
+                    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+                    if (hipStreamIsCapturing(os, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) { (void)hipGetLastError(); continue; }
+                    if (hipStreamQuery(os) != hipSuccess) { (void)hipGetLastError(); continue; }
+                }
+                take(lo->second);
+                return PGK_OK;
+            }
+        }
+    }
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, cls);
+    if (e != hipSuccess) {
+        // Out of memory: give cached blocks back to the driver and retry once.
+        (void)hipGetLastError();
+        pgk_pool_trim();
+        e = hipMalloc(&p, cls);
+    }
+    if (e != hipSuccess)
+        return set_error(PGK_ERR_HIP, "pgk_malloc(%zu bytes): %s", nbytes, hipGetErrorString(e));
+    std::lock_guard<std::mutex> lk(P.mu);
+    P.live[p] = Block{dev, cls, owner, g_capture_id};
+    P.st.n_device_malloc++;
+    P.st.bytes_in_use += cls;
+    P.reserved += cls;
+    if (P.reserved > P.st.bytes_reserved_peak) P.st.bytes_reserved_peak = P.reserved;
+    *ptr = p;
+    return PGK_OK;
+}
+
+pgk_status pool_malloc_on(void** ptr, size_t nbytes, hipStream_t st) {
+    bool ours = st == resolve_stream(nullptr);
+    if (!ours) {
+        Pool& P = pool();
+        std::lock_guard<std::mutex> lk(P.mu);
+        ours = P.streams.count(st) != 0;
+    }
+    if (!ours) return set_error(PGK_ERR_UNSUPPORTED, "scratch memory on a stream that is neither current nor this library's");
+    return malloc_owned(ptr, nbytes, st);
+}
+
 template <class T>
 __global__ void fill_kernel(T* p, T v, size_t n) {
     size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
@@ -166,63 +236,7 @@ pgk_status pgk_mem_info(size_t* free_bytes, size_t* total_bytes) {
 // ------------------------------------------------------------------------------ memory ----
 pgk_status pgk_malloc(void** ptr, size_t nbytes) {
     PGK_REQUIRE(ptr, "pgk_malloc: null output");
-    *ptr = nullptr;
-    int dev = 0;
-    PGK_CHECK_HIP(hipGetDevice(&dev));
-    const size_t cls = size_class(nbytes ? nbytes : 1);
-    hipStream_t owner = resolve_stream(nullptr);
-    Pool& P = pool();
-    {
-        std::lock_guard<std::mutex> lk(P.mu);
-        P.st.n_alloc++;
-        auto take = [&](std::vector<void*>& list) {
-            void* p = list.back();
-            list.pop_back();
-            P.live[p] = Block{dev, cls, owner, g_capture_id};
-            P.st.n_pool_hit++;
-            P.st.bytes_cached -= cls;
-            P.st.bytes_in_use += cls;
-            *ptr = p;
-        };
-        auto it = P.free_lists.find({dev, cls, owner});
-        if (it != P.free_lists.end() && !it->second.empty()) { take(it->second); return PGK_OK; }
-        // another stream's cached block of this class: only once that stream has drained (never while capturing: a
-        // query on a capturing stream is an error, and the answer would say nothing about replays)
-        // key stream == nullptr: blocks whose owner was destroyed (after a sync) - free for anyone
-        if (g_capture_id == 0) {
-            for (auto lo = P.free_lists.lower_bound({dev, cls, nullptr}); lo != P.free_lists.end(); ++lo) {
-                if (std::get<0>(lo->first) != dev || std::get<1>(lo->first) != cls) break;
-                if (lo->second.empty()) continue;
-                hipStream_t os = std::get<2>(lo->first);
-                if (os != nullptr) {
-                    if (!P.streams.count(os)) continue;                     // not ours to query
-                    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-                    if (hipStreamIsCapturing(os, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) { (void)hipGetLastError(); continue; }
-                    if (hipStreamQuery(os) != hipSuccess) { (void)hipGetLastError(); continue; }
-                }
-                take(lo->second);
-                return PGK_OK;
-            }
-        }
-    }
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, cls);
-    if (e != hipSuccess) {
-        // Out of memory: give cached blocks back to the driver and retry once.
-        (void)hipGetLastError();
-        pgk_pool_trim();
-        e = hipMalloc(&p, cls);
-    }
-    if (e != hipSuccess)
-        return set_error(PGK_ERR_HIP, "pgk_malloc(%zu bytes): %s", nbytes, hipGetErrorString(e));
-    std::lock_guard<std::mutex> lk(P.mu);
-    P.live[p] = Block{dev, cls, owner, g_capture_id};
-    P.st.n_device_malloc++;
-    P.st.bytes_in_use += cls;
-    P.reserved += cls;
-    if (P.reserved > P.st.bytes_reserved_peak) P.st.bytes_reserved_peak = P.reserved;
-    *ptr = p;
-    return PGK_OK;
+    return malloc_owned(ptr, nbytes, resolve_stream(nullptr));
 }
 
 pgk_status pgk_free(void* ptr) {

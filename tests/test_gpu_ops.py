@@ -749,6 +749,43 @@ def test_sdpa_runs_of_any_count(cfg):
     test_sdpa_few_rows_over_a_long_context("bfloat16", cfg)
 
 
+@pytest.mark.parametrize("ql", [42, 200])
+def test_sdpa_scratch_belongs_to_the_stream_the_call_names(ql):
+    """A call on an explicit stream, other than the current one: its partial rows are not handed to the current stream while the kernels that
+    use them are still queued (the stream has tens of milliseconds of work in front of them)."""
+    from pygpukit_amd import _hip
+    from pygpukit_amd.core.stream import Stream
+
+    b, st = pk.get_backend(), Stream()
+    hq, hkv, kl, d = 8, 2, 2142, 128
+    rng = np.random.default_rng(ql)
+    q, k, v = (dev(rng.standard_normal(s).astype(np.float32), "bfloat16") for s in ((hq, ql, d), (hkv, kl, d), (hkv, kl, d)))
+    big = [dev(np.zeros((n, 4096, d), np.float32), "bfloat16") for n in (32, 8, 8, 32)]
+    out = dev(np.zeros((hq, ql, d), np.float32), "bfloat16")
+
+    def on(stream, q, k, v, o):
+        (hq, ql, d), (hkv, kl, _) = q.shape, k.shape
+        _hip.call("pgk_sdpa_causal", q._p, k._p, v._p, o._p, hq, hkv, ql, kl, d, 0.0, ql * d, d, kl * d, d, ql * d, d, q.dtype.code, stream)
+
+    want = host(ops.sdpa_causal(q, k, v))
+    _hip.call("pgk_device_sync")
+    b.pool_trim()
+    for _ in range(200):
+        on(st.handle, *big)                             # one run each: no scratch
+    s0 = b.pool_stats()
+    on(st.handle, q, k, v, out)
+    s1 = b.pool_stats()
+    scratch = s1["bytes_cached"] - s0["bytes_cached"]
+    other = pk.zeros((scratch // 4,), "float32")
+    s2 = b.pool_stats()
+    assert s1["n_device_malloc"] == s0["n_device_malloc"] + 1 and scratch > 0
+    assert s2["n_pool_hit"] == s1["n_pool_hit"] and s2["n_device_malloc"] == s1["n_device_malloc"] + 1
+    st.synchronize()
+    np.testing.assert_array_equal(host(out), want)
+    del other
+    st.destroy()
+
+
 @pytest.mark.parametrize("ql", [128, 192])   # 128: first-generation kernel, 192: transposed-score kernel
 def test_sdpa_softmax_max_jump(ql):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
