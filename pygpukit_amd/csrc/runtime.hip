@@ -155,8 +155,10 @@ static pgk_status malloc_owned(void** ptr, size_t nbytes, hipStream_t owner) {
         pgk_pool_trim();
         e = hipMalloc(&p, cls);
     }
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();      // reported here, and not again by the next launch: callers go on with less
         return set_error(PGK_ERR_HIP, "pgk_malloc(%zu bytes): %s", nbytes, hipGetErrorString(e));
+    }
     std::lock_guard<std::mutex> lk(P.mu);
     P.live[p] = Block{dev, cls, owner, g_capture_id};
     P.st.n_device_malloc++;

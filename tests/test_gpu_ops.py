@@ -102,6 +102,18 @@ def test_device_is_mi355x_and_pool_works():
     assert s1["n_pool_hit"] >= s0["n_pool_hit"] + 1
 
 
+def test_a_refused_allocation_is_not_the_next_launchs_error():
+    """The call that asked for more than the card has raises; operators after it run (their launches ask for the last error)."""
+    from pygpukit_amd import _hip
+    import ctypes as C
+
+    a = dev(np.arange(8, dtype=np.float32))
+    p = C.c_void_p()
+    with pytest.raises(RuntimeError, match="pgk_malloc"):
+        _hip.call("pgk_malloc", C.byref(p), 1 << 50)
+    np.testing.assert_array_equal(host(ops.add(a, a)), 2 * np.arange(8, dtype=np.float32))
+
+
 def test_roundtrip_and_views():
     x = np.arange(24, dtype=np.float32).reshape(4, 6)
     a = from_numpy(x)
