@@ -2118,6 +2118,8 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         if (e->pf) PGK_CHECK_HIP(hipStreamSynchronize(st));
         if (e->pf) pgk_free(e->pf);
         e->pf = nullptr;
+        e->pf_bytes = 0;              // (a smaller prompt after a refusal must ask again)
+        if (need > e->pf_most) return set_error(PGK_ERR_HIP, "pgk_engine_prefill: %d rows need %zu bytes of workspace, PGK_PREFILL_MEM allows %zu", n, need, e->pf_most);
         if (pgk_status r = pgk_malloc(&e->pf, need)) return r;
         e->pf_bytes = need;
     }
@@ -2564,6 +2566,7 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
         // Costs the layers' bytes again; skipped when that is more than a quarter of the device's free memory.
         const int QDp = c.num_heads * D, NQ = e->qkv_dim(), I = c.intermediate_size;
         const char* ep = getenv("PGK_PACKED_PREFILL");
+        if (const char* em = getenv("PGK_PREFILL_MEM")) e->pf_most = (size_t)atoll(em) << 20;
         const size_t per_layer = ((size_t)NQ * H + (size_t)H * QDp + (size_t)2 * I * H + (size_t)H * I) * 2;
         size_t free_b = 0, total_b = 0;
         const bool fits = hipMemGetInfo(&free_b, &total_b) == hipSuccess && per_layer * c.num_layers < free_b / 4;

@@ -2,6 +2,7 @@
 // engine_stack.hip: layer lists).  The C entry points that do not depend on the kind are in engine_api.hip.
 #pragma once
 
+#include <cstdint>
 #include <cstdlib>
 #include <type_traits>
 #include <vector>
@@ -174,7 +175,7 @@ struct Engine {
     bool packed_decode = false;
     // prefill workspace (grown on demand, outside capture)
     void* pf = nullptr;
-    size_t pf_bytes = 0;
+    size_t pf_bytes = 0, pf_most = SIZE_MAX;   // PGK_PREFILL_MEM=MiB: more than that is refused, as memory that is not there would be
     int32_t* pf_tokens = nullptr;
     int pf_tokens_cap = 0;
     // captured step: [0] the long-context launch sequence, [1] the short-context one (when the engine has both)
