@@ -2058,8 +2058,9 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* x, const i
 
 // One pass over the weights for the prompt rows of one or several sequences (h_tokens: their rows one behind the other).  all_logits: bf16 logits
 // of every row (one sequence only).  h_want, n_want: row indices whose fp32 logits go to h_logits, the last rows of the sequences h_want_slots.
+// no_room: set where the pass failed because its workspace was refused, before anything was enqueued.
 static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slots, const int32_t* h_lens, const int32_t* h_starts, const int32_t* h_tokens, void* all_logits,
-                                     int n_want, const int32_t* h_want, const int32_t* h_want_slots, float* h_logits, hipStream_t st) {
+                                     int n_want, const int32_t* h_want, const int32_t* h_want_slots, float* h_logits, hipStream_t st, bool* no_room = nullptr) {
     const auto& c = e->cfg;
     int n = 0, n_items = 0, longest = 0;
     for (int i = 0; i < n_seqs; ++i) {
@@ -2119,9 +2120,11 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         if (e->pf) pgk_free(e->pf);
         e->pf = nullptr;
         e->pf_bytes = 0;              // (a smaller prompt after a refusal must ask again)
+        if (no_room) *no_room = true;
         if (need > e->pf_most) return set_error(PGK_ERR_HIP, "pgk_engine_prefill: %d rows need %zu bytes of workspace, PGK_PREFILL_MEM allows %zu", n, need, e->pf_most);
         if (pgk_status r = pgk_malloc(&e->pf, need)) return r;
         e->pf_bytes = need;
+        if (no_room) *no_room = false;
     }
     // one upload: token ids | (position, slot) of every row | attention tiles | wanted rows  (the last three for several sequences)
     const int at_off = (n + 3) & ~3, item_off = at_off + ((2 * n + 3) & ~3), want_off = item_off + 4 * n_items, meta = many ? want_off + n_want : n;
@@ -2392,9 +2395,9 @@ static pgk_status dense_prefill(Engine* e, int seq, const int32_t* h_tokens, int
 }
 
 // Sequences share passes over the weights, up to PREFILL_ROWS rows each (one longer prompt: a pass of its own), which is past what a pass needs to
-// be bound by its products and bounds the scratch memory; only the logits of a sequence's last row.  Sixteen prompts of 20..400 tokens on
-// Qwen3-0.6B: 31.4 -> 5.7 ms (6.3 before the staged GEMMs fetched whole lines).  fp8 x fp8 engines keep a sequence to a pass: there a prompt's length decides whether its activations are rounded
-// to e4m3.
+// be bound by its products and bounds the scratch memory (fewer rows, down to a sequence, where that memory is not there); only the logits of a
+// sequence's last row.  Sixteen prompts of 20..400 tokens on Qwen3-0.6B: 31.4 -> 5.7 ms (6.3 before the staged GEMMs fetched whole lines).  fp8 x
+// fp8 engines keep a sequence to a pass: there a prompt's length decides whether its activations are rounded to e4m3.
 constexpr int PREFILL_ROWS = 8192;
 static pgk_status dense_prefill_batch(Engine* e, int n_seqs, const int32_t* h_slots, const int32_t* h_lens, const int32_t* h_starts, const int32_t* h_tokens,
                                       int n_want, const int32_t* h_want, float* h_logits, hipStream_t st) {
@@ -2406,6 +2409,7 @@ static pgk_status dense_prefill_batch(Engine* e, int n_seqs, const int32_t* h_sl
     }
     PGK_REQUIRE(w == n_want, "pgk_engine_prefill_batch: wanted rows must be ascending last rows");
     std::vector<int32_t> want, slots;
+    int most = PREFILL_ROWS;
     row0 = w = 0;
     for (int i0 = 0; i0 < n_seqs;) {
         int i = i0, rows = 0;
@@ -2415,10 +2419,14 @@ static pgk_status dense_prefill_batch(Engine* e, int n_seqs, const int32_t* h_sl
             rows += h_lens[i];
             if (w + (int)want.size() < n_want && h_want[w + want.size()] == row0 + rows - 1) { want.push_back(rows - 1); slots.push_back(h_slots[i]); }
             ++i;
-        } while (i < n_seqs && e->cfg.weight_format != 2 && rows + h_lens[i] <= PREFILL_ROWS && e->cfg.max_batch <= FLASH_MOST_SLOTS);
+        } while (i < n_seqs && e->cfg.weight_format != 2 && rows + h_lens[i] <= most && e->cfg.max_batch <= FLASH_MOST_SLOTS);
+        bool no_room = false;
         if (pgk_status r = dense_prefill_rows(e, i - i0, h_slots + i0, h_lens + i0, h_starts + i0, h_tokens + row0, nullptr, (int)want.size(), want.data(), slots.data(),
-                                              h_logits + (size_t)w * e->cfg.vocab_size, st))
-            return r;
+                                              h_logits + (size_t)w * e->cfg.vocab_size, st, &no_room)) {
+            if (!no_room || i - i0 == 1) return r;
+            most = rows / 2;                               // the same sequences again, fewer to a pass
+            continue;
+        }
         w += (int)want.size();
         row0 += rows;
         i0 = i;
