@@ -2536,14 +2536,16 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
     A((void**)&e->act, (size_t)B * c.intermediate_size * 4, &e->ws_bytes);
     A((void**)&e->logits, (size_t)B * c.vocab_size * 4, &e->ws_bytes);
     e->lm_cap = e->lm_blocks > ceil_div(c.vocab_size, 16) ? e->lm_blocks : ceil_div(c.vocab_size, 16);   // per-sequence argmax partial slots
+    bool gemv_only = false;
     {
         const char* ev = getenv("PGK_BATCHED_MFMA");
+        gemv_only = ev && atoi(ev) == 0;
         e->batched_min = (ev && atoi(ev) == 2) ? 3 : 5;   // 2: from 3 up
         // every projection's K must suit the MFMA decode kernels: K = 128 S with S in {8, 16, 24, 32} (activation
         // fragments in registers) or an LDS image of K x 16 bf16 that fits (K <= 4096); Llama-3-8B's down_proj
         // (K = 14336) does neither, so such models decode batches in GEMV chunks of 8 / 4 / 2 / 1
         auto k_ok = [](int K) { return K % 128 == 0 && K <= 4096; };
-        e->batched_mfma = !(ev && atoi(ev) == 0) && k_ok(c.hidden_size) && k_ok(c.intermediate_size) && k_ok(c.num_heads * c.head_dim);
+        e->batched_mfma = !gemv_only && k_ok(c.hidden_size) && k_ok(c.intermediate_size) && k_ok(c.num_heads * c.head_dim);
         // 17..64 sequences in one weight pass (batched_mt_kernel) need K = 128 S with S instantiated; otherwise chunks of 16
         auto k_tiled = [](int K) { const int s = K / 128; return K % 128 == 0 && (s == 2 || s == 4 || s == 8 || s == 16 || s == 24 || s == 32); };
         e->batched_max = (k_tiled(c.hidden_size) && k_tiled(c.intermediate_size) && k_tiled(c.num_heads * c.head_dim)) ? 64 : 16;
@@ -2561,7 +2563,7 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
         const int I = c.intermediate_size, QD = c.num_heads * D, NQ = e->qkv_dim(), nw = f8 ? 16 : 8;
         auto fixed = [&](int N, int K) { return K % (64 * nw) == 0 && K / (64 * nw) <= (N >= 4096 ? 3 : 6); };
         const bool ok = wide_proj_ok(NQ, H, false) && wide_proj_ok(H, QD, false) && wide_proj_ok(I, H, false) && wide_proj_ok(H, I, true) && wide_proj_ok(c.vocab_size, H, false) &&
-                        (size_t)I * 8 <= 156 * 1024 && wide_aligned(e);
+                        (size_t)I * 8 <= 156 * 1024 && wide_aligned(e) && !gemv_only;
         const bool all_fixed = fixed(NQ, H) && fixed(H, QD) && fixed(I, H) && fixed(H, I);
         if (ok) e->wide = 0xE8 | (H >= 1536 || !all_fixed ? 0x10 : 0) | (H >= 1536 && !all_fixed ? 0x06 : 0);
     }
