@@ -1529,8 +1529,8 @@ static hipError_t launch_attn_mfma(dim3 grid, hipStream_t st, const AttnArgs& a)
 }
 
 // Slices per sequence of m sequences' split attention on attn_stream_kernel, or 0 where that kernel does not take them (launch_attn says where).  At
-// least 128 positions each, enough for two workgroups per CU and none longer than 512: contexts of a batch differ, and its longest sequence must
-// not be what the launch waits for.  But one slice, and no merge, where that is one and a half workgroups per CU already and no
+// least 128 positions each, enough for two workgroups per CU and none longer than 512 (as far as the records go, 64 slices: beyond
+// 32768 positions longer): contexts of a batch differ, and its longest sequence must not be what the launch waits for.  But one slice, and no merge, where that is one and a half workgroups per CU already and no
 // context exceeds 2048 (Qwen3-0.6B, four steps, ms, slices of 512 and one: 54 sequences of 890..1151 9.35 and 8.41, 64 of 60..1200 7.96 and 7.54,
 // 64 of 100..2000 10.15 and 9.80; 40 of 1350..1500, 1.25 workgroups per CU, 8.84 and 9.18, merged).
 static int attn_span(const Engine* e) { return (e->step_span > 0 && e->step_span < e->cfg.max_seq_len) ? e->step_span : e->cfg.max_seq_len; }
@@ -1595,7 +1595,10 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
     // fits one round of the CUs, and where one or two query heads share a kv head and slices of 128 positions fit two: there the first bytes'
     // latency counts, and attn_decode_kernel requests them before it knows the position (Qwen3-0.6B, us per step, that kernel and this one:
     // 4 sequences of 1500 positions 937 and 984, 8 of 600 828 and 855; 12 of 1000 1301 and 1250; Llama-3-8B shape, four query heads, 6 of 1100
-    // 3434 and 3338).
+    // 3434 and 3338).  Whole contexts beyond one round of the CUs (Qwen3-0.6B, 64 sequences of the same context, that kernel and this one: 60 positions
+    // 1078 and 1057, 100 1118 and 1097, 130 1138 and 1149, 190 1200 and 1206, 250 1308 and 1271, 500 1621 and 1585; 48 of 130 1109 and 1121): a
+    // group that starts a wave's second trip costs 0.4 us a layer, so between 129 and about 220 positions that kernel is up to 1 % faster.
+    // It is not taken there: it reads 128 rows whatever the context, so the largest position, all that is known here, does not say.
     const bool whole = direct && (G == 1 || G == 2 || G == 4) && m * (int)c.num_kv_heads <= e->cu_count;
     const int chunk = direct || fused || merged ? 0 : stream_chunk(e, m);
     const bool stream = m >= 2 && !fused && !merged && G <= AS_HEADS && (direct ? !whole : chunk > 0);
@@ -1799,7 +1802,6 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
         mark(KC_OPROJ);
         a = FusedArgs{};
         a.w = L.w_o; a.wscale = (const bf16*)L.s_o; a.N = H; a.K = QD;
-        a.xin = e->attnv + (size_t)b0 * QD;
         a.xin16 = e->attnv16 + (size_t)b0 * QD;               // attention left bf16 rows
         a.res = h; a.out = h; a.ld_out = H;
         if (pgk_status r = batched_proj(FP8, PRO_PLAIN, EPI_RESID, a, M, st)) return r;
@@ -1819,7 +1821,6 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
         mark(KC_DOWN);
         a = FusedArgs{};
         a.w = L.w_down; a.wscale = (const bf16*)L.s_down; a.N = H; a.K = I;
-        a.xin = e->act + (size_t)b0 * I;
         a.xin16 = e->act16 + (size_t)b0 * I;
         a.res = h; a.out = h; a.ld_out = H;
         if (pgk_status r = batched_proj(FP8, PRO_PLAIN, EPI_RESID, a, M, st)) return r;
@@ -2047,12 +2048,12 @@ static pgk_status decode_step(Engine* e, int batch, hipStream_t st, int* launche
     return decode_step_impl<bf16>(e, batch, st, launches, short_ctx);
 }
 
-// out[i] = the rows `want` of x, as they are and in fp32
+// The rows `want` of x, as they are (out) or in fp32 (out32)
 __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* x, const int32_t* want, bf16* out, float* out32, int H) {
     const bf16* row = x + (size_t)want[blockIdx.x] * H;
     for (int i = threadIdx.x; i < H; i += 256) {
-        out[(size_t)blockIdx.x * H + i] = row[i];
-        out32[(size_t)blockIdx.x * H + i] = to_f(row[i]);
+        if (out) out[(size_t)blockIdx.x * H + i] = row[i];
+        else out32[(size_t)blockIdx.x * H + i] = to_f(row[i]);
     }
 }
 
@@ -2355,7 +2356,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     if (many && in_order && (mfma || wide) && NQKV + QD + 3 * I >= H) {
         float* lg = e->logits + h_want_slots[0] * V;
         bf16* rows16 = qkv;                       // free by now: [n_want][H], n_want <= n
-        gather_rows_kernel<<<n_want, 256, 0, st>>>(x, e->pf_tokens + want_off, rows16, h32, H);
+        gather_rows_kernel<<<n_want, 256, 0, st>>>(x, e->pf_tokens + want_off, mfma ? rows16 : (bf16*)nullptr, h32, H);
         PGK_LAUNCH_CHECK();
         const int most = mfma ? e->batched_max : 8, nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
         for (int i = 0; i < n_want; i += most) {
@@ -2364,7 +2365,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             a.w = e->lm_head; a.N = c.vocab_size; a.K = H;
             a.out = lg + i * V; a.ld_out = c.vocab_size;
             if (mfma) {
-                a.xin = h32 + (size_t)i * H; a.xin16 = rows16 + (size_t)i * H; a.wp = e->packed_lm;
+                a.xin16 = rows16 + (size_t)i * H; a.wp = e->packed_lm;
                 a.amax_val = e->amax_val; a.amax_idx = e->amax_idx;
                 if (pgk_status r = batched_proj(false, PRO_PLAIN, EPI_LOGITS, a, m, st, nblk)) return r;
             } else {

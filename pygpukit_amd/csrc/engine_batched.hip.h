@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void batched_mfma_kernel(unsigned long long* t
     // Rows are unrolled to MP with clamped addresses and masked use (a runtime row loop would index registers
     // dynamically and wait per load); chunk loops have a uniform trip count for the same reason.
     const int nchunk = K >> 3;
-    const float* src = (PRO == PRO_NORM) ? a.h : a.xin;
+    const float* src = a.h;
     if constexpr (PRO == PRO_NORM) {
         float ss[MP];
 #pragma unroll
@@ -85,41 +85,35 @@ __global__ __launch_bounds__(256) void batched_mfma_kernel(unsigned long long* t
     }
     for (int c0 = 0; c0 < nchunk; c0 += 256) {
         const int c = min(c0 + tid, nchunk - 1);
-        float g[8];
         if constexpr (PRO == PRO_NORM) {
             Vec<bf16> gr;
             gr.load(a.gamma + c * 8);
+            float g[8];
             gr.to_float(g);
-        }
-        if constexpr (PRO != PRO_NORM) {
-            if (a.xin16) {                                  // bf16 hand-off: copy the stored chunks into the image
+            float4 v0[MP], v1[MP];
 #pragma unroll
-                for (int m = 0; m < MP; ++m) {
-                    uint4 raw = *reinterpret_cast<const uint4*>(a.xin16 + (size_t)min(m, M - 1) * K + c * 8);
-                    if (m >= M) raw = make_uint4(0, 0, 0, 0);
-                    *reinterpret_cast<uint4*>(smem + ((size_t)c * MP + m) * 16) = raw;
-                }
-                continue;
+            for (int m = 0; m < MP; ++m) {
+                v0[m] = *reinterpret_cast<const float4*>(src + (size_t)min(m, M - 1) * K + c * 8);
+                v1[m] = *reinterpret_cast<const float4*>(src + (size_t)min(m, M - 1) * K + c * 8 + 4);
             }
-        }
-        float4 v0[MP], v1[MP];
 #pragma unroll
-        for (int m = 0; m < MP; ++m) {
-            v0[m] = *reinterpret_cast<const float4*>(src + (size_t)min(m, M - 1) * K + c * 8);
-            v1[m] = *reinterpret_cast<const float4*>(src + (size_t)min(m, M - 1) * K + c * 8 + 4);
-        }
-#pragma unroll
-        for (int m = 0; m < MP; ++m) {
-            float f[8] = {v0[m].x, v0[m].y, v0[m].z, v0[m].w, v1[m].x, v1[m].y, v1[m].z, v1[m].w};
-            if constexpr (PRO == PRO_NORM) {
+            for (int m = 0; m < MP; ++m) {
+                float f[8] = {v0[m].x, v0[m].y, v0[m].z, v0[m].w, v1[m].x, v1[m].y, v1[m].z, v1[m].w};
                 const float inv = 1.0f / sqrtf((s_ss[0][m] + s_ss[1][m] + s_ss[2][m] + s_ss[3][m]) / K + a.eps);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) f[j] = f[j] * inv * g[j];
+                Vec<bf16> o;
+                o.from_float(f);
+                if (m >= M) o.raw = make_uint4(0, 0, 0, 0);     // unused rows of the image are zero
+                *reinterpret_cast<uint4*>(smem + ((size_t)c * MP + m) * 16) = o.raw;   // (duplicate writes of the clamped tail chunk are identical)
             }
-            Vec<bf16> o;
-            o.from_float(f);
-            if (m >= M) o.raw = make_uint4(0, 0, 0, 0);     // unused rows of the image are zero
-            *reinterpret_cast<uint4*>(smem + ((size_t)c * MP + m) * 16) = o.raw;   // (duplicate writes of the clamped tail chunk are identical)
+        } else {                                            // bf16 hand-off: copy the stored chunks into the image
+#pragma unroll
+            for (int m = 0; m < MP; ++m) {
+                uint4 raw = *reinterpret_cast<const uint4*>(a.xin16 + (size_t)min(m, M - 1) * K + c * 8);
+                if (m >= M) raw = make_uint4(0, 0, 0, 0);
+                *reinterpret_cast<uint4*>(smem + ((size_t)c * MP + m) * 16) = raw;
+            }
         }
     }
     __syncthreads();
@@ -241,7 +235,7 @@ template <class WT, int PRO, int EPI, int S, int RPG>
 __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl, const void* w_, const bf16* wp_, const float* x_, const bf16* gamma_,
                                                           int N_, int K_, int M, int nblk_logits, FusedArgs a) {
     // the first 14 dwords of the arguments - everything the load-issue phase needs - arrive preloaded in SGPRs (see fused_gemv_kernel,
-    // engine.hip): w_ / wp_ = FusedArgs::w / wp, x_ = the fp32 input rows (h for the norm prologue, xin otherwise), gamma_, N_, K_
+    // engine.hip): w_ / wp_ = FusedArgs::w / wp, x_ = the fp32 input rows of the norm prologue (h), gamma_, N_, K_
     const TLStamp tls(tl);
     constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value;
     constexpr int NT = (EPI == EPI_SWIGLU) ? 2 : 1;
@@ -343,17 +337,10 @@ __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl
                 af[s] = pack8(u, v, inv, g);
             }
         }
-    } else if (a.xin16) {                                  // bf16 hand-off: the fragment is the stored 16-byte chunk
+    } else {                                               // bf16 hand-off: the fragment is the stored 16-byte chunk
         const bf16* src16 = a.xin16 + (size_t)min(l15, M - 1) * K + kw0 + 8 * q;
 #pragma unroll
         for (int s = 0; s < S; ++s) af[s] = *reinterpret_cast<const uint4*>(src16 + s * 32);
-    } else {
-        const float one[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const float4 u = *reinterpret_cast<const float4*>(src + s * 32), v = *reinterpret_cast<const float4*>(src + s * 32 + 4);
-            af[s] = pack8(u, v, 1.0f, one);
-        }
     }
     if (l15 >= M) {
 #pragma unroll
@@ -662,7 +649,7 @@ static pgk_status launch_batched_reg(const FusedArgs& a, int M, hipStream_t st, 
     // enough workgroups to pull HBM bandwidth: fewer weight rows per workgroup when N / 16 would leave CUs idle
     int rpg = (EPI == EPI_LOGITS || ceil_div(a.N, 16) >= 192) ? 16 : (ceil_div(a.N, 8) >= 192 ? 8 : 4);
     const int grid = (EPI == EPI_LOGITS) ? nblk_logits : ceil_div(a.N, rpg);
-    const float* x = (PRO == PRO_NORM) ? a.h : a.xin;
+    const float* x = a.h;
     hipError_t he;
     if (rpg == 16) he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, 16>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
     else if (rpg == 8) he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, 8>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
@@ -686,6 +673,7 @@ static pgk_status launch_batched_s(const FusedArgs& a, int M, int steps, int gri
 template <class WT, int PRO, int EPI>
 static pgk_status launch_batched(const FusedArgs& a, int M, hipStream_t st, int nblk_logits = 0) {
     PGK_REQUIRE(a.K % 128 == 0 && M >= 1 && M <= 16, "batched decode projection: K=%d must be a multiple of 128 and M=%d in [1,16]", a.K, M);
+    PGK_REQUIRE(PRO == PRO_NORM ? a.h != nullptr : a.xin16 != nullptr, "batched decode projection: no input rows");
     const int steps = a.K / 128, ngroups = ceil_div(a.N, 16);
     // register-resident activations at the instantiated widths; the LDS-image kernel below for every other K
     if (steps == 8) return launch_batched_reg<WT, PRO, EPI, 8>(a, M, st, nblk_logits);

@@ -115,7 +115,7 @@ struct FusedArgs {
     const float* h;       // PRO_NORM / PRO_NORM_SUM: [M][K] residual stream
     const bf16* gamma;
     float eps;
-    const float* xin;     // PRO_PLAIN: [M][K]
+    const float* xin;     // PRO_PLAIN: [M][K] (GEMV and wide kernels)
     const float* part;    // PRO_NORM_SUM: [M][n_part][K]
     int nsplit;           // PRO_NORM_SUM: number of partial vectors to add
     float* h_out;         // PRO_NORM_SUM: workgroup 0 stores h + sum(part) here ([M][K])
@@ -126,14 +126,13 @@ struct FusedArgs {
     int* amax_idx;
     // batched MFMA path only: bf16 hand-off between projections (the consumer rounds to bf16 anyway, so the producer
     // does it once and every consuming workgroup reads half the bytes)
-    const bf16* xin16;    // PRO_PLAIN: [M][K] bf16, used instead of xin when set
+    const bf16* xin16;    // PRO_PLAIN: [M][K] bf16
     bf16* out16;          // EPI_SWIGLU: [M][ld_out] bf16, written instead of out when set
 };
 
 // engine_batched.hip: projections for 3..64 sequences on MFMA.  `pro`/`epi` are the codes above; `fp8` selects e4m3
-// weights with 128x128 bf16 block scales.  M <= 16 accepts PRO_NORM (RMSNorm fused) or PRO_PLAIN; 17 <= M <= 64 takes
-// PRO_PLAIN with a.xin16 set (rows already normalised to bf16 by norm_rows_bf16) and reads each weight byte ONCE for
-// all M rows.
+// weights with 128x128 bf16 block scales.  M <= 16 accepts PRO_NORM (RMSNorm fused) or PRO_PLAIN (bf16 rows, a.xin16);
+// 17 <= M <= 64 takes PRO_PLAIN (rows normalised by norm_rows_bf16) and reads each weight byte ONCE for all M rows.
 pgk_status batched_proj(bool fp8, int pro, int epi, const FusedArgs& a, int M, hipStream_t st, int nblk_logits = 0);
 // x16[m][:] = bf16(rmsnorm(h[m][:]) * gamma): one workgroup per row
 pgk_status norm_rows_bf16(const float* h, const bf16* gamma, bf16* x16, int M, int K, float eps, hipStream_t st);

@@ -9,7 +9,7 @@ namespace pgk {
 struct FlashItem { int row0, q_len, kv_len, slot_tile; };       // slot_tile: slot << 16 | query tile
 
 constexpr int FLASH_ITEM_ROWS = 128;                            // query rows of a tile
-constexpr int FLASH_MOST_SLOTS = 1 << 15, FLASH_MOST_TILES = 1 << 16;
+constexpr int FLASH_MOST_SLOTS = 1 << 15;                       // (a tile of several sequences' rows is at most a pass's rows / 128)
 
 // items: room for sum(ceil(lens / FLASH_ITEM_ROWS)); returns how many, the heaviest first
 int flash_items(FlashItem* items, const int* lens, const int* starts, const int* slots, int n);

@@ -1021,7 +1021,6 @@ pgk_status gemm256_fp8_swiglu_nt(const uint8_t* a, const float* sa, const uint8_
     return PGK_OK;
 }
 
-// bf16 NT on the 256^2 structure; caller guarantees K % 64 == 0 and 16-byte aligned rows
 // 192-column tiles when they fill the rounds of the chip better (cost = rounds x work per tile)
 static bool gemm256_narrow(int M, int N) {
     const int ntm = ceil_div(M, G2_BM);
@@ -1043,6 +1042,7 @@ pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, in
     return PGK_OK;
 }
 
+// bf16 NT on the 256^2 structure; caller guarantees K % 64 == 0 and 16-byte aligned rows
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
                            hipStream_t st, bool packed, const ActArgs* act) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64, "gemm256: K=%d must be a multiple of 64", K);
