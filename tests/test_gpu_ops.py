@@ -798,7 +798,27 @@ def test_sdpa_scratch_belongs_to_the_stream_the_call_names(ql):
     st.destroy()
 
 
-@pytest.mark.parametrize("ql", [128, 192])   # 128: first-generation kernel, 192: transposed-score kernel
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(4, 2, 1, 129, 128), (4, 2, 70, 300, 64), (6, 3, 128, 641, 128), (2, 1, 200, 200, 64), (2, 2, 40, 100, 64)])
+def test_sdpa_rows_that_only_the_first_kernel_stores(dt, cfg):
+    """Output rows that are not whole groups of four elements apart stay on flash_prefill_kernel at every length (64-row tiles, a loop over the
+    context): several turns of its loop, ragged ends, the diagonal inside a tile.  Same roundings as the other kernel, uncut: p and the output;
+    bar twice that of test_sdpa_few_rows_over_a_long_context's two."""
+    from pygpukit_amd.ops.nn.attention import sdpa_causal_strided
+
+    hq, hkv, ql, kl, d = cfg
+    rng = np.random.default_rng(kl)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((hq, ql, d), (hkv, kl, d), (hkv, kl, d)))
+    qr, kr, vr = rounded(q, dt), rounded(k, dt), rounded(v, dt)
+    ref = O.sdpa_causal(qr.astype(np.float64), np.repeat(kr, hq // hkv, axis=0), np.repeat(vr, hq // hkv, axis=0))
+    out = dev(np.full((hq, ql, d + 2), 7.0, np.float32), dt)
+    sdpa_causal_strided(dev(q, dt), dev(k, dt), dev(v, dt), out, hq, hkv, ql, kl, d, (ql * d, d), (kl * d, d), (ql * (d + 2), d + 2))
+    got = host(out)
+    assert rel_err(got[..., :d], ref) < 2 * (2.0**-9 if dt == "bfloat16" else 2.0**-12)
+    assert (got[..., d:] == 7.0).all()
+
+
+@pytest.mark.parametrize("ql", [128, 192])   # 128: the whole context in one tile (attn_short_kernel), 192: transposed-score kernel
 def test_sdpa_softmax_max_jump(ql):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
     rng = np.random.default_rng(11)
