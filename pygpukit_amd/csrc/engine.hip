@@ -2555,7 +2555,7 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
     {
         // How many sequences decode on ops_wide.hip, one pass over the weights (us per step before -> after, 8 layers, bf16 unless said):
         //   * 3, 5, 6, 7, where the batch kernels of engine_batched.hip do not take the model: the GEMV kernels pass over the weights two or
-        //     three times (width 2048, 7 sequences: 2012 -> 409; Llama-3-8B shape, 6: 15300 -> 3430);
+        //     three times (width 2048, feed-forward 8192, 7 sequences: 2147 -> 436; Llama-3-8B shape, 6: 15300 -> 3430);
         //   * 4 from width 1536 on, or where a row is not among the GEMV kernels' compile-time lengths (width 2048 e4m3 405 -> 355, 1536 691 ->
         //     455, 1024 with such a row 362 -> 318; but Qwen3-0.6B, all lengths fixed: 771 against 980 here);
         //   * 1 and 2 where both hold (Llama-3-8B shape 5340 -> 3080; 1536: 416 -> 411; 1024: 254 against 277 here).

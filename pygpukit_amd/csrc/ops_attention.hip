@@ -450,7 +450,8 @@ static pgk_status sdpa_dispatch(const void* q, const void* k, const void* v, voi
         // second generation: 128-row query tiles, transposed-score orientation (ops_flash.hip).  Few rows over a long context
         // too, since it cuts the context into runs (prompt pieces, whole model: Llama-3-8B shape, 100 rows at position 1800:
         // 11.1 -> 7.8 ms; Qwen3-0.6B, 42 rows at position 100: 1.38 -> 1.21 ms, 120 at 3000: 7.1 -> 1.7 ms); the
-        // first-generation kernel keeps what attn_short_kernel does not take of contexts up to 128
+        // first-generation kernel keeps what attn_short_kernel does not take of contexts up to 128, and outputs whose rows are not whole
+        // groups of four elements apart
         const bool gen2_ok = mfma_ok && (reinterpret_cast<uintptr_t>(out) & 7u) == 0 && sd.os % 4 == 0 && sd.oh % 4 == 0;
         if (gen2_ok && (q_len > 128 || kv_len > 128))
             return flash_prefill(q, k, v, out, hq, hkv, q_len, kv_len, d, scale, sd.qh, sd.qs, sd.kh, sd.ks, sd.oh, sd.os,

@@ -519,7 +519,9 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
     int nsplit = WIN ? flash_window_runs((long long)tiles * hq, span) : flash_runs((long long)tiles * hq, q_len, kv_len, 16);
     const bool wide = many.items || q_len <= 128;
-    if (nsplit > 1 && q_len <= 128) {      // up to 128 rows need no scratch memory to be captured
+    // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
+    // tiles of the first-generation kernel 61, 31 and 239)
+    if (nsplit > 1 && q_len <= 128) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) nsplit = 1;
     }
