@@ -20,41 +20,47 @@ struct QkvHeadArgs {
 };
 struct ActArgs { float pos, neg; bool gelu; };     // pgk_device.hip.h: xielu's factors, or gelu_erf
 
-// Head slot `slot` of the bf16-rounded QKV projection of ROWS token rows, row0 + STEP i: 16 lanes hold one row's 128 dims, 8 each (sub = lane's
-// chunk; load(i) gives them).  The arithmetic of qknorm_rope_kvwrite_kernel, operation for operation, then the store.  All lanes must be active.
-// Four rows' places and angles are requested together, ahead of the stores, which the compiler cannot move them across: a row at a time the
-// epilogue was a chain of ROWS round trips (QKV of Qwen3-0.6B, 3365 rows in 256-tiles 45 -> 42 us, 384 rows in 128-tiles 16.9 -> 15.2).
-template <int ROWS, int STEP, class Load>
-__device__ __forceinline__ void qkv_heads_finish(int sub, int slot, int row0, int M, const QkvHeadArgs& hd, bf16* qkv, int ldq, Load load) {
-    const bool is_q = slot < hd.hq, is_k = !is_q && slot < hd.hq + hd.hkv;
-    const bf16* gamma = is_q ? hd.q_gamma : hd.k_gamma;
-    Vec<bf16> gr;
-    gr.raw = make_uint4(0, 0, 0, 0);
-    if (gamma) gr.raw = *reinterpret_cast<const uint4*>(gamma + sub * 8);
-    float gm[8];
-    gr.to_float(gm);
-    const int dd = (sub * 8) % 64;
-    const bool lo = sub < 8;
+// Head slots of the bf16-rounded QKV projection of ROWS token rows, row0 + step i: 16 lanes hold one row's 128 dims, 8 each (sub = lane's chunk).
+// finish() does the arithmetic of qknorm_rope_kvwrite_kernel, operation for operation, then the store (load(i) gives a row's dims); all lanes must be active.
+// The rows' places and angles are asked for by places() and angles(), which callers put ahead of and behind the writes of the tile to LDS: two round trips that
+// the tile's barrier hides.  Asked for four rows at a time between the stores, the epilogue of a 256-row tile (two heads) took 9.9 us of the 32 of a product of
+// 3365 x 4096 x 1024, and 4.3 of 14 for a 128-row tile.
+template <int ROWS>
+struct HeadRows {
+    int2 place[ROWS];
+    float4 cs[ROWS][2], sn[ROWS][2];
+    __device__ __forceinline__ void places(int row0, int step, int M, const QkvHeadArgs& hd) {
 #pragma unroll
-    for (int i0 = 0; i0 < ROWS; i0 += 4) {
-        int2 place[4];
-        float4 cs[4][2], sn[4][2];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int grow = row0 + (i0 + u) * STEP;
-            place[u] = hd.at ? hd.at[min(grow, M - 1)] : make_int2(hd.start_pos + grow, 0);
+        for (int i = 0; i < ROWS; ++i) {
+            const int grow = row0 + i * step;
+            place[i] = hd.at ? hd.at[min(grow, M - 1)] : make_int2(hd.start_pos + grow, 0);
         }
+    }
+    __device__ __forceinline__ void angles(int sub, int first_slot, const QkvHeadArgs& hd) {
+        if (first_slot >= hd.hq + hd.hkv) return;            // value heads are stored as they are
+        const int dd = (sub * 8) % 64;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const size_t at = (size_t)min(place[u].x, hd.max_seq - 1) * 64 + dd;
-            cs[u][0] = *reinterpret_cast<const float4*>(hd.rope_cos + at); cs[u][1] = *reinterpret_cast<const float4*>(hd.rope_cos + at + 4);
-            sn[u][0] = *reinterpret_cast<const float4*>(hd.rope_sin + at); sn[u][1] = *reinterpret_cast<const float4*>(hd.rope_sin + at + 4);
+        for (int i = 0; i < ROWS; ++i) {
+            const size_t at = (size_t)min(place[i].x, hd.max_seq - 1) * 64 + dd;
+            cs[i][0] = *reinterpret_cast<const float4*>(hd.rope_cos + at); cs[i][1] = *reinterpret_cast<const float4*>(hd.rope_cos + at + 4);
+            sn[i][0] = *reinterpret_cast<const float4*>(hd.rope_sin + at); sn[i][1] = *reinterpret_cast<const float4*>(hd.rope_sin + at + 4);
         }
+    }
+    template <class Load>
+    __device__ __forceinline__ void finish(int sub, int slot, int row0, int step, int M, const QkvHeadArgs& hd, bf16* qkv, int ldq, Load load) const {
+        const bool is_q = slot < hd.hq, is_k = !is_q && slot < hd.hq + hd.hkv;
+        const bf16* gamma = is_q ? hd.q_gamma : hd.k_gamma;
+        Vec<bf16> gr;
+        gr.raw = make_uint4(0, 0, 0, 0);
+        if (gamma) gr.raw = *reinterpret_cast<const uint4*>(gamma + sub * 8);
+        float gm[8];
+        gr.to_float(gm);
+        const float sign = sub < 8 ? -1.f : 1.f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int grow = row0 + (i0 + u) * STEP, pos = place[u].x;
+        for (int i = 0; i < ROWS; ++i) {
+            const int grow = row0 + i * step, pos = place[i].x;
             float x[8];
-            load(i0 + u, x);
+            load(i, x);
             if (is_q || is_k) {
                 if (gamma) {
                     float ss = 0.f;
@@ -65,14 +71,12 @@ __device__ __forceinline__ void qkv_heads_finish(int sub, int slot, int row0, in
 #pragma unroll
                     for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * gm[j];
                 }
-                const float c[8] = {cs[u][0].x, cs[u][0].y, cs[u][0].z, cs[u][0].w, cs[u][1].x, cs[u][1].y, cs[u][1].z, cs[u][1].w};
-                const float s[8] = {sn[u][0].x, sn[u][0].y, sn[u][0].z, sn[u][0].w, sn[u][1].x, sn[u][1].y, sn[u][1].z, sn[u][1].w};
+                const float c[8] = {cs[i][0].x, cs[i][0].y, cs[i][0].z, cs[i][0].w, cs[i][1].x, cs[i][1].y, cs[i][1].z, cs[i][1].w};
+                const float s[8] = {sn[i][0].x, sn[i][0].y, sn[i][0].z, sn[i][0].w, sn[i][1].x, sn[i][1].y, sn[i][1].z, sn[i][1].w};
                 float o[8];
+                // x c -+ other s
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float other = xor_half<16>(x[j]);
-                    o[j] = lo ? (x[j] * c[j] - other * s[j]) : (x[j] * c[j] + other * s[j]);
-                }
+                for (int j = 0; j < 8; ++j) o[j] = fmaf(x[j], c[j], xor_half<16>(x[j]) * (s[j] * sign));
 #pragma unroll
                 for (int j = 0; j < 8; ++j) x[j] = o[j];
             }
@@ -83,11 +87,11 @@ __device__ __forceinline__ void qkv_heads_finish(int sub, int slot, int row0, in
                     ov.store(qkv + (size_t)grow * ldq + slot * 128 + sub * 8);
                 } else if (pos < hd.max_seq) {
                     const int kvh = is_k ? slot - hd.hq : slot - hd.hq - hd.hkv;
-                    ov.store((is_k ? hd.kcache : hd.vcache) + place[u].y * hd.slot_stride + ((size_t)kvh * hd.max_seq + pos) * 128 + sub * 8);
+                    ov.store((is_k ? hd.kcache : hd.vcache) + place[i].y * hd.slot_stride + ((size_t)kvh * hd.max_seq + pos) * 128 + sub * 8);
                 }
             }
         }
     }
-}
+};
 
 }  // namespace pgk

@@ -172,6 +172,9 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
+    const int c = tid & 15, r0 = tid >> 4;                   // 16 lanes take both heads of rows r0 + 32 i, whose angles they share
+    HeadRows<8> hr;
+    hr.places(m0 + r0, 32, M, hd);
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -182,14 +185,16 @@ __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g 
                 const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
                 *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
             }
+    hr.angles(c, 2 * tn, hd);
     __syncthreads();
-    const int c = tid & 31;
-    qkv_heads_finish<16, 16>(c & 15, 2 * tn + (c >> 4), m0 + (tid >> 5), M, hd, qkv, N, [&](int i, float (&x)[8]) {
-        const int row = i * 16 + (tid >> 5), sw = ((row >> 2) & 3) << 5;
-        Vec<bf16> raw;
-        raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((c * 16) ^ sw));
-        raw.to_float(x);
-    });
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        hr.finish(c, 2 * tn + h, m0 + r0, 32, M, hd, qkv, N, [&](int i, float (&x)[8]) {
+            const int row = i * 32 + r0, sw = ((row >> 2) & 3) << 5;
+            Vec<bf16> raw;
+            raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((h * 256 + c * 16) ^ sw));
+            raw.to_float(x);
+        });
 }
 
 template <int EPI>   // 0: bf16 C store (+bias); 1: fp32 C +=
@@ -483,29 +488,37 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     }
 }
 
-// ---- bf16, 128 x 128 tiles on the same staged LDS-DMA pipeline: the shapes too small for 192 tiles of 256 x 256 -------------
-// (Qwen3-0.6B at S = 2048: N = 1024 projections = 128 tiles, QKV 512 tiles with K = 1024.)  The register-staged 128-tile
-// kernel of ops_gemm.hip keeps ONE K step in flight (global -> registers -> LDS -> barrier): with one or two workgroups
-// per CU every step costs a memory round trip - 1.9 us per 64 k at M = 2048, N = 1024 (30 us for 8.6 GFLOP).  Here: 4 waves
-// (2 x 2, 64 x 64 each = 64 accumulator registers), stages of 32 k (16 KiB, the images, rings and counts of gemm256s: A a pair of stages at a
-// time in whole lines, packed W as it lies), three stages in flight behind a counted vmcnt(8), ONE barrier per stage; 80 KiB
-// of LDS and < 128 registers, so two workgroups share a CU and one's MFMAs cover the other's barrier and fragment reads -
-// no stagger needed.  blockIdx.y = K split (EPI 2: fp32 slab z of [splits][M][N], summed by the consumer).
-// (Reading the next stage's fragments under this one's MFMAs, or eight stages, changes nothing: the loop waits for what the DMA delivers.  M = 1531,
-// N = 4096, K = 1024, us: row-major W, 64-byte rows of A 20.6; packed 25.6 -> 19.2.  M = 384, N = 1024, K = 3072 in four splits: 12.4; 13.7 -> 10.9.)
-// Epilogue through LDS: the fp32 tile (64 KiB of the stages) is written with the lane quarters XOR-ed apart, then read
-// back as rows - 32 lanes x 16 B = one 512-byte row segment per instruction - for coalesced stores (EPI 1: float4
-// read-modify-write of the residual stream, all loads issued before the first store).
-constexpr int G1_THREADS = 256, G1_HALF = 128 * 64;
+// ---- bf16, smaller tiles: four waves multiply, four others fetch ------------------------------------------------------------
+// For the shapes too small for 192 tiles of 256 x 256.  Tiles of 32 WM x 32 WN, 2 x 2 waves of 16 WM x 16 WN, stages of 32 k in the images, rings and
+// counts of gemm256s (A a pair of stages at a time in whole lines, packed W as it lies).  A wave that issues an LDS-DMA instruction stands still until
+// the CU's one texture path has taken its 64 addresses, 20 clocks and those of the waves in front of it: with the DMA in the multiplying waves a stage
+// of a 128 x 128 tile took 0.25 us with one workgroup on the CU, half of it DMA issue (0.19 without the fragment reads, 0.12 for the DMA alone, 0.11 for
+// the products alone).  So waves 4-7 issue all of it and waves 0-3 never do; the fragments of stage s + 1 are requested between the products of stage s,
+// each into the registers its row of products has just read (W's, and the last row's, into a second set).  0.17-0.18 us a stage.
+// One barrier per stage: behind it stage s + 1 has landed (the DMA waves have waited for their shares) and stage s has been read, so W of s + 4 and,
+// where s is odd, A of s + 5 and s + 6 take its place.  Between W of a stage and the wait for it lie W of two stages and A of one pair.
+//   us a launch, before / after (K = 1024, packed W): 1531 rows, N = 6144 28.0 / 23.0 on 192 x 192 tiles, N = 4096 20.3 / 16.6 on 192 x 128; 384 rows,
+//   N = 6144 12.7 / 10.8; K = 3072, N = 1024, 3365 rows 28.3 / 23.4.
+// blockIdx.y = K split (EPI 2: fp32 slab z of [splits][M][N], summed by the consumer).
+// Epilogue through LDS, by all eight waves: the tile as fp32 (as bf16 where the values are rounded to it first anyway, EPI 3 and 4) with the lane
+// quarters XOR-ed apart, then back as rows for coalesced stores (EPI 1: float4 read-modify-write of the residual stream, all loads issued before the first
+// store).
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: fp32 split-K slab; 3: QKV heads (QkvHeadArgs: tile column = head slot);
-// 4: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]; tile tn = act columns [64 tn, +64)); 5: xIELU, 7: gelu, bf16 store
+// 4: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]; tile tn = act columns [16 WN tn, +16 WN)); 5: xIELU, 7: gelu, bf16 store
 // GRP: rows sorted by expert (GroupArgs), every tile with its expert's weight; EPI 4, 7, or 6: bf16 rows times their weight, each at its place
-template <int EPI, bool GRP>
-__device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                              int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga) {
-    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 8 KiB | W: 4 stages of 8 KiB
+constexpr int GP_THREADS = 512;
+template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
+    const size_t ring = G2S_ARING * (size_t)(32 * WM * 64) + 4 * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
+    return ring > tile ? ring : tile;
+}
+template <int EPI, bool GRP, int WM, int WN>
+__device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
+                                           int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga) {
+    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of AH bytes | W: 4 stages of WH
+    constexpr int BM = 32 * WM, BN = 32 * WN, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
+    constexpr bool B16 = EPI == 3 || EPI == 4;
+    static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int wr = wid >> 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
     int tm, tn, m0;
     if constexpr (GRP) {
         ntm = *ga.n_tiles;
@@ -517,220 +530,255 @@ __device__ __forceinline__ void gemm128s_body(const bf16* A, const bf16* W, cons
         m0 = t.row0;
         M = t.row0 + t.rows;
         W += t.expert * ga.w_stride;
-    } else m0 = tm * 128;
-    const int n0 = tn * 128;
+    } else m0 = tm * BM;
+    const int n0 = tn * BN;
     const int kbeg = (int)blockIdx.y * kps, kend = min(K, kbeg + kps);
+    const int nh = (kend - kbeg) / 32;                       // (kend - kbeg) % 64 == 0: an even number of stages
 
-    const int drow = wid * 32 + (lane >> 2);                 // one DMA instruction = 16 rows x 64 B
-    const int dchunk = (lane & 3) ^ ((lane >> 4) & 2);
-    auto a_row = [&](int r) -> int {
-        r = min(r, M - 1);
-        if constexpr (GRP) return ga.div > 0 ? ga.order[r] / ga.div : r;
-        else return r;
-    };
-    const bf16* a_src[4];
+    f32x4_g acc[WM][WN];
+    const int wr = (wid >> 1) & 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
+    if (wid >= 4) {
+        const int pw = __builtin_amdgcn_readfirstlane(wid & 3);
+        auto a_row = [&](int r) -> int {
+            r = min(r, M - 1);
+            if constexpr (GRP) return ga.div > 0 ? ga.order[r] / ga.div : r;
+            else return r;
+        };
+        const bf16* a_src[NA];                               // 8 rows x 128 B, two stages
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a_src[i] = A + (size_t)a_row(m0 + wid * 32 + 8 * i + (lane >> 3)) * K + kbeg + ((lane & 7) ^ (lane >> 3)) * 8;
-    // EPI 4: B-tile rows 0-63 = gate rows 64 tn .., rows 64-127 = the matching up rows N + 64 tn .. (N = I); a wave's 32 rows stay in one half
-    const int wrow = (EPI == 4) ? (drow < 64 ? tn * 64 + drow : N + tn * 64 + drow - 64) : n0 + drow;
-    const int wlast = (EPI == 4) ? 2 * N - 1 : N - 1;
-    // W row-major, or (packed) the fragment-major copy: see gemm256s_bf16_kernel
-    const bf16 *w_src0, *w_src1;
-    const int wk = packed ? 512 : 32;
-    if (packed) {
-        const int r_in = lane >> 2, nt_last = (wlast >> 4);
-        w_src0 = W + (((size_t)min((wrow - r_in) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + lane) * 8;
-        w_src1 = W + (((size_t)min((wrow - r_in + 16) >> 4, nt_last) * (K >> 5) + (kbeg >> 5)) * 64 + lane) * 8;
+        for (int i = 0; i < NA; ++i) a_src[i] = A + (size_t)a_row(m0 + (pw * NA + i) * 8 + (lane >> 3)) * K + kbeg + ((lane & 7) ^ (lane >> 3)) * 8;
+        // one instruction of W = 16 rows x 64 B of the row-major weight, or (packed) a block of the fragment-major copy as it lies: see gemm256s_bf16_kernel.
+        // EPI 4: the tile's first half are gate rows, the second the matching up rows N further on (N = I)
+        const bf16* w_src[NW];
+        const int wk = packed ? 512 : 32, wlast = (EPI == 4) ? 2 * N - 1 : N - 1;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const int r0 = (pw * NW + i) * 16;
+            const int row = (EPI == 4) ? (r0 < BN / 2 ? tn * (BN / 2) + r0 : N + tn * (BN / 2) + r0 - BN / 2) : n0 + r0;
+            if (packed) w_src[i] = W + (((size_t)min(row >> 4, wlast >> 4) * (K >> 5) + (kbeg >> 5)) * 64 + lane) * 8;
+            else w_src[i] = W + (size_t)min(row + (lane >> 2), wlast) * K + kbeg + ((lane & 3) ^ ((lane >> 4) & 2)) * 8;
+        }
+        const uint32_t lds0 = g2_lds_addr(g2_smem);
+        // past the end of K the last stage is read again (never consumed): the counts below stay constant
+        auto stage_a = [&](int h, int at) {                  // `at`: byte offset of the ring's slot
+            const int k = min(h, nh - 2) * 32;
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + at + pw * NA * 1024);
+#pragma unroll
+            for (int i = 0; i < NA; ++i) g2_dma16(a_src[i] + k, dst + i * 1024);
+        };
+        auto stage_w = [&](int h, int buf) {
+            const size_t kw = (size_t)min(h, nh - 1) * wk;
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + G2S_ARING * AH + buf * WH + pw * NW * 1024);
+#pragma unroll
+            for (int i = 0; i < NW; ++i) g2_dma16(w_src[i] + kw, dst + i * 1024);
+        };
+        auto wait_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + 2 * NW) : "memory"); };
+        stage_a(0, 0);
+        stage_w(0, 0);
+        stage_a(2, 2 * AH);
+        stage_w(1, 1);
+        stage_w(2, 2);
+        stage_a(4, 4 * AH);
+        stage_w(3, 3);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NA + 3 * NW) : "memory");   // stage 0
+        __builtin_amdgcn_s_barrier();
+        int at = 0;
+        for (int s = 0; s < nh; s += 2) {
+            wait_landed();                                   // stage s + 1
+            __builtin_amdgcn_s_barrier();
+            stage_w(s + 4, s & 3);
+            wait_landed();
+            __builtin_amdgcn_s_barrier();
+            stage_a(s + 6, at);
+            stage_w(s + 5, (s + 1) & 3);
+            at = at == 4 * AH ? 0 : at + 2 * AH;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // retire the phantom DMAs: the stages become the C tile
+        __builtin_amdgcn_s_barrier();
     } else {
-        w_src0 = W + (size_t)min(wrow, wlast) * K + kbeg + dchunk * 8;
-        w_src1 = W + (size_t)min(wrow + 16, wlast) * K + kbeg + dchunk * 8;
-    }
-    const uint32_t lds0 = g2_lds_addr(g2_smem);
-    const int nh = (kend - kbeg) / 32;
-    // past the end of K the last stage is read again (never consumed): the counts below stay constant
-    auto stage_a = [&](int h, int at) {
-        const int k = min(h, nh - 2) * 32;
-        const uint32_t a_dst = __builtin_amdgcn_readfirstlane(lds0 + at + wid * 4096);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) g2_dma16(a_src[i] + k, a_dst + i * 1024);
-    };
-    auto stage_w = [&](int h, int buf) {
-        const size_t kw = (size_t)min(h, nh - 1) * wk;
-        const uint32_t w_dst = __builtin_amdgcn_readfirstlane(lds0 + (G2S_ARING + buf) * G1_HALF + wid * 2048);
-        g2_dma16(w_src0 + kw, w_dst);
-        g2_dma16(w_src1 + kw, w_dst + 1024);
-    };
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
+        const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
+        const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
+        const int a_base = wr * 16 * WM * 128, w_base = G2S_ARING * AH + wc * 16 * WN * 64 + w_off;
+        auto frag = [&](const char* p) { return *reinterpret_cast<const bf16x8_g*>(p); };
+        bf16x8_g fa[WM - 1], fl[2], fb[2][WN];               // A's rows but the last, the last, W's
+        __builtin_amdgcn_s_barrier();
+        {
+            const char *As = g2_smem + a_base + a_off0, *Ws = g2_smem + w_base;
+#pragma unroll
+            for (int i = 0; i < WM - 1; ++i) fa[i] = frag(As + i * 2048);
+            fl[0] = frag(As + (WM - 1) * 2048);
+#pragma unroll
+            for (int j = 0; j < WN; ++j) fb[0][j] = frag(Ws + j * 1024);
+        }
+        int a_cur = 0;                                       // ring slot of A's stage s
+#define GP_MFMA(I, F, P)                                                                                     \
+    _Pragma("unroll") for (int j = 0; j < WN; ++j) acc[I][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(F, fb[P][j], acc[I][j], 0, 0, 0); \
+    __builtin_amdgcn_sched_barrier(0);
+#define GP_STEP(BUF)                                                                                         \
+    {                                                                                                        \
+        constexpr int P = (BUF) & 1;                                                                         \
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   /* stage s in registers: its place may be refilled */ \
+        __builtin_amdgcn_s_barrier();                                                                        \
+        __builtin_amdgcn_sched_barrier(0);                                                                   \
+        const int a_nxt = P ? (a_cur == 4 * AH ? 0 : a_cur + 2 * AH) : a_cur;                                \
+        const char* As = g2_smem + a_nxt + a_base + (P ? a_off0 : a_off1);                                   \
+        const char* Ws = g2_smem + (((BUF) + 1) & 3) * WH + w_base;                                          \
+        GP_MFMA(0, fa[0], P)                                                                                 \
+        fa[0] = frag(As);                                                                                    \
+        fl[P ^ 1] = frag(As + (WM - 1) * 2048);                                                              \
+        _Pragma("unroll") for (int j = 0; j < WN / 2; ++j) fb[P ^ 1][j] = frag(Ws + j * 1024);               \
+        __builtin_amdgcn_sched_barrier(0);                                                                   \
+        GP_MFMA(1, fa[1], P)                                                                                 \
+        fa[1] = frag(As + 2048);                                                                             \
+        _Pragma("unroll") for (int j = WN / 2; j < WN; ++j) fb[P ^ 1][j] = frag(Ws + j * 1024);              \
+        __builtin_amdgcn_sched_barrier(0);                                                                   \
+        _Pragma("unroll") for (int i = 2; i < WM - 1; ++i) {                                                 \
+            GP_MFMA(i, fa[i], P)                                                                             \
+            fa[i] = frag(As + i * 2048);                                                                     \
+            __builtin_amdgcn_sched_barrier(0);                                                               \
+        }                                                                                                    \
+        GP_MFMA(WM - 1, fl[P], P)                                                                            \
+        a_cur = a_nxt;                                                                                       \
+    }
+        int s = 0;
+        for (; s + 4 <= nh; s += 4) {
+            GP_STEP(0) GP_STEP(1) GP_STEP(2) GP_STEP(3)
+        }
+        if (s < nh) {
+            GP_STEP(0) GP_STEP(1)
+        }
+#undef GP_STEP
+#undef GP_MFMA
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads past the last stage, before the stages become the C tile
+        __builtin_amdgcn_s_barrier();
+    }
 
-    f32x4_g acc[4][4];
+    // rows of the tile: fp32, 64-byte group g at g ^ ((R >> 2) & 3), or bf16, 32-byte group likewise - (R >> 2) & 3 == q for the accumulator layout
+    constexpr int ROWB = BN * (B16 ? 2 : 4);
+    constexpr int QS = B16 ? 5 : 6;
+    HeadRows<EPI == 3 ? BM / 32 : 1> hr;
+    const int hrow = tid >> 4;                               // EPI 3: 16 consecutive lanes = one (token row, head)
+    if constexpr (EPI == 3) hr.places(m0 + hrow, 32, M, hd);
+    if (wid < 4) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
-    const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
-    const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
-    const int a_base = wr * 64 * 128, w_base = G2S_ARING * G1_HALF + wc * 64 * 64;
-    uint4 fa[4], fb[4];
-
-    stage_a(0, 0);
-    stage_w(0, 0);
-    stage_a(2, 2 * G1_HALF);
-    stage_w(1, 1);
-    stage_w(2, 2);
-    int a_cur = 0;                                           // ring slot of A's stage s
-    // iteration s: own share of stage s landed (two younger stages may stay in flight) | barrier: everyone's share landed AND
-    // everyone finished reading stage s - 1, whose buffer the DMA of stage s + 3 - issued right behind the reads - refills
-#define G1S_STEP(S, BUF)                                                                                      \
-    {                                                                                                         \
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                                                      \
-        __builtin_amdgcn_s_barrier();                                                                         \
-        const char* As = g2_smem + a_cur + a_base + (((BUF) & 1) ? a_off1 : a_off0);                         \
-        const char* Ws = g2_smem + (BUF) * G1_HALF + w_base + w_off;                                      \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 2048); \
-        _Pragma("unroll") for (int j = 0; j < 4; ++j) fb[j] = *reinterpret_cast<const uint4*>(Ws + j * 1024); \
-        __builtin_amdgcn_sched_barrier(0);                                                                    \
-        if (((BUF) & 1) == 0) {                                                                               \
-            const int a_new = a_cur >= 2 * G1_HALF ? a_cur - 2 * G1_HALF : a_cur + 4 * G1_HALF;               \
-            stage_a((S) + 4, a_new);                                                                          \
-        }                                                                                                     \
-        stage_w((S) + 3, ((BUF) + 3) & 3);                                                                    \
-        if (((BUF) & 1) == 1) a_cur = a_cur == 4 * G1_HALF ? 0 : a_cur + 2 * G1_HALF;                         \
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                    \
-        __builtin_amdgcn_sched_barrier(0);                                                                    \
-        __builtin_amdgcn_s_setprio(1);                                                                        \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                         \
-            _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                     \
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_g, fa[i]),      \
-                                                                    __builtin_bit_cast(bf16x8_g, fb[j]), acc[i][j], 0, 0, 0); \
-        __builtin_amdgcn_s_setprio(0);                                                                        \
-        __builtin_amdgcn_sched_barrier(0);                                                                    \
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = wr * 16 * WM + i * 16 + q * 4 + r, col = wc * 16 * WN + j * 16 + l15;
+                    if constexpr (B16) *reinterpret_cast<bf16*>(g2_smem + row * ROWB + ((col * 2) ^ (q << QS))) = from_f<bf16>(acc[i][j][r]);
+                    else *reinterpret_cast<float*>(g2_smem + row * ROWB + ((col * 4) ^ (q << QS))) = acc[i][j][r];
+                }
     }
-    int s = 0;
-    for (; s + 4 <= nh; s += 4) {
-        G1S_STEP(s, 0) G1S_STEP(s + 1, 1) G1S_STEP(s + 2, 2) G1S_STEP(s + 3, 3)
+    if constexpr (EPI == 3) hr.angles((tid & 15), tn, hd);
+    auto tile4 = [&](int row, int byte) { return *reinterpret_cast<const float4*>(g2_smem + row * ROWB + (byte ^ (((row >> 2) & 3) << QS))); };
+    if constexpr (EPI == 1) {
+        constexpr int IT = BM * (BN / 4) / GP_THREADS;
+        float4 old[IT];
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / (BN / 4), c = item % (BN / 4);
+            old[it] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(Cv) + (size_t)min(m0 + row, M - 1) * N + min(n0 + c * 4, N - 4));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / (BN / 4), c = item % (BN / 4);
+            float4 v = tile4(row, c * 16);
+            const int grow = m0 + row, gcol = n0 + c * 4;
+            if (grow >= M || gcol >= N) continue;
+            v.x += old[it].x; v.y += old[it].y; v.z += old[it].z; v.w += old[it].w;
+            *reinterpret_cast<float4*>(reinterpret_cast<float*>(Cv) + (size_t)grow * N + gcol) = v;
+        }
+        return;
     }
-    if (s < nh) {   // (kend - kbeg) % 64 == 0: an even number of stages, so two remain at most
-        G1S_STEP(s, 0) G1S_STEP(s + 1, 1)
-    }
-#undef G1S_STEP
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // retire the phantom DMAs: the stages become the C tile
-    __builtin_amdgcn_s_barrier();
-
-    // fp32 tile [128][128]: row R's 64-byte group g at g ^ ((R >> 2) & 3) - (R >> 2) & 3 == q for the accumulator layout
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 64 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 4;
-                *reinterpret_cast<float*>(g2_smem + row * 512 + (colb ^ (q << 6))) = acc[i][j][r];
-            }
     __syncthreads();
     if constexpr (EPI == 4) {
-        // act = bf16(silu(g) * u) from the bf16-rounded g and u (the arithmetic of swiglu_rows_kernel / g2_swiglu_epilogue): 8 lanes per row
+        // act = bf16(silu(g) * u) from the bf16-rounded g and u (the arithmetic of swiglu_rows_kernel / g2_swiglu_epilogue)
+        constexpr int CH = BN / 16;                          // chunks of 8 act columns in a row
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int item = it * G1_THREADS + tid, row = item >> 3, c = item & 7, sw = ((row >> 2) & 3) << 6;
-            const char* rp = g2_smem + row * 512;
-            const float4 g0 = *reinterpret_cast<const float4*>(rp + ((c * 32) ^ sw)), g1 = *reinterpret_cast<const float4*>(rp + ((c * 32 + 16) ^ sw));
-            const float4 u0 = *reinterpret_cast<const float4*>(rp + ((256 + c * 32) ^ sw)), u1 = *reinterpret_cast<const float4*>(rp + ((256 + c * 32 + 16) ^ sw));
-            const float gfr[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, ufr[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+        for (int it = 0; it < (BM * CH + GP_THREADS - 1) / GP_THREADS; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / CH, c = item % CH, sw = ((row >> 2) & 3) << QS;
+            if (BM * CH % GP_THREADS != 0 && row >= BM) break;
             Vec<bf16> g, u;
-            g.from_float(gfr);
-            u.from_float(ufr);
+            g.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((c * 16) ^ sw));
+            u.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((BN + c * 16) ^ sw));
             float gf[8], uf[8];
             g.to_float(gf);
             u.to_float(uf);
 #pragma unroll
             for (int e = 0; e < 8; ++e) gf[e] = gf[e] / (1.0f + __expf(-gf[e])) * uf[e];
             g.from_float(gf);
-            const int grow = m0 + row, gcol = tn * 64 + c * 8;
+            const int grow = m0 + row, gcol = tn * (BN / 2) + c * 8;
             if (grow < M && gcol < N) g.store(reinterpret_cast<bf16*>(Cv) + (size_t)grow * N + gcol);
         }
     } else if constexpr (EPI == 3) {
-        // 16 consecutive lanes = one (token row, head): the arithmetic of qknorm_rope_kvwrite_kernel on the bf16-rounded row,
-        // so the result is bit-identical to GEMM (bf16 store) + that kernel.  Tile column tn is the head slot.
+        // the arithmetic of qknorm_rope_kvwrite_kernel on the bf16-rounded row, so the result is bit-identical to GEMM (bf16 store) + that kernel
         const int c = tid & 15;
-        qkv_heads_finish<8, 16>(c, tn, m0 + (tid >> 4), M, hd, reinterpret_cast<bf16*>(Cv), N, [&](int i, float (&x)[8]) {
-            const int row = i * 16 + (tid >> 4), sw = ((row >> 2) & 3) << 6;
-            const float4 v0 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32) ^ sw));
-            const float4 v1 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32 + 16) ^ sw));
-            const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        hr.finish(c, tn, m0 + hrow, 32, M, hd, reinterpret_cast<bf16*>(Cv), N, [&](int i, float (&x)[8]) {
+            const int row = i * 32 + hrow;
             Vec<bf16> raw;
-            raw.from_float(f);
+            raw.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((c * 16) ^ (((row >> 2) & 3) << QS)));
             raw.to_float(x);
         });
-    } else if constexpr (EPI == 6) {
+    } else if constexpr (EPI == 2) {
+        float* C = reinterpret_cast<float*>(Cv) + (size_t)blockIdx.y * M * N;
 #pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int item = it * G1_THREADS + tid, row = item >> 4, c = item & 15, sw = ((row >> 2) & 3) << 6;
-            const float4 v0 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32) ^ sw));
-            const float4 v1 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32 + 16) ^ sw));
-            const int grow = m0 + row, gcol = n0 + c * 8;
-            if (grow >= M || gcol >= N) continue;
-            const int place = ga.order[grow];
-            const float w = ga.wts[place];
-            const float f[8] = {v0.x * w, v0.y * w, v0.z * w, v0.w * w, v1.x * w, v1.y * w, v1.z * w, v1.w * w};
-            Vec<bf16> o;
-            o.from_float(f);
-            o.store(reinterpret_cast<bf16*>(Cv) + (size_t)place * N + gcol);
+        for (int it = 0; it < BM * (BN / 4) / GP_THREADS; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / (BN / 4), c = item % (BN / 4);
+            const float4 v = tile4(row, c * 16);
+            const int grow = m0 + row, gcol = n0 + c * 4;
+            if (grow < M && gcol < N) *reinterpret_cast<float4*>(C + (size_t)grow * N + gcol) = v;
         }
-    } else if constexpr (EPI == 0 || EPI == 5 || EPI == 7) {
+    } else {
         // 8 columns per lane: two float4 -> 16 bytes of bf16
 #pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int item = it * G1_THREADS + tid, row = item >> 4, c = item & 15, sw = ((row >> 2) & 3) << 6;
-            const float4 v0 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32) ^ sw));
-            const float4 v1 = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 32 + 16) ^ sw));
+        for (int it = 0; it < BM * (BN / 8) / GP_THREADS; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / (BN / 8), c = item % (BN / 8);
+            const float4 v0 = tile4(row, c * 32), v1 = tile4(row, c * 32 + 16);
             const int grow = m0 + row, gcol = n0 + c * 8;
             if (grow >= M || gcol >= N) continue;
             float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-            if (bias) {
+            size_t orow = grow;
+            if constexpr (EPI == 6) {
+                orow = ga.order[grow];
+                const float w = ga.wts[orow];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) f[e] += to_f(bias[gcol + e]);
-            }
-            if constexpr (EPI == 5) {
+                for (int e = 0; e < 8; ++e) f[e] *= w;
+            } else {
+                if (bias) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) f[e] = xielu<false>(f[e], xa.pos, xa.neg);
-            }
-            if constexpr (EPI == 7) {
+                    for (int e = 0; e < 8; ++e) f[e] += to_f(bias[gcol + e]);
+                }
+                if constexpr (EPI == 5) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) f[e] = gelu_erf(f[e]);
+                    for (int e = 0; e < 8; ++e) f[e] = xielu<false>(f[e], xa.pos, xa.neg);
+                }
+                if constexpr (EPI == 7) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) f[e] = gelu_erf(f[e]);
+                }
             }
             Vec<bf16> o;
             o.from_float(f);
-            o.store(reinterpret_cast<bf16*>(Cv) + (size_t)grow * N + gcol);
-        }
-    } else {
-        float* C = reinterpret_cast<float*>(Cv) + (EPI == 2 ? (size_t)blockIdx.y * M * N : 0);
-        float4 old[16];
-        if constexpr (EPI == 1) {
-#pragma unroll
-            for (int it = 0; it < 16; ++it) {
-                const int item = it * G1_THREADS + tid, row = item >> 5, c = item & 31;
-                const int grow = min(m0 + row, M - 1), gcol = min(n0 + c * 4, N - 4);
-                old[it] = *reinterpret_cast<const float4*>(C + (size_t)grow * N + gcol);
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < 16; ++it) {
-            const int item = it * G1_THREADS + tid, row = item >> 5, c = item & 31, sw = ((row >> 2) & 3) << 6;
-            float4 v = *reinterpret_cast<const float4*>(g2_smem + row * 512 + ((c * 16) ^ sw));
-            const int grow = m0 + row, gcol = n0 + c * 4;
-            if (grow >= M || gcol >= N) continue;
-            if constexpr (EPI == 1) { v.x += old[it].x; v.y += old[it].y; v.z += old[it].z; v.w += old[it].w; }
-            *reinterpret_cast<float4*>(C + (size_t)grow * N + gcol) = v;
+            o.store(reinterpret_cast<bf16*>(Cv) + orow * N + gcol);
         }
     }
 }
-template <int EPI>
-__global__ __launch_bounds__(G1_THREADS, 2) void gemm128s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa = ActArgs{}) {
-    gemm128s_body<EPI, false>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{});
+// (128 x 128: two workgroups a CU, 80 KiB of LDS and 128 registers each; the larger ones have a CU to themselves)
+template <int EPI, int WM, int WN>
+__global__ __launch_bounds__(GP_THREADS, WM * WN == 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
+                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa) {
+    gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{});
 }
 template <int EPI>
-__global__ __launch_bounds__(G1_THREADS, 2) void gemm128s_grouped_kernel(const bf16* A, const bf16* W, bf16* C, int N, int K, int ntn, GroupArgs ga) {
-    gemm128s_body<EPI, true>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga);
+__global__ __launch_bounds__(GP_THREADS, 4) void gemmp_grouped_kernel(const bf16* A, const bf16* W, bf16* C, int N, int K, int ntn, GroupArgs ga) {
+    gemmp_body<EPI, true, 4, 4>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga);
 }
 
 // ---- fp8 x fp8 with 128-wide block scales on the same structure --------------------------------------------
@@ -1117,7 +1165,39 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
     return PGK_OK;
 }
 
-// 128 x 128 tiles; mode 0: bf16 C (+bias, or with `act` its activation), 1: fp32 C +=, 2: fp32 slabs [splits][M][N] (K split into `splits` runs of whole 64-k steps)
+template <int EPI, int WM, int WN>
+static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, void* C, int M, int N, int K, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa,
+                               hipStream_t st) {
+    constexpr size_t LDS = gemmp_lds<WM, WN, EPI == 3 || EPI == 4>();
+    static bool attr_done = false;
+    if (!attr_done) {
+        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemmp_bf16_kernel<EPI, WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
+        attr_done = true;
+    }
+    const int ntm = ceil_div(M, 32 * WM), ntn = EPI == 4 ? ceil_div(N, 16 * WN) : ceil_div(N, 32 * WN);      // SwiGLU: N = I act columns, half a tile's
+    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa);
+    PGK_CHECK_HIP(hipGetLastError());
+    return PGK_OK;
+}
+
+// Tile of an unsplit product of `cols` weight rows: the cheapest by rounds of workgroups x (time of a stage x stages + start and epilogue), in 0.01 us as measured
+// with the chip full.  128 x 128 runs two workgroups on a CU where there are more than 256.  (256 x 128 fills a round only where two of 128 x 128 on a CU do as well.)
+// 0: 128 x 128, 1: 192 x 128, 2: 192 x 192 (SwiGLU alone: heads are 128 columns).
+static int gemmp_tile(int M, int cols, int K, bool wide) {
+    constexpr struct { int bm, bn, stage, fixed; } t[] = {{128, 128, 18, 260}, {192, 128, 27, 350}, {192, 192, 40, 460}};
+    int best = 0;
+    long long least = 0;
+    for (int i = 0; i < (wide ? 3 : 2); ++i) {
+        const long long n = (long long)ceil_div(M, t[i].bm) * ceil_div(cols, t[i].bn), stages = K / 32;
+        long long cost = ceil_div(n, 256LL) * (stages * t[i].stage + t[i].fixed);
+        if (i == 0) cost = n / 512 * (stages * 29 + 420) + (n % 512 > 256 ? stages * 29 + 420 : n % 512 > 0 ? stages * 18 + 260 : 0);
+        if (i == 0 || cost < least) { best = i; least = cost; }
+    }
+    return best;
+}
+
+// mode 0: bf16 C (+bias, or with `act` its activation), 1: fp32 C +=, 2: fp32 slabs [splits][M][N] (K split into `splits` runs of whole 64-k steps),
+// 3: QKV heads, 4: SwiGLU
 bool gemm128s_shape_ok(int N, int K) { return K % 64 == 0 && K >= 64 && N % 8 == 0 && N >= 8; }
 bool gemm128s_ok(int M, int N, int K) { return M > 128 && gemm128s_shape_ok(N, K); }
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
@@ -1128,49 +1208,42 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
     PGK_REQUIRE(mode != 4 || N % 64 == 0, "gemm128s: the SwiGLU epilogue needs I=%d to be a multiple of 64", N);
     PGK_REQUIRE(mode != 3 || (heads && N == (heads->hq + 2 * heads->hkv) * 128), "gemm128s: the QKV-heads epilogue needs N=%d = (Hq + 2 Hkv) x 128", N);
     const QkvHeadArgs hd = heads ? *heads : QkvHeadArgs{};
-    constexpr size_t LDS = (G2S_ARING + 4) * (size_t)G1_HALF;
+    const int kps = ceil_div(ceil_div(K, splits), 64) * 64;
+    PGK_REQUIRE(ceil_div(K, kps) == splits, "gemm128s: K=%d does not split into %d runs of whole 64-k steps", K, splits);
+    const ActArgs none{};
+    if (mode == 0 && act && act->gelu) return gemmp_launch<7, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, st);
+    if (mode == 0 && act) return gemmp_launch<5, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, st);
+    if (mode == 0) return gemmp_launch<0, 4, 4>(A, W, bias, C, M, N, K, kps, hd, pk, none, st);
+    if (mode == 1) return gemmp_launch<1, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    if (mode == 2) return gemmp_launch<2, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    const int t = gemmp_tile(M, mode == 4 ? 2 * N : N, K, mode == 4);
+    if (mode == 3) {
+        if (t == 1) return gemmp_launch<3, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+        return gemmp_launch<3, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    }
+    if (t == 1) return gemmp_launch<4, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    if (t == 2) return gemmp_launch<4, 6, 6>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    return gemmp_launch<4, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+}
+
+template <int EPI>
+static pgk_status gemmp_grouped_launch(const bf16* A, const bf16* W, bf16* C, const GroupArgs& g, int max_tiles, int ntn, int N, int K, hipStream_t st) {
+    constexpr size_t LDS = gemmp_lds<4, 4, EPI == 4>();
     static bool attr_done = false;
     if (!attr_done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<5>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_bf16_kernel<7>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
+        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemmp_grouped_kernel<EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
         attr_done = true;
     }
-    const int ntm = ceil_div(M, 128), ntn = mode == 4 ? N / 64 : ceil_div(N, 128);      // SwiGLU: N = I act columns, 64 per tile
-    const int kps = ceil_div(ceil_div(K, splits), 64) * 64;
-    const dim3 grid(ntm * ntn, ceil_div(K, kps));
-    PGK_REQUIRE((int)grid.y == splits, "gemm128s: K=%d does not split into %d runs of whole 64-k steps", K, splits);
-    if (mode == 0 && act && act->gelu) gemm128s_bf16_kernel<7><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, *act);
-    else if (mode == 0 && act) gemm128s_bf16_kernel<5><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, *act);
-    else if (mode == 0) gemm128s_bf16_kernel<0><<<grid, G1_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, pk, ActArgs{});
-    else if (mode == 1) gemm128s_bf16_kernel<1><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, ActArgs{});
-    else if (mode == 2) gemm128s_bf16_kernel<2><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, ActArgs{});
-    else if (mode == 3) gemm128s_bf16_kernel<3><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, ActArgs{});
-    else gemm128s_bf16_kernel<4><<<grid, G1_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, kps, hd, pk, ActArgs{});
+    gemmp_grouped_kernel<EPI><<<max_tiles * ntn, GP_THREADS, LDS, st>>>(A, W, C, N, K, ntn, g);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
-
 pgk_status gemm128s_grouped(const bf16* A, const bf16* W, bf16* C, MoeProduct what, const GroupArgs& g, int max_tiles, int rows, int N, int K, hipStream_t st) {
     PGK_REQUIRE(K % 64 == 0 && N % 64 == 0 && max_tiles >= 1 && g.tiles && g.n_tiles && g.order && g.wts, "gemm128s_grouped: N=%d K=%d", N, K);
-    constexpr size_t LDS = (G2S_ARING + 4) * (size_t)G1_HALF;
-    static bool attr_done = false;
-    if (!attr_done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_grouped_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_grouped_kernel<6>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm128s_grouped_kernel<7>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        attr_done = true;
-    }
     const int ntn = what == MOE_SWIGLU ? N / 64 : ceil_div(N, 128);
-    if (what == MOE_GELU) gemm128s_grouped_kernel<7><<<max_tiles * ntn, G1_THREADS, LDS, st>>>(A, W, C, N, K, ntn, g);
-    else if (what == MOE_DOWN) gemm128s_grouped_kernel<6><<<max_tiles * ntn, G1_THREADS, LDS, st>>>(A, W, C, N, K, ntn, g);
-    else gemm128s_grouped_kernel<4><<<max_tiles * ntn, G1_THREADS, LDS, st>>>(A, W, C, N, K, ntn, g);
-    PGK_CHECK_HIP(hipGetLastError());
-    return PGK_OK;
+    if (what == MOE_GELU) return gemmp_grouped_launch<7>(A, W, C, g, max_tiles, ntn, N, K, st);
+    if (what == MOE_DOWN) return gemmp_grouped_launch<6>(A, W, C, g, max_tiles, ntn, N, K, st);
+    return gemmp_grouped_launch<4>(A, W, C, g, max_tiles, ntn, N, K, st);
 }
 
 }  // namespace pgk
