@@ -34,7 +34,10 @@
 namespace pgk {
 
 pgk_status engine_gemm_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, void* C, bool accum_f32, int M,
-                          int N, int K, hipStream_t st, bool packed = false);      // packed: W = the fragment-major bf16 copy
+                          int N, int K, hipStream_t st, bool packed = false, const NormIn& ni = NormIn{});      // packed: W = the fragment-major bf16 copy
+bool engine_gemm_carry_ok(int M, int N, int K);                // ops_gemm.hip: RMSNorm carried by the products around it (NormIn, NormOut)
+bool engine_gemm_resid_pays(int M, int N, int K, int splits);
+pgk_status engine_gemm_resid_nt(const bf16* A, const void* W, float* h, int M, int N, int K, const NormOut& no, hipStream_t st, bool packed);
 bool engine_gemm_packed_ok(int M, int N, int K);
 int wsgemm_pick_splits(int N, int K, bool allow_split);
 int engine_gemm_pick_splits(int M, int N, int K);
@@ -50,9 +53,9 @@ bool sdpa_flash_enabled();                                     // ops_attention.
 pgk_status flash_prefill_q8(const void* q, const void* k, const void* v, uint8_t* q8, float* q8s, int hq, int hkv, int q_len, int kv_len,
                             float scale, long long qh, long long qs, long long kh, long long ks, hipStream_t st);   // ops_flash.hip
 bool engine_gemm_qkv_heads_ok(int M, int N, int K);            // ops_gemm.hip: QKV projection with per-head norm + RoPE + cache write as its epilogue
-pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed = false);
+pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni);
 bool engine_gemm_swiglu_ok(int M, int I, int K, bool fp8);     // ops_gemm.hip: gate / up projection with the SwiGLU epilogue
-pgk_status engine_gemm_swiglu_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, bf16* act, int M, int I, int K, hipStream_t st, bool packed = false);
+pgk_status engine_gemm_swiglu_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, bf16* act, int M, int I, int K, hipStream_t st, bool packed, const NormIn& ni);
 bool gemm_fp8_qkv_heads_ok(int M, int N, int K);               // ops_fp8_gemm.hip: the same epilogue on the fp8 x fp8 256-tile kernel
 pgk_status gemm_fp8_qkv_heads_nt(const uint8_t* a, const float* sa, const uint8_t* w, const bf16* sw, bf16* qkv, int M, int N, int K,
                                  const QkvHeadArgs& hd, hipStream_t st);
@@ -2107,6 +2110,10 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     const bool gsplit = !ws && (c.weight_format == 0 || pkd);
     auto hidden_splits = [&](int K_) { return !gsplit ? 1 : staged ? engine_gemm_short_splits(H, K_) : engine_gemm_pick_splits(n, H, K_); };
     const int g_so = hidden_splits(QD), g_sd = hidden_splits(I), g_sq = gsplit ? engine_gemm_qkv_splits(n, NQKV, H, D == 128) : 1;
+    // RMSNorm without a pass of its own: o_proj and down_proj leave x = bf16(h gamma) and h's sums of squares, gate_up and QKV scale their rows
+    // (Qwen3-0.6B, 1531 rows: a layer 124 -> 115 us, 3365 rows 193 -> 181).  From 512 rows on: 384 rows took the same with it and without.
+    const bool carry = n >= 512 && !ws && !staged && (c.weight_format == 0 || pkd) && engine_gemm_carry_ok(n, NQKV, H) && engine_gemm_carry_ok(n, 2 * I, H);
+    const bool carry_o = carry && engine_gemm_resid_pays(n, H, QD, g_so), carry_d = carry && g_sq == 1 && engine_gemm_resid_pays(n, H, I, g_sd);
     const bool use_slabs = ws || g_so > 1 || g_sd > 1 || g_sq > 1;
     size_t slab_elems = (size_t)(s_o > s_d ? s_o : s_d) * n * H;
     if ((size_t)(g_so > g_sd ? g_so : g_sd) * n * H > slab_elems) slab_elems = (size_t)(g_so > g_sd ? g_so : g_sd) * n * H;
@@ -2115,7 +2122,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     if (g_sq > 1 && (size_t)g_sq * n * NQKV > slab_elems) slab_elems = (size_t)g_sq * n * NQKV;
     if (s_gu > 1 && (size_t)s_gu * n * 2 * I > slab_elems) slab_elems = (size_t)s_gu * n * 2 * I;
     const size_t need = (size_t)n * H * 4 + ((size_t)n * H + (size_t)n * NQKV + (size_t)n * QD + (size_t)n * 2 * I + (size_t)n * I) * 2 +
-                        (use_slabs ? slab_elems * 4 : 0) + 512 + (c.weight_format == 2 ? 2 * ((size_t)n * maxk + (size_t)n * (maxk / 128) * 4 + 512) : 0);
+                        (use_slabs ? slab_elems * 4 : 0) + (carry ? (size_t)n * ceil_div(H, 64) * 4 : 0) + 512 + (c.weight_format == 2 ? 2 * ((size_t)n * maxk + (size_t)n * (maxk / 128) * 4 + 512) : 0);
     if (need > e->pf_bytes) {
         if (e->pf) PGK_CHECK_HIP(hipStreamSynchronize(st));
         if (e->pf) pgk_free(e->pf);
@@ -2162,10 +2169,12 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     bf16* gu = (bf16*)p; p += (size_t)n * 2 * I * 2;
     bf16* act = (bf16*)p; p += (size_t)n * I * 2;
     float* slabs = (float*)(((uintptr_t)p + 255) & ~(uintptr_t)255);
+    float* row_ss = slabs + (use_slabs ? slab_elems : 0);                                                     // carried norms: [ceil(H / 64)][n]
     uint8_t* q8 = (uint8_t*)(((uintptr_t)slabs + (use_slabs ? slab_elems * 4 : 0) + 255) & ~(uintptr_t)255);   // fp8 activations [n][maxk]
     float* q8s = (float*)(q8 + (size_t)n * maxk);                                                          // their scales [n][maxk/128]
     uint8_t* q8b = (uint8_t*)(((uintptr_t)(q8s + (size_t)n * (maxk / 128)) + 255) & ~(uintptr_t)255);      // second pair: the gate / up GEMM's
     float* q8bs = (float*)(q8b + (size_t)n * maxk);                                                        // SwiGLU epilogue writes while q8 is its operand
+    NormIn carried_x{};   // how the products that read x scale its rows (null: x is normalised)
     int pending = 0;   // split-K slabs of the previous projection still to be added into h32 by the next norm
     // fp8act: RMSNorm and SwiGLU leave their result in q8/q8s themselves (x_in == nullptr); attention output is
     // quantised here (its rows span all heads, a flash workgroup only sees one)
@@ -2200,6 +2209,13 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         pending = splits;
         return wsgemm_nt(x_in, K_, w, (const bf16*)sc, fp8, slabs, nullptr, 1, splits, n, N_, K_, st);
     };
+    // an N = hidden projection and the norm behind it, where that is carried
+    auto proj_resid = [&](const bf16* x_in, const void* w, const bf16* wp, int K_, const void* gamma) -> pgk_status {
+        NormOut no{};
+        no.gamma = (const bf16*)gamma; no.x = x; no.ss = row_ss;
+        carried_x.ss = row_ss; carried_x.n = H / 64; carried_x.eps = c.norm_eps;
+        return engine_gemm_resid_nt(x_in, pkd ? (const void*)wp : w, h32, n, H, K_, no, st, pkd);
+    };
     // with splits > 1 the result is left as fp32 split-K slabs for the consumer kernel to sum
     auto proj_store = [&](const bf16* x_in, const void* w, const void* sc, bf16* out_, int N_, int K_, int splits, const bf16* wp = nullptr) -> pgk_status {
         if (fp8act) {
@@ -2207,8 +2223,8 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
                 if (pgk_status r = quantize_fp8_rows_bf16(x_in, q8, q8s, n, K_, st)) return r;
             return gemm_fp8_nt(q8, q8s, (const uint8_t*)w, (const bf16*)sc, out_, false, n, N_, K_, st);
         }
-        if (!ws && pkd && wp != nullptr) return engine_gemm_nt(x_in, wp, nullptr, false, out_, false, n, N_, K_, st, true);
-        if (!ws) return engine_gemm_nt(x_in, w, (const bf16*)sc, fp8, out_, false, n, N_, K_, st);
+        if (!ws && pkd && wp != nullptr) return engine_gemm_nt(x_in, wp, nullptr, false, out_, false, n, N_, K_, st, true, carried_x);
+        if (!ws) return engine_gemm_nt(x_in, w, (const bf16*)sc, fp8, out_, false, n, N_, K_, st, false, carried_x);
         if (splits > 1) return wsgemm_nt(x_in, K_, w, (const bf16*)sc, fp8, slabs, nullptr, 1, splits, n, N_, K_, st);
         return wsgemm_nt(x_in, K_, w, (const bf16*)sc, fp8, out_, nullptr, 0, 1, n, N_, K_, st);
     };
@@ -2220,6 +2236,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             rmsnorm_f32_bf16_kernel<16><<<n, 256, 0, st>>>(h32, gamma, x, n, H, c.norm_eps, slabs, pending, to_fp8 ? q8 : nullptr,
                                                            to_fp8 ? q8s : nullptr);
         pending = 0;
+        carried_x = NormIn{};
         PGK_LAUNCH_CHECK();
         return PGK_OK;
     };
@@ -2236,7 +2253,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         const bool carried = pk && e->packed_resid;
         PkArgs nrm{};                                   // how the consumer of x scales its rows (all null: x is normalised)
         if (carried && l > 0) { nrm.ss_in = e->pk_ss; nrm.ss_n = ss_n; nrm.ss_eps = c.norm_eps; }
-        else if (pgk_status r = norm((const bf16*)L.attn_norm, fuse_q)) return r;
+        else if (!carried_x.ss) { if (pgk_status r = norm((const bf16*)L.attn_norm, fuse_q)) return r; }
         if (pk_heads) {
             PkArgs hd = nrm;
             hd.q_gamma = c.use_qk_norm ? (const bf16*)L.q_norm : nullptr;
@@ -2257,7 +2274,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
                 if (pgk_status r = gemm_fp8_qkv_heads_nt(q8, q8s, (const uint8_t*)L.w_qkv, (const bf16*)L.s_qkv, qkv, n, NQKV, H, hd, st)) return r;
             } else if (staged) {
                 if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].qkv : L.w_qkv, qkv, 3, 1, n, NQKV, H, st, pkd, &hd)) return r;
-            } else if (pgk_status r = engine_gemm_qkv_heads_nt(x, pkd ? e->packed[l].qkv : (const bf16*)L.w_qkv, qkv, n, NQKV, H, hd, st, pkd)) return r;
+            } else if (pgk_status r = engine_gemm_qkv_heads_nt(x, pkd ? e->packed[l].qkv : (const bf16*)L.w_qkv, qkv, n, NQKV, H, hd, st, pkd, carried_x)) return r;
         } else if (staged || g_sq > 1) {
             if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].qkv : L.w_qkv, g_sq > 1 ? (void*)slabs : qkv, g_sq > 1 ? 2 : 0, g_sq, n, NQKV, H, st, pkd)) return r;
         } else {
@@ -2314,8 +2331,15 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             continue;
         }
         if (pk) { if (pgk_status r = pk_accum(attn, e->packed[l].o, QD, pk_so)) return r; }
+        else if (carry_o) { if (pgk_status r = proj_resid(attn, L.w_o, pkd ? e->packed[l].o : nullptr, QD, L.mlp_norm)) return r; }
         else if (pgk_status r = proj_accum(attn_q8 ? nullptr : attn, L.w_o, L.s_o, H, QD, s_o, pkd ? e->packed[l].o : nullptr)) return r;
-        if (pgk_status r = norm((const bf16*)L.mlp_norm, fuse_q)) return r;
+        if (!carry_o)
+            if (pgk_status r = norm((const bf16*)L.mlp_norm, fuse_q)) return r;
+        auto down = [&]() -> pgk_status {       // (behind the last layer: the norm's own pass)
+            if (carry_d && l + 1 < c.num_layers) return proj_resid(act, L.w_down, pkd ? e->packed[l].down : nullptr, I, e->layers[l + 1].attn_norm);
+            carried_x = NormIn{};
+            return proj_accum(fuse_q ? nullptr : act, L.w_down, L.s_down, H, I, s_d, pkd ? e->packed[l].down : nullptr);
+        };
         if (pk) {
             // SwiGLU inside the gate_up projection: the gate tile and its up tile live in the same wave
             if (pgk_status r = pkgemm_nt(x, H, e->packed[l].gate_up, act, I, PK_EPI_SWIGLU, 1, n, 2 * I, H, nullptr, st)) return r;
@@ -2331,15 +2355,15 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         if (fuse_sw16) {
             if (staged) {
                 if (pgk_status r = engine_gemm_short(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, act, 4, 1, n, I, H, st, pkd)) return r;
-            } else if (pgk_status r = engine_gemm_swiglu_nt(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, (const bf16*)L.s_gate_up, fp8 && !pkd, act, n, I, H, st, pkd)) return r;
-            if (pgk_status r = proj_accum(act, L.w_down, L.s_down, H, I, s_d, pkd ? e->packed[l].down : nullptr)) return r;
+            } else if (pgk_status r = engine_gemm_swiglu_nt(x, pkd ? (const void*)e->packed[l].gate_up : L.w_gate_up, (const bf16*)L.s_gate_up, fp8 && !pkd, act, n, I, H, st, pkd, carried_x)) return r;
+            if (pgk_status r = down()) return r;
             continue;
         }
         if (pgk_status r = proj_store(fuse_q ? nullptr : x, L.w_gate_up, L.s_gate_up, gu, 2 * I, H, s_gu, pkd ? e->packed[l].gate_up : nullptr)) return r;
         swiglu_rows_kernel<<<ceil_div((long long)n * I / 8, 256) > 2048 ? 2048 : ceil_div((long long)n * I / 8, 256), 256, 0, st>>>(
             gu, act, n, I, slabs, s_gu > 1 ? s_gu : 0, fuse_q ? q8 : nullptr, fuse_q ? q8s : nullptr);
         PGK_LAUNCH_CHECK();
-        if (pgk_status r = proj_accum(fuse_q ? nullptr : act, L.w_down, L.s_down, H, I, s_d, pkd ? e->packed[l].down : nullptr)) return r;
+        if (pgk_status r = down()) return r;
     }
     if (pgk_status r = norm(e->final_norm)) return r;
     if (all_logits) {

@@ -18,6 +18,32 @@ struct QkvHeadArgs {
     const int2* at;
     long long slot_stride;
 };
+// An RMSNorm between two products without a pass of its own.  The product before it (its residual epilogue) leaves x = bf16(h gamma) and, per row and 64
+// columns, h's sum of squares; the product behind it reads x and scales its result rows by 1 / rms, which a factor per row may as well do after the sum.
+struct NormIn { const float* ss; int n; float eps; };      // ss [n][rows]; null: x is normalised
+struct NormOut { const bf16* gamma; bf16* x; float* ss; };  
+// 1 / rms of a row of K values
+__device__ __forceinline__ float norm_in_scale(const NormIn& nn, int row, int rows, int K) {
+    float s = 0.f;
+    for (int i = 0; i < nn.n; i += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = nn.ss[(size_t)min(i + j, nn.n - 1) * rows + row];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += i + j < nn.n ? v[j] : 0.f;
+    }
+    return 1.0f / sqrtf(s / K + nn.eps);
+}
+// Residual epilogue of four columns of a row (gamma: g), held by one of 16 lanes that have 64: h (already stored) -> x and the sum of squares.  All lanes must be active.
+__device__ __forceinline__ void norm_out_row(const float4& v, uint2 g, bool live, int row, int col, int rows, int N, const NormOut& no) {
+    const float ss = group16_sum(live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f);
+    if (!live) return;
+    uint2 o;
+    o.x = pack_bf16x2(v.x * __uint_as_float(g.x << 16), v.y * __uint_as_float(g.x & 0xFFFF0000u));
+    o.y = pack_bf16x2(v.z * __uint_as_float(g.y << 16), v.w * __uint_as_float(g.y & 0xFFFF0000u));
+    *reinterpret_cast<uint2*>(no.x + (size_t)row * N + col) = o;
+    if ((col & 63) == 0) no.ss[(size_t)(col >> 6) * rows + row] = ss;
+}
 struct ActArgs { float pos, neg; bool gelu; };     // pgk_device.hip.h: xielu's factors, or gelu_erf
 
 // Head slots of the bf16-rounded QKV projection of ROWS token rows, row0 + step i: 16 lanes hold one row's 128 dims, 8 each (sub = lane's chunk).

@@ -23,14 +23,15 @@ pgk_status wsgemm_nt(const bf16* a, int lda, const void* w, const bf16* wscale, 
 // (packed: W is the fragment-major bf16 copy of ops_pkgemm.hip instead of the row-major weight - the staged kernels' DMA
 // instruction moves 16 rows x 32 k, which is one block of that layout)
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
-                           hipStream_t st, bool packed = false, const ActArgs* act = nullptr);
-pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed = false);
+                           hipStream_t st, bool packed = false, const ActArgs* act = nullptr, const NormIn& ni = NormIn{});
+pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed = false, const NormIn& ni = NormIn{});
 bool gemm256_bf16_qkv_heads_ok(int M, int N, int K);
-pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed);
+pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni);
 bool gemm128s_shape_ok(int N, int K);
 bool gemm128s_ok(int M, int N, int K);    // ops_gemm256.hip: 128 x 128 tiles on the staged LDS-DMA pipeline (bf16, M > 128, K % 64 == 0, N % 8 == 0)
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
-                            const QkvHeadArgs* heads = nullptr, bool packed = false, const ActArgs* act = nullptr);
+                            const QkvHeadArgs* heads = nullptr, bool packed = false, const ActArgs* act = nullptr, const NormIn& ni = NormIn{}, const NormOut& no = NormOut{});
+bool gemm128s_resid_pays(int M, int N, int K, int splits);
 // the 256 x 256 structure needs enough tiles to fill the chip and whole 128-byte K rows
 // PGK_GEMM256 = 0 / 1 forces the choice (read per call: tests flip it to drive small shapes through both kernels); shared
 // with the fp8 x fp8 GEMM (ops_fp8_gemm.hip)
@@ -439,15 +440,25 @@ pgk_status engine_gemm_nt_slabs(const bf16* A, const void* W, float* slabs, int 
 // internal (engine prefill): bf16 A against a bf16 or fp8 (+128x128 bf16 block scales) weight W[N,K];
 // either a bf16 result or an fp32 "+=" into the residual stream.
 // the shapes whose kernels can read the fragment-major bf16 copy (engine_gemm_nt and friends with packed = true)
+// the shapes whose kernels scale the rows of a carried norm (NormIn), bf16 weights, row-major or packed
+bool engine_gemm_carry_ok(int M, int N, int K) { return use_gemm256(M, N, K) || gemm128s_ok(M, N, K); }
+// h += A . W^T with x = bf16(h gamma) and h's sums of squares for the next product; `splits`: what the product would be split into without.  Not on the 256-tile
+// kernel: 4096 rows of Llama-3-8B take as long with it, what the two passes of 18 us cost comes back in its epilogues (o 108 / 114, down 323 / 333, gate_up 670 / 678).
+bool engine_gemm_resid_pays(int M, int N, int K, int splits) { return !use_gemm256(M, N, K) && gemm128s_ok(M, N, K) && gemm128s_resid_pays(M, N, K, splits); }
+pgk_status engine_gemm_resid_nt(const bf16* A, const void* W, float* h, int M, int N, int K, const NormOut& no, hipStream_t st, bool packed) {
+    PGK_REQUIRE(gemm128s_ok(M, N, K), "engine_gemm_resid: M=%d N=%d K=%d outside the fused kernel's shapes", M, N, K);
+    return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, h, 5, 1, M, N, K, st, nullptr, packed, nullptr, NormIn{}, no);
+}
 bool engine_gemm_packed_ok(int M, int N, int K) { return N % 16 == 0 && K % 64 == 0 && (use_gemm256(M, N, K) || gemm128s_ok(M, N, K)); }
 
 pgk_status engine_gemm_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, void* C, bool accum_f32, int M,
-                          int N, int K, hipStream_t st, bool packed) {
+                          int N, int K, hipStream_t st, bool packed, const NormIn& ni) {
     if (packed) {
         PGK_REQUIRE(!fp8 && engine_gemm_packed_ok(M, N, K), "engine_gemm_nt: M=%d N=%d K=%d has no kernel that reads the fragment-major copy", M, N, K);
-        if (use_gemm256(M, N, K)) return gemm256_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32, M, N, K, st, true);
-        return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32 ? 1 : 0, 1, M, N, K, st, nullptr, true);
+        if (use_gemm256(M, N, K)) return gemm256_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32, M, N, K, st, true, nullptr, ni);
+        return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32 ? 1 : 0, 1, M, N, K, st, nullptr, true, nullptr, ni);
     }
+    PGK_REQUIRE(!ni.ss || (!fp8 && engine_gemm_carry_ok(M, N, K)), "engine_gemm_nt: M=%d N=%d K=%d has no kernel that scales its rows", M, N, K);
     if (fp8 && use_gemm256(M, N, K) && K % 128 == 0 && N % 128 == 0) {
         // large w8a16 products: dequantise the weight once into a bf16 scratch (a ~10 % extra pass over memory) and run
         // the LDS-DMA bf16 kernel, instead of dequantising in the staging path of the 128-tile kernel (0.58 vs ~1 PFLOP/s)
@@ -464,8 +475,8 @@ pgk_status engine_gemm_nt(const bf16* A, const void* W, const bf16* wscale, bool
         if (accum_f32) return dispatch_mfma<bf16, B_NT_FP8, 1>(A, W, wscale, nullptr, C, M, N, K, st);
         return dispatch_mfma<bf16, B_NT_FP8, 0>(A, W, wscale, nullptr, C, M, N, K, st);
     }
-    if (use_gemm256(M, N, K)) return gemm256_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32, M, N, K, st);
-    if (gemm128s_ok(M, N, K)) return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32 ? 1 : 0, 1, M, N, K, st);
+    if (use_gemm256(M, N, K)) return gemm256_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32, M, N, K, st, false, nullptr, ni);
+    if (gemm128s_ok(M, N, K)) return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, C, accum_f32 ? 1 : 0, 1, M, N, K, st, nullptr, false, nullptr, ni);
     if (accum_f32) return dispatch_mfma<bf16, B_NT, 1>(A, W, nullptr, nullptr, C, M, N, K, st);
     return dispatch_mfma<bf16, B_NT, 0>(A, W, nullptr, nullptr, C, M, N, K, st);
 }
@@ -484,10 +495,10 @@ pgk_status engine_gemm_act_nt(const bf16* A, const bf16* W, bf16* act, int M, in
 bool engine_gemm_qkv_heads_ok(int M, int N, int K) {
     return use_gemm256(M, N, K) ? gemm256_bf16_qkv_heads_ok(M, N, K) : N % 128 == 0 && gemm128s_ok(M, N, K);
 }
-pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed) {
+pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni) {
     PGK_REQUIRE(engine_gemm_qkv_heads_ok(M, N, K), "engine_gemm_qkv_heads: M=%d N=%d K=%d outside the fused kernels' shapes", M, N, K);
-    if (use_gemm256(M, N, K)) return gemm256_bf16_qkv_heads_nt(A, W, qkv, M, N, K, hd, st, packed);
-    return gemm128s_bf16_nt(A, W, nullptr, qkv, 3, 1, M, N, K, st, &hd, packed);
+    if (use_gemm256(M, N, K)) return gemm256_bf16_qkv_heads_nt(A, W, qkv, M, N, K, hd, st, packed, ni);
+    return gemm128s_bf16_nt(A, W, nullptr, qkv, 3, 1, M, N, K, st, &hd, packed, nullptr, ni);
 }
 
 // internal (engine prefill): act[M][I] = bf16(silu(A . Wg^T) * (A . Wu^T)) on the fused [2 I, K] gate / up weight (bf16, or fp8 with
@@ -498,10 +509,11 @@ bool engine_gemm_swiglu_ok(int M, int I, int K, bool fp8) {
     if (I % 128 == 0 && use_gemm256(M, 2 * I, K) && (!fp8 || K % 128 == 0)) return true;
     return !fp8 && I % 64 == 0 && gemm128s_ok(M, I, K);
 }
-pgk_status engine_gemm_swiglu_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, bf16* act, int M, int I, int K, hipStream_t st, bool packed) {
+pgk_status engine_gemm_swiglu_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, bf16* act, int M, int I, int K, hipStream_t st, bool packed, const NormIn& ni) {
     PGK_REQUIRE(engine_gemm_swiglu_ok(M, I, K, fp8) && !(packed && fp8), "engine_gemm_swiglu: M=%d I=%d K=%d outside the fused kernel's shapes", M, I, K);
-    if (!(I % 128 == 0 && use_gemm256(M, 2 * I, K))) return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, act, 4, 1, M, I, K, st, nullptr, packed);
-    if (!fp8) return gemm256_bf16_swiglu_nt(A, (const bf16*)W, act, M, I, K, st, packed);
+    if (!(I % 128 == 0 && use_gemm256(M, 2 * I, K))) return gemm128s_bf16_nt(A, (const bf16*)W, nullptr, act, 4, 1, M, I, K, st, nullptr, packed, nullptr, ni);
+    if (!fp8) return gemm256_bf16_swiglu_nt(A, (const bf16*)W, act, M, I, K, st, packed, ni);
+    PGK_REQUIRE(!ni.ss, "engine_gemm_swiglu: e4m3 weights without a copy take normalised rows");
     void* wb = nullptr;
     if (pgk_status r = pgk_malloc(&wb, (size_t)2 * I * K * sizeof(bf16))) return r;
     const size_t chunks = (size_t)2 * I * K / 16;
@@ -571,7 +583,7 @@ pgk_status pgk_w8a16_gemm_nk(const void* a, const uint8_t* w_nk, const void* sca
     PGK_REQUIRE(aligned16(a) && aligned16(w_nk), "pgk_w8a16_gemm_nk: operands must be 16-byte aligned");
     if (!m) return PGK_OK;
     if (m <= 128) return wsgemm_nt((const bf16*)a, k, w_nk, (const bf16*)scale, true, c, nullptr, 0, 1, m, n, k, resolve_stream(s));
-    return engine_gemm_nt((const bf16*)a, w_nk, (const bf16*)scale, true, c, false, m, n, k, resolve_stream(s), false);
+    return engine_gemm_nt((const bf16*)a, w_nk, (const bf16*)scale, true, c, false, m, n, k, resolve_stream(s), false, NormIn{});
 }
 
 pgk_status pgk_w8a16_gemm_kn(const void* a, const uint8_t* b_kn, const void* scale, void* c, int m, int n, int k,

@@ -21,6 +21,8 @@
 #include "moe.hip.h"
 #include "pgk_internal.h"
 
+#include <climits>
+
 namespace pgk {
 
 typedef __bf16 bf16x8_g __attribute__((ext_vector_type(8)));
@@ -333,10 +335,11 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256_bf16_kernel(const bf16* A,
 constexpr int G2S_ARING = 6;      // slots of A, in stages
 constexpr size_t G2S_LDS = (G2S_ARING + 4) * (size_t)256 * 64;
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store;
-// 5: QKV heads (QkvHeadArgs; a tile holds two head slots, N % 256 == 0).  Qwen3-0.6B, 3365 rows: 38 us and 14 of the separate pass -> 42.
+// 5: QKV heads (QkvHeadArgs; a tile holds two head slots, N % 256 == 0).  Qwen3-0.6B, 3365 rows: 38 us and 14 of the separate pass -> 38.
+// EPI 0, 2, 5: rows scaled by NormIn where given.
 template <int EPI, int TN = 4>
 __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                    int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa = ActArgs{}, QkvHeadArgs hd = QkvHeadArgs{}) {
+                                                                    int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa, QkvHeadArgs hd, NormIn ni) {
     static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
@@ -412,6 +415,12 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     stage_w(1, 1);
     stage_w(2, 2);
     int a_cur = 0;                                           // ring slot of A's stage s
+    // 1 / rms of row tid, where a register is left for it through the loop
+    constexpr bool EARLY = (EPI == 0 || EPI == 2) && TN == 3;
+    float mine = 0.f;
+    if constexpr (EARLY) {
+        if (ni.ss && tid < 256) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
+    }
     wait_two_younger();
     __builtin_amdgcn_s_barrier();
     if (late) __builtin_amdgcn_s_barrier();                  // waves 4-7 start one phase behind
@@ -454,6 +463,21 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     if (!late) __builtin_amdgcn_s_barrier();                 // match the extra barrier of waves 4-7
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // retire the phantom DMAs before the LDS is given back
 
+    if constexpr (EPI == 0 || EPI == 2 || EPI == 5) {
+        if (ni.ss) {
+            float* inv = reinterpret_cast<float*>(g2_smem + 256 * 512);          // behind the epilogues' tile
+            if (!EARLY && tid < 256) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
+            __builtin_amdgcn_s_barrier();                    // every wave is past its last operand read
+            if (tid < 256) inv[tid] = mine;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f32x4_g f = *reinterpret_cast<const f32x4_g*>(inv + wr * 128 + i * 16 + q * 4);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] *= f;
+            }
+        }
+    }
     if constexpr (EPI == 2) {
         g2_swiglu_epilogue<false, TN>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
         return;
@@ -495,8 +519,8 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 // of a 128 x 128 tile took 0.25 us with one workgroup on the CU, half of it DMA issue (0.19 without the fragment reads, 0.12 for the DMA alone, 0.11 for
 // the products alone).  So waves 4-7 issue all of it and waves 0-3 never do; the fragments of stage s + 1 are requested between the products of stage s,
 // each into the registers its row of products has just read (W's, and the last row's, into a second set).  0.17-0.18 us a stage.
-// One barrier per stage: behind it stage s + 1 has landed (the DMA waves have waited for their shares) and stage s has been read, so W of s + 4 and,
-// where s is odd, A of s + 5 and s + 6 take its place.  Between W of a stage and the wait for it lie W of two stages and A of one pair.
+// One barrier per stage: behind it stage s + 1 has landed (the DMA waves have waited for their shares) and stage s has been read, so W of s + RW and,
+// where s is odd, A of s + RA - 1 and s + RA take its place.
 //   us a launch, before / after (K = 1024, packed W): 1531 rows, N = 6144 28.0 / 23.0 on 192 x 192 tiles, N = 4096 20.3 / 16.6 on 192 x 128; 384 rows,
 //   N = 6144 12.7 / 10.8; K = 3072, N = 1024, 3365 rows 28.3 / 23.4.
 // blockIdx.y = K split (EPI 2: fp32 slab z of [splits][M][N], summed by the consumer).
@@ -504,19 +528,23 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 // quarters XOR-ed apart, then back as rows for coalesced stores (EPI 1: float4 read-modify-write of the residual stream, all loads issued before the first
 // store).
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: fp32 split-K slab; 3: QKV heads (QkvHeadArgs: tile column = head slot);
-// 4: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]; tile tn = act columns [16 WN tn, +16 WN)); 5: xIELU, 7: gelu, bf16 store
+// 4: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]; tile tn = act columns [16 WN tn, +16 WN)); 5: xIELU, 7: gelu, bf16 store;
+// 8: 1, and what the next RMSNorm leaves to do (NormOut).  EPI 0, 3, 4: rows scaled by NormIn where given
 // GRP: rows sorted by expert (GroupArgs), every tile with its expert's weight; EPI 4, 7, or 6: bf16 rows times their weight, each at its place
 constexpr int GP_THREADS = 512;
+// stages of W that the ring holds; A's has two more.  The smaller tiles' stages are shorter, and latency asks for more of them
+constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 ? 4 : 6; }
 template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
-    const size_t ring = G2S_ARING * (size_t)(32 * WM * 64) + 4 * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
+    const size_t RW = gemmp_ring(WM, WN), ring = (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
     return ring > tile ? ring : tile;
 }
 template <int EPI, bool GRP, int WM, int WN>
 __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                           int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga) {
-    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of AH bytes | W: 4 stages of WH
-    constexpr int BM = 32 * WM, BN = 32 * WN, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
-    constexpr bool B16 = EPI == 3 || EPI == 4;
+                                           int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no) {
+    extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
+    constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
+    constexpr bool B16 = EPI == 3 || EPI == 4, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4);
+    static_assert(!SCALED || BM <= 256, "a row for each of the waves that multiply");
     static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     int tm, tn, m0;
@@ -536,6 +564,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     const int nh = (kend - kbeg) / 32;                       // (kend - kbeg) % 64 == 0: an even number of stages
 
     f32x4_g acc[WM][WN];
+    float mine = 0.f;                                        // 1 / rms of row tid
     const int wr = (wid >> 1) & 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
     if (wid >= 4) {
         const int pw = __builtin_amdgcn_readfirstlane(wid & 3);
@@ -568,41 +597,45 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         };
         auto stage_w = [&](int h, int buf) {
             const size_t kw = (size_t)min(h, nh - 1) * wk;
-            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + G2S_ARING * AH + buf * WH + pw * NW * 1024);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + RA * AH + buf * WH + pw * NW * 1024);
 #pragma unroll
             for (int i = 0; i < NW; ++i) g2_dma16(w_src[i] + kw, dst + i * 1024);
         };
-        auto wait_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + 2 * NW) : "memory"); };
+        // between W of a stage and the wait for it: W of RW - 2 stages and their A
+        auto wait_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RW - 2) * NW + (RW - 2) / 2 * NA) : "memory"); };
         stage_a(0, 0);
-        stage_w(0, 0);
-        stage_a(2, 2 * AH);
-        stage_w(1, 1);
-        stage_w(2, 2);
-        stage_a(4, 4 * AH);
-        stage_w(3, 3);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NA + 3 * NW) : "memory");   // stage 0
+#pragma unroll
+        for (int t = 0; t < RW; ++t) {
+            if (t & 1) stage_a(t + 1, (t + 1) * AH);
+            stage_w(t, t);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RW - 1) * NW + RW / 2 * NA) : "memory");   // stage 0
         __builtin_amdgcn_s_barrier();
-        int at = 0;
+        int at = 0, buf = 0;
         for (int s = 0; s < nh; s += 2) {
             wait_landed();                                   // stage s + 1
             __builtin_amdgcn_s_barrier();
-            stage_w(s + 4, s & 3);
+            stage_w(s + RW, buf);
             wait_landed();
             __builtin_amdgcn_s_barrier();
-            stage_a(s + 6, at);
-            stage_w(s + 5, (s + 1) & 3);
-            at = at == 4 * AH ? 0 : at + 2 * AH;
+            stage_a(s + RA, at);
+            stage_w(s + RW + 1, buf + 1);
+            at = at == (RA - 2) * AH ? 0 : at + 2 * AH;
+            buf = buf == RW - 2 ? 0 : buf + 2;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // retire the phantom DMAs: the stages become the C tile
         __builtin_amdgcn_s_barrier();
     } else {
+        if constexpr (SCALED && EPI != 0) {
+            if (ni.ss && tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
+        }
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
             for (int j = 0; j < WN; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
         const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
         const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
-        const int a_base = wr * 16 * WM * 128, w_base = G2S_ARING * AH + wc * 16 * WN * 64 + w_off;
+        const int a_base = wr * 16 * WM * 128, w_base = RA * AH + wc * 16 * WN * 64 + w_off;
         auto frag = [&](const char* p) { return *reinterpret_cast<const bf16x8_g*>(p); };
         bf16x8_g fa[WM - 1], fl[2], fb[2][WN];               // A's rows but the last, the last, W's
         __builtin_amdgcn_s_barrier();
@@ -614,7 +647,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 #pragma unroll
             for (int j = 0; j < WN; ++j) fb[0][j] = frag(Ws + j * 1024);
         }
-        int a_cur = 0;                                       // ring slot of A's stage s
+        int a_cur = 0, w_cur = 0;                            // ring slots of stage s
 #define GP_MFMA(I, F, P)                                                                                     \
     _Pragma("unroll") for (int j = 0; j < WN; ++j) acc[I][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(F, fb[P][j], acc[I][j], 0, 0, 0); \
     __builtin_amdgcn_sched_barrier(0);
@@ -624,21 +657,18 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   /* stage s in registers: its place may be refilled */ \
         __builtin_amdgcn_s_barrier();                                                                        \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
-        const int a_nxt = P ? (a_cur == 4 * AH ? 0 : a_cur + 2 * AH) : a_cur;                                \
+        const int a_nxt = P ? (a_cur == (RA - 2) * AH ? 0 : a_cur + 2 * AH) : a_cur;                         \
+        if constexpr (RW == 4) w_cur = (((BUF) + 1) & 3) * WH;                                               \
+        else w_cur = w_cur == (RW - 1) * WH ? 0 : w_cur + WH;                                                \
         const char* As = g2_smem + a_nxt + a_base + (P ? a_off0 : a_off1);                                   \
-        const char* Ws = g2_smem + (((BUF) + 1) & 3) * WH + w_base;                                          \
-        GP_MFMA(0, fa[0], P)                                                                                 \
-        fa[0] = frag(As);                                                                                    \
-        fl[P ^ 1] = frag(As + (WM - 1) * 2048);                                                              \
-        _Pragma("unroll") for (int j = 0; j < WN / 2; ++j) fb[P ^ 1][j] = frag(Ws + j * 1024);               \
-        __builtin_amdgcn_sched_barrier(0);                                                                   \
-        GP_MFMA(1, fa[1], P)                                                                                 \
-        fa[1] = frag(As + 2048);                                                                             \
-        _Pragma("unroll") for (int j = WN / 2; j < WN; ++j) fb[P ^ 1][j] = frag(Ws + j * 1024);              \
-        __builtin_amdgcn_sched_barrier(0);                                                                   \
-        _Pragma("unroll") for (int i = 2; i < WM - 1; ++i) {                                                 \
+        const char* Ws = g2_smem + w_cur + w_base;                                                           \
+        _Pragma("unroll") for (int i = 0; i < WM - 1; ++i) {                                                 \
             GP_MFMA(i, fa[i], P)                                                                             \
             fa[i] = frag(As + i * 2048);                                                                     \
+            if (i == 0) fl[P ^ 1] = frag(As + (WM - 1) * 2048);                                              \
+            if (i < 2) {                                                                                     \
+                _Pragma("unroll") for (int j = i * (WN / 2); j < (WM == 2 ? WN : (i + 1) * (WN / 2)); ++j) fb[P ^ 1][j] = frag(Ws + j * 1024); \
+            }                                                                                                \
             __builtin_amdgcn_sched_barrier(0);                                                               \
         }                                                                                                    \
         GP_MFMA(WM - 1, fl[P], P)                                                                            \
@@ -663,6 +693,24 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     HeadRows<EPI == 3 ? BM / 32 : 1> hr;
     const int hrow = tid >> 4;                               // EPI 3: 16 consecutive lanes = one (token row, head)
     if constexpr (EPI == 3) hr.places(m0 + hrow, 32, M, hd);
+    if constexpr (SCALED) {
+        if (ni.ss) {
+            float* inv = reinterpret_cast<float*>(g2_smem + BM * ROWB);          // behind the tile, where the last stages were
+            if constexpr (EPI == 0) {                        // (held through the loop it is spilled; no engine's step comes here unless PGK_FUSED_EPILOGUES is 0)
+                if (tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
+            }
+            if (tid < BM) inv[tid] = mine;
+            __syncthreads();
+            if (wid < 4) {
+#pragma unroll
+                for (int i = 0; i < WM; ++i) {
+                    const f32x4_g f = *reinterpret_cast<const f32x4_g*>(inv + wr * 16 * WM + i * 16 + q * 4);
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) acc[i][j] *= f;
+                }
+            }
+        }
+    }
     if (wid < 4) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
@@ -677,23 +725,25 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     }
     if constexpr (EPI == 3) hr.angles((tid & 15), tn, hd);
     auto tile4 = [&](int row, int byte) { return *reinterpret_cast<const float4*>(g2_smem + row * ROWB + (byte ^ (((row >> 2) & 3) << QS))); };
-    if constexpr (EPI == 1) {
+    if constexpr (EPI == 1 || EPI == 8) {
         constexpr int IT = BM * (BN / 4) / GP_THREADS;
+        const int c = tid % (BN / 4), gcol = n0 + c * 4;     // a thread's columns are the same in all its rows
         float4 old[IT];
+        uint2 gamma = make_uint2(0, 0);
+        if constexpr (EPI == 8) gamma = *reinterpret_cast<const uint2*>(no.gamma + min(gcol, N - 4));
 #pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int item = it * GP_THREADS + tid, row = item / (BN / 4), c = item % (BN / 4);
-            old[it] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(Cv) + (size_t)min(m0 + row, M - 1) * N + min(n0 + c * 4, N - 4));
-        }
+        for (int it = 0; it < IT; ++it)
+            old[it] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(Cv) + (size_t)min(m0 + (it * GP_THREADS + tid) / (BN / 4), M - 1) * N + min(gcol, N - 4));
         __syncthreads();
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
-            const int item = it * GP_THREADS + tid, row = item / (BN / 4), c = item % (BN / 4);
+            const int row = (it * GP_THREADS + tid) / (BN / 4), grow = m0 + row;
             float4 v = tile4(row, c * 16);
-            const int grow = m0 + row, gcol = n0 + c * 4;
-            if (grow >= M || gcol >= N) continue;
+            const bool live = grow < M && gcol < N;
+            if (EPI == 1 && !live) continue;
             v.x += old[it].x; v.y += old[it].y; v.z += old[it].z; v.w += old[it].w;
-            *reinterpret_cast<float4*>(reinterpret_cast<float*>(Cv) + (size_t)grow * N + gcol) = v;
+            if (live) *reinterpret_cast<float4*>(reinterpret_cast<float*>(Cv) + (size_t)grow * N + gcol) = v;
+            if constexpr (EPI == 8) norm_out_row(v, gamma, live, grow, gcol, M, N, no);
         }
         return;
     }
@@ -770,15 +820,15 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
     }
 }
-// (128 x 128: two workgroups a CU, 80 KiB of LDS and 128 registers each; the larger ones have a CU to themselves)
+// (up to 128 x 128: two workgroups a CU, 80 KiB of LDS and 128 registers each; the larger ones have a CU to themselves)
 template <int EPI, int WM, int WN>
-__global__ __launch_bounds__(GP_THREADS, WM * WN == 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa) {
-    gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{});
+__global__ __launch_bounds__(GP_THREADS, WM * WN <= 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
+                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa, NormIn ni, NormOut no) {
+    gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{}, ni, no);
 }
 template <int EPI>
 __global__ __launch_bounds__(GP_THREADS, 4) void gemmp_grouped_kernel(const bf16* A, const bf16* W, bf16* C, int N, int K, int ntn, GroupArgs ga) {
-    gemmp_body<EPI, true, 4, 4>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga);
+    gemmp_body<EPI, true, 4, 4>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga, NormIn{}, NormOut{});
 }
 
 // ---- fp8 x fp8 with 128-wide block scales on the same structure --------------------------------------------
@@ -1077,7 +1127,7 @@ static bool gemm256_narrow(int M, int N) {
 
 // QKV projection finished head by head: where whole 256-column tiles are what gemm256_bf16_nt would take
 bool gemm256_bf16_qkv_heads_ok(int M, int N, int K) { return K % 64 == 0 && K >= 64 && N % 256 == 0 && !gemm256_narrow(M, N); }
-pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed) {
+pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni) {
     PGK_REQUIRE(gemm256_bf16_qkv_heads_ok(M, N, K) && N == (hd.hq + 2 * hd.hkv) * 128, "gemm256 heads: N=%d K=%d (%d + 2 x %d heads)", N, K, hd.hq, hd.hkv);
     static bool attr_done = false;
     if (!attr_done) {
@@ -1085,14 +1135,14 @@ pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, in
         attr_done = true;
     }
     const int ntm = ceil_div(M, G2_BM), ntn = N / G2_BN;
-    gemm256s_bf16_kernel<5><<<ntm * ntn, G2_THREADS, G2S_LDS, st>>>(A, W, nullptr, qkv, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, hd);
+    gemm256s_bf16_kernel<5><<<ntm * ntn, G2_THREADS, G2S_LDS, st>>>(A, W, nullptr, qkv, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, hd, ni);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
 
 // bf16 NT on the 256^2 structure; caller guarantees K % 64 == 0 and 16-byte aligned rows
 pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, bool accum_f32, int M, int N, int K,
-                           hipStream_t st, bool packed, const ActArgs* act) {
+                           hipStream_t st, bool packed, const ActArgs* act, const NormIn& ni) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64, "gemm256: K=%d must be a multiple of 64", K);
     PGK_REQUIRE(!packed || N % 16 == 0, "gemm256: the fragment-major weight copy has whole 16-row tiles (N=%d)", N);
     constexpr size_t LDS = G2S_LDS;
@@ -1104,7 +1154,7 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
     }
     const int ntm = ceil_div(M, G2_BM), ntn = ceil_div(N, G2_BN);
     const char* e = getenv("PGK_GEMM256S");          // 0: two full stages, waves in lockstep; default: staggered phases
-    if (packed || act || !e || atoi(e) != 0) {
+    if (packed || act || ni.ss || !e || atoi(e) != 0) {
         static bool attr_s = false;
         if (!attr_s) {
             PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
@@ -1124,16 +1174,16 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
                 static bool attr_x[2] = {false, false};
                 if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
                 attr_x[act->gelu] = true;
-                kfn<<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn3, packed ? 1 : 0, *act, QkvHeadArgs{});
-            } else gemm256s_bf16_kernel<0, 3><<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn3, packed ? 1 : 0, ActArgs{});
+                kfn<<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn3, packed ? 1 : 0, *act, QkvHeadArgs{}, NormIn{});
+            } else gemm256s_bf16_kernel<0, 3><<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn3, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
         } else if (act) {
             auto kfn = act->gelu ? &gemm256s_bf16_kernel<4> : &gemm256s_bf16_kernel<3>;
             static bool attr_x[2] = {false, false};
             if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
             attr_x[act->gelu] = true;
-            kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, *act, QkvHeadArgs{});
-        } else if (accum_f32) gemm256s_bf16_kernel<1><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{});
-        else gemm256s_bf16_kernel<0><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{});
+            kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, *act, QkvHeadArgs{}, NormIn{});
+        } else if (accum_f32) gemm256s_bf16_kernel<1><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, NormIn{});
+        else gemm256s_bf16_kernel<0><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
         PGK_CHECK_HIP(hipGetLastError());
         return PGK_OK;
     }
@@ -1144,7 +1194,7 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
 }
 
 // act[M][I] = bf16(silu(A . Wg^T) * (A . Wu^T)), W = fused [2 I, K] gate / up weight (staggered kernel, SwiGLU epilogue)
-pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed) {
+pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M, int I, int K, hipStream_t st, bool packed, const NormIn& ni) {
     PGK_REQUIRE(K % 64 == 0 && K >= 64 && I % 128 == 0, "gemm256 swiglu: K=%d must be a multiple of 64 and I=%d of 128", K, I);
     constexpr size_t LDS = G2S_LDS;
     static bool attr_done = false;
@@ -1157,9 +1207,9 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
     // 96 act columns per tile (192-column B tiles) when that fills the rounds of the chip better: Qwen3-0.6B at S = 2048 is
     // 8 x 24 = 192 tiles of 128 (three quarters of the CUs, one round) or 8 x 32 = 256 tiles of 96 (all of them)
     if (I % 96 == 0 && 0.75 * ceil_div(ntm * (I / 96), 256) < (double)ceil_div(ntm * ntn, 256) - 0.01) {
-        gemm256s_bf16_kernel<2, 3><<<ntm * (I / 96), G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, I / 96, packed ? 1 : 0, ActArgs{});
+        gemm256s_bf16_kernel<2, 3><<<ntm * (I / 96), G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, I / 96, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
     } else {
-        gemm256s_bf16_kernel<2><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, ntn, packed ? 1 : 0, ActArgs{});
+        gemm256s_bf16_kernel<2><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
     }
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
@@ -1167,7 +1217,7 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
 
 template <int EPI, int WM, int WN>
 static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, void* C, int M, int N, int K, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa,
-                               hipStream_t st) {
+                               const NormIn& ni, const NormOut& no, hipStream_t st) {
     constexpr size_t LDS = gemmp_lds<WM, WN, EPI == 3 || EPI == 4>();
     static bool attr_done = false;
     if (!attr_done) {
@@ -1175,7 +1225,7 @@ static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, v
         attr_done = true;
     }
     const int ntm = ceil_div(M, 32 * WM), ntn = EPI == 4 ? ceil_div(N, 16 * WN) : ceil_div(N, 32 * WN);      // SwiGLU: N = I act columns, half a tile's
-    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa);
+    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa, ni, no);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
@@ -1196,34 +1246,66 @@ static int gemmp_tile(int M, int cols, int K, bool wide) {
     return best;
 }
 
+// The same for a product that ends in the residual epilogue with a norm (nothing of it splits along K, so few rows ask for small tiles).
+// 0: 128 x 128, 1: 128 x 64, 2: 64 x 64, two workgroups on a CU for 0 and 2
+static int gemmp_resid_tile(int M, int N, int K, int* cost) {
+    constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 450, 29, 640}, {128, 64, 14, 400, 0, 0}, {64, 64, 11, 300, 16, 400}};
+    int best = 0;
+    for (int i = 0; i < 3; ++i) {
+        const long long n = (long long)ceil_div(M, t[i].bm) * ceil_div(N, t[i].bn), stages = K / 32;
+        const long long one = stages * t[i].one + t[i].one_fixed, two = stages * t[i].two + t[i].two_fixed;
+        const long long c = t[i].two ? n / 512 * two + (n % 512 > 256 ? two : n % 512 > 0 ? one : 0) : ceil_div(n, 256LL) * one;
+        if (i == 0 || c < *cost) { best = i; *cost = (int)(c < INT_MAX ? c : INT_MAX); }
+    }
+    return best;
+}
+// Whether that epilogue pays against a product in `splits` slabs (or `splits` = 1, fp32 +=) and the norm's pass, which takes 6 us and a launch, less what
+// the scaled rows cost the next product.  Qwen3-0.6B, us with the norm: 1531 rows o 20.7 / 14.5, down 25 / 20; 384 rows 15 / 11, 17.5 / 14.5.
+bool gemm128s_resid_pays(int M, int N, int K, int splits) {
+    if (N % 64 != 0) return false;
+    if (splits == 1) return true;
+    int cost;
+    gemmp_resid_tile(M, N, K, &cost);
+    return cost <= K / splits / 32 * 18 + 260 + 720;
+}
+
 // mode 0: bf16 C (+bias, or with `act` its activation), 1: fp32 C +=, 2: fp32 slabs [splits][M][N] (K split into `splits` runs of whole 64-k steps),
-// 3: QKV heads, 4: SwiGLU
+// 3: QKV heads, 4: SwiGLU, 5: 1 with what the next RMSNorm leaves to do (NormOut); 0, 3, 4: rows scaled by NormIn where given
 bool gemm128s_shape_ok(int N, int K) { return K % 64 == 0 && K >= 64 && N % 8 == 0 && N >= 8; }
 bool gemm128s_ok(int M, int N, int K) { return M > 128 && gemm128s_shape_ok(N, K); }
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
-                            const QkvHeadArgs* heads, bool packed, const ActArgs* act) {
+                            const QkvHeadArgs* heads, bool packed, const ActArgs* act, const NormIn& ni, const NormOut& no) {
     PGK_REQUIRE(!packed || N % 16 == 0, "gemm128s: the fragment-major weight copy has whole 16-row tiles (N=%d)", N);
     const int pk = packed ? 1 : 0;
-    PGK_REQUIRE(M >= 1 && gemm128s_shape_ok(N, K) && mode >= 0 && mode <= 4 && splits >= 1 && (splits == 1 || mode == 2), "gemm128s: M=%d N=%d K=%d mode=%d splits=%d", M, N, K, mode, splits);
+    PGK_REQUIRE(M >= 1 && gemm128s_shape_ok(N, K) && mode >= 0 && mode <= 5 && splits >= 1 && (splits == 1 || mode == 2), "gemm128s: M=%d N=%d K=%d mode=%d splits=%d", M, N, K, mode, splits);
     PGK_REQUIRE(mode != 4 || N % 64 == 0, "gemm128s: the SwiGLU epilogue needs I=%d to be a multiple of 64", N);
     PGK_REQUIRE(mode != 3 || (heads && N == (heads->hq + 2 * heads->hkv) * 128), "gemm128s: the QKV-heads epilogue needs N=%d = (Hq + 2 Hkv) x 128", N);
+    PGK_REQUIRE(mode != 5 || (N % 64 == 0 && no.gamma && no.x && no.ss), "gemm128s: the residual epilogue with a norm needs N=%d to be a multiple of 64", N);
+    PGK_REQUIRE(!ni.ss || mode == 0 || mode == 3 || mode == 4, "gemm128s: mode %d does not scale its rows", mode);
     const QkvHeadArgs hd = heads ? *heads : QkvHeadArgs{};
     const int kps = ceil_div(ceil_div(K, splits), 64) * 64;
     PGK_REQUIRE(ceil_div(K, kps) == splits, "gemm128s: K=%d does not split into %d runs of whole 64-k steps", K, splits);
     const ActArgs none{};
-    if (mode == 0 && act && act->gelu) return gemmp_launch<7, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, st);
-    if (mode == 0 && act) return gemmp_launch<5, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, st);
-    if (mode == 0) return gemmp_launch<0, 4, 4>(A, W, bias, C, M, N, K, kps, hd, pk, none, st);
-    if (mode == 1) return gemmp_launch<1, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
-    if (mode == 2) return gemmp_launch<2, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    if (mode == 0 && act && act->gelu) return gemmp_launch<7, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, ni, no, st);
+    if (mode == 0 && act) return gemmp_launch<5, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, ni, no, st);
+    if (mode == 0) return gemmp_launch<0, 4, 4>(A, W, bias, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (mode == 1) return gemmp_launch<1, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (mode == 2) return gemmp_launch<2, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (mode == 5) {
+        int cost;
+        const int t = gemmp_resid_tile(M, N, K, &cost);
+        if (t == 1) return gemmp_launch<8, 4, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        if (t == 2) return gemmp_launch<8, 2, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        return gemmp_launch<8, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    }
     const int t = gemmp_tile(M, mode == 4 ? 2 * N : N, K, mode == 4);
     if (mode == 3) {
-        if (t == 1) return gemmp_launch<3, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
-        return gemmp_launch<3, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+        if (t == 1) return gemmp_launch<3, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        return gemmp_launch<3, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
     }
-    if (t == 1) return gemmp_launch<4, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
-    if (t == 2) return gemmp_launch<4, 6, 6>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
-    return gemmp_launch<4, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, st);
+    if (t == 1) return gemmp_launch<4, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (t == 2) return gemmp_launch<4, 6, 6>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    return gemmp_launch<4, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
 }
 
 template <int EPI>

@@ -4,6 +4,7 @@
 
 #include <type_traits>
 
+#include "gemm_epilogues.hip.h"
 #include "moe.hip.h"
 
 namespace pgk {
@@ -15,7 +16,7 @@ bool gemm128s_ok(int M, int N, int K);
 struct QkvHeadArgs;
 struct ActArgs;
 pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void* C, int mode, int splits, int M, int N, int K, hipStream_t st,
-                            const QkvHeadArgs* heads, bool packed, const ActArgs* act);
+                            const QkvHeadArgs* heads, bool packed, const ActArgs* act, const NormIn& ni, const NormOut& no);
 
 // -------------------------------------------------------------------------------------------- choice and sorting
 // A wave per row; logits are the sum of `slabs` fp32 slabs
@@ -280,7 +281,7 @@ pgk_status moe_rows(const MoeArgs& a, pgk_dtype dt, hipStream_t st) {
     } else {
         if (dt == PGK_F32) { if (pgk_status q = pgk_gemm_nt(a.x, a.w_router, nullptr, logits, a.n, p.Ep, a.W, PGK_F32, st)) return q; }
         else if (a.n <= 128) { if (pgk_status q = wsgemm_nt((const bf16*)a.x, a.W, a.w_router, nullptr, false, logits, nullptr, 1, p.slabs, a.n, p.Ep, a.W, st)) return q; }
-        else if (pgk_status q = gemm128s_bf16_nt((const bf16*)a.x, (const bf16*)a.w_router, nullptr, logits, 2, p.slabs, a.n, p.Ep, a.W, st, nullptr, false, nullptr)) return q;
+        else if (pgk_status q = gemm128s_bf16_nt((const bf16*)a.x, (const bf16*)a.w_router, nullptr, logits, 2, p.slabs, a.n, p.Ep, a.W, st, nullptr, false, nullptr, NormIn{}, NormOut{})) return q;
         const size_t lds = (size_t)4 * route_floats(r) * 4;
         PGK_REQUIRE(lds <= 60 * 1024, "moe: %d experts", r.E);
         moe_route_kernel<<<ceil_div(a.n, 4), 256, lds, st>>>(r, logits, p.Ep, p.slabs, (size_t)a.n * p.Ep, a.n, ids, wts);
