@@ -15,8 +15,8 @@
 // (V used to be transposed by a pass of its own over the whole context: 5.3 us of a 1531-token prompt's 42 us of
 // attention per layer, 5.8 of 42 for 384 tokens at position 3201.)
 // Workgroup = 4 waves = 128 query rows of one head; KV tiles of 64 positions, K and V [64][D] double
-// buffered in LDS (64 KiB at D = 128: two workgroups per CU); the global loads of tile t+1 are issued before the
-// MFMAs of tile t and written to the other buffer after them: one barrier per tile.
+// buffered in LDS (64 KiB at D = 128: two workgroups per CU), fetched by LDS-DMA, K a tile ahead of V: the products
+// S(t + 1) run between the exponentials of S(t).  One barrier per tile.
 // Workgroups are ordered heavy-first (causal: late query tiles see more keys) and all query heads of a kv head
 // share id % Hkv, i.e. an XCD when Hkv is a multiple of 8, so the K/V stream of a head is served by one L2.
 // Mask: kv_pos <= (kv_len - q_len) + q_pos  (reference: native/ops/nn/attention_kernels.cuh:32-148).
@@ -49,6 +49,14 @@ template <> __device__ __forceinline__ uint32_t pack16x2<f16>(float lo, float hi
 }
 
 struct FlashStrides { long long qh, qs, kh, ks, oh, os; };
+
+// One wave-instruction of LDS-DMA: 64 lanes x 16 bytes at per-lane byte offsets of a buffer to LDS [lds, +1024), zeros beyond its end.  (Inline asm: for the
+// builtin hipcc waits for the DMA in front of the next LDS read, whichever buffer that reads.  The waits are the explicit ones in the kernel.)
+typedef uint32_t fl_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void fl_dma16(const fl_u32x4& buffer, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buffer), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t fl_lds_addr(const char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p; }
 
 constexpr int FL_BQ = FLASH_ITEM_ROWS, FL_BKV = 64, FL_THREADS = 256;
 
@@ -119,13 +127,12 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     constexpr int NC = D / 8;            // 16-byte chunks per K row
     constexpr int KS = D / 16;           // k-steps of Q.K^T
     constexpr int DT = D / 32;           // 32-row tiles of O^T
-    constexpr int KCH = 64 * NC / FL_THREADS;   // K chunks staged per thread
     constexpr int K_BYTES = 64 * D * 2, V_BYTES = K_BYTES;
     extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // K[2] | V[2]
     auto Ks = [&](int buf) -> char* { return fl_smem + buf * K_BYTES; };
     auto Vs = [&](int buf) -> char* { return fl_smem + 2 * K_BYTES + buf * V_BYTES; };
 
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, ql = lane & 31, h = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), ql = lane & 31, h = lane >> 5;
     // workgroup id -> (kv head, query head in its group, query tile, KV run), heavy tiles first
     const int rep = hq / hkv;
     const int id = blockIdx.x;
@@ -162,13 +169,7 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     const T* kh = k + (size_t)kvh * sd.kh;
     const T* vh = v + (size_t)kvh * sd.kh;
 
-    // Q^T fragments (B operand): lane = query column, k = d
     uint4 qf[KS];
-    {
-        const T* qrow = qh + (size_t)min(qw0 + ql, q_len - 1) * sd.qs + 8 * h;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const uint4*>(qrow + ks * 16);
-    }
     f32x16_fl o[DT];
 #pragma unroll
     for (int i = 0; i < DT; ++i)
@@ -184,60 +185,35 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     const int tb = WIN && first_kv > 0 ? first_kv / FL_BKV : 0;            // tiles before it are outside every row's window
     const int t0 = tb + (int)((long long)(nt_all - tb) * split / sp.nsplit), t1 = tb + (int)((long long)(nt_all - tb) * (split + 1) / sp.nsplit);
 
-    // staging in NAMED registers (an array here ends up in scratch memory at this register pressure, see
-    // ops_fp8_gemm.hip): chunk i of this thread is c = tid + 256 i; KCH = VCH = D / 32 chunks each
-    static_assert(KCH == 2 || KCH == 4, "staging is written for D = 64 / 128");
-    uint4 rk0, rk1, rk2, rk3, rv0, rv1, rv2, rv3;
-    const int kr = tid / NC, kc16 = tid % NC;               // row kr + (256/NC) i, chunk kc16
-    constexpr int KR_STEP = FL_THREADS / NC;
-    // Whole tiles address their rows as (wave-uniform tile base) + (per-lane element offset fixed for the kernel): the
-    // per-tile address arithmetic is scalar.  (Recomputing min(row, kv_len - 1) * stride per chunk cost 48 vector
-    // instructions per tile - 64-bit multiplies included - in a loop that is bound by vector issue.)  Only the ragged
-    // last tile clamps its rows (their probabilities are zero).
-    const uint32_t ko0 = (uint32_t)(kr * sd.ks + kc16 * 8), ko_step = (uint32_t)(KR_STEP * sd.ks);
-    auto load_rows = [&](const T* base, int t, uint4& r0, uint4& r1, uint4& r2, uint4& r3) {
-        const int kv0 = t * FL_BKV;
-        if (kv0 + FL_BKV <= kv_len) {      // wave-uniform
-            const T* tile = base + (size_t)kv0 * sd.ks;
-            r0 = *reinterpret_cast<const uint4*>(tile + ko0);
-            r1 = *reinterpret_cast<const uint4*>(tile + ko0 + ko_step);
-            if constexpr (KCH == 4) {
-                r2 = *reinterpret_cast<const uint4*>(tile + ko0 + 2 * ko_step);
-                r3 = *reinterpret_cast<const uint4*>(tile + ko0 + 3 * ko_step);
-            }
-        } else {
-            auto src = [&](int i) { return base + (size_t)min(kv0 + kr + KR_STEP * i, kv_len - 1) * sd.ks + kc16 * 8; };
-            r0 = *reinterpret_cast<const uint4*>(src(0));
-            r1 = *reinterpret_cast<const uint4*>(src(1));
-            if constexpr (KCH == 4) {
-                r2 = *reinterpret_cast<const uint4*>(src(2));
-                r3 = *reinterpret_cast<const uint4*>(src(3));
-            }
-        }
+    // One wave-instruction of LDS-DMA moves 1 KiB = ROWS rows; the images' swizzles are applied on the source side (lane l of a row fetches the chunk that belongs
+    // into its 16 bytes).  A wave moves NI instructions of K and of V per tile.  A tile is a buffer of the rows that are there: what lies beyond comes as zeros
+    // without a branch (their probabilities are zero too), and a tile past the run's end reads nothing.
+    constexpr int ROWS = 64 / NC, NI = 64 / ROWS / 4;
+    const int dr = lane / NC, ds = lane % NC;
+    uint32_t ko[NI], vo[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = wid * 16 + i * ROWS + dr;
+        ko[i] = (uint32_t)(r * sd.ks + (ds ^ (r & (NC - 1))) * 8) * 2;
+        vo[i] = (uint32_t)(r * sd.ks + (ds ^ fl_v_sw<D>(r)) * 8) * 2;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(fl_lds_addr(fl_smem) + wid * NI * 1024), row_bytes = (uint32_t)(sd.ks * 2);
+    auto tile_of = [&](const T* base, int t) {
+        const uint64_t at = (uint64_t)(uintptr_t)(base + (size_t)t * FL_BKV * sd.ks);
+        const int last = t < t1 ? min(kv_len - t * FL_BKV, FL_BKV) - 1 : -1;     // last row that is there
+        return fl_u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xFFFFu, last < 0 ? 0u : last * row_bytes + 2 * D, 0x00020000u};   // raw, 32-bit words
     };
-    auto load_k = [&](int t) { load_rows(kh, t, rk0, rk1, rk2, rk3); };
-    auto load_v = [&](int t) { load_rows(vh, t, rv0, rv1, rv2, rv3); };
-    auto store_k = [&](int buf) {
-        char* kb = Ks(buf);
-        *reinterpret_cast<uint4*>(kb + fl_k_off<D>(kr, kc16)) = rk0;
-        *reinterpret_cast<uint4*>(kb + fl_k_off<D>(kr + KR_STEP, kc16)) = rk1;
-        if constexpr (KCH == 4) {
-            *reinterpret_cast<uint4*>(kb + fl_k_off<D>(kr + 2 * KR_STEP, kc16)) = rk2;
-            *reinterpret_cast<uint4*>(kb + fl_k_off<D>(kr + 3 * KR_STEP, kc16)) = rk3;
-        }
-    };
-    auto store_v = [&](int buf) {
-        char* vb = Vs(buf);
-        *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr, kc16)) = rv0;
-        *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + KR_STEP, kc16)) = rv1;
-        if constexpr (KCH == 4) {
-            *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + 2 * KR_STEP, kc16)) = rv2;
-            *reinterpret_cast<uint4*>(vb + fl_v_off<D>(kr + 3 * KR_STEP, kc16)) = rv3;
-        }
+    auto dma_k = [&](const fl_u32x4& tile, int t, int i) { fl_dma16(tile, ko[i], lds0 + (t & 1) * K_BYTES + i * 1024); };
+    auto dma_v = [&](const fl_u32x4& tile, int t, int i) { fl_dma16(tile, vo[i], lds0 + 2 * K_BYTES + (t & 1) * V_BYTES + i * 1024); };
+    // what iteration t requests, in KS pieces: K of t + 2, V of t + 1
+    static_assert(2 * NI == KS, "a piece of the DMA per k-step");
+    auto dma_next = [&](int t, int piece) {
+        if (piece < NI) dma_k(tile_of(kh, t + 2), t + 2, piece);
+        else dma_v(tile_of(vh, t + 1), t + 1, piece - NI);
     };
     // S^T = K . Q^T of one tile: two 32-kv sub-tiles (rows = positions, column = this lane's query)
     const float slope = BIAS ? win.slopes[head] * win.inv_scale : 0.f;
-    auto qk = [&](int buf, int t, f32x16_fl& s0, f32x16_fl& s1) {
+    auto s_init = [&](int t, f32x16_fl& s0, f32x16_fl& s1) {
         if constexpr (BIAS) {            // rows are keys kv0 + (r & 3) + 8 (r >> 2) + 4 h (+ 32), this lane's query is position qpos
             const float b0 = slope * (float)(t * FL_BKV + 4 * h - (causal_off + qw0 + ql));
 #pragma unroll
@@ -249,36 +225,45 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
 #pragma unroll
             for (int r = 0; r < 16; ++r) { s0[r] = 0.f; s1[r] = 0.f; }
         }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uint4 a0 = *reinterpret_cast<const uint4*>(Ks(buf) + fl_k_off<D>(ql, 2 * ks + h));
-            const uint4 a1 = *reinterpret_cast<const uint4*>(Ks(buf) + fl_k_off<D>(32 + ql, 2 * ks + h));
-            s0 = mfma32<T>(a0, qf[ks], s0);
-            s1 = mfma32<T>(a1, qf[ks], s1);
-        }
     };
+    auto k_frag = [&](const char* kb, int half, int ks) { return *reinterpret_cast<const uint4*>(kb + fl_k_off<D>(32 * half + ql, 2 * ks + h)); };
     // tiles entirely above this wave's diagonal contribute nothing (wave-uniform)
     auto live = [&](int t) -> bool {
         return t < t1 && t * FL_BKV <= causal_off + qw0 + 31 && (!WIN || t * FL_BKV + FL_BKV - 1 > causal_off + qw0 - win.window);
     };
 
-    // One KV tile per iteration: S = K . Q^T, softmax, O += V . P; the global loads of tile t + 1 are issued before the MFMAs of
-    // tile t and parked in the other LDS buffer after them: one barrier per tile.  (Tried in round 3: multiplying S(t + 1) under
-    // the softmax of S(t).  As two conditional blocks hipcc keeps them apart - QK block, 64 register copies, softmax - and
-    // the kernel lost 2 %; it needs a branch-free, two-tile-unrolled body to interleave.)
+    // One KV tile per iteration: softmax of S(t) with the products S(t + 1) = K(t + 1) . Q^T between its exponentials - in one basic block, a matrix instruction
+    // behind every two of them - then O += V(t) . P.  So K runs a tile ahead of V: the DMA of K(t + 2) and V(t + 1) goes out behind the barrier at which K(t + 1)
+    // and V(t) have landed and S(t) and O(t - 1) have been read.  Attention with merge, us, staged through registers with S(t) in front of its softmax / this: 16
+    // heads, 1531 rows 35.4 / 30.6, 384 at 3585 34.0 / 29.0; 32 heads, 4096 rows 180 / 151.  (As two conditional blocks hipcc keeps S(t + 1) and the softmax apart; the
+    // DMA a piece behind each k-step, inside the block, spills 74 registers.)
     f32x16_fl sc0, sc1;
-    if (t0 < t1) {
-        load_k(t0);
-        load_v(t0);
-        store_k(t0 & 1);
-        store_v(t0 & 1);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) dma_k(tile_of(kh, t0), t0, i);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) dma_k(tile_of(kh, t0 + 1), t0 + 1, i);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) dma_v(tile_of(vh, t0), t0, i);
+    // Q^T fragments (B operand): lane = query column, k = d
+    {
+        const T* qrow = qh + (size_t)min(qw0 + ql, q_len - 1) * sd.qs + 8 * h;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const uint4*>(qrow + ks * 16);
     }
-    // Retire the Q loads HERE: if they are still counted as pending at the loop header, hipcc's conservative
-    // vmcnt bookkeeping waits for them in every iteration - behind the tile prefetch issued at the top of the
-    // loop, i.e. it drains the prefetch before the first MFMA.
+    // Retire the Q loads (and with them the first tiles) HERE: still counted as pending at the loop header, they would be waited for in every iteration, behind
+    // the DMA that it has just issued.
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
-    __syncthreads();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    s_init(t0, sc0, sc1);
+    if (live(t0)) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            sc0 = mfma32<T>(k_frag(Ks(t0 & 1), 0, ks), qf[ks], sc0);
+            sc1 = mfma32<T>(k_frag(Ks(t0 & 1), 1, ks), qf[ks], sc1);
+        }
+    }
     // V^T fragments: lane l gets dim 32 i + (l & 31) of rows 16 s + 8 u + 4 h .. + 3.  A 16-lane group's transposing read covers 4 rows x 16
     // dims: lane l15 of it supplies the address of row l15 >> 2, dims 4 (l15 & 3) .. + 3.  The swizzle of such a row depends on l15 >> 2, h and
     // u only, so the addresses of (i, u) serve every s with an immediate offset of 16 rows.
@@ -287,10 +272,13 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     const int tr = (lane & 15) >> 2, tc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), t8 = 8 * (lane & 1);
     for (int t = t0; t < t1; ++t) {
         const int buf = t & 1, kv0 = t * FL_BKV;
-        if (t + 1 < t1) { load_k(t + 1); load_v(t + 1); }
-        const bool cur = live(t);
-        if (cur) qk(buf, t, sc0, sc1);
-        if (cur) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // this wave's share of K(t + 1) and V(t)
+        __syncthreads();                                                 // ... everyone's; and everyone has read K(t) and V(t - 1)
+#pragma unroll
+        for (int i = 0; i < KS; ++i) dma_next(t, i);
+        if (live(t)) {
+            f32x16_fl sn0, sn1;                                          // S(t + 1); behind the last tile of what K's other buffer holds, and unused
+            const char* kn = Ks(buf ^ 1);
             // ---- mask, online softmax (this lane: query qw0 + ql, kv rows (r&3) + 8(r>>2) + 4h of each sub-tile) ----
             const bool need_mask = kv0 + FL_BKV - 1 > causal_off + qw0 || kv0 + FL_BKV > kv_len ||
                                    (WIN && kv0 <= causal_off + qw0 + 31 - win.window);   // wave-uniform
@@ -309,7 +297,10 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
             // v_max_f32 x, x, x of its own - 60 instructions for these 32 values instead of 16 v_max3_f32)
 #pragma unroll
             for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(fmaxf(sc0[r], sc1[r]), fmaxf(sc0[r + 1], sc1[r + 1])), mx);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            {   // with the other half of the rows, lane ^ 32
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+                mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+            }
             mx *= scale_log2e;                                           // -inf stays -inf (scale > 0)
             // Deferred rescale: the reference point of a row only moves when its maximum grew by more than 6 (log2
             // domain), so probabilities stay <= 64 (exact in fp32 sums, fine in 16-bit P) and on most tiles - for the whole
@@ -318,21 +309,40 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
             const float m_use = m_new == -INFINITY ? 0.f : m_new;        // a fully masked row so far: p = exp2(-inf) = 0
             const bool moved = __builtin_amdgcn_ballot_w64(m_new != m_run) != 0;   // wave-uniform
             const float alpha = moved ? __builtin_amdgcn_exp2f(m_run - m_use) : 1.0f;   // m_run = -inf -> 0 (accumulators are 0 anyway)
-            float ls = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                sc0[r] = __builtin_amdgcn_exp2f(fmaf(sc0[r], scale_log2e, -m_use));
-                sc1[r] = __builtin_amdgcn_exp2f(fmaf(sc1[r], scale_log2e, -m_use));
-                ls += sc0[r] + sc1[r];
-            }
-            l_run = l_run * alpha + ls;
-            m_run = m_new;
-            if (moved) {
+            if (moved) {                                                 // (in front of the block below, which it would cut in two)
 #pragma unroll
                 for (int i = 0; i < DT; ++i)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
             }
+            float ls = 0.f;
+            uint32_t pw0[8], pw1[8];                                     // P, packed
+            s_init(t + 1, sn0, sn1);
+            uint4 ka = k_frag(kn, 0, 0), kb2 = k_frag(kn, 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int PER = 16 / KS;                                 // rows of S(t) per k-step of S(t + 1)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const uint4 na = k_frag(kn, 0, ks + 1 < KS ? ks + 1 : ks), nb = k_frag(kn, 1, ks + 1 < KS ? ks + 1 : ks);
+                sn0 = mfma32<T>(ka, qf[ks], sn0);
+#pragma unroll
+                for (int r = ks * PER; r < (ks + 1) * PER; ++r) {
+                    sc0[r] = __builtin_amdgcn_exp2f(fmaf(sc0[r], scale_log2e, -m_use));
+                    sc1[r] = __builtin_amdgcn_exp2f(fmaf(sc1[r], scale_log2e, -m_use));
+                    ls += sc0[r] + sc1[r];
+                    if (r == ks * PER + PER / 2 - 1) sn1 = mfma32<T>(kb2, qf[ks], sn1);
+                }
+#pragma unroll
+                for (int r = ks * PER; r < (ks + 1) * PER; r += 2) {
+                    pw0[r / 2] = pack16x2<T>(sc0[r], sc0[r + 1]);
+                    pw1[r / 2] = pack16x2<T>(sc1[r], sc1[r + 1]);
+                }
+                ka = na;
+                kb2 = nb;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            l_run = l_run * alpha + ls;
+            m_run = m_new;
             // ---- O^T += V^T . P^T : 4 k-steps of 16 kv ----
             const char* vb = Vs(buf);
             const char* va[DT][2];
@@ -342,14 +352,8 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
                 for (int u = 0; u < 2; ++u) va[i][u] = vb + fl_v_off<D>(8 * u + 4 * h + tr, 4 * i + tc) + t8;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                uint4 pb;
-                if (s < 2) {
-                    pb = make_uint4(pack16x2<T>(sc0[8 * s + 0], sc0[8 * s + 1]), pack16x2<T>(sc0[8 * s + 2], sc0[8 * s + 3]),
-                                    pack16x2<T>(sc0[8 * s + 4], sc0[8 * s + 5]), pack16x2<T>(sc0[8 * s + 6], sc0[8 * s + 7]));
-                } else {
-                    pb = make_uint4(pack16x2<T>(sc1[8 * (s - 2) + 0], sc1[8 * (s - 2) + 1]), pack16x2<T>(sc1[8 * (s - 2) + 2], sc1[8 * (s - 2) + 3]),
-                                    pack16x2<T>(sc1[8 * (s - 2) + 4], sc1[8 * (s - 2) + 5]), pack16x2<T>(sc1[8 * (s - 2) + 6], sc1[8 * (s - 2) + 7]));
-                }
+                const uint32_t* w = s < 2 ? pw0 + 4 * s : pw1 + 4 * (s - 2);
+                const uint4 pb = make_uint4(w[0], w[1], w[2], w[3]);
 #pragma unroll
                 for (int i = 0; i < DT; ++i) {
                     const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][0] + s * 32 * D)));
@@ -357,9 +361,18 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
                     o[i] = mfma32<T>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb, o[i]);
                 }
             }
+            sc0 = sn0;
+            sc1 = sn1;
+        } else {
+            if (WIN && live(t + 1)) {                                    // left of this wave's windows: the next tile's scores alone
+                s_init(t + 1, sc0, sc1);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    sc0 = mfma32<T>(k_frag(Ks(buf ^ 1), 0, ks), qf[ks], sc0);
+                    sc1 = mfma32<T>(k_frag(Ks(buf ^ 1), 1, ks), qf[ks], sc1);
+                }
+            }
         }
-        if (t + 1 < t1) { store_k(buf ^ 1); store_v(buf ^ 1); }
-        __syncthreads();
     }
 
     // ---- normalise and store: lane = query row, registers 4g..4g+3 of tile i are d = 32i + 8g + 4h .. +3 ----
@@ -490,13 +503,15 @@ static int flash_cus() {
     return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
-// KV runs per query tile, at least four KV tiles to a run, as many as one round of workgroups holds: of two per CU (the kernel's occupancy), a heavy
-// and a light one, where the causal edge makes query tiles differ; of one per CU where a long context makes all runs alike and that many still
-// cut it well.  A second round costs more than the shorter runs save, and every run costs the merge.  Launch and merge, us, runs that reached two
-// per CU / this rule: 1531 rows, 16 heads 37.4 (4) / 35.8 (2); 3500 rows 95.9 (2) / 92.3 (1); 800 rows at 1200 39.3 (8) / 33.4 (4);
-// 384 at 3201 33.8 (8) / 32.5 (5); 250 at 1750, 32 heads 29.4 (8) / 25.9 (4); 900 at 2800, 16 heads one per CU 56.0 (2), two 47.0 (4).
+// KV runs per query tile, at least four KV tiles to a run.  Where the causal edge is most of the work (contexts under twice the rows) two, of which a heavy and a light
+// one share a CU, if one round holds them and the heaviest tile is long enough for the merge to pay; elsewhere as many as one round of workgroups holds: of two per
+// CU (the kernel's occupancy), or of one per CU where a long context makes all runs alike and that many still cut it well.  A second round costs more than the
+// shorter runs save, and every run costs the merge.  Launch and merge, us (runs): 16 heads, 512 rows 14.8 (1) 16.2 (2); 1000 23.8 (1) 23.2 (2) 25.5 (4); 1200 27.2 (1)
+// 27.5 (2); 1531 34.1 (1) 31.4 (2); 2000 44.7 (1) 38.9 (2); 3000 63.6 (1) 66.3 (2); 800 at 1200 28.9 (1) 25.2 (2) 26.2 (4); 32 heads, 500 14.9 (1) 18.6 (2), 1000 25.5 (1) 30.2
+// (2); longer contexts, 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5) 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).
 static int flash_runs(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
+    if (kv_len < 2LL * q_len) return wgs <= cus && kv_len >= 1200 && most >= 2 ? 2 : 1;
     long long n = cus / wgs;
     if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
     if (n > most) n = most;

@@ -923,6 +923,23 @@ def test_sdpa_fixed_cache_multi_query():
         ops.sdpa_causal_fixed_cache(dev(q, "bfloat16"), dev(kc, "bfloat16"), dev(vc, "bfloat16"), out, max_seq + 1)
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(4, 2, 129, 129, 128), (4, 2, 130, 191, 128), (2, 2, 200, 257, 64), (2, 1, 256, 320, 128), (2, 1, 140, 1345, 64), (1, 1, 129, 2049, 128)])
+def test_sdpa_reads_nothing_behind_the_context(dt, cfg):
+    """A cache whose rows behind the context are NaN: tiles of 64 keys with 1, 63, 1, 64, 1 and 1 rows that are there, one run of the context or several, of
+    which one may be a single tile.  Bar: that of the long-context test, p, a run's output and the output rounded to 16 bits."""
+    hq, hc, ql, ctx, d = cfg
+    rng = np.random.default_rng(ctx)
+    q = rng.standard_normal((hq, ql, d)).astype(np.float32)
+    kc, vc = (rng.standard_normal((hc, ctx + 70, d)).astype(np.float32) for _ in range(2))
+    ref = O.sdpa_causal_fixed_cache(rounded(q, dt).astype(np.float64), rounded(kc, dt), rounded(vc, dt), ctx)
+    kc[:, ctx:], vc[:, ctx:] = np.nan, np.nan
+    out = pk.empty((hq, ql, d), dt)
+    ops.sdpa_causal_fixed_cache(dev(q, dt), dev(kc, dt), dev(vc, dt), out, ctx)
+    bar = 2 * (2.0**-9 if dt == "bfloat16" else 2.0**-12)
+    assert rel_err(host(out), ref) < bar, rel_err(host(out), ref)
+
+
 # ----------------------------------------------------------------------------- paged KV cache / continuous batching
 def _paged_setup(rng, num_seqs, hkv, bs, d, ctxs, dt, num_blocks=None):
     max_blocks = max((c + bs - 1) // bs for c in ctxs) + 1
