@@ -39,6 +39,8 @@ bool engine_gemm_carry_ok(int M, int N, int K);                // ops_gemm.hip: 
 bool engine_gemm_resid_pays(int M, int N, int K, int splits);
 pgk_status engine_gemm_resid_nt(const bf16* A, const void* W, float* h, int M, int N, int K, const NormOut& no, hipStream_t st, bool packed);
 bool engine_gemm_packed_ok(int M, int N, int K);
+bool gemm_few_swiglu_ok(int I, int K);                         // ops_gemm256.hip
+pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, int I, int K, const NormIn& ni, hipStream_t st);
 int wsgemm_pick_splits(int N, int K, bool allow_split);
 int engine_gemm_pick_splits(int M, int N, int K);
 int engine_gemm_qkv_splits(int M, int N, int K, bool fused);
@@ -1858,6 +1860,13 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
     *launches += 2;
     return PGK_OK;
 }
+// gate_up with SwiGLU of up to 128 rows on the fragment-major copy (carried: how x's rows are scaled)
+static pgk_status packed_swiglu(const bf16* x, const bf16* wp, bf16* act, int M, int I, int H, const PkArgs* carried, hipStream_t st) {
+    if (M <= 32 || !gemm_few_swiglu_ok(I, H)) return pkgemm_nt(x, H, wp, act, I, PK_EPI_SWIGLU, 1, M, 2 * I, H, carried, st);
+    NormIn ni{};
+    if (carried && carried->ss_in) ni = NormIn{carried->ss_in, carried->ss_n, carried->ss_eps, PK_SS_LD};
+    return gemm_few_swiglu_nt(x, wp, act, M, I, H, ni, st);
+}
 
 // 17..64 sequences, bf16 layers: the step on the fragment-major weight copy (ops_pkgemm.hip) - the prefill's kernels with
 // one row per SEQUENCE.  Seven launches per layer as on the tiled path, but the projections stream coalesced 1 KiB
@@ -1902,7 +1911,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
             mark(KC_GATEUP);
             PkArgs gn{};
             gn.ss_in = e->pk_ss; gn.ss_n = ss_n; gn.ss_eps = c.norm_eps;
-            if (pgk_status r = pkgemm_nt(x16, H, P.gate_up, act16, I, PK_EPI_SWIGLU, 1, M, 2 * I, H, &gn, st)) return r;
+            if (pgk_status r = packed_swiglu(x16, P.gate_up, act16, M, I, H, &gn, st)) return r;
             mark(KC_DOWN);
             const bf16* gnext = l + 1 < c.num_layers ? (const bf16*)e->layers[l + 1].attn_norm : nullptr;
             if (pgk_status r = pkgemm_resid_nt(act16, I, P.down, h, M, H, I, gnext, x16, e->pk_ss, &ss_n, st)) return r;
@@ -1913,7 +1922,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
         pending = s_o;
         if (pgk_status r = norm((const bf16*)L.mlp_norm)) return r;
         mark(KC_GATEUP);
-        if (pgk_status r = pkgemm_nt(x16, H, P.gate_up, act16, I, PK_EPI_SWIGLU, 1, M, 2 * I, H, nullptr, st)) return r;
+        if (pgk_status r = packed_swiglu(x16, P.gate_up, act16, M, I, H, nullptr, st)) return r;
         mark(KC_DOWN);
         if (pgk_status r = pkgemm_nt(act16, I, P.down, e->dec_slabs, H, PK_EPI_SLAB, s_d, M, H, I, nullptr, st)) return r;
         pending = s_d;
@@ -2325,7 +2334,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
             if (pgk_status r = pkgemm_resid_nt(attn, QD, e->packed[l].o, h32, n, H, QD, (const bf16*)L.mlp_norm, x, e->pk_ss, &ss_n, st)) return r;
             PkArgs gn{};
             gn.ss_in = e->pk_ss; gn.ss_n = ss_n; gn.ss_eps = c.norm_eps;
-            if (pgk_status r = pkgemm_nt(x, H, e->packed[l].gate_up, act, I, PK_EPI_SWIGLU, 1, n, 2 * I, H, &gn, st)) return r;
+            if (pgk_status r = packed_swiglu(x, e->packed[l].gate_up, act, n, I, H, &gn, st)) return r;
             const bf16* gnext = l + 1 < c.num_layers ? (const bf16*)e->layers[l + 1].attn_norm : nullptr;
             if (pgk_status r = pkgemm_resid_nt(act, I, e->packed[l].down, h32, n, H, I, gnext, x, e->pk_ss, &ss_n, st)) return r;
             continue;
@@ -2342,7 +2351,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         };
         if (pk) {
             // SwiGLU inside the gate_up projection: the gate tile and its up tile live in the same wave
-            if (pgk_status r = pkgemm_nt(x, H, e->packed[l].gate_up, act, I, PK_EPI_SWIGLU, 1, n, 2 * I, H, nullptr, st)) return r;
+            if (pgk_status r = packed_swiglu(x, e->packed[l].gate_up, act, n, I, H, nullptr, st)) return r;
             if (pgk_status r = pk_accum(act, e->packed[l].down, I, pk_sd)) return r;
             continue;
         }

@@ -20,7 +20,8 @@ struct QkvHeadArgs {
 };
 // An RMSNorm between two products without a pass of its own.  The product before it (its residual epilogue) leaves x = bf16(h gamma) and, per row and 64
 // columns, h's sum of squares; the product behind it reads x and scales its result rows by 1 / rms, which a factor per row may as well do after the sum.
-struct NormIn { const float* ss; int n; float eps; };      // ss [n][rows]; null: x is normalised
+// ss [n][rows], or (ld = 64) [rows][64] of which n <= 64 count, as pkgemm_resid_nt leaves them; null: x is normalised
+struct NormIn { const float* ss; int n; float eps; int ld; };
 struct NormOut { const bf16* gamma; bf16* x; float* ss; };  
 // 1 / rms of a row of K values
 __device__ __forceinline__ float norm_in_scale(const NormIn& nn, int row, int rows, int K) {
