@@ -1862,7 +1862,7 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
 }
 // gate_up with SwiGLU of up to 128 rows on the fragment-major copy (carried: how x's rows are scaled)
 static pgk_status packed_swiglu(const bf16* x, const bf16* wp, bf16* act, int M, int I, int H, const PkArgs* carried, hipStream_t st) {
-    if (M <= 32 || !gemm_few_swiglu_ok(I, H)) return pkgemm_nt(x, H, wp, act, I, PK_EPI_SWIGLU, 1, M, 2 * I, H, carried, st);
+    if (!gemm_few_swiglu_ok(I, H)) return pkgemm_nt(x, H, wp, act, I, PK_EPI_SWIGLU, 1, M, 2 * I, H, carried, st);
     NormIn ni{};
     if (carried && carried->ss_in) ni = NormIn{carried->ss_in, carried->ss_n, carried->ss_eps, PK_SS_LD};
     return gemm_few_swiglu_nt(x, wp, act, M, I, H, ni, st);

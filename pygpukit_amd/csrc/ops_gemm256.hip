@@ -533,7 +533,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 // GRP: rows sorted by expert (GroupArgs), every tile with its expert's weight; EPI 4, 7, or 6: bf16 rows times their weight, each at its place
 constexpr int GP_THREADS = 512;
 // stages of W that the ring holds; A's has two more.  The smaller tiles' stages are shorter, and latency asks for more of them
-constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 ? 4 : 6; }
+constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 || (WM == 2 && WN == 4) ? 4 : 6; }
 template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
     const size_t RW = gemmp_ring(WM, WN), ring = (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
     return ring > tile ? ring : tile;
@@ -564,7 +564,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     const int nh = (kend - kbeg) / 32;                       // (kend - kbeg) % 64 == 0: an even number of stages
 
     f32x4_g acc[WM][WN];
-    float mine = 0.f;                                        // 1 / rms of row tid (64 rows: tid / 4)
+    float mine = 0.f;                                        // 1 / rms of row tid (ni.ld: of tid / 4)
     const int wr = (wid >> 1) & 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
     if (wid >= 4) {
         const int pw = __builtin_amdgcn_readfirstlane(wid & 3);
@@ -627,8 +627,8 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         __builtin_amdgcn_s_barrier();
     } else {
         if constexpr (SCALED && EPI != 0) {
-            if constexpr (BM == 64) {                        // (ld = 64) four threads to a row, 16 parts each
-                if (ni.ss) {
+            if (BM == 64 && ni.ss && ni.ld) {                // four threads to a row, 16 parts each
+                {
                     const float* p = ni.ss + (size_t)min(m0 + (tid >> 2), M - 1) * 64 + (tid & 3) * 16;
                     float4 v[4];
 #pragma unroll
@@ -714,7 +714,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
             if constexpr (EPI == 0) {                        // (held through the loop it is spilled; no engine's step comes here unless PGK_FUSED_EPILOGUES is 0)
                 if (tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
             }
-            if constexpr (BM == 64) { if (tid < 256 && (tid & 3) == 0) inv[tid >> 2] = mine; }
+            if (BM == 64 && ni.ld) { if (tid < 256 && (tid & 3) == 0) inv[tid >> 2] = mine; }
             else if (tid < BM) inv[tid] = mine;
             __syncthreads();
             if (wid < 4) {
@@ -1246,17 +1246,19 @@ static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, v
     return PGK_OK;
 }
 
-// Tile of an unsplit product of `cols` weight rows: the cheapest by rounds of workgroups x (time of a stage x stages + start and epilogue), in 0.01 us as measured
-// with the chip full.  128 x 128 runs two workgroups on a CU where there are more than 256.  (256 x 128 fills a round only where two of 128 x 128 on a CU do as well.)
-// 0: 128 x 128, 1: 192 x 128, 2: 192 x 192 (SwiGLU alone: heads are 128 columns).
-static int gemmp_tile(int M, int cols, int K, bool wide) {
-    constexpr struct { int bm, bn, stage, fixed; } t[] = {{128, 128, 18, 260}, {192, 128, 27, 350}, {192, 192, 40, 460}};
+// Tile of a product of `cols` weight rows in `splits` runs of K: the cheapest by rounds of workgroups x (time of a stage x stages + start and epilogue), in 0.01 us as
+// measured with the chip full, with one and where the LDS lets it with two workgroups on a CU.  `most`: how far down the list the product's epilogue goes (QKV heads
+// are 128 columns, split products leave most of a round idle anyway).  Us a launch, K = 1024: 384 rows, N = 4096 10.1 (128 x 128) 8.4 (64 x 128); 93 rows, N = 6144 9.8,
+// 7.5, 6.3 (64 x 64); 1531 rows, N = 4096 18.7 (128 x 128) 16.6 (192 x 128), N = 6144 27.8, 31.9, 23.0 (192 x 192).
+enum { GP_128, GP_64_128, GP_192_128, GP_192, GP_64 };
+static int gemmp_tile(int M, int cols, int K, int splits, int most) {
+    constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 260, 29, 420}, {64, 128, 13, 200, 20, 330}, {192, 128, 27, 350, 0, 0}, {192, 192, 40, 460, 0, 0}, {64, 64, 11, 150, 16, 260}};
     int best = 0;
     long long least = 0;
-    for (int i = 0; i < (wide ? 3 : 2); ++i) {
-        const long long n = (long long)ceil_div(M, t[i].bm) * ceil_div(cols, t[i].bn), stages = K / 32;
-        long long cost = ceil_div(n, 256LL) * (stages * t[i].stage + t[i].fixed);
-        if (i == 0) cost = n / 512 * (stages * 29 + 420) + (n % 512 > 256 ? stages * 29 + 420 : n % 512 > 0 ? stages * 18 + 260 : 0);
+    for (int i = 0; i <= most; ++i) {
+        const long long n = (long long)ceil_div(M, t[i].bm) * ceil_div(cols, t[i].bn) * splits, stages = K / splits / 32;
+        const long long one = stages * t[i].one + t[i].one_fixed, two = stages * t[i].two + t[i].two_fixed;
+        const long long cost = t[i].two ? n / 512 * two + (n % 512 > 256 ? two : n % 512 > 0 ? one : 0) : ceil_div(n, 256LL) * one;
         if (i == 0 || cost < least) { best = i; least = cost; }
     }
     return best;
@@ -1306,7 +1308,10 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
     if (mode == 0 && act) return gemmp_launch<5, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, *act, ni, no, st);
     if (mode == 0) return gemmp_launch<0, 4, 4>(A, W, bias, C, M, N, K, kps, hd, pk, none, ni, no, st);
     if (mode == 1) return gemmp_launch<1, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
-    if (mode == 2) return gemmp_launch<2, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (mode == 2) {
+        if (gemmp_tile(M, N, K, splits, GP_64_128) == GP_64_128) return gemmp_launch<2, 2, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        return gemmp_launch<2, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    }
     if (mode == 5) {
         int cost;
         const int t = gemmp_resid_tile(M, N, K, &cost);
@@ -1314,19 +1319,23 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
         if (t == 2) return gemmp_launch<8, 2, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
         return gemmp_launch<8, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
     }
-    const int t = gemmp_tile(M, mode == 4 ? 2 * N : N, K, mode == 4);
     if (mode == 3) {
-        if (t == 1) return gemmp_launch<3, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        const int t = gemmp_tile(M, N, K, 1, GP_192_128);
+        if (t == GP_64_128) return gemmp_launch<3, 2, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        if (t == GP_192_128) return gemmp_launch<3, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
         return gemmp_launch<3, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
     }
-    if (t == 1) return gemmp_launch<4, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
-    if (t == 2) return gemmp_launch<4, 6, 6>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    const int t = gemmp_tile(M, 2 * N, K, 1, GP_64);
+    if (t == GP_64_128) return gemmp_launch<4, 2, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (t == GP_192_128) return gemmp_launch<4, 6, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (t == GP_192) return gemmp_launch<4, 6, 6>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+    if (t == GP_64) return gemmp_launch<4, 2, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
     return gemmp_launch<4, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
 }
 
 // act[M][I] = SwiGLU of few rows (a prompt of up to 128, the step of a batch) against the fragment-major gate / up copy: 64 x 64 tiles, 32 act columns each.  The
 // packed kernel gives a wave the weights in registers and a workgroup 32 rows: us a launch there / here, K = 1024, I = 3072: 93 rows 10.9 / 7.8, 64 rows 8.5 / 7.3,
-// 37 rows 8.1 / 7.2.
+// 37 rows 8.1 / 7.2; ms, 4 steps of 24 sequences 4.07 / 3.97, a prompt of 9 1.083 / 1.051.
 bool gemm_few_swiglu_ok(int I, int K) { return K % 64 == 0 && K >= 64 && I % 32 == 0; }
 pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, int I, int K, const NormIn& ni, hipStream_t st) {
     PGK_REQUIRE(M >= 1 && gemm_few_swiglu_ok(I, K) && (!ni.ss || (ni.ld == 64 && ni.n <= 64)), "gemm_few_swiglu: M=%d I=%d K=%d", M, I, K);
