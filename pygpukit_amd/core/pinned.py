@@ -1,0 +1,60 @@
+"""NumPy arrays on pinned host memory, for results that a call copies back from the device.
+
+Into pageable memory the runtime copies by way of its own pinned buffers and touches every fresh page of the result: a prompt of 93 tokens with its
+151936 fp32 logits took 1.23 ms that way, 1.15 into a pinned array, sixteen prompts in one call 5.4 and 5.0.  A block returns to the pool with the last view of its array; the pool keeps at most POOL_BYTES of free blocks
+and gives the rest back."""
+
+from __future__ import annotations
+
+import ctypes as C
+import sys
+import threading
+
+import numpy as np
+
+from pygpukit_amd import _hip
+
+POOL_BYTES = 64 << 20
+_lock = threading.Lock()
+_free: dict[int, list[int]] = {}
+_free_bytes = 0
+
+
+class _Block:
+    """Owner of one pinned allocation; the array made from it keeps it alive."""
+
+    def __init__(self, address: int, nbytes: int, shape: tuple, typestr: str):
+        self.address, self.nbytes = address, nbytes
+        self.__array_interface__ = {"data": (address, False), "shape": shape, "typestr": typestr, "version": 3}
+
+    def __del__(self):
+        global _free_bytes
+        if sys is None or sys.is_finalizing():   # the process's memory goes with it
+            return
+        with _lock:
+            keep = _free_bytes + self.nbytes <= POOL_BYTES
+            if keep:
+                _free.setdefault(self.nbytes, []).append(self.address)
+                _free_bytes += self.nbytes
+        if not keep:
+            _hip.load().pgk_host_free(C.c_void_p(self.address))
+
+
+def empty(shape: tuple, dtype=np.float32) -> np.ndarray:
+    """np.empty on pinned memory; on ordinary memory where none is to be had."""
+    global _free_bytes
+    dtype = np.dtype(dtype)
+    nbytes = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+    if nbytes == 0:
+        return np.empty(shape, dtype)
+    address = None
+    with _lock:
+        if _free.get(nbytes):
+            address = _free[nbytes].pop()
+            _free_bytes -= nbytes
+    if address is None:
+        p = C.c_void_p()
+        if _hip.load().pgk_host_alloc(C.byref(p), nbytes) != 0 or not p.value:
+            return np.empty(shape, dtype)
+        address = p.value
+    return np.asarray(_Block(address, nbytes, tuple(int(n) for n in shape), dtype.str))

@@ -2164,8 +2164,7 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         flash_items((FlashItem*)(host.data() + item_off), h_lens, h_starts, h_slots, n_seqs);
         std::copy(h_want, h_want + n_want, host.begin() + want_off);
     }
-    PGK_CHECK_HIP(hipMemcpyAsync(e->pf_tokens, many ? host.data() : h_tokens, (size_t)meta * 4, hipMemcpyHostToDevice, st));
-    PGK_CHECK_HIP(hipStreamSynchronize(st));  // h_tokens may be pageable: make the copy complete before returning control
+    if (pgk_status r = stage_upload(e->up, e->pf_tokens, many ? host.data() : h_tokens, (size_t)meta * 4, st)) return r;
     const int2* d_at = many ? (const int2*)(e->pf_tokens + at_off) : nullptr;
     const FlashItem* d_items = (const FlashItem*)(e->pf_tokens + item_off);
     const bool fp8 = c.weight_format != 0;

@@ -3,7 +3,23 @@
 
 #include "engine_state.hip.h"
 
+#include <algorithm>
+
 namespace pgk {
+
+// Tokens and positions of a state travel as the launch's arguments: no copy to set up, nothing of the caller's to wait for.
+struct StateArgs {
+    static constexpr int MOST = 64;
+    int n;
+    int32_t tokens[MOST], positions[MOST];
+};
+__global__ void set_state_kernel(StateArgs a, int32_t* tokens, int32_t* positions) {
+    const int b = threadIdx.x;
+    if (b < a.n) {
+        tokens[b] = a.tokens[b];
+        positions[b] = a.positions[b];
+    }
+}
 
 thread_local Probe* g_probe = nullptr;   // measurement hooks: engine_common.hip.h
 
@@ -24,6 +40,8 @@ pgk_status pgk_engine_destroy(pgk_engine eh) {
     if (e->u_ring) (void)pgk_free(e->u_ring);
     if (e->sampled) (void)pgk_free(e->sampled);
     if (e->sample_scratch) (void)pgk_free(e->sample_scratch);
+    stage_free(e->up);
+    stage_free(e->down);
     delete e;
     return PGK_OK;
 }
@@ -83,8 +101,14 @@ pgk_status pgk_engine_set_state(pgk_engine eh, const int32_t* h_tokens, const in
     hipStream_t st = resolve_stream(s);
     e->pos_hi = 0;
     for (int b = 0; b < batch; ++b) e->pos_hi = h_positions[b] > e->pos_hi ? h_positions[b] : e->pos_hi;
-    PGK_CHECK_HIP(hipMemcpyAsync(e->tokens, h_tokens, (size_t)batch * 4, hipMemcpyHostToDevice, st));
-    PGK_CHECK_HIP(hipMemcpyAsync(e->positions, h_positions, (size_t)batch * 4, hipMemcpyHostToDevice, st));
+    for (int b = 0; b < batch; b += StateArgs::MOST) {
+        StateArgs a;
+        a.n = batch - b < StateArgs::MOST ? batch - b : StateArgs::MOST;
+        std::copy(h_tokens + b, h_tokens + b + a.n, a.tokens);
+        std::copy(h_positions + b, h_positions + b + a.n, a.positions);
+        set_state_kernel<<<1, StateArgs::MOST, 0, st>>>(a, e->tokens + b, e->positions + b);
+        PGK_LAUNCH_CHECK();
+    }
     // the residual stream enters a step already holding the embeddings of the state tokens
     if (pgk_status r = e->kind->embed_state(e, batch, st)) return r;
     PGK_CHECK_HIP(hipStreamSynchronize(st));
@@ -292,8 +316,11 @@ pgk_status pgk_engine_read_tokens(pgk_engine eh, int32_t* h_out, int batch, int 
     PGK_REQUIRE(batch >= 1 && batch <= e->cfg.max_batch, "pgk_engine_read_tokens: bad batch %d", batch);
     hipStream_t st = resolve_stream(s);
     // log rows are max_batch wide; return the first `batch` columns, step-major
-    std::vector<int32_t> tmp((size_t)n_steps * e->cfg.max_batch);
-    if (n_steps) PGK_CHECK_HIP(hipMemcpyAsync(tmp.data(), e->token_log, tmp.size() * 4, hipMemcpyDeviceToHost, st));
+    const size_t words = (size_t)n_steps * e->cfg.max_batch;
+    std::vector<int32_t> pageable;
+    int32_t* tmp = (int32_t*)stage_room(e->down, words * 4);     // (into pageable memory the copy is set up when the last step has ended)
+    if (!tmp) { pageable.resize(words); tmp = pageable.data(); }
+    if (n_steps) PGK_CHECK_HIP(hipMemcpyAsync(tmp, e->token_log, words * 4, hipMemcpyDeviceToHost, st));
     PGK_CHECK_HIP(hipStreamSynchronize(st));
     for (int t = 0; t < n_steps; ++t)
         for (int b = 0; b < batch; ++b) h_out[(size_t)t * batch + b] = tmp[(size_t)t * e->cfg.max_batch + b];

@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <cstdlib>
 #include <type_traits>
+#include <cstring>
 #include <vector>
 
 #include "engine_common.hip.h"
@@ -123,6 +124,14 @@ struct EngineKind {
     void (*destroy)(Engine* e);                                          // null: nothing beyond Engine itself
 };
 
+// Pinned host memory of an engine; `sent`: the end of the copy that last read it
+struct HostStage {
+    void* p = nullptr;
+    size_t cap = 0;
+    hipEvent_t sent = nullptr;
+    bool busy = false;
+};
+
 struct Engine {
     const EngineKind* kind = nullptr;
     void* kind_state = nullptr;
@@ -188,10 +197,50 @@ struct Engine {
     int step_span = 0;          // the split-KV slicing of the step being enqueued (launch_attn); 0: the whole cache
     int launches_per_step = 0;
     std::vector<void*> allocs;
+    HostStage up, down;         // uploads and read-backs of a few bytes
 
     size_t kv_layer_elems() const { return (size_t)cfg.max_batch * cfg.num_kv_heads * cfg.max_seq_len * cfg.head_dim; }
     int qkv_dim() const { return (cfg.num_heads + 2 * cfg.num_kv_heads) * cfg.head_dim; }
 };
+
+// `bytes` of pinned host memory in s.p, free to be written (null: none to be had)
+inline void* stage_room(HostStage& s, size_t bytes) {
+    if (s.busy && hipEventSynchronize(s.sent) == hipSuccess) s.busy = false;
+    if (s.busy) return nullptr;
+    if (bytes > s.cap) {
+        if (s.p) (void)hipHostFree(s.p);
+        s.p = nullptr;
+        s.cap = 0;
+        const size_t want = bytes > 16384 ? bytes : 16384;
+        if (hipHostMalloc(&s.p, want, hipHostMallocDefault) != hipSuccess) { s.p = nullptr; (void)hipGetLastError(); return nullptr; }
+        s.cap = want;
+    }
+    if (!s.sent && hipEventCreateWithFlags(&s.sent, hipEventDisableTiming) != hipSuccess) { s.sent = nullptr; (void)hipGetLastError(); return nullptr; }
+    return s.p;
+}
+// Upload of host memory that is the caller's again on return, without a wait: by way of the stage, whose next use waits for this one's end.  Not inside a capture,
+// which would read the stage again at every replay.
+inline pgk_status stage_upload(HostStage& s, void* dst, const void* src, size_t bytes, hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    PGK_CHECK_HIP(hipStreamIsCapturing(st, &cs));
+    PGK_REQUIRE(cs == hipStreamCaptureStatusNone, "upload of host data inside a stream capture");
+    if (void* p = stage_room(s, bytes)) {
+        memcpy(p, src, bytes);
+        PGK_CHECK_HIP(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, st));
+        PGK_CHECK_HIP(hipEventRecord(s.sent, st));
+        s.busy = true;
+        return PGK_OK;
+    }
+    PGK_CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+    PGK_CHECK_HIP(hipStreamSynchronize(st));
+    return PGK_OK;
+}
+inline void stage_free(HostStage& s) {
+    if (s.busy) (void)hipEventSynchronize(s.sent);
+    if (s.p) (void)hipHostFree(s.p);
+    if (s.sent) (void)hipEventDestroy(s.sent);
+    s = HostStage{};
+}
 
 inline pgk_status dev_alloc(Engine* e, void** p, size_t bytes, size_t* acct) {
     pgk_status r = pgk_malloc(p, bytes);

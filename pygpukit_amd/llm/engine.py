@@ -12,6 +12,7 @@ import ctypes as C
 import numpy as np
 
 from pygpukit_amd import _hip
+from pygpukit_amd.core import pinned
 from pygpukit_amd.core.array import GPUArray
 from pygpukit_amd.core.dtypes import bfloat16, float32, int32
 from pygpukit_amd.core.factory import from_numpy, zeros
@@ -72,7 +73,7 @@ class Engine:
         """Run the prompt through the MFMA path, filling sequence slot `seq`'s KV rows; returns the last
         row's logits (fp32 [V]) when asked.  all_logits: optional bf16 [n, V] device buffer."""
         toks = np.ascontiguousarray(tokens, dtype=np.int32)
-        out = np.empty(self.config["vocab_size"], np.float32) if want_last_logits else None
+        out = pinned.empty((self.config["vocab_size"],)) if want_last_logits else None
         _hip.call("pgk_engine_prefill", self.handle, seq, toks.ctypes.data_as(_hip.c_i32_p), len(toks), start_pos,
                   all_logits._p if all_logits is not None else None,
                   out.ctypes.data_as(C.POINTER(C.c_float)) if out is not None else None, None)
@@ -98,7 +99,7 @@ class Engine:
                 raise ValueError("prefill_batch: wanted row outside its prompt")
         w = np.asarray([f + i for f, r in zip(first, rows) for i in r], np.int32)
         toks = np.ascontiguousarray(np.concatenate([np.asarray(p, np.int32) for p in prompts]))
-        out = np.empty((len(w), self.config["vocab_size"]), np.float32)
+        out = pinned.empty((len(w), self.config["vocab_size"]))
         i32 = lambda a: a.ctypes.data_as(_hip.c_i32_p)  # noqa: E731
         _hip.call("pgk_engine_prefill_batch", self.handle, len(prompts), i32(slots), i32(lens), i32(starts), i32(toks), len(w),
                   i32(w) if len(w) else None, out.ctypes.data_as(C.POINTER(C.c_float)) if len(w) else None, None)
