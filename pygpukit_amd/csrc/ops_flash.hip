@@ -14,7 +14,7 @@
 //   * alpha (the running-max rescale) and 1/l are per-lane scalars for the O^T accumulators (q is again the lane).
 // (V used to be transposed by a pass of its own over the whole context: 5.3 us of a 1531-token prompt's 42 us of
 // attention per layer, 5.8 of 42 for 384 tokens at position 3201.)
-// Workgroup = 4 waves = 128 query rows of one head; KV tiles of 64 positions, K and V [64][D] double
+// Workgroup = 4 waves (or two sides of 4, each with half the KV tiles: flash_plan) = 128 query rows of one head; KV tiles of 64 positions, K and V [64][D] double
 // buffered in LDS (64 KiB at D = 128: two workgroups per CU), fetched by LDS-DMA, K a tile ahead of V: the products
 // S(t + 1) run between the exponentials of S(t).  One barrier per tile.
 // Workgroups are ordered heavy-first (causal: late query tiles see more keys) and all query heads of a kv head
@@ -74,11 +74,8 @@ struct FlashMany {
     long long slot_stride;         // elements between the caches of two slots
 };
 
-// KV split (short prompts): nsplit > 1 cuts a query tile's KV tiles into nsplit contiguous runs, one workgroup each; every
-// workgroup leaves a NORMALISED partial output (type T) and its (m, l) per row, and flash_merge_kernel combines them.
-// Without it the causal imbalance sets the time of a short prompt: at S = 2048 with 16 heads there are 256 workgroups -
-// one per CU, the heaviest walks 32 KV tiles, the lightest 2 - and the launch lasts as long as the heaviest (52 us for
-// 17 GFLOP).  Cut in two and dealt heavy-first, two half-runs share a CU and the CUs finish together.
+// KV split: nsplit > 1 cuts a query tile's KV tiles into nsplit contiguous runs, one workgroup each; every workgroup leaves a
+// NORMALISED partial output (type T) and its (m, l) per row, and flash_merge_kernel combines them.
 struct FlashSplit {
     int nsplit;
     float* ml;      // [nsplit][Hq][q_len][2]  (m in the exp2 domain, l)
@@ -120,19 +117,20 @@ template <class T, int N> __device__ __forceinline__ void flash_gate_cols(const 
     }
 }
 
-template <class T, int D, bool WIN = false, bool BIAS = false>
-__global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
+template <class T, int D, bool WIN = false, bool BIAS = false, int SIDES = 1>
+__global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
                                                               int q_len, int kv_len, float scale_log2e, FlashStrides sd,
                                                               FlashSplit sp, FlashWindow win, FlashMany many) {
     constexpr int NC = D / 8;            // 16-byte chunks per K row
     constexpr int KS = D / 16;           // k-steps of Q.K^T
     constexpr int DT = D / 32;           // 32-row tiles of O^T
     constexpr int K_BYTES = 64 * D * 2, V_BYTES = K_BYTES;
-    extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // K[2] | V[2]
-    auto Ks = [&](int buf) -> char* { return fl_smem + buf * K_BYTES; };
-    auto Vs = [&](int buf) -> char* { return fl_smem + 2 * K_BYTES + buf * V_BYTES; };
+    extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // of each side K[2] | V[2]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wid = wave & 3, ql = lane & 31, h = lane >> 5;
+    const int side = SIDES == 1 ? 0 : wave >> 2, side_at = side * (2 * K_BYTES + 2 * V_BYTES);
+    auto Ks = [&](int buf) -> char* { return fl_smem + side_at + buf * K_BYTES; };
+    auto Vs = [&](int buf) -> char* { return fl_smem + side_at + 2 * K_BYTES + buf * V_BYTES; };
 
-    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), ql = lane & 31, h = lane >> 5;
     // workgroup id -> (kv head, query head in its group, query tile, KV run), heavy tiles first
     const int rep = hq / hkv;
     const int id = blockIdx.x;
@@ -183,7 +181,14 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     // this workgroup's run of KV tiles [t0, t1)
     const int first_kv = WIN ? causal_off + qt * FL_BQ - win.window + 1 : 0;
     const int tb = WIN && first_kv > 0 ? first_kv / FL_BKV : 0;            // tiles before it are outside every row's window
-    const int t0 = tb + (int)((long long)(nt_all - tb) * split / sp.nsplit), t1 = tb + (int)((long long)(nt_all - tb) * (split + 1) / sp.nsplit);
+    int t0 = tb + (int)((long long)(nt_all - tb) * split / sp.nsplit), t1 = tb + (int)((long long)(nt_all - tb) * (split + 1) / sp.nsplit);
+    int last = t1;                                  // where the loop ends; both sides pass as many barriers
+    if constexpr (SIDES == 2) {
+        const int half = (t1 - t0 + 1) / 2;
+        if (side) t0 += half;
+        else t1 = t0 + half;
+        last = t0 + half;
+    }
 
     // One wave-instruction of LDS-DMA moves 1 KiB = ROWS rows; the images' swizzles are applied on the source side (lane l of a row fetches the chunk that belongs
     // into its 16 bytes).  A wave moves NI instructions of K and of V per tile.  A tile is a buffer of the rows that are there: what lies beyond comes as zeros
@@ -197,7 +202,7 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
         ko[i] = (uint32_t)(r * sd.ks + (ds ^ (r & (NC - 1))) * 8) * 2;
         vo[i] = (uint32_t)(r * sd.ks + (ds ^ fl_v_sw<D>(r)) * 8) * 2;
     }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(fl_lds_addr(fl_smem) + wid * NI * 1024), row_bytes = (uint32_t)(sd.ks * 2);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(fl_lds_addr(fl_smem) + side_at + wid * NI * 1024), row_bytes = (uint32_t)(sd.ks * 2);
     auto tile_of = [&](const T* base, int t) {
         const uint64_t at = (uint64_t)(uintptr_t)(base + (size_t)t * FL_BKV * sd.ks);
         const int last = t < t1 ? min(kv_len - t * FL_BKV, FL_BKV) - 1 : -1;     // last row that is there
@@ -270,7 +275,7 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
     typedef short fl_v4s __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) fl_v4s* fl_lds_v4;
     const int tr = (lane & 15) >> 2, tc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), t8 = 8 * (lane & 1);
-    for (int t = t0; t < t1; ++t) {
+    for (int t = t0; t < last; ++t) {
         const int buf = t & 1, kv0 = t * FL_BKV;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // this wave's share of K(t + 1) and V(t)
         __syncthreads();                                                 // ... everyone's; and everyone has read K(t) and V(t - 1)
@@ -373,6 +378,36 @@ __global__ __launch_bounds__(FL_THREADS, 2) void flash_fwd_kernel(const T* q, co
                 }
             }
         }
+    }
+
+    if constexpr (SIDES == 2) {      // the second side's state comes to the first by way of the tiles' place
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // requests past the run's end
+        __syncthreads();
+        float4* mine = reinterpret_cast<float4*>(fl_smem) + wid * (4 * DT + 1) * 64 + lane;
+        if (side) {
+#pragma unroll
+            for (int i = 0; i < DT; ++i)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) mine[(4 * i + g) * 64] = make_float4(o[i][4 * g], o[i][4 * g + 1], o[i][4 * g + 2], o[i][4 * g + 3]);
+            mine[4 * DT * 64] = make_float4(m_run, l_run, 0.f, 0.f);
+        }
+        __syncthreads();
+        if (side) return;
+        const float4 ml = mine[4 * DT * 64];
+        const float m = fmaxf(m_run, ml.x), m_use = m == -INFINITY ? 0.f : m;
+        const float a0 = __builtin_amdgcn_exp2f(m_run - m_use), a1 = __builtin_amdgcn_exp2f(ml.x - m_use);
+        l_run = l_run * a0 + ml.y * a1;
+        m_run = m;
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 v = mine[(4 * i + g) * 64];
+                o[i][4 * g] = fmaf(v.x, a1, o[i][4 * g] * a0);
+                o[i][4 * g + 1] = fmaf(v.y, a1, o[i][4 * g + 1] * a0);
+                o[i][4 * g + 2] = fmaf(v.z, a1, o[i][4 * g + 2] * a0);
+                o[i][4 * g + 3] = fmaf(v.w, a1, o[i][4 * g + 3] * a0);
+            }
     }
 
     // ---- normalise and store: lane = query row, registers 4g..4g+3 of tile i are d = 32i + 8g + 4h .. +3 ----
@@ -503,20 +538,29 @@ static int flash_cus() {
     return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
-// KV runs per query tile, at least four KV tiles to a run.  Where the causal edge is most of the work (contexts under twice the rows) two, of which a heavy and a light
-// one share a CU, if one round holds them and the heaviest tile is long enough for the merge to pay; elsewhere as many as one round of workgroups holds: of two per
-// CU (the kernel's occupancy), or of one per CU where a long context makes all runs alike and that many still cut it well.  A second round costs more than the
-// shorter runs save, and every run costs the merge.  Launch and merge, us (runs): 16 heads, 512 rows 14.8 (1) 16.2 (2); 1000 23.8 (1) 23.2 (2) 25.5 (4); 1200 27.2 (1)
-// 27.5 (2); 1531 34.1 (1) 31.4 (2); 2000 44.7 (1) 38.9 (2); 3000 63.6 (1) 66.3 (2); 800 at 1200 28.9 (1) 25.2 (2) 26.2 (4); 32 heads, 500 14.9 (1) 18.6 (2), 1000 25.5 (1) 30.2
-// (2); longer contexts, 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5) 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).
-static int flash_runs(long long wgs, int q_len, int kv_len, int most) {
+// KV runs per query tile and sides of a workgroup (1 or 2: half a run's tiles each), at least four KV tiles to a run.
+// Where the causal edge is most of the work (contexts under twice the rows) a launch of up to two workgroups per CU lasts as long as its heaviest tile, alone on its CU for
+// most of that, 1.47 us a KV tile; with two sides it has the CU's other half too, 1.1 us, and nothing to merge outside.  Beyond, two workgroups of their own time per CU do
+// more (one barrier makes the sides wait for each other); up to ten KV tiles the sides' merge costs what they save.  Where at most every CU has a workgroup and the context
+// is long enough for the merge, two runs do better, of which a heavy and a light one share a CU.  In an engine's prompts, us a launch, one run / two runs with merge / two
+// sides: 16 heads, 550 rows 16.0 / - / 16.6, 1024 26.0 / - / 24.4, 1531 - / 31.5 / 34.2, 1800 - / 36.9 / 39.0, 2300 54.2 / - / 47.5, 3000 71.2 / - / 60.0; 32 heads, 700 20.2 / - / 19.6, 1100 31.1 / - / 28.0.  By themselves:
+// 16 heads, 512 rows 15.0 / 16.1 / 15.9; 1000 24.9 / 24.0 / 22.8; 2300 49.6 / 46.7 / 41.5; 3300 72.9 / 72.0 / 58.3; 4000 94.9 / 98.5 / 81.0; 5000 127 / - / 132; 32 heads, 700
+// 19.6 / 25.5 / 18.2, 1100 28.7 / 37.5 / 24.6, 2500 69.9 / - / 78.0; 8 heads, 4000 79.4 / 57.0 / 63.9; head dim 64, 16 heads, 700 13.5 / 14.0 / 12.1, 2300 35.7 / 33.0 / 29.0.
+// Longer contexts: as many runs as one round of workgroups holds: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and that many
+// still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
+// 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
+struct FlashPlan { int runs, sides; };
+static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
-    if (kv_len < 2LL * q_len) return wgs <= cus && kv_len >= 1200 && most >= 2 ? 2 : 1;
+    if (kv_len < 2LL * q_len) {
+        if (wgs <= cus && kv_len >= 1200 && most >= 2) return {2, 1};
+        return {1, kv_len > 10 * FL_BKV && wgs <= 2 * cus ? 2 : 1};
+    }
     long long n = cus / wgs;
     if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
     if (n > most) n = most;
     if (n > ceil_div(kv_len, FL_BKV) / 4) n = ceil_div(kv_len, FL_BKV) / 4;
-    return n < 1 ? 1 : (int)n;
+    return {n < 1 ? 1 : (int)n, 1};
 }
 // with a sliding window: up to four runs over the `span` keys that the heaviest query tile walks, until two workgroups per CU are reached
 static int flash_window_runs(long long wgs, int span) {
@@ -532,7 +576,8 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
                                const FlashMany& many = FlashMany{}) {
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-    int nsplit = WIN ? flash_window_runs((long long)tiles * hq, span) : flash_runs((long long)tiles * hq, q_len, kv_len, 16);
+    const FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
+    int nsplit = plan.runs;
     const bool wide = many.items || q_len <= 128;
     // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
     // tiles of the first-generation kernel 61, 31 and 239)
@@ -551,16 +596,21 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
             nsplit = sp.nsplit = 1;        // no memory, or a stream whose end the pool cannot see: slower, and right
         }
     }
-    constexpr size_t LDS = 4 * (size_t)(64 * D * 2);
-    static bool attr_done = false;
-    if (LDS > 48 * 1024 && !attr_done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<T, D, WIN, BIAS>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        attr_done = true;
-    }
-    flash_fwd_kernel<T, D, WIN, BIAS><<<tiles * hq * nsplit, FL_THREADS, LDS, st>>>(q, k, v, out, hq, hkv, q_len, kv_len,
-                                                                      scale * 1.4426950408889634f, sd, sp, win, many);
-    hipError_t e = hipGetLastError();
+    auto launch = [&](auto sides) -> hipError_t {
+        constexpr int SIDES = decltype(sides)::value;
+        constexpr size_t LDS = SIDES * 4 * (size_t)(64 * D * 2);
+        auto kernel = &flash_fwd_kernel<T, D, WIN, BIAS, SIDES>;
+        static bool attr_done = false;
+        if (LDS > 48 * 1024 && !attr_done) {
+            if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS); e != hipSuccess) return e;
+            attr_done = true;
+        }
+        kernel<<<tiles * hq * nsplit, SIDES * FL_THREADS, LDS, st>>>(q, k, v, out, hq, hkv, q_len, kv_len, scale * 1.4426950408889634f, sd, sp, win, many);
+        return hipGetLastError();
+    };
+    hipError_t e;
+    if constexpr (WIN) e = launch(std::integral_constant<int, 1>{});
+    else e = plan.sides == 2 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
     if (e == hipSuccess && nsplit > 1) {
         const size_t work = (size_t)q_len * hq * (D / 8);
         const unsigned grid = (unsigned)((work + 255) / 256);

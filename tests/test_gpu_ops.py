@@ -940,6 +940,17 @@ def test_sdpa_reads_nothing_behind_the_context(dt, cfg):
     assert rel_err(host(out), ref) < bar, rel_err(host(out), ref)
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(2, 1, 641, 641, 128), (4, 2, 699, 705, 64), (2, 2, 500, 768, 128), (1, 1, 700, 1199, 128), (33, 3, 1281, 1281, 128)])
+def test_sdpa_with_the_tiles_of_a_run_shared_by_two_sides(dt, cfg):
+    """11 and 12 KV tiles in the heaviest query tile and 2 in the lightest, a context before the rows, more workgroups than CUs: the bars of the tests that are
+    called."""
+    test_sdpa_few_rows_over_a_long_context(dt, cfg)
+    test_sdpa_reads_nothing_behind_the_context(dt, cfg)
+    if dt == "bfloat16" and cfg[1] == 2:                # (a key head that stays as it is, a position that every row sees)
+        test_sdpa_nan_and_infinite_keys(cfg)
+
+
 # ----------------------------------------------------------------------------- paged KV cache / continuous batching
 def _paged_setup(rng, num_seqs, hkv, bs, d, ctxs, dt, num_blocks=None):
     max_blocks = max((c + bs - 1) // bs for c in ctxs) + 1
