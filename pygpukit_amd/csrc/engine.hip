@@ -56,6 +56,8 @@ pgk_status flash_prefill_q8(const void* q, const void* k, const void* v, uint8_t
                             float scale, long long qh, long long qs, long long kh, long long ks, hipStream_t st);   // ops_flash.hip
 bool engine_gemm_qkv_heads_ok(int M, int N, int K);            // ops_gemm.hip: QKV projection with per-head norm + RoPE + cache write as its epilogue
 pgk_status engine_gemm_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni);
+pgk_status flash_prefill(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, int d, float scale, long long qh, long long qs,
+                         long long kh, long long ks, long long oh, long long os, int dt16, hipStream_t st, bool one_side);
 bool engine_gemm_swiglu_ok(int M, int I, int K, bool fp8);     // ops_gemm.hip: gate / up projection with the SwiGLU epilogue
 pgk_status engine_gemm_swiglu_nt(const bf16* A, const void* W, const bf16* wscale, bool fp8, bf16* act, int M, int I, int K, hipStream_t st, bool packed, const NormIn& ni);
 bool gemm_fp8_qkv_heads_ok(int M, int N, int K);               // ops_fp8_gemm.hip: the same epilogue on the fp8 x fp8 256-tile kernel
@@ -2312,6 +2314,9 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
         } else if (many && sdpa_flash_enabled()) {
             if (pgk_status r = flash_many(qkv, kc, vc, attn, d_items, n_items, n, longest, slot_stride, c.num_heads, c.num_kv_heads, D, 1.0f / sqrtf((float)D), D, NQKV,
                                           (long long)c.max_seq_len * D, D, D, QD, st))
+                return r;
+        } else if (c.weight_format == 2 && n > 128 && !many && sdpa_flash_enabled()) {     // e4m3 rounding follows, in a pass of its own: the sums of flash_prefill_q8
+            if (pgk_status r = flash_prefill(qkv, kc, vc, attn, c.num_heads, c.num_kv_heads, n, kv_len, D, 1.0f / sqrtf((float)D), D, NQKV, (long long)c.max_seq_len * D, D, D, QD, 0, st, true))
                 return r;
         } else {
             for (int i = 0, r0 = 0; i < n_seqs; r0 += h_lens[i++]) {

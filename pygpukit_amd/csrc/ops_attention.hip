@@ -422,7 +422,7 @@ pgk_status attn_short_gated(const void* q, const void* k, const void* v, void* o
 
 pgk_status flash_prefill(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, int d,
                          float scale, long long qh, long long qs, long long kh, long long ks, long long oh, long long os,
-                         int dt16, hipStream_t st);
+                         int dt16, hipStream_t st, bool one_side = false);
 
 // The reference's A/B switches, same names and values (native/ops/nn/attention/sdpa_causal.inl:380-447), read per call:
 //   PYGPUKIT_FLASH_ATTENTION  "0"/"false": never the tiled MFMA flash kernels (one-workgroup-per-row fallback, kv_len <= 15360);

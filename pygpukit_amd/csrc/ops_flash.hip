@@ -549,6 +549,8 @@ static int flash_cus() {
 // Longer contexts: as many runs as one round of workgroups holds: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and that many
 // still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
 // 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
+// (Results that are rounded to e4m3 next, by whichever kernel, ask for one side: the codes magnify a sum's last bit to a sixteenth, and a prompt in one pass and in pieces would
+// no longer agree - 4096 rows of 32 heads at once and as two of 2048, which alone had two sides, were 0.028 apart in the logits, with one side each under 0.01.)
 struct FlashPlan { int runs, sides; };
 static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
@@ -573,7 +575,7 @@ static int flash_window_runs(long long wgs, int span) {
 template <class T, int D, bool WIN = false, bool BIAS = false>
 static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int hq, int hkv, int q_len, int kv_len, float scale,
                                const FlashStrides& sd, hipStream_t st, uint8_t* q8 = nullptr, float* q8s = nullptr, const FlashWindow& win = FlashWindow{},
-                               const FlashMany& many = FlashMany{}) {
+                               const FlashMany& many = FlashMany{}, bool one_side = false) {
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
     const FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
@@ -610,7 +612,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     };
     hipError_t e;
     if constexpr (WIN) e = launch(std::integral_constant<int, 1>{});
-    else e = plan.sides == 2 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
+    else e = plan.sides == 2 && !one_side ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
     if (e == hipSuccess && nsplit > 1) {
         const size_t work = (size_t)q_len * hq * (D / 8);
         const unsigned grid = (unsigned)((work + 255) / 256);
@@ -623,17 +625,17 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     return PGK_OK;
 }
 
-// entry used by ops_attention.hip's dispatcher; dt16: 0 = bf16, 1 = f16
+// entry used by ops_attention.hip's dispatcher and by an engine whose next step rounds the result to e4m3 (one_side); dt16: 0 = bf16, 1 = f16
 pgk_status flash_prefill(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, int d,
                          float scale, long long qh, long long qs, long long kh, long long ks, long long oh, long long os,
-                         int dt16, hipStream_t st) {
+                         int dt16, hipStream_t st, bool one_side) {
     const FlashStrides sd{qh, qs, kh, ks, oh, os};
     if (dt16 == 0) {
-        if (d == 128) return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, q_len, kv_len, scale, sd, st);
-        return flash_launch<bf16, 64>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, q_len, kv_len, scale, sd, st);
+        if (d == 128) return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, q_len, kv_len, scale, sd, st, nullptr, nullptr, FlashWindow{}, FlashMany{}, one_side);
+        return flash_launch<bf16, 64>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, q_len, kv_len, scale, sd, st, nullptr, nullptr, FlashWindow{}, FlashMany{}, one_side);
     }
-    if (d == 128) return flash_launch<f16, 128>((const f16*)q, (const f16*)k, (const f16*)v, (f16*)out, hq, hkv, q_len, kv_len, scale, sd, st);
-    return flash_launch<f16, 64>((const f16*)q, (const f16*)k, (const f16*)v, (f16*)out, hq, hkv, q_len, kv_len, scale, sd, st);
+    if (d == 128) return flash_launch<f16, 128>((const f16*)q, (const f16*)k, (const f16*)v, (f16*)out, hq, hkv, q_len, kv_len, scale, sd, st, nullptr, nullptr, FlashWindow{}, FlashMany{}, one_side);
+    return flash_launch<f16, 64>((const f16*)q, (const f16*)k, (const f16*)v, (f16*)out, hq, hkv, q_len, kv_len, scale, sd, st, nullptr, nullptr, FlashWindow{}, FlashMany{}, one_side);
 }
 
 // sliding-window causal attention with an optional output gate and distance bias (bf16, head_dim 64 / 128, one key head per query head or
@@ -656,7 +658,7 @@ pgk_status flash_prefill_q8(const void* q, const void* k, const void* v, uint8_t
                             float scale, long long qh, long long qs, long long kh, long long ks, hipStream_t st) {
     PGK_REQUIRE(q8 && q8s && q_len > 128, "flash_prefill_q8: needs output buffers and q_len > 128 (got %d)", q_len);
     const FlashStrides sd{qh, qs, kh, ks, 0, 0};
-    return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, nullptr, hq, hkv, q_len, kv_len, scale, sd, st, q8, q8s);
+    return flash_launch<bf16, 128>((const bf16*)q, (const bf16*)k, (const bf16*)v, nullptr, hq, hkv, q_len, kv_len, scale, sd, st, q8, q8s, FlashWindow{}, FlashMany{}, true);
 }
 
 int flash_items(FlashItem* items, const int* lens, const int* starts, const int* slots, int n) {
