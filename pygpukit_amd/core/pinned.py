@@ -1,8 +1,8 @@
 """NumPy arrays on pinned host memory, for results that a call copies back from the device.
 
 Into pageable memory the runtime copies by way of its own pinned buffers and touches every fresh page of the result: a prompt of 93 tokens with its
-151936 fp32 logits took 1.23 ms that way, 1.15 into a pinned array, sixteen prompts in one call 5.4 and 5.0.  A block returns to the pool with the last view of its array; the pool keeps at most POOL_BYTES of free blocks
-and gives the rest back."""
+151936 fp32 logits took 1.23 ms that way, 1.15 into a pinned array, sixteen prompts in one call 5.4 and 5.0.  A block returns to the pool with the last view
+of its array; the pool keeps at most POOL_BYTES of free blocks and gives the rest back.  Larger arrays, which the pool could never keep, are ordinary ones."""
 
 from __future__ import annotations
 
@@ -15,7 +15,7 @@ import numpy as np
 from pygpukit_amd import _hip
 
 POOL_BYTES = 64 << 20
-_lock = threading.Lock()
+_lock = threading.RLock()   # a garbage collection under it may end another block in the same thread
 _free: dict[int, list[int]] = {}
 _free_bytes = 0
 
@@ -41,11 +41,11 @@ class _Block:
 
 
 def empty(shape: tuple, dtype=np.float32) -> np.ndarray:
-    """np.empty on pinned memory; on ordinary memory where none is to be had."""
+    """np.empty on pinned memory; on ordinary memory for more than POOL_BYTES and where no pinned memory is to be had."""
     global _free_bytes
     dtype = np.dtype(dtype)
     nbytes = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
-    if nbytes == 0:
+    if nbytes == 0 or nbytes > POOL_BYTES:
         return np.empty(shape, dtype)
     address = None
     with _lock:
