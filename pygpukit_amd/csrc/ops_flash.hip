@@ -380,8 +380,8 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
         }
     }
 
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                     // requests past the run's end, before the LDS is given back
     if constexpr (SIDES == 2) {      // the second side's state comes to the first by way of the tiles' place
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // requests past the run's end
         __syncthreads();
         float4* mine = reinterpret_cast<float4*>(fl_smem) + wid * (4 * DT + 1) * 64 + lane;
         if (side) {
