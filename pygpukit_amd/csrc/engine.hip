@@ -41,6 +41,9 @@ pgk_status engine_gemm_resid_nt(const bf16* A, const void* W, float* h, int M, i
 bool engine_gemm_packed_ok(int M, int N, int K);
 bool gemm_few_swiglu_ok(int I, int K);                         // ops_gemm256.hip
 pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, int I, int K, const NormIn& ni, hipStream_t st);
+bool gemm_few_logits_ok(int M, int V, int K);
+int gemm_few_logits_blocks(int V);
+pgk_status gemm_few_logits_nt(const bf16* A, const bf16* wp, float* logits, float* best_val, int* best_idx, int M, int V, int K, hipStream_t st);
 int wsgemm_pick_splits(int N, int K, bool allow_split);
 int engine_gemm_pick_splits(int M, int N, int K);
 int engine_gemm_qkv_splits(int M, int N, int K, bool fused);
@@ -811,7 +814,7 @@ __global__ __launch_bounds__(256) void attn_oproj_kernel(unsigned long long* tl,
 // attn_oproj_kernel above spends 2.1 of its 5.5 us in the score / P.V loop: one wave per SIMD, ~750 VALU instructions per 48
 // positions (v_dot2c at ~10 cycles of issue, DPP reductions).  The first attempt to move Q.K^T to MFMA loaded the K rows
 // from global memory in A-fragment shape (lane = row): 64 separate 16-byte pieces per instruction, and the kernel lost
-// more in its load issue phase than the MFMAs won (DESIGN.md 7).  Here the cached rows are staged ROW-MAJOR by LDS-DMA -
+// more in its load issue phase than the MFMAs won.  Here the cached rows are staged ROW-MAJOR by LDS-DMA -
 // the same bytes per instruction as the register loads they replace, 1 KiB contiguous each - and the fragments come out
 // of LDS: the one-tile prefill kernel's scheme (ops_attention.hip, attn_short_kernel) with the G query heads of the kv
 // head as the only live columns:
@@ -1800,7 +1803,7 @@ static pgk_status decode_chunk_batched(Engine* e, int b0, int M, bool last, hipS
             a.xin16 = x16;
         }
         // 16-row workgroups (N / 16 >= 192) stream the fragment-major copy where the engine holds one: one coalesced KiB per
-        // load instead of 64 separate 16-byte pieces of the row-major matrix (the batched lm_head's gain, DESIGN.md 4.1)
+        // load instead of 64 separate 16-byte pieces of the row-major matrix (the batched lm_head's gain)
         if (!FP8 && e->packed_ok) a.wp = e->packed[l].qkv;
         if (pgk_status r = batched_proj(FP8, tiled ? PRO_PLAIN : PRO_NORM, EPI_STORE, a, M, st)) return r;
         mark(KC_ATTN);
@@ -1930,7 +1933,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
         pending = s_d;
         *launches += (direct || stream_slices(e, M) == 1 ? 7 : 8) + gqa_chunks(c.num_heads / c.num_kv_heads, M) - 1;
     }
-    const int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
+    int nblk = ceil_div(c.vocab_size, 16) < 2048 ? ceil_div(c.vocab_size, 16) : 2048;
     if (pgk_status r = norm(e->final_norm)) return r;     // also folds the last down_proj's slabs into the residual stream
     mark(KC_LMHEAD);
     FusedArgs a{};
@@ -1939,10 +1942,11 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
     a.out = e->logits + (size_t)b0 * c.vocab_size; a.ld_out = c.vocab_size;
     a.amax_val = e->amax_val + (size_t)b0 * e->lm_cap; a.amax_idx = e->amax_idx + (size_t)b0 * e->lm_cap;
     a.xin16 = x16;
-    a.wp = e->packed_lm;                                  // the M-tiled lm_head streams the fragment-major copy too
-    // (lm_head on a packed copy with an argmax epilogue was built and measured: 1.342 ms per step against 1.331 at 64
-    // sequences - its 39 MB of fp32 logits stores, not the weight loads, are what the row-major kernel's 95 us are made of)
-    if (pgk_status r = batched_proj(false, PRO_PLAIN, EPI_LOGITS, a, M, st, nblk)) return r;
+    a.wp = e->packed_lm;
+    if (e->packed_lm && gemm_few_logits_ok(M, c.vocab_size, H)) {
+        nblk = gemm_few_logits_blocks(c.vocab_size);
+        if (pgk_status r = gemm_few_logits_nt(x16, e->packed_lm, a.out, a.amax_val, a.amax_idx, M, c.vocab_size, H, st)) return r;
+    } else if (pgk_status r = batched_proj(false, PRO_PLAIN, EPI_LOGITS, a, M, st, nblk)) return r;
     mark(KC_ARGMAX);
     const int32_t* sampled = nullptr;
     if (e->sample_temperature > 0.f) {

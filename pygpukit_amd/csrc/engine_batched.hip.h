@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl
     // ---- activation fragments of this wave's K quarter ----
     // Issue order = arrival order: the activation rows (L2) are requested BEFORE the weight stream (HBM), so the RMSNorm
     // statistic, its barrier and the bf16 conversion run while the weights are still in flight (the other way round the
-    // prologue started when the last weight byte had landed - the batch-1 kernels' lesson, DESIGN.md 4.1).
+    // prologue started when the last weight byte had landed - the batch-1 kernels' lesson).
     const float* src = x_ + (size_t)min(l15, M - 1) * K + kw0 + 8 * q;
     uint4 af[S];
     constexpr bool HOLD_FIRST = PRO == PRO_NORM && S <= 8;      // raw rows held in registers across the reduction

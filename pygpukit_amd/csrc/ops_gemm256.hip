@@ -170,7 +170,7 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
 
 // ---- QKV-heads epilogue (EPI 3 of the fp8 kernel, 5 of the bf16 one): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
 // g2_swiglu_epilogue), a tile = 256 token rows x two head slots, 16 consecutive lanes take one (row, head) and finish it
-// (qkv_heads_finish: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
+// (HeadRows: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 // store).
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: fp32 split-K slab; 3: QKV heads (QkvHeadArgs: tile column = head slot);
 // 4: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]; tile tn = act columns [16 WN tn, +16 WN)); 5: xIELU, 7: gelu, bf16 store;
-// 8: 1, and what the next RMSNorm leaves to do (NormOut).  EPI 0, 3, 4: rows scaled by NormIn where given
+// 8: 1, and what the next RMSNorm leaves to do (NormOut); 9: fp32 store and each row's best column of the tile (BestOut).  EPI 0, 3, 4: rows scaled by NormIn where given
 // GRP: rows sorted by expert (GroupArgs), every tile with its expert's weight; EPI 4, 7, or 6: bf16 rows times their weight, each at its place
 constexpr int GP_THREADS = 512;
 // stages of W that the ring holds; A's has two more.  The smaller tiles' stages are shorter, and latency asks for more of them
@@ -538,9 +538,10 @@ template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
     const size_t RW = gemmp_ring(WM, WN), ring = (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
     return ring > tile ? ring : tile;
 }
+struct BestOut { float* val; int* idx; };                    // [M][tiles of columns]
 template <int EPI, bool GRP, int WM, int WN>
 __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                           int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no) {
+                                           int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no, const BestOut& bo) {
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
     constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
     constexpr bool B16 = EPI == 3 || EPI == 4, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4);
@@ -801,6 +802,34 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
             const int grow = m0 + row, gcol = n0 + c * 4;
             if (grow < M && gcol < N) *reinterpret_cast<float4*>(C + (size_t)grow * N + gcol) = v;
         }
+    } else if constexpr (EPI == 9) {
+        constexpr int LN = BN / 4;                           // lanes that hold a row
+#pragma unroll
+        for (int it = 0; it < BM * LN / GP_THREADS; ++it) {
+            const int item = it * GP_THREADS + tid, row = item / LN, c = item % LN;
+            const float4 v = tile4(row, c * 16);
+            const int grow = m0 + row, gcol = n0 + c * 4;
+            const bool live = grow < M && gcol < N;
+            if (live) *reinterpret_cast<float4*>(reinterpret_cast<float*>(Cv) + (size_t)grow * N + gcol) = v;
+            float best = -INFINITY;                          // the lowest column of the largest value; NaN is never the best
+            int at = 0x7FFFFFFF;
+            if (live) {
+                if (v.x > best) { best = v.x; at = gcol; }
+                if (v.y > best) { best = v.y; at = gcol + 1; }
+                if (v.z > best) { best = v.z; at = gcol + 2; }
+                if (v.w > best) { best = v.w; at = gcol + 3; }
+            }
+#pragma unroll
+            for (int off = LN / 2; off >= 1; off >>= 1) {
+                const float ov = __shfl_xor(best, off, 64);
+                const int oi = __shfl_xor(at, off, 64);
+                if (ov > best || (ov == best && oi < at)) { best = ov; at = oi; }
+            }
+            if (c == 0 && grow < M) {
+                bo.val[(size_t)grow * ntn + tn] = best;
+                bo.idx[(size_t)grow * ntn + tn] = at;
+            }
+        }
     } else {
         // 8 columns per lane: two float4 -> 16 bytes of bf16
 #pragma unroll
@@ -839,12 +868,12 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 // (up to 128 x 128: two workgroups a CU, 80 KiB of LDS and 128 registers each; the larger ones have a CU to themselves)
 template <int EPI, int WM, int WN>
 __global__ __launch_bounds__(GP_THREADS, WM * WN <= 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa, NormIn ni, NormOut no) {
-    gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{}, ni, no);
+                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa, NormIn ni, NormOut no, BestOut bo) {
+    gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{}, ni, no, bo);
 }
 template <int EPI>
 __global__ __launch_bounds__(GP_THREADS, 4) void gemmp_grouped_kernel(const bf16* A, const bf16* W, bf16* C, int N, int K, int ntn, GroupArgs ga) {
-    gemmp_body<EPI, true, 4, 4>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga, NormIn{}, NormOut{});
+    gemmp_body<EPI, true, 4, 4>(A, W, nullptr, C, 0, N, K, 0, ntn, K, QkvHeadArgs{}, 0, ActArgs{}, ga, NormIn{}, NormOut{}, BestOut{});
 }
 
 // ---- fp8 x fp8 with 128-wide block scales on the same structure --------------------------------------------
@@ -1233,7 +1262,7 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
 
 template <int EPI, int WM, int WN>
 static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, void* C, int M, int N, int K, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa,
-                               const NormIn& ni, const NormOut& no, hipStream_t st) {
+                               const NormIn& ni, const NormOut& no, hipStream_t st, const BestOut& bo = BestOut{}) {
     constexpr size_t LDS = gemmp_lds<WM, WN, EPI == 3 || EPI == 4>();
     static bool attr_done = false;
     if (!attr_done) {
@@ -1241,7 +1270,7 @@ static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, v
         attr_done = true;
     }
     const int ntm = ceil_div(M, 32 * WM), ntn = EPI == 4 ? ceil_div(N, 16 * WN) : ceil_div(N, 32 * WN);      // SwiGLU: N = I act columns, half a tile's
-    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa, ni, no);
+    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa, ni, no, bo);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
@@ -1340,6 +1369,17 @@ bool gemm_few_swiglu_ok(int I, int K) { return K % 64 == 0 && K >= 64 && I % 32 
 pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, int I, int K, const NormIn& ni, hipStream_t st) {
     PGK_REQUIRE(M >= 1 && gemm_few_swiglu_ok(I, K) && (!ni.ss || (ni.ld == 64 && ni.n <= 64)), "gemm_few_swiglu: M=%d I=%d K=%d", M, I, K);
     return gemmp_launch<4, 2, 2>(A, wp, nullptr, act, M, I, K, K, QkvHeadArgs{}, 1, ActArgs{}, ni, NormOut{}, st);
+}
+
+// Logits of a batch's step against the fragment-major lm_head: 64 x 128 tiles, bound by the stream of the weights and the fp32 rows (5.6 TB/s at 64 rows).  The kernel of
+// 16 columns a workgroup stores 64 bytes of a row at a time; here 512.  K = 1024, 151936 columns, us a launch there / here: 64 rows 82 / 62; us a step
+// of Qwen3-0.6B: 64 sequences 1172 / 1154, 48 1118 / 1104, 33 1093 / 1084, 24 1030 / 1029, 17 1011 / 1013: from 33 on.
+constexpr int GP_LOGITS_COLS = 128;
+bool gemm_few_logits_ok(int M, int V, int K) { return M > 32 && K % 64 == 0 && K >= 64 && V % 16 == 0; }
+int gemm_few_logits_blocks(int V) { return ceil_div(V, GP_LOGITS_COLS); }     // parts per row of best_val and best_idx
+pgk_status gemm_few_logits_nt(const bf16* A, const bf16* wp, float* logits, float* best_val, int* best_idx, int M, int V, int K, hipStream_t st) {
+    PGK_REQUIRE(gemm_few_logits_ok(M, V, K) && best_val && best_idx, "gemm_few_logits: M=%d V=%d K=%d", M, V, K);
+    return gemmp_launch<9, 2, GP_LOGITS_COLS / 32>(A, wp, nullptr, logits, M, V, K, K, QkvHeadArgs{}, 1, ActArgs{}, NormIn{}, NormOut{}, st, BestOut{best_val, best_idx});
 }
 
 template <int EPI>
