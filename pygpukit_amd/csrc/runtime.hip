@@ -292,7 +292,10 @@ pgk_status pgk_pool_trim(void) {
 
 pgk_status pgk_host_alloc(void** h_ptr, size_t nbytes) {
     PGK_REQUIRE(h_ptr, "pgk_host_alloc: null output");
-    PGK_CHECK_HIP(hipHostMalloc(h_ptr, nbytes ? nbytes : 1, hipHostMallocDefault));
+    if (const hipError_t e = hipHostMalloc(h_ptr, nbytes ? nbytes : 1, hipHostMallocDefault); e != hipSuccess) {
+        (void)hipGetLastError();      // reported here, and not again by the next launch: callers go on with pageable memory
+        return set_error(PGK_ERR_HIP, "pgk_host_alloc(%zu bytes): %s", nbytes, hipGetErrorString(e));
+    }
     return PGK_OK;
 }
 pgk_status pgk_host_free(void* h_ptr) {

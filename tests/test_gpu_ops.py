@@ -114,6 +114,33 @@ def test_a_refused_allocation_is_not_the_next_launchs_error():
     np.testing.assert_array_equal(host(ops.add(a, a)), 2 * np.arange(8, dtype=np.float32))
 
 
+def test_a_refused_pinned_allocation_is_not_the_next_launchs_error(monkeypatch):
+    """Pinned memory that is not to be had: the call that asked for it raises, the pool of result arrays takes ordinary memory, and operators after either run."""
+    from pygpukit_amd import _hip
+    from pygpukit_amd.core import pinned
+    import ctypes as C
+
+    a = dev(np.arange(8, dtype=np.float32))
+    p = C.c_void_p()
+    with pytest.raises(RuntimeError, match="pgk_host_alloc"):
+        _hip.call("pgk_host_alloc", C.byref(p), 1 << 50)
+    np.testing.assert_array_equal(host(ops.add(a, a)), 2 * np.arange(8, dtype=np.float32))
+
+    lib = _hip.load()
+
+    class Refusing:
+        def __getattr__(self, name):
+            return (lambda p, nbytes: lib.pgk_host_alloc(p, 1 << 50)) if name == "pgk_host_alloc" else getattr(lib, name)
+
+    monkeypatch.setattr(pinned._hip, "load", Refusing)
+    monkeypatch.setattr(pinned, "_free", {})
+    out = pinned.empty((54321,))
+    monkeypatch.undo()
+    out[:] = 1
+    assert out.base is None
+    np.testing.assert_array_equal(host(ops.add(a, a)), 2 * np.arange(8, dtype=np.float32))
+
+
 def test_roundtrip_and_views():
     x = np.arange(24, dtype=np.float32).reshape(4, 6)
     a = from_numpy(x)
