@@ -1,6 +1,8 @@
 """The pool of pinned result blocks, with host memory in the library's place."""
 
 import ctypes as C
+import mmap
+import os
 import threading
 
 import numpy as np
@@ -118,3 +120,40 @@ def test_a_refused_allocation_leaves_an_ordinary_array_and_the_counts(memory):
     memory.pgk_host_alloc = lambda p, n: 2
     held = pinned._held_bytes
     assert pinned.empty((100000,)).base is None and pinned._held_bytes == held
+
+
+def test_a_forked_process_reads_the_arrays_that_were_there(memory, monkeypatch):
+    """With memory that is not inherited, as the driver's: blocks of their own and two that share a page."""
+    maps = []
+
+    def alloc(p, nbytes):
+        if nbytes > 4096 or not maps:
+            maps.append(mmap.mmap(-1, max(nbytes, 4096)))
+            maps[-1].madvise(mmap.MADV_DONTFORK)
+            at = 0
+        else:
+            at = 1024
+        p._obj.value = C.addressof(C.c_char.from_buffer(maps[-1])) + at
+        return 0
+
+    memory.pgk_host_alloc = alloc
+    held = [pinned.empty((n,)) for n in (100, 200, 30000, 200000)]
+    gone = pinned.empty((300000,))
+    del gone
+    for i, a in enumerate(held):
+        a[:] = np.arange(a.size) + i
+    part = held[3][777:]
+    child = os.fork()
+    if child == 0:
+        status = 1
+        try:
+            ok = all((a == np.arange(a.size) + i).all() for i, a in enumerate(held)) and part[0] == 780
+            held[2][:] = 0
+            ok = ok and pinned.empty((300000,)).base is None
+            held.clear()
+            status = 0 if ok else 2
+        finally:
+            os._exit(status)
+    assert os.waitpid(child, 0)[1] == 0
+    assert all((a == np.arange(a.size) + i).all() for i, a in enumerate(held))
+    assert not pinned._at_fork and pinned.empty((300000,)).base is not None
