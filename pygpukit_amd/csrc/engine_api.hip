@@ -318,7 +318,8 @@ pgk_status pgk_engine_read_tokens(pgk_engine eh, int32_t* h_out, int batch, int 
     // log rows are max_batch wide; return the first `batch` columns, step-major
     const size_t words = (size_t)n_steps * e->cfg.max_batch;
     std::vector<int32_t> pageable;
-    int32_t* tmp = (int32_t*)stage_room(e->down, words * 4);     // (into pageable memory the copy is set up when the last step has ended)
+    std::unique_lock<std::mutex> stage(e->down_mu, std::try_to_lock);
+    int32_t* tmp = stage.owns_lock() ? (int32_t*)stage_room(e->down, words * 4) : nullptr;     // (into pageable memory the copy is set up when the last step has ended)
     if (!tmp) { pageable.resize(words); tmp = pageable.data(); }
     if (n_steps) PGK_CHECK_HIP(hipMemcpyAsync(tmp, e->token_log, words * 4, hipMemcpyDeviceToHost, st));
     PGK_CHECK_HIP(hipStreamSynchronize(st));

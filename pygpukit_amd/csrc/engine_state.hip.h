@@ -4,8 +4,9 @@
 
 #include <cstdint>
 #include <cstdlib>
-#include <type_traits>
 #include <cstring>
+#include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "engine_common.hip.h"
@@ -198,6 +199,7 @@ struct Engine {
     int launches_per_step = 0;
     std::vector<void*> allocs;
     HostStage up, down;         // uploads and read-backs of a few bytes
+    std::mutex down_mu;         // two threads may read at a time
 
     size_t kv_layer_elems() const { return (size_t)cfg.max_batch * cfg.num_kv_heads * cfg.max_seq_len * cfg.head_dim; }
     int qkv_dim() const { return (cfg.num_heads + 2 * cfg.num_kv_heads) * cfg.head_dim; }
