@@ -23,7 +23,7 @@ import numpy as np
 from pygpukit_amd import _hip
 
 POOL_BYTES = 64 << 20
-CLASS_BYTES = 64 << 10
+CLASS_BYTES = 32 << 10
 _lock = threading.RLock()   # a garbage collection under it may end another block in the same thread
 _free: dict[int, list[int]] = {}
 _free_bytes = 0
