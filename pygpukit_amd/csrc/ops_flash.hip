@@ -538,31 +538,42 @@ static int flash_cus() {
     return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
-// KV runs per query tile and sides of a workgroup (1 or 2: half a run's tiles each), at least four KV tiles to a run.
-// Where the causal edge is most of the work (contexts under twice the rows) a launch of up to two workgroups per CU lasts as long as its heaviest tile, alone on its CU for
-// most of that, 1.47 us a KV tile; with two sides it has the CU's other half too, 1.1 us, and nothing to merge outside.  Beyond, two workgroups of their own time per CU do
-// more (one barrier makes the sides wait for each other); up to ten KV tiles the sides' merge costs what they save.  Where at most every CU has a workgroup and the context
-// is long enough for the merge, two runs do better, of which a heavy and a light one share a CU.  In an engine's prompts, us a launch, one run / two runs with merge / two
-// sides: 16 heads, 550 rows 16.0 / - / 16.6, 1024 26.0 / - / 24.4, 1531 - / 31.5 / 34.2, 1800 - / 36.9 / 39.0, 2300 54.2 / - / 47.5, 3000 71.2 / - / 60.0; 32 heads, 700 20.2 / - / 19.6, 1100 31.1 / - / 28.0.  By themselves:
-// 16 heads, 512 rows 15.0 / 16.1 / 15.9; 1000 24.9 / 24.0 / 22.8; 2300 49.6 / 46.7 / 41.5; 3300 72.9 / 72.0 / 58.3; 4000 94.9 / 98.5 / 81.0; 5000 127 / - / 132; 32 heads, 700
-// 19.6 / 25.5 / 18.2, 1100 28.7 / 37.5 / 24.6, 2500 69.9 / - / 78.0; 8 heads, 4000 79.4 / 57.0 / 63.9; head dim 64, 16 heads, 700 13.5 / 14.0 / 12.1, 2300 35.7 / 33.0 / 29.0.
-// Longer contexts: as many runs as one round of workgroups holds: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and that many
-// still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
+// KV runs per query tile and sides of a workgroup (1 or 2: half a run's tiles each).
+// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile, 1.47 us a KV tile for a workgroup that has its
+// CU to itself; two sides take 1.1, and merge in LDS.
+//  * Few workgroups (short of 5/8 of the CUs, 1200 positions and more): as many runs as two to a CU hold, of at least 2.5 KV tiles - more where many rows make the merge's
+//    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 23.3 / 15.9, 5000 56.3 / 26.3; 4 heads, 2048
+//    30.3 / 25.8; 8 heads, 2048 33.5 / 29.3.
+//  * Up to a workgroup per CU: two runs, of which a heavy and a light one share a CU.  16 heads, 1531 rows 31.5 (two sides 34.2), 1800 36.9 (39.0).
+//  * Shorter contexts, at most a workgroup to four CUs: three or four runs whose rows stay fp32.  In 16 bits they were rounded twice: 2.27e-3 of float64 for 700 rows of 4 heads
+//    where two sides leave 2.00e-3 and these 1.98e-3.  1 head, 1024 rows 23.3 (two sides) / 14.6, 8 heads, 900 21.9 / 21.1.
+//  * Otherwise two sides beyond ten KV tiles, up to five workgroups to four CUs: 16 heads, 2300 rows 54.2 (one side) / 47.5; 32 heads, 1100 31.1 / 28.0.  Up to two to a CU only where
+//    nearly all of the context is causal and long: 16 heads, 3000 rows 71.2 / 60.0; but 64 heads, 900 rows 26.8 / 34.1, 32 heads, 1300 at 650 47.1 / 52.6.  Beyond, two workgroups
+//    of their own time per CU do more (one barrier makes the sides wait for each other).
+// Longer contexts: as many runs as one round of workgroups holds, at least four KV tiles each: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and
+// that many still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
 // 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
 // (Results that are rounded to e4m3 next, by whichever kernel, ask for one side: the codes magnify a sum's last bit to a sixteenth, and a prompt in one pass and in pieces would
 // no longer agree - 4096 rows of 32 heads at once and as two of 2048, which alone had two sides, were 0.028 apart in the logits, with one side each under 0.01.)
-struct FlashPlan { int runs, sides; };
+struct FlashPlan { int runs, sides; bool fp32; };       // fp32: of partial rows
 static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
     if (kv_len < 2LL * q_len) {
-        if (wgs <= cus && kv_len >= 1200 && most >= 2) return {2, 1};
-        return {1, kv_len > 10 * FL_BKV && wgs <= 2 * cus ? 2 : 1};
+        const int nt = ceil_div(kv_len, FL_BKV);
+        const bool fp32 = kv_len < 1200;
+        long long n = 1;
+        if (!fp32) n = 8 * wgs <= 5 * cus ? std::min({8 * wgs > cus ? 12LL : 8LL, 2 * cus / wgs, nt * 40 / (100 + wgs * 256 / cus)}) : wgs <= cus ? 2 : 1;
+        else if (4 * wgs <= cus) n = 8 * wgs <= cus ? std::min(nt / 3, 4) : std::min(nt / 4, 3);
+        if (fp32 && n < 3) n = 1;
+        n = std::min<long long>(n, most);
+        if (n > 1) return {(int)n, 1, fp32};
+        return {1, nt > 10 && (4 * wgs <= 5 * cus || (wgs <= 2 * cus && !fp32 && 4LL * kv_len <= 5LL * q_len)) ? 2 : 1, false};
     }
     long long n = cus / wgs;
     if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
     if (n > most) n = most;
     if (n > ceil_div(kv_len, FL_BKV) / 4) n = ceil_div(kv_len, FL_BKV) / 4;
-    return {n < 1 ? 1 : (int)n, 1};
+    return {n < 1 ? 1 : (int)n, 1, false};
 }
 // with a sliding window: up to four runs over the `span` keys that the heaviest query tile walks, until two workgroups per CU are reached
 static int flash_window_runs(long long wgs, int span) {
@@ -578,9 +589,9 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
                                const FlashMany& many = FlashMany{}, bool one_side = false) {
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-    const FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
+    const FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1, false} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
     int nsplit = plan.runs;
-    const bool wide = many.items || q_len <= 128;
+    const bool wide = many.items || q_len <= 128 || plan.fp32;
     // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
     // tiles of the first-generation kernel 61, 31 and 239)
     if (nsplit > 1 && q_len <= 128) {

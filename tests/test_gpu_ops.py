@@ -968,13 +968,25 @@ def test_sdpa_reads_nothing_behind_the_context(dt, cfg):
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("cfg", [(2, 1, 641, 641, 128), (4, 2, 699, 705, 64), (2, 2, 500, 768, 128), (1, 1, 700, 1199, 128), (33, 3, 1281, 1281, 128)])
+@pytest.mark.parametrize("cfg", [(16, 1, 641, 641, 128), (12, 2, 699, 705, 64), (20, 2, 500, 768, 128), (12, 1, 700, 1199, 128), (33, 3, 1281, 1281, 128)])
 def test_sdpa_with_the_tiles_of_a_run_shared_by_two_sides(dt, cfg):
-    """11 and 12 KV tiles in the heaviest query tile and 2 in the lightest, a context before the rows, more workgroups than CUs: the bars of the tests that are
-    called."""
+    """72 to 96 workgroups, and more than there are CUs: 11 and 12 KV tiles in the heaviest query tile and 2 in the lightest, a context before the rows.  The bars of the
+    tests that are called."""
     test_sdpa_few_rows_over_a_long_context(dt, cfg)
     test_sdpa_reads_nothing_behind_the_context(dt, cfg)
     if dt == "bfloat16" and cfg[1] == 2:                # (a key head that stays as it is, a position that every row sees)
+        test_sdpa_nan_and_infinite_keys(cfg)
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(2, 1, 575, 576, 64), (2, 1, 641, 641, 128), (4, 2, 699, 705, 64), (2, 2, 500, 768, 128), (8, 1, 513, 769, 128), (1, 1, 700, 1199, 128), (1, 1, 700, 1200, 64),
+                                 (1, 1, 2049, 2049, 64), (2, 1, 2500, 2501, 128), (9, 3, 1800, 1806, 64), (10, 2, 2000, 2006, 128)])
+def test_sdpa_of_few_workgroups_in_runs(dt, cfg):
+    """Prompts of few heads on a card of 256 CUs: 3, 3, 4, 4, 3 and 4 runs of fp32 rows up to 1199 positions, from 1200 on 7, 8, 11, 3 and 3 (2.5 tiles each and more) whose
+    first query tiles leave most runs empty.  The bars of the tests that are called."""
+    test_sdpa_few_rows_over_a_long_context(dt, cfg)
+    test_sdpa_reads_nothing_behind_the_context(dt, cfg)
+    if dt == "bfloat16" and cfg[1] == 2 and cfg[3] - cfg[2] > 5:
         test_sdpa_nan_and_infinite_keys(cfg)
 
 
