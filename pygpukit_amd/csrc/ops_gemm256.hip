@@ -1364,8 +1364,10 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
 
 // act[M][I] = SwiGLU of few rows (a prompt of up to 128, the step of a batch) against the fragment-major gate / up copy: 64 x 64 tiles, 32 act columns each.  The
 // packed kernel gives a wave the weights in registers and a workgroup 32 rows: us a launch there / here, K = 1024, I = 3072: 93 rows 10.9 / 7.8, 64 rows 8.5 / 7.3,
-// 37 rows 8.1 / 7.2; ms, 4 steps of 24 sequences 4.07 / 3.97, a prompt of 9 1.083 / 1.051.
-bool gemm_few_swiglu_ok(int I, int K) { return K % 64 == 0 && K >= 64 && I % 32 == 0; }
+// 37 rows 8.1 / 7.2; ms, 4 steps of 24 sequences 4.07 / 3.97, a prompt of 9 1.083 / 1.051.  Smaller weights stay there, where more workgroups start earlier: us a layer there / here, K = 512,
+// I = 1024 1 row 28.3 / 29.2, 96 rows 32.4 / 32.7; K = 1024, I = 2048 9 rows 32.9 / 33.4, 96 rows 38.4 / 38.6; but I = 3072 9 rows 35.0 / 34.3, 96 rows 41.1 / 39.5, and K = 1536, I = 1024
+// 9 rows 46.9 / 45.8, 96 rows 50.1 / 49.5.
+bool gemm_few_swiglu_ok(int I, int K) { return K % 64 == 0 && I % 32 == 0 && (K >= 1536 || (K >= 1024 && I >= 3072)); }
 pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, int I, int K, const NormIn& ni, hipStream_t st) {
     PGK_REQUIRE(M >= 1 && gemm_few_swiglu_ok(I, K) && (!ni.ss || (ni.ld == 64 && ni.n <= 64)), "gemm_few_swiglu: M=%d I=%d K=%d", M, I, K);
     return gemmp_launch<4, 2, 2>(A, wp, nullptr, act, M, I, K, K, QkvHeadArgs{}, 1, ActArgs{}, ni, NormOut{}, st);
