@@ -1375,9 +1375,10 @@ pgk_status gemm_few_swiglu_nt(const bf16* A, const bf16* wp, bf16* act, int M, i
 
 // Logits of a batch's step against the fragment-major lm_head: 64 x 128 tiles, bound by the stream of the weights and the fp32 rows (5.6 TB/s at 64 rows).  The kernel of
 // 16 columns a workgroup stores 64 bytes of a row at a time; here 512.  K = 1024, 151936 columns, us a launch there / here: 64 rows 82 / 62; us a step
-// of Qwen3-0.6B: 64 sequences 1172 / 1154, 48 1118 / 1104, 33 1093 / 1084, 24 1030 / 1029, 17 1011 / 1013: from 33 on.
+// of Qwen3-0.6B: 64 sequences 1172 / 1154, 48 1118 / 1104, 33 1093 / 1084, 24 1030 / 1029, 17 1011 / 1013: from 33 on.  From 64 tiles of columns on: 33 and 64 sequences, 4096 columns
+// 136.0 / 137.3 and 140.3 / 140.4, 8192 139.5 / 137.3 and 145.2 / 140.5.
 constexpr int GP_LOGITS_COLS = 128;
-bool gemm_few_logits_ok(int M, int V, int K) { return M > 32 && K % 64 == 0 && K >= 64 && V % 16 == 0; }
+bool gemm_few_logits_ok(int M, int V, int K) { return M > 32 && V >= 64 * GP_LOGITS_COLS && K % 64 == 0 && K >= 64 && V % 16 == 0; }
 int gemm_few_logits_blocks(int V) { return ceil_div(V, GP_LOGITS_COLS); }     // parts per row of best_val and best_idx
 pgk_status gemm_few_logits_nt(const bf16* A, const bf16* wp, float* logits, float* best_val, int* best_idx, int M, int V, int K, hipStream_t st) {
     PGK_REQUIRE(gemm_few_logits_ok(M, V, K) && best_val && best_idx, "gemm_few_logits: M=%d V=%d K=%d", M, V, K);
