@@ -13,6 +13,7 @@ their values at the same addresses in the child, and the child's own results are
 from __future__ import annotations
 
 import ctypes as C
+import math
 import mmap
 import os
 import sys
@@ -53,15 +54,17 @@ class _Block:
 
 def _take(size: int):
     """(address, size) of the smallest free block that serves `size` bytes, or None; under the lock"""
-    fits = [n for n in list(_free) if _free[n] and (n == size or n >= size >= CLASS_BYTES)]
+    if _free.get(size):
+        return _free[size].pop(), size
+    fits = [n for n in list(_free) if _free[n] and n >= size >= CLASS_BYTES]
     return (_free[min(fits)].pop(), min(fits)) if fits else None
 
 
 def empty(shape: tuple, dtype=np.float32) -> np.ndarray:
     """np.empty on pinned memory; on ordinary memory for what the pool has no room for and where no pinned memory is to be had."""
     global _free_bytes, _held_bytes
-    dtype = np.dtype(dtype)
-    size = nbytes = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+    dtype, shape = np.dtype(dtype), tuple(int(n) for n in shape)
+    size = nbytes = math.prod(shape) * dtype.itemsize
     if nbytes >= CLASS_BYTES:
         size = 1 << (nbytes - 1).bit_length()
     if nbytes == 0 or size > POOL_BYTES or _forked:
@@ -89,7 +92,7 @@ def empty(shape: tuple, dtype=np.float32) -> np.ndarray:
                 _held_bytes -= size
             return np.empty(shape, dtype)
         address = p.value
-    return np.asarray(_Block(address, size, nbytes, tuple(int(n) for n in shape), dtype.str))
+    return np.asarray(_Block(address, size, nbytes, shape, dtype.str))
 
 
 _at_fork: list[tuple[int, bytes]] = []
