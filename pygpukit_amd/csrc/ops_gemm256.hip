@@ -544,7 +544,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
                                            int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no, const BestOut& bo) {
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
     constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
-    constexpr bool B16 = EPI == 3 || EPI == 4, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4);
+    constexpr bool B16 = EPI == 3 || EPI == 4, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4), PARTS = SCALED && EPI == 4 && BM == 64;   // PARTS: may come as ni.ld says
     static_assert(!SCALED || BM <= 256, "a row for each of the waves that multiply");
     static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -627,23 +627,24 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // retire the phantom DMAs: the stages become the C tile
         __builtin_amdgcn_s_barrier();
     } else {
-        if constexpr (SCALED && EPI != 0) {
-            if (BM == 64 && ni.ss && ni.ld) {                // four threads to a row, 16 parts each
-                {
-                    const float* p = ni.ss + (size_t)min(m0 + (tid >> 2), M - 1) * 64 + (tid & 3) * 16;
-                    float4 v[4];
+        if constexpr (PARTS) {
+            if (ni.ss && ni.ld) {                            // four threads to a row, 16 parts each
+                const float* p = ni.ss + (size_t)min(m0 + (tid >> 2), M - 1) * 64 + (tid & 3) * 16;
+                float4 v[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float4*>(p + 4 * j);
+                for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float4*>(p + 4 * j);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int i = (tid & 3) * 16 + 4 * j;
-                        mine += ((i < ni.n ? v[j].x : 0.f) + (i + 1 < ni.n ? v[j].y : 0.f)) + ((i + 2 < ni.n ? v[j].z : 0.f) + (i + 3 < ni.n ? v[j].w : 0.f));
-                    }
-                    mine += dpp_f<DPP_XOR1>(mine);
-                    mine += dpp_f<DPP_XOR2>(mine);
-                    mine = 1.0f / sqrtf(mine / K + ni.eps);
+                for (int j = 0; j < 4; ++j) {
+                    const int i = (tid & 3) * 16 + 4 * j;
+                    mine += ((i < ni.n ? v[j].x : 0.f) + (i + 1 < ni.n ? v[j].y : 0.f)) + ((i + 2 < ni.n ? v[j].z : 0.f) + (i + 3 < ni.n ? v[j].w : 0.f));
                 }
-            } else if (ni.ss && tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
+                mine += dpp_f<DPP_XOR1>(mine);
+                mine += dpp_f<DPP_XOR2>(mine);
+                mine = 1.0f / sqrtf(mine / K + ni.eps);
+            }
+        }
+        if constexpr (SCALED && EPI != 0) {
+            if (ni.ss && !(PARTS && ni.ld) && tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
         }
 #pragma unroll
         for (int i = 0; i < WM; ++i)
@@ -712,10 +713,10 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     if constexpr (SCALED) {
         if (ni.ss) {
             float* inv = reinterpret_cast<float*>(g2_smem + BM * ROWB);          // behind the tile, where the last stages were
-            if constexpr (EPI == 0) {                        // (held through the loop it is spilled; no engine's step comes here unless PGK_FUSED_EPILOGUES is 0)
+            if constexpr (EPI == 0) {                        // (held through the loop it is spilled; QKV of heads that are not 128 columns, and all where PGK_FUSED_EPILOGUES is 0)
                 if (tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
             }
-            if (BM == 64 && ni.ld) { if (tid < 256 && (tid & 3) == 0) inv[tid >> 2] = mine; }
+            if (PARTS && ni.ld) { if (tid < 256 && (tid & 3) == 0) inv[tid >> 2] = mine; }
             else if (tid < BM) inv[tid] = mine;
             __syncthreads();
             if (wid < 4) {
@@ -865,7 +866,8 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
     }
 }
-// (up to 128 x 128: two workgroups a CU, 80 KiB of LDS and 128 registers each; the larger ones have a CU to themselves)
+// (up to 128 x 128: two workgroups a CU, at most 80 KiB of LDS and 128 registers each - but for 128 x 64, whose ring of six takes 88 KiB; the larger ones have a CU to
+// themselves)
 template <int EPI, int WM, int WN>
 __global__ __launch_bounds__(GP_THREADS, WM * WN <= 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                                                        int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa, NormIn ni, NormOut no, BestOut bo) {
@@ -1275,10 +1277,11 @@ static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, v
     return PGK_OK;
 }
 
-// Tile of a product of `cols` weight rows in `splits` runs of K: the cheapest by rounds of workgroups x (time of a stage x stages + start and epilogue), in 0.01 us as
-// measured with the chip full, with one and where the LDS lets it with two workgroups on a CU.  `most`: how far down the list the product's epilogue goes (QKV heads
-// are 128 columns, split products leave most of a round idle anyway).  Us a launch, K = 1024: 384 rows, N = 4096 10.1 (128 x 128) 8.4 (64 x 128); 93 rows, N = 6144 9.8,
-// 7.5, 6.3 (64 x 64); 1531 rows, N = 4096 18.7 (128 x 128) 16.6 (192 x 128), N = 6144 27.8, 31.9, 23.0 (192 x 192).
+// Tile of a product of `cols` weight rows in `splits` runs of K: the cheapest by rounds of workgroups x (time of a stage x stages + start and epilogue), in 0.01 us for
+// one and, where the LDS lets it, for two workgroups on a CU.  The prices rank the tiles and are not a launch's time, which is 1.2 to 1.4 times as
+// long.  `most`: how far down the list the product's epilogue goes (QKV heads are 128 columns, split products leave most
+// of a round idle anyway).  Us a launch, K = 1024, measured (priced): 384 rows, N = 4096 10.1 (8.4) on 128 x 128, 8.4 (6.2) on 64 x 128; 93 rows, N = 6144 9.8 (8.4),
+// 7.5 (6.2), 6.3 (5.0) on 64 x 64; 1531 rows, N = 4096 18.7 (13.5) on 128 x 128, 16.6 (12.1) on 192 x 128, N = 6144 27.8 (21.8) on 128 x 128, 23.0 (17.4) on 192 x 192.
 enum { GP_128, GP_64_128, GP_192_128, GP_192, GP_64 };
 static int gemmp_tile(int M, int cols, int K, int splits, int most) {
     constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 260, 29, 420}, {64, 128, 13, 200, 20, 330}, {192, 128, 27, 350, 0, 0}, {192, 192, 40, 460, 0, 0}, {64, 64, 11, 150, 16, 260}};
