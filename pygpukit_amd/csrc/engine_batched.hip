@@ -78,13 +78,13 @@ static pgk_status batched_proj_t(int pro, int epi, const FusedArgs& a, int M, hi
         switch (epi) {
             case EPI_STORE: return launch_batched<WT, PRO_NORM, EPI_STORE>(a, M, st);
             case EPI_SWIGLU: return launch_batched<WT, PRO_NORM, EPI_SWIGLU>(a, M, st);
-            case EPI_LOGITS: return launch_batched<WT, PRO_NORM, EPI_LOGITS>(a, M, st, nblk);
+            case EPI_LOGITS:                       // (the lm_head is bf16 whatever the layers are)
+                if constexpr (!std::is_same<WT, fp8e4m3>::value) return launch_batched<WT, PRO_NORM, EPI_LOGITS>(a, M, st, nblk);
+                break;
         }
     } else if (pro == PRO_PLAIN) {
         switch (epi) {
-            case EPI_STORE: return launch_batched<WT, PRO_PLAIN, EPI_STORE>(a, M, st);
             case EPI_RESID: return launch_batched<WT, PRO_PLAIN, EPI_RESID>(a, M, st);
-            case EPI_SWIGLU: return launch_batched<WT, PRO_PLAIN, EPI_SWIGLU>(a, M, st);
             case EPI_LOGITS:                       // rows a prompt left, already normalised
                 if constexpr (!std::is_same<WT, fp8e4m3>::value) return launch_batched<WT, PRO_PLAIN, EPI_LOGITS>(a, M, st, nblk);
                 break;

@@ -223,159 +223,246 @@ __global__ __launch_bounds__(256) void batched_mfma_kernel(unsigned long long* t
 //
 // The LDS-image kernel above spends its time before the first MFMA: every workgroup reads all M rows twice (sum of
 // squares, then normalise), writes a K x 16 image to LDS and crosses two barriers - 9-13 us per projection at M = 16
-// where the M = 1 GEMV kernels take 4.6-5.8.  A wave only ever multiplies ITS quarter of K, so here each wave loads that
-// quarter of the activation rows straight from global memory in A-fragment shape (lane l: row l & 15, k = 32 s + 8 (l >> 4)
-// .. + 8), keeps the raw fp32 values in registers while the row sums of squares cross the waves (64 floats of LDS,
-// one barrier), and converts in place: no activation image, one pass over the rows.
+// where the M = 1 GEMV kernels take 4.6-5.8.  A wave only ever multiplies ITS quarter of K, so here each wave takes that
+// quarter of the activation rows: raw fp32 values in registers while the row sums of squares cross the waves (64 floats of LDS,
+// one barrier), then bf16 through LDS of its own into A fragments: one pass over the rows, no other barrier.
+// The rows are loaded along K, 1 KiB contiguous per wave instruction.  Loaded in fragment shape (lane l: row l & 15, k = 32 s + 8 (l >> 4) .. + 8) an instruction
+// is 64 pieces of 16 bytes, which a CU's texture path takes at one a clock: S = 24 kept it busy for 2.8 us of a 5.5 us launch.  Us a launch of 5 rows, then and now: QKV
+// (N = 4096, K = 1024) 4.0 / 2.6, o_proj (1024, 2048) 3.4 / 2.5, gate_up (6144, 1024) 4.6 / 3.4, down (1024, 3072) 4.3 / 2.8; a step of Qwen3-0.6B at contexts to 300, us: 3
+// sequences 815 / 692, 8 893 / 723, 9 912 / 786, 16 1013 / 843, with e4m3 weights 8 1016 / 743; 8 layers of K = 4096 1111 / 565.
 // RPG = weight rows per workgroup (16, 8 or 4): the N = hidden projections have only N / 16 = 64 row groups at
 // N = 1024, far too few workgroups to pull HBM bandwidth; with RPG < 16 the lanes of the unused B columns load nothing
 // and the epilogue ignores those columns (the MFMA computes them on whatever the registers hold - columns are
-// independent).
-template <class WT, int PRO, int EPI, int S, int RPG>
+// independent).  MR = rows that are loaded, 8 or 16: those past the batch repeat its last one, and their results are dropped.
+template <class WT, int PRO, int EPI, int S, int RPG, int MR>
 __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl, const void* w_, const bf16* wp_, const float* x_, const bf16* gamma_,
                                                           int N_, int K_, int M, int nblk_logits, FusedArgs a) {
     // the first 14 dwords of the arguments - everything the load-issue phase needs - arrive preloaded in SGPRs (see fused_gemv_kernel,
-    // engine.hip): w_ / wp_ = FusedArgs::w / wp, x_ = the fp32 input rows of the norm prologue (h), gamma_, N_, K_
+    // engine.hip): w_ / wp_ = FusedArgs::w / wp, x_ = the input rows (fp32 h for the norm prologue, else xin16), gamma_, N_, K_
     const TLStamp tls(tl);
     constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value;
     constexpr int NT = (EPI == EPI_SWIGLU) ? 2 : 1;
-    __shared__ float s_ss[4][16];
+    constexpr int NC = S / 8;                              // chunks of 256 k of a wave's quarter
+    static_assert(S % 8 == 0 && (MR == 8 || MR == 16), "whole chunks; 8 or 16 rows");
+    __shared__ __attribute__((aligned(16))) float s_ss[MR][20];        // sums of squares: of 16 lanes of a wave, 16 parts a row
     __shared__ float red[NT * 4 * 256];                    // [NT][4 waves][16 m][16 n]
+    __shared__ __attribute__((aligned(16))) char s_img[4][MR * 512];   // a wave's chunk: 8 k of row m at slot m ^ (k / 8) of MR
     const int K = K_, N = N_;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, q = lane >> 4, l15 = lane & 15;
     const int ngroups = (N + RPG - 1) / RPG;
     const int kw0 = wid * S * 32;
-    const bool wlane = l15 < RPG;                          // this lane holds a real weight row
-    uint4 wv[NT][S];
-    float wsc[NT][S];
+    // Weights of a group, every load unconditional (one under a branch is waited for where the branches meet again, in front of the whole prologue).
+    // 16 rows: in fragment shape, a step (e4m3: two, a lane's 16 bytes are 8 k of each, so that a load takes 64 bytes of a row; the activations follow) to a load -
+    // of the fragment-major copy (ops_pkgemm.hip: block (n-tile, k-step) is this very fragment, 1 KiB in lane order) where there is one.
+    // Fewer: along K like the activations, and through the wave's LDS.
+    constexpr bool FRAG = RPG == 16;
+    constexpr int RL = FP8 ? 4 : 2;                        // rows of a chunk to a load
+    constexpr int WS = FRAG ? (FP8 ? S / 2 : S) : NC * RPG / RL;
+    uint4 wv[NT][WS];
+    float wsc[NT][FRAG ? WS : NC * 2];                     // e4m3 block scales: of a load; of a half chunk of this lane's column
     auto load_w = [&](int n0) {
-        const int nrow = min(n0 + l15, N - 1);
-        if constexpr (!FP8 && RPG == 16) {
-            // fragment-major copy (ops_pkgemm.hip): block (n-tile, k-step) is this very fragment, 1 KiB in lane order - one
-            // coalesced load per k-step instead of 64 separate 16-byte pieces of a row-major matrix (3.5x the texture
-            // addresser's time per instruction, tools/micro/ta_probe.hip).  Used where a workgroup streams many groups (lm_head).
-            if (wp_ != nullptr && n0 + 16 <= N) {
-                const int ksn = K >> 5;
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const bf16* run = wp_ + (((size_t)((t == 0 ? n0 : N + n0) >> 4) * ksn + (kw0 >> 5)) * 64 + lane) * 8;
+        for (int t = 0; t < NT; ++t) {
+            auto row_of = [&](int r) { return (size_t)(t == 0 ? 0 : N) + min(n0 + r, N - 1); };
+            if constexpr (FRAG && !FP8) {
+                const bool pk = wp_ != nullptr && n0 + 16 <= N;
+                const bf16* p = pk ? wp_ + (((size_t)((t == 0 ? n0 : N + n0) >> 4) * (K >> 5) + (kw0 >> 5)) * 64 + lane) * 8
+                                   : reinterpret_cast<const bf16*>(w_) + row_of(l15) * K + kw0 + 8 * q;
+                const size_t step = pk ? 512 : 32;
 #pragma unroll
-                    for (int s = 0; s < S; ++s) wv[t][s] = load_nt16(run + (size_t)s * 512);
+                for (int s = 0; s < S; ++s) wv[t][s] = load_nt16(p + (size_t)s * step);
+            } else if constexpr (FRAG) {
+                const size_t row = row_of(l15);
+#pragma unroll
+                for (int s = 0; s < WS; ++s) {
+                    const int k = kw0 + s * 64 + 16 * q;
+                    wv[t][s] = load_nt16(reinterpret_cast<const uint8_t*>(w_) + row * K + k);
+                    wsc[t][s] = to_f(a.wscale[(row >> 7) * (size_t)(K >> 7) + (k >> 7)]);
                 }
-                return;
-            }
-        }
-        if (wlane) {
+            } else {
+                constexpr int LR = 64 / RL;                // lanes to a row's chunk
+                constexpr int B = FP8 ? 1 : 2;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const size_t row = (size_t)(t == 0 ? nrow : N + nrow);
+                for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const int k = kw0 + s * 32 + 8 * q;
-                    if constexpr (FP8) {
-                        const uint2 v = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(w_) + row * K + k);
-                        wv[t][s] = make_uint4(v.x, v.y, 0, 0);
-                        wsc[t][s] = to_f(a.wscale[(row >> 7) * (size_t)(K >> 7) + (k >> 7)]);
-                    } else {
-                        wv[t][s] = load_nt16(reinterpret_cast<const bf16*>(w_) + row * K + k);
-                    }
+                    for (int i = 0; i < RPG / RL; ++i)
+                        wv[t][c * (RPG / RL) + i] = load_nt16(reinterpret_cast<const char*>(w_) + (row_of(i * RL + lane / LR) * K + kw0 + c * 256) * B + (lane % LR) * 16);
+                if constexpr (FP8) {
+#pragma unroll
+                    for (int i = 0; i < 2 * NC; ++i) wsc[t][i] = to_f(a.wscale[(row_of(l15 % RPG) >> 7) * (size_t)(K >> 7) + (kw0 >> 7) + i]);
                 }
             }
         }
     };
     const int em = tid >> 4, en = tid & 15;
+    float res0 = 0.f;                                      // of the first group
+    if constexpr (EPI == EPI_RESID) res0 = a.res[(size_t)min(em, M - 1) * a.ld_out + min((int)blockIdx.x * RPG + en, N - 1)];
 
     // ---- activation fragments of this wave's K quarter ----
-    // Issue order = arrival order: the activation rows (L2) are requested BEFORE the weight stream (HBM), so the RMSNorm
+    // Issue order = arrival order: rows, gamma and residual (L2) are requested BEFORE the weight stream (HBM), so the RMSNorm
     // statistic, its barrier and the bf16 conversion run while the weights are still in flight (the other way round the
     // prologue started when the last weight byte had landed - the batch-1 kernels' lesson).
-    const float* src = x_ + (size_t)min(l15, M - 1) * K + kw0 + 8 * q;
     uint4 af[S];
-    constexpr bool HOLD_FIRST = PRO == PRO_NORM && S <= 8;      // raw rows held in registers across the reduction
-    if constexpr (!HOLD_FIRST) load_w(blockIdx.x * RPG);        // (deep K: the rows are re-read after the barrier anyway)
-    auto pack8 = [](const float4& u, const float4& v, float inv, const float* g) {
-        return make_uint4(pack_bf16x2(u.x * inv * g[0], u.y * inv * g[1]), pack_bf16x2(u.z * inv * g[2], u.w * inv * g[3]),
-                          pack_bf16x2(v.x * inv * g[4], v.y * inv * g[5]), pack_bf16x2(v.z * inv * g[6], v.w * inv * g[7]));
+    char* img = s_img[wid];
+    auto slot = [&](int c8, int m) { return (c8 * MR + (m ^ (c8 & (MR - 1)))) * 16; };
+    auto order = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    auto take = [&](int c) {                               // behind the wave's own writes; the next chunk's come behind it
+        order();
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const int c8 = FP8 ? 8 * (s >> 1) + 2 * q + (s & 1) : 4 * s + q;
+            af[8 * c + s] = *reinterpret_cast<const uint4*>(img + slot(c8, l15 & (MR - 1)));
+        }
+        order();
     };
     if constexpr (PRO == PRO_NORM) {
-        constexpr bool HOLD = S <= 8;                      // raw rows stay in registers across the reduction
-        float4 r0[HOLD ? S : 1], r1[HOLD ? S : 1];
-        float ss = 0.f;
+        constexpr bool HOLD = MR * NC <= 32;               // raw rows stay in registers across the reduction
+        const float* src = x_ + kw0 + 4 * lane;
+        auto row = [&](int m, int c) { return *reinterpret_cast<const float4*>(src + (size_t)min(m, M - 1) * K + 256 * c); };
+        float4 r[HOLD ? NC : 1][MR];
+        uint2 g[NC];
+        float ss[MR];
         if constexpr (HOLD) {
 #pragma unroll
-            for (int s = 0; s < S; ++s) { r0[s] = *reinterpret_cast<const float4*>(src + s * 32); r1[s] = *reinterpret_cast<const float4*>(src + s * 32 + 4); }
-            __builtin_amdgcn_sched_barrier(0);
-            load_w(blockIdx.x * RPG);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const float4 u = r0[s], v = r1[s];
-                ss += u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w + v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-            }
-        } else {
+                for (int m = 0; m < MR; ++m) r[c][m] = row(m, c);
+        }
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const float4 u = *reinterpret_cast<const float4*>(src + s * 32), v = *reinterpret_cast<const float4*>(src + s * 32 + 4);
-                ss += u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w + v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+        for (int c = 0; c < NC; ++c) g[c] = *reinterpret_cast<const uint2*>(gamma_ + kw0 + 256 * c + 4 * lane);
+        if constexpr (!HOLD) {
+#pragma unroll
+            for (int m = 0; m < MR; ++m) ss[m] = 0.f;
+            for (int c = 0; c < NC; ++c) {
+#pragma unroll
+                for (int m = 0; m < MR; ++m) r[0][m] = row(m, c);
+#pragma unroll
+                for (int m = 0; m < MR; ++m) ss[m] += r[0][m].x * r[0][m].x + r[0][m].y * r[0][m].y + r[0][m].z * r[0][m].z + r[0][m].w * r[0][m].w;
             }
         }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
-        if (q == 0) s_ss[wid][l15] = ss;
-        __syncthreads();
-        const float inv = 1.0f / sqrtf((s_ss[0][l15] + s_ss[1][l15] + s_ss[2][l15] + s_ss[3][l15]) / K + a.eps);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(blockIdx.x * RPG);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            Vec<bf16> gr;
-            gr.load(gamma_ + kw0 + s * 32 + 8 * q);
-            float g[8];
-            gr.to_float(g);
+        for (int m = 0; m < MR; ++m) {
             if constexpr (HOLD) {
-                af[s] = pack8(r0[s], r1[s], inv, g);
-            } else {
-                const float4 u = *reinterpret_cast<const float4*>(src + s * 32), v = *reinterpret_cast<const float4*>(src + s * 32 + 4);
-                af[s] = pack8(u, v, inv, g);
+                ss[m] = 0.f;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) ss[m] += r[c][m].x * r[c][m].x + r[c][m].y * r[c][m].y + r[c][m].z * r[c][m].z + r[c][m].w * r[c][m].w;
             }
         }
-    } else {                                               // bf16 hand-off: the fragment is the stored 16-byte chunk
-        const bf16* src16 = a.xin16 + (size_t)min(l15, M - 1) * K + kw0 + 8 * q;
+        // 16 lanes, 16 (8) rows: at each step a lane keeps the half of the rows that its bit names and hands the other half over, so it ends with row lane & (MR - 1)
+        const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+        if constexpr (MR == 16) {
 #pragma unroll
-        for (int s = 0; s < S; ++s) af[s] = *reinterpret_cast<const uint4*>(src16 + s * 32);
-    }
-    if (l15 >= M) {
+            for (int i = 0; i < 8; ++i) ss[i] = (b3 ? ss[i + 8] : ss[i]) + dpp_f<DPP_MIRROR>(b3 ? ss[i] : ss[i + 8]);
+        }
 #pragma unroll
-        for (int s = 0; s < S; ++s) af[s] = make_uint4(0, 0, 0, 0);      // rows past the batch contribute nothing
+        for (int i = 0; i < 4; ++i) ss[i] = (b2 ? ss[i + 4] : ss[i]) + dpp_f<DPP_HALF_MIRROR>(b2 ? ss[i] : ss[i + 4]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ss[i] = (b1 ? ss[i + 2] : ss[i]) + dpp_f<DPP_XOR2>(b1 ? ss[i] : ss[i + 2]);
+        ss[0] = (b0 ? ss[1] : ss[0]) + dpp_f<DPP_XOR1>(b0 ? ss[0] : ss[1]);
+        if constexpr (MR == 8) ss[0] += dpp_f<DPP_ROR8>(ss[0]);
+        const int mr = lane & (MR - 1);                    // a lane's row; the others' come from their lanes
+        s_ss[mr][4 * wid + q] = ss[0];
+        __syncthreads();
+        float tot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 v = *reinterpret_cast<const float4*>(&s_ss[mr][4 * i]);
+            tot += (v.x + v.y) + (v.z + v.w);
+        }
+        const float mine = 1.0f / sqrtf(tot / K + a.eps);
+        float inv[MR];
+#pragma unroll
+        for (int m = 0; m < MR; ++m) inv[m] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), m));
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float g0 = __uint_as_float(g[c].x << 16), g1 = __uint_as_float(g[c].x & 0xFFFF0000u), g2 = __uint_as_float(g[c].y << 16), g3 = __uint_as_float(g[c].y & 0xFFFF0000u);
+            if constexpr (!HOLD) {
+#pragma unroll
+                for (int m = 0; m < MR; ++m) r[0][m] = row(m, c);
+            }
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                const float4 v = r[HOLD ? c : 0][m];
+                *reinterpret_cast<uint2*>(img + slot(lane >> 1, m) + (lane & 1) * 8) =
+                    make_uint2(pack_bf16x2(v.x * inv[m] * g0, v.y * inv[m] * g1), pack_bf16x2(v.z * inv[m] * g2, v.w * inv[m] * g3));
+            }
+            take(c);
+        }
+    } else {                                               // bf16 hand-off: 32 lanes to the 512 bytes of a row's chunk
+        const bf16* src = reinterpret_cast<const bf16*>(x_) + kw0 + 8 * (lane & 31);
+        u32x4 r[NC][MR / 2];
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < MR / 2; ++i) r[c][i] = *reinterpret_cast<const u32x4*>(src + (size_t)min(2 * i + (lane >> 5), M - 1) * K + 256 * c);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(blockIdx.x * RPG);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+#pragma unroll
+            for (int i = 0; i < MR / 2; ++i) *reinterpret_cast<u32x4*>(img + slot(lane & 31, 2 * i + (lane >> 5))) = r[c][i];
+            take(c);
+        }
     }
 
-    auto bfrag = [&](int t, int s) -> uint4 {
-        if constexpr (FP8) {
-            const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].x, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].x, true);
-            const f32x2 c2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].y, false), c3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].y, true);
-            const float sc = wsc[t][s];
-            return make_uint4(pack_bf16x2(c0.x * sc, c0.y * sc), pack_bf16x2(c1.x * sc, c1.y * sc), pack_bf16x2(c2.x * sc, c2.y * sc),
-                              pack_bf16x2(c3.x * sc, c3.y * sc));
-        } else {
-            return wv[t][s];
-        }
+    // 8 k of e4m3 codes, scaled
+    auto widen = [](uint32_t lo, uint32_t hi, float sc) {
+        const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, true);
+        const f32x2 c2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, false), c3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, true);
+        return make_uint4(pack_bf16x2(c0.x * sc, c0.y * sc), pack_bf16x2(c1.x * sc, c1.y * sc), pack_bf16x2(c2.x * sc, c2.y * sc), pack_bf16x2(c3.x * sc, c3.y * sc));
     };
+    auto half = [&](const uint4& v, int h, float sc) { return h ? widen(v.z, v.w, sc) : widen(v.x, v.y, sc); };
     float bv = -INFINITY;
     int bi = 0x7FFFFFFF;
     for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
         const int n0 = g * RPG;
-        float resv = 0.f;
-        if constexpr (EPI == EPI_RESID) resv = a.res[(size_t)min(em, M - 1) * a.ld_out + min(n0 + en, N - 1)];
+        float resv = res0;
+        if constexpr (EPI == EPI_RESID) {
+            if (g != (int)blockIdx.x) resv = a.res[(size_t)min(em, M - 1) * a.ld_out + min(n0 + en, N - 1)];
+        }
         f32x4_b acc[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = f32x4_b{0.f, 0.f, 0.f, 0.f};
+        auto mul = [&](int t, int s, const uint4& w) {
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_b, af[s]), __builtin_bit_cast(bf16x8_b, w), acc[t], 0, 0, 0);
+        };
+        if constexpr (FRAG) {
 #pragma unroll
-        for (int s = 0; s < S; ++s)
+            for (int s = 0; s < S; ++s)
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_b, af[s]), __builtin_bit_cast(bf16x8_b, bfrag(t, s)), acc[t], 0, 0, 0);
+                for (int t = 0; t < NT; ++t) {
+                    if constexpr (FP8) mul(t, s, half(wv[t][s / 2], s & 1, wsc[t][s / 2]));
+                    else mul(t, s, wv[t][s]);
+                }
+        } else {
+            constexpr int LR = 64 / RL;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    auto at = [&](int c16, int r) { return img + (c16 * RPG + (r ^ (c16 & (RPG - 1)))) * 16; };
+#pragma unroll
+                    for (int i = 0; i < RPG / RL; ++i) *reinterpret_cast<uint4*>(at(lane % LR, i * RL + lane / LR)) = wv[t][c * (RPG / RL) + i];
+                    order();
+                    uint4 w[FP8 ? 4 : 8];
+#pragma unroll
+                    for (int s = 0; s < (FP8 ? 4 : 8); ++s) w[s] = *reinterpret_cast<const uint4*>(at(4 * s + q, l15 % RPG));
+                    order();
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) {
+                        if constexpr (FP8) mul(t, 8 * c + s, half(w[s / 2], s & 1, wsc[t][2 * c + s / 4]));
+                        else mul(t, 8 * c + s, w[s]);
+                    }
+                }
+        }
         // the next group's weights (lm_head: a workgroup walks several groups) travel while this one is reduced and stored
         if (g + (int)gridDim.x < ngroups) load_w((g + (int)gridDim.x) * RPG);
         __syncthreads();                                    // the previous trip's partial tiles have been read
-        if (wlane) {
+        if (l15 < RPG) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -644,18 +731,27 @@ static pgk_status launch_batched_tiled(const FusedArgs& a, int M, hipStream_t st
     return set_error(PGK_ERR_UNSUPPORTED, "batched decode projection: K=%d is not 128 x {2,4,8,16,24,32}", a.K);
 }
 
+template <class WT, int PRO, int EPI, int S, int RPG>
+static pgk_status launch_batched_rows(const FusedArgs& a, int M, int grid, hipStream_t st, int nblk_logits) {
+    const float* x = PRO == PRO_NORM ? a.h : reinterpret_cast<const float*>(a.xin16);
+    hipError_t he;
+    if (M <= 8) he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, RPG, 8>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
+    else he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, RPG, 16>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
+    PGK_CHECK_HIP(he);
+    return PGK_OK;
+}
+
 template <class WT, int PRO, int EPI, int S>
 static pgk_status launch_batched_reg(const FusedArgs& a, int M, hipStream_t st, int nblk_logits) {
     // enough workgroups to pull HBM bandwidth: fewer weight rows per workgroup when N / 16 would leave CUs idle
-    int rpg = (EPI == EPI_LOGITS || ceil_div(a.N, 16) >= 192) ? 16 : (ceil_div(a.N, 8) >= 192 ? 8 : 4);
-    const int grid = (EPI == EPI_LOGITS) ? nblk_logits : ceil_div(a.N, rpg);
-    const float* x = a.h;
-    hipError_t he;
-    if (rpg == 16) he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, 16>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
-    else if (rpg == 8) he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, 8>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
-    else he = launch_k(batched_reg_kernel<WT, PRO, EPI, S, 4>, dim3(grid), dim3(256), 0, st, a.w, a.wp, x, a.gamma, a.N, a.K, M, nblk_logits, a);
-    PGK_CHECK_HIP(he);
-    return PGK_OK;
+    const int rpg = (EPI == EPI_LOGITS || ceil_div(a.N, 16) >= 192) ? 16 : (ceil_div(a.N, 8) >= 192 ? 8 : 4);
+    if constexpr (EPI == EPI_LOGITS) return launch_batched_rows<WT, PRO, EPI, S, 16>(a, M, nblk_logits, st, nblk_logits);
+    else {
+        const int grid = ceil_div(a.N, rpg);
+        if (rpg == 16) return launch_batched_rows<WT, PRO, EPI, S, 16>(a, M, grid, st, nblk_logits);
+        if (rpg == 8) return launch_batched_rows<WT, PRO, EPI, S, 8>(a, M, grid, st, nblk_logits);
+        return launch_batched_rows<WT, PRO, EPI, S, 4>(a, M, grid, st, nblk_logits);
+    }
 }
 
 template <class WT, int PRO, int EPI, int MP, int S>
@@ -687,15 +783,7 @@ static pgk_status launch_batched(const FusedArgs& a, int M, hipStream_t st, int 
     const size_t lds = (size_t)(a.K / 8) * mp * 16 + (size_t)NT * 4 * 256 * 4;
     PGK_REQUIRE(lds <= 158 * 1024, "batched decode projection: K=%d does not fit the LDS image", a.K);
 #define PGK_BS(MPV, SV) return launch_batched_s<WT, PRO, EPI, MPV, SV>(a, M, steps, grid, lds, st, nblk_logits);
-    if (mp == 8) {
-        if (steps == 8) PGK_BS(8, 8)
-        if (steps == 16) PGK_BS(8, 16)
-        if (steps == 24) PGK_BS(8, 24)
-        PGK_BS(8, 0)
-    }
-    if (steps == 8) PGK_BS(16, 8)
-    if (steps == 16) PGK_BS(16, 16)
-    if (steps == 24) PGK_BS(16, 24)
+    if (mp == 8) PGK_BS(8, 0)
     PGK_BS(16, 0)
 #undef PGK_BS
 }
