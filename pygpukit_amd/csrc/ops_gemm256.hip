@@ -66,6 +66,18 @@ __device__ __forceinline__ void g2_tile_of(int id, int nwg, int ntm, int ntn, in
     tn = in / gsz;
 }
 
+// ---- bf16 C tiles in LDS, for the epilogues.  Kernels with such a tile multiply W fragments by A fragments, so a lane of a 16 x 16 product holds four consecutive columns of
+// one row (row lane & 15, columns 4 (lane >> 4) .. + 4) and puts them down in one 8-byte instruction, where four rows of a column took four of 2 bytes.
+// 16-byte chunks are XOR-ed by the row so that the 16 rows of an instruction meet different banks; whole rows are read back.
+//   us a launch, the other way and this: 1531 rows, K = 1024: SwiGLU (192 x 192) 23.5 / 23.0, QKV heads (192 x 128) 20.0 / 19.5; 4096 rows, K = 4096: SwiGLU, N = 14336 714 /
+// 708, QKV stored from registers (N = 6144) 177 / 172.  fp32 tiles (16 bytes for four of 4) lost as much: += of N = 4096, K = 4096 107 / 113.
+template <int ROWB> __device__ __forceinline__ int ct_off(int row, int byte) {
+    static_assert(ROWB % 128 == 0, "chunks are exchanged in groups of 8, or of 16");
+    const int sw = ROWB % 256 == 0 ? row & 15 : (row >> 1) & 7;
+    return row * ROWB + (((byte >> 4) ^ sw) << 4) + (byte & 15);
+}
+__device__ __forceinline__ uint2 ct_bf16(const f32x4_g& v) { return make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])); }
+
 // ---- SwiGLU epilogue (EPI 2 of the kernels below): W is the fused [2 I, K] gate / up weight, the workgroup's 256 B-tile rows are
 // gate rows [128 tn, +128) followed by up rows [I + 128 tn, +128), so output tile tn holds act columns [128 tn, +128): waves
 // wc 0 / 1 hold gate columns, wc 2 / 3 the matching up columns.  The accumulators go to LDS as the bf16 tile the plain kernel
@@ -76,7 +88,7 @@ __device__ __forceinline__ void g2_tile_of(int id, int nwg, int ntm, int ntn, in
 // store 16 bytes of bf16, or (QOUT) 8 e4m3 codes with the row's scale for this 128-column block (absmax / 448 over the 16
 // lanes, quantize_fp8_rows' contract): exactly the fp8 x fp8 down projection's A operand.  Saves the [M][2 I] bf16 round
 // trip through HBM (Llama-3-8B shape, S = 4096: 235 MB written + read back = ~75 us of a 1.4 ms layer) and a launch.
-template <bool QOUT, int TN = 4>   // TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
+template <bool QOUT, int TN = 4, bool ROWS = false>   // ROWS: a lane holds columns of a row (ct_off), otherwise rows of a column; TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
 __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&acc)[8][TN], int tid, int m0, int tn, int M, int I,
                                                    void* outv, float* out_scales) {
     static_assert(TN == 4 || !QOUT, "the e4m3 epilogue needs whole 128-column scale blocks");
@@ -86,19 +98,25 @@ __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&a
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<uint2*>(smem + ct_off<ROWB>(wr * 128 + i * 16 + l15, (wc * WN + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
-                *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
+                for (int r = 0; r < 4; ++r) {
+                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
+                    *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
+                }
             }
+        }
+    auto at = [&](int row, int byte) { return smem + (ROWS ? ct_off<ROWB>(row, byte) : row * ROWB + (byte ^ (((row >> 2) & 3) << 5))); };
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < 256 * CH / G2_THREADS; ++it) {
-        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH, sw = ((row >> 2) & 3) << 5;
+        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH;
         Vec<bf16> g, u;
-        g.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((c * 16) ^ sw));
-        u.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((ACT * 2 + c * 16) ^ sw));
+        g.raw = *reinterpret_cast<const uint4*>(at(row, c * 16));
+        u.raw = *reinterpret_cast<const uint4*>(at(row, ACT * 2 + c * 16));
         float gf[8], uf[8];
         g.to_float(gf);
         u.to_float(uf);
@@ -171,6 +189,7 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
 // ---- QKV-heads epilogue (EPI 3 of the fp8 kernel, 5 of the bf16 one): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
 // g2_swiglu_epilogue), a tile = 256 token rows x two head slots, 16 consecutive lanes take one (row, head) and finish it
 // (HeadRows: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
+template <bool ROWS = false>
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -181,20 +200,25 @@ __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g 
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<uint2*>(smem + ct_off<512>(wr * 128 + i * 16 + l15, (wc * 64 + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
-                *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
+                for (int r = 0; r < 4; ++r) {
+                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
+                    *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
+                }
             }
+        }
     hr.angles(c, 2 * tn, hd);
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         hr.finish(c, 2 * tn + h, m0 + r0, 32, M, hd, qkv, N, [&](int i, float (&x)[8]) {
-            const int row = i * 32 + r0, sw = ((row >> 2) & 3) << 5;
+            const int row = i * 32 + r0, byte = h * 256 + c * 16;
             Vec<bf16> raw;
-            raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((h * 256 + c * 16) ^ sw));
+            raw.raw = *reinterpret_cast<const uint4*>(smem + (ROWS ? ct_off<512>(row, byte) : row * 512 + (byte ^ (((row >> 2) & 3) << 5))));
             raw.to_float(x);
         });
 }
@@ -343,6 +367,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
+    constexpr bool ROWS = EPI != 1;                          // a lane holds columns of a row: ct_off
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
     const int late = __builtin_amdgcn_readfirstlane(wr);     // wave-uniform by construction: scalar branches around barriers
@@ -445,8 +470,8 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
         __builtin_amdgcn_s_setprio(1);                                                                       \
         _Pragma("unroll") for (int i = 0; i < 8; ++i)                                                        \
             _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                   \
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_g, fa[i]),     \
-                                                                    __builtin_bit_cast(bf16x8_g, fb[j]), acc[i][j], 0, 0, 0); \
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_g, ROWS ? fb[j] : fa[i]),     \
+                                                                    __builtin_bit_cast(bf16x8_g, ROWS ? fa[i] : fb[j]), acc[i][j], 0, 0, 0); \
         __builtin_amdgcn_s_setprio(0);                                                                       \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
         if (!late) wait_two_younger();                                                                       \
@@ -472,18 +497,18 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const f32x4_g f = *reinterpret_cast<const f32x4_g*>(inv + wr * 128 + i * 16 + q * 4);
+                const float f = inv[wr * 128 + i * 16 + l15];
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] *= f;
             }
         }
     }
     if constexpr (EPI == 2) {
-        g2_swiglu_epilogue<false, TN>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
+        g2_swiglu_epilogue<false, TN, true>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
         return;
     }
     if constexpr (EPI == 5) {
-        g2_qkv_heads_epilogue(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
+        g2_qkv_heads_epilogue<true>(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
         return;
     }
     if constexpr (EPI == 1 && TN == 4) {
@@ -492,23 +517,53 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
             return;
         }
     }
+    if constexpr (!ROWS) {                                   // N % 4 != 0
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = n0 + wc * WN + j * 16 + l15;
+            if (col >= N) continue;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = m0 + wr * 128 + i * 16 + q * 4 + r;
+                    if (row < M) reinterpret_cast<float*>(Cv)[(size_t)row * N + col] += acc[i][j][r];
+                }
+        }
+        return;
+    }
+    // four columns of a row to a lane: one 8-byte store where every row is aligned to it
+    const bool whole = (N & 3) == 0 && ((uintptr_t)Cv & 7) == 0;
+    bf16* C = reinterpret_cast<bf16*>(Cv);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wc * WN + j * 16 + l15;
-        if (col >= N) continue;
-        float b = 0.f;
-        if constexpr (EPI == 0) b = bias ? to_f(bias[col]) : 0.f;
+        const int col = n0 + wc * WN + j * 16 + q * 4;
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (EPI == 0) {
+            if (bias) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+                for (int r = 0; r < 4; ++r) b[r] = to_f(bias[min(col + r, N - 1)]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int row = m0 + wr * 128 + i * 16 + l15;
+            if (row >= M) continue;
+            f32x4_g v = acc[i][j];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wr * 128 + i * 16 + q * 4 + r;
-                if (row >= M) continue;
-                if constexpr (EPI == 0) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(acc[i][j][r] + b);
-                else if constexpr (EPI == 3) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(xielu<false>(acc[i][j][r], xa.pos, xa.neg));
-                else if constexpr (EPI == 4) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(gelu_erf(acc[i][j][r]));
-                else reinterpret_cast<float*>(Cv)[(size_t)row * N + col] += acc[i][j][r];
+                if constexpr (EPI == 0) v[r] += b[r];
+                else if constexpr (EPI == 3) v[r] = xielu<false>(v[r], xa.pos, xa.neg);
+                else if constexpr (EPI == 4) v[r] = gelu_erf(v[r]);
             }
+            if (whole) {
+                if (col < N) *reinterpret_cast<uint2*>(C + (size_t)row * N + col) = ct_bf16(v);
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (col + r < N) C[(size_t)row * N + col + r] = from_f<bf16>(v[r]);
+        }
     }
 }
 
@@ -544,7 +599,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
                                            int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no, const BestOut& bo) {
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
     constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
-    constexpr bool B16 = EPI == 3 || EPI == 4, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4), PARTS = SCALED && EPI == 4 && BM == 64;   // PARTS: may come as ni.ld says
+    constexpr bool B16 = EPI == 3 || EPI == 4, ROWS = B16, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4), PARTS = SCALED && EPI == 4 && BM == 64;   // PARTS: may come as ni.ld says
     static_assert(!SCALED || BM <= 256, "a row for each of the waves that multiply");
     static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -666,7 +721,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
         int a_cur = 0, w_cur = 0;                            // ring slots of stage s
 #define GP_MFMA(I, F, P)                                                                                     \
-    _Pragma("unroll") for (int j = 0; j < WN; ++j) acc[I][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(F, fb[P][j], acc[I][j], 0, 0, 0); \
+    _Pragma("unroll") for (int j = 0; j < WN; ++j) acc[I][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ROWS ? fb[P][j] : F, ROWS ? F : fb[P][j], acc[I][j], 0, 0, 0); \
     __builtin_amdgcn_sched_barrier(0);
 #define GP_STEP(BUF)                                                                                         \
     {                                                                                                        \
@@ -704,9 +759,8 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         __builtin_amdgcn_s_barrier();
     }
 
-    // rows of the tile: fp32, 64-byte group g at g ^ ((R >> 2) & 3), or bf16, 32-byte group likewise - (R >> 2) & 3 == q for the accumulator layout
+    // rows of the tile: bf16 (ROWS: ct_off), or fp32, 64-byte group g at g ^ ((R >> 2) & 3), which is q for a lane's rows
     constexpr int ROWB = BN * (B16 ? 2 : 4);
-    constexpr int QS = B16 ? 5 : 6;
     HeadRows<EPI == 3 ? BM / 32 : 1> hr;
     const int hrow = tid >> 4;                               // EPI 3: 16 consecutive lanes = one (token row, head)
     if constexpr (EPI == 3) hr.places(m0 + hrow, 32, M, hd);
@@ -722,7 +776,11 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
             if (wid < 4) {
 #pragma unroll
                 for (int i = 0; i < WM; ++i) {
-                    const f32x4_g f = *reinterpret_cast<const f32x4_g*>(inv + wr * 16 * WM + i * 16 + q * 4);
+                    f32x4_g f;
+                    if constexpr (ROWS) {
+                        const float one = inv[wr * 16 * WM + i * 16 + l15];
+                        f = f32x4_g{one, one, one, one};
+                    } else f = *reinterpret_cast<const f32x4_g*>(inv + wr * 16 * WM + i * 16 + q * 4);
 #pragma unroll
                     for (int j = 0; j < WN; ++j) acc[i][j] *= f;
                 }
@@ -733,16 +791,18 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
-            for (int j = 0; j < WN; ++j)
+            for (int j = 0; j < WN; ++j) {
+                if constexpr (ROWS) {
+                    *reinterpret_cast<uint2*>(g2_smem + ct_off<ROWB>(wr * 16 * WM + i * 16 + l15, (wc * 16 * WN + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
+                } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = wr * 16 * WM + i * 16 + q * 4 + r, col = wc * 16 * WN + j * 16 + l15;
-                    if constexpr (B16) *reinterpret_cast<bf16*>(g2_smem + row * ROWB + ((col * 2) ^ (q << QS))) = from_f<bf16>(acc[i][j][r]);
-                    else *reinterpret_cast<float*>(g2_smem + row * ROWB + ((col * 4) ^ (q << QS))) = acc[i][j][r];
+                    for (int r = 0; r < 4; ++r)
+                        *reinterpret_cast<float*>(g2_smem + (wr * 16 * WM + i * 16 + q * 4 + r) * ROWB + (((wc * 16 * WN + j * 16 + l15) * 4) ^ (q << 6))) = acc[i][j][r];
                 }
+            }
     }
     if constexpr (EPI == 3) hr.angles((tid & 15), tn, hd);
-    auto tile4 = [&](int row, int byte) { return *reinterpret_cast<const float4*>(g2_smem + row * ROWB + (byte ^ (((row >> 2) & 3) << QS))); };
+    auto tile4 = [&](int row, int byte) { return *reinterpret_cast<const float4*>(g2_smem + row * ROWB + (byte ^ (((row >> 2) & 3) << 6))); };
     if constexpr (EPI == 1 || EPI == 8) {
         constexpr int IT = BM * (BN / 4) / GP_THREADS;
         const int c = tid % (BN / 4), gcol = n0 + c * 4;     // a thread's columns are the same in all its rows
@@ -771,11 +831,11 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         constexpr int CH = BN / 16;                          // chunks of 8 act columns in a row
 #pragma unroll
         for (int it = 0; it < (BM * CH + GP_THREADS - 1) / GP_THREADS; ++it) {
-            const int item = it * GP_THREADS + tid, row = item / CH, c = item % CH, sw = ((row >> 2) & 3) << QS;
+            const int item = it * GP_THREADS + tid, row = item / CH, c = item % CH;
             if (BM * CH % GP_THREADS != 0 && row >= BM) break;
             Vec<bf16> g, u;
-            g.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((c * 16) ^ sw));
-            u.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((BN + c * 16) ^ sw));
+            g.raw = *reinterpret_cast<const uint4*>(g2_smem + ct_off<ROWB>(row, c * 16));
+            u.raw = *reinterpret_cast<const uint4*>(g2_smem + ct_off<ROWB>(row, BN + c * 16));
             float gf[8], uf[8];
             g.to_float(gf);
             u.to_float(uf);
@@ -791,7 +851,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         hr.finish(c, tn, m0 + hrow, 32, M, hd, reinterpret_cast<bf16*>(Cv), N, [&](int i, float (&x)[8]) {
             const int row = i * 32 + hrow;
             Vec<bf16> raw;
-            raw.raw = *reinterpret_cast<const uint4*>(g2_smem + row * ROWB + ((c * 16) ^ (((row >> 2) & 3) << QS)));
+            raw.raw = *reinterpret_cast<const uint4*>(g2_smem + ct_off<ROWB>(row, c * 16));
             raw.to_float(x);
         });
     } else if constexpr (EPI == 2) {

@@ -535,6 +535,18 @@ def test_gemm256_exact_integers(N, monkeypatch):
     np.testing.assert_array_equal(c, O.bf16_round(a @ w.T))
 
 
+@pytest.mark.parametrize("M,N", [(300, 260), (257, 263), (256, 774), (129, 130), (300, 577)])
+def test_gemm256_stores_of_four_columns_exact_integers(M, N, monkeypatch):
+    """The 256-tile kernels store four columns of a row at once where N % 4 == 0 and single ones elsewhere, with a bias, at the ends of rows and of tiles."""
+    rng = np.random.default_rng(M + N)
+    K = 64
+    a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    w = rng.integers(-3, 4, (N, K)).astype(np.float32)
+    bias = rng.integers(-8, 9, N).astype(np.float32)
+    monkeypatch.setenv("PGK_GEMM256", "1")
+    np.testing.assert_array_equal(host(ops.matmul_nt(dev(a, "bfloat16"), dev(w, "bfloat16"), dev(bias, "bfloat16"))), O.bf16_round(a @ w.T + bias))
+
+
 @pytest.mark.parametrize("tile", ["0", "1"])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
 def test_staged_gemm_rings_exact_integers(K, tile, monkeypatch):
