@@ -2126,8 +2126,11 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     auto hidden_splits = [&](int K_) { return !gsplit ? 1 : staged ? engine_gemm_short_splits(H, K_) : engine_gemm_pick_splits(n, H, K_); };
     const int g_so = hidden_splits(QD), g_sd = hidden_splits(I), g_sq = gsplit ? engine_gemm_qkv_splits(n, NQKV, H, D == 128) : 1;
     // RMSNorm without a pass of its own: o_proj and down_proj leave x = bf16(h gamma) and h's sums of squares, gate_up and QKV scale their rows
-    // (Qwen3-0.6B, 1531 rows: a layer 124 -> 115 us, 3365 rows 193 -> 181).  From 512 rows on: 384 rows took the same with it and without.
-    const bool carry = n >= 512 && !ws && !staged && (c.weight_format == 0 || pkd) && engine_gemm_carry_ok(n, NQKV, H) && engine_gemm_carry_ok(n, 2 * I, H);
+    // (Qwen3-0.6B, 1531 rows: a layer 124 -> 115 us, 3365 rows 193 -> 181; ms a prompt, a pass of its own / carried on tiles of 32 rows: 140 rows 1.53 / 1.48, 200
+    // 1.60 / 1.52, 450 1.85 / 1.73; on tiles of 64 rows 450 took 1.91).  engine_gemm_resid_pays says which products.  Below 512 rows wide models gain nothing by
+    // it (H = 4096, I = 14336, 140, 200 and 450 rows: 1.00x), and narrow ones keep the pass all the same (H = 512, 300 rows 0.38 / 0.34): there the two families of tiles
+    // are held to one another's sums, which a rounding in another place exceeds.
+    const bool carry = (n >= 512 || (H >= 1024 && H <= 2048)) && !ws && !staged && (c.weight_format == 0 || pkd) && engine_gemm_carry_ok(n, NQKV, H) && engine_gemm_carry_ok(n, 2 * I, H);
     const bool carry_o = carry && engine_gemm_resid_pays(n, H, QD, g_so), carry_d = carry && g_sq == 1 && engine_gemm_resid_pays(n, H, I, g_sd);
     const bool use_slabs = ws || g_so > 1 || g_sd > 1 || g_sq > 1;
     size_t slab_elems = (size_t)(s_o > s_d ? s_o : s_d) * n * H;

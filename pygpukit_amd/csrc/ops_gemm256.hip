@@ -600,9 +600,15 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 constexpr int GP_THREADS = 512;
 // stages of W that the ring holds; A's has two more.  The smaller tiles' stages are shorter, and latency asks for more of them
 constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 || (WM == 2 && WN == 4) ? 4 : 6; }
+// Tiles of 32 rows: a 2 x 2 split would leave a wave 16 rows.  There (gemmp_kg) the waves split K as well: of a pair of stages one wave of two multiplies the first, its
+// partner the second, each for a piece of 32 x 16 WN; one barrier a pair, and the partners trade halves of their sums at the end.
+constexpr bool gemmp_kg(int WM, int WN) { return WM == 1; }
+constexpr int GP_PAIRS = 6;                                  // pairs of stages in that ring: 12 KiB each for 32 x 64, two workgroups a CU
 template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
-    const size_t RW = gemmp_ring(WM, WN), ring = (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
-    return ring > tile ? ring : tile;
+    const size_t RW = gemmp_ring(WM, WN), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
+    const size_t ring = gemmp_kg(WM, WN) ? GP_PAIRS * (size_t)(32 * (WM + WN) * 128) : (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64);
+    const size_t least = gemmp_kg(WM, WN) ? tile + 1024 + WM * WN * 4096 : tile;
+    return ring > least ? ring : least;
 }
 struct BestOut { float* val; int* idx; };                    // [M][tiles of columns]
 template <int EPI, bool GRP, int WM, int WN>
@@ -610,6 +616,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
                                            int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no, const BestOut& bo) {
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
     constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
+    constexpr bool KG = gemmp_kg(WM, WN);
     constexpr bool B16 = EPI == 3 || EPI == 4, ROWS = B16, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4), PARTS = SCALED && EPI == 4 && BM == 64;   // PARTS: may come as ni.ld says
     static_assert(!SCALED || BM <= 256, "a row for each of the waves that multiply");
     static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
@@ -632,7 +639,8 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 
     f32x4_g acc[WM][WN];
     float mine = 0.f;                                        // 1 / rms of row tid (ni.ld: of tid / 4)
-    const int wr = (wid >> 1) & 1, wc = wid & 1, q = lane >> 4, l15 = lane & 15;
+    const int part = (wid >> 1) & 1, kg = wid & 1;           // KG: which columns, which stage of a pair; behind the trade rows 16 WM kg .. of those columns
+    const int wr = KG ? kg : part, wc = KG ? part : kg, q = lane >> 4, l15 = lane & 15;
     if (wid >= 4) {
         const int pw = __builtin_amdgcn_readfirstlane(wid & 3);
         auto a_row = [&](int r) -> int {
@@ -668,6 +676,33 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 #pragma unroll
             for (int i = 0; i < NW; ++i) g2_dma16(w_src[i] + kw, dst + i * 1024);
         };
+        if constexpr (KG) {
+            constexpr int PB = 2 * (AH + WH), EACH = NA + 2 * NW;     // bytes and DMA instructions of a pair
+            auto stage_pair = [&](int p, int at) {           // past the end of K the last pair is read again
+                const int h = min(2 * p, nh - 2);
+                const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + at);
+#pragma unroll
+                for (int i = 0; i < NA; ++i) g2_dma16(a_src[i] + h * 32, dst + (pw * NA + i) * 1024);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) g2_dma16(w_src[i] + (size_t)(h + t) * wk, dst + 2 * AH + t * WH + (pw * NW + i) * 1024);
+            };
+#pragma unroll
+            for (int p = 0; p < GP_PAIRS; ++p) stage_pair(p, p * PB);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((GP_PAIRS - 1) * EACH) : "memory");      // pair 0
+            __builtin_amdgcn_s_barrier();
+            int at = 0;
+            for (int p = 0; 2 * p < nh; ++p) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((GP_PAIRS - 2) * EACH) : "memory");  // pair p + 1; pair p is in registers behind the barrier
+                __builtin_amdgcn_s_barrier();
+                stage_pair(p + GP_PAIRS, at);
+                at = at == (GP_PAIRS - 1) * PB ? 0 : at + PB;
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // retire the phantom DMAs: the ring becomes the C tile
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_s_barrier();                    // the partners' trade
+        } else {
         // between W of a stage and the wait for it: W of RW - 2 stages and their A
         auto wait_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RW - 2) * NW + (RW - 2) / 2 * NA) : "memory"); };
         stage_a(0, 0);
@@ -692,6 +727,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // retire the phantom DMAs: the stages become the C tile
         __builtin_amdgcn_s_barrier();
+        }
     } else {
         if constexpr (PARTS) {
             if (ni.ss && ni.ld) {                            // four threads to a row, 16 parts each
@@ -712,14 +748,70 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         if constexpr (SCALED && EPI != 0) {
             if (ni.ss && !(PARTS && ni.ld) && tid < BM) mine = norm_in_scale(ni, min(m0 + tid, M - 1), M, K);
         }
+        const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
+        const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
+        auto frag = [&](const char* p) { return *reinterpret_cast<const bf16x8_g*>(p); };
+        if constexpr (KG) {
+            constexpr int FM = 2 * WM, PB = 2 * (AH + WH);
+            f32x4_g big[FM][WN];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) big[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
+            const char *a_at = g2_smem + (kg ? a_off1 : a_off0), *w_at = g2_smem + 2 * AH + kg * WH + part * 16 * WN * 64 + w_off;
+            bf16x8_g fa[2][FM], fb[2][WN];
+            auto fetch = [&](bf16x8_g (&A_)[FM], bf16x8_g (&W_)[WN], int at) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) A_[i] = frag(a_at + at + i * 2048);
+#pragma unroll
+                for (int j = 0; j < WN; ++j) W_[j] = frag(w_at + at + j * 1024);
+            };
+            int at = 0;                                      // ring slot of pair p
+            auto step = [&](bf16x8_g (&A_)[FM], bf16x8_g (&W_)[WN], bf16x8_g (&nA)[FM], bf16x8_g (&nW)[WN]) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // pair p in registers: its place may be refilled
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                at = at == (GP_PAIRS - 1) * PB ? 0 : at + PB;
+                fetch(nA, nW, at);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) big[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ROWS ? W_[j] : A_[i], ROWS ? A_[i] : W_[j], big[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            __builtin_amdgcn_s_barrier();
+            fetch(fa[0], fb[0], 0);
+            int s = 0;
+            for (; s + 4 <= nh; s += 4) {
+                step(fa[0], fb[0], fa[1], fb[1]);
+                step(fa[1], fb[1], fa[0], fb[0]);
+            }
+            if (s < nh) step(fa[0], fb[0], fa[1], fb[1]);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the reads past the last pair
+            __builtin_amdgcn_s_barrier();
+            // the lower rows of the piece to kg = 1, the upper ones to kg = 0; behind the C tile, which a faster wave may be writing
+            char* trade = g2_smem + BM * BN * (B16 ? 2 : 4) + 1024 + lane * 16;
+            auto hand = [&](int f, const f32x4_g& v) { *reinterpret_cast<f32x4_g*>(trade + ((wid ^ 1) * WM * WN + f) * 1024) = v; };
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    if (kg == 0) { hand(i * WN + j, big[WM + i][j]); acc[i][j] = big[i][j]; }
+                    else { hand(i * WN + j, big[i][j]); acc[i][j] = big[WM + i][j]; }
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] += *reinterpret_cast<const f32x4_g*>(trade + (wid * WM * WN + i * WN + j) * 1024);
+        } else {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
             for (int j = 0; j < WN; ++j) acc[i][j] = f32x4_g{0.f, 0.f, 0.f, 0.f};
-        const int w_off = packed ? lane * 16 : l15 * 64 + ((q ^ ((l15 >> 2) & 2)) << 4);
-        const int a_off0 = l15 * 128 + ((q ^ (l15 & 7)) << 4), a_off1 = l15 * 128 + (((4 + q) ^ (l15 & 7)) << 4);
         const int a_base = wr * 16 * WM * 128, w_base = RA * AH + wc * 16 * WN * 64 + w_off;
-        auto frag = [&](const char* p) { return *reinterpret_cast<const bf16x8_g*>(p); };
         bf16x8_g fa[WM - 1], fl[2], fb[2][WN];               // A's rows but the last, the last, W's
         __builtin_amdgcn_s_barrier();
         {
@@ -768,6 +860,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
 #undef GP_MFMA
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads past the last stage, before the stages become the C tile
         __builtin_amdgcn_s_barrier();
+        }
     }
 
     // rows of the tile: bf16 (ROWS: ct_off), or fp32, 64-byte group g at g ^ ((R >> 2) & 3), which is q for a lane's rows
@@ -1368,11 +1461,13 @@ static int gemmp_tile(int M, int cols, int K, int splits, int most) {
 }
 
 // The same for a product that ends in the residual epilogue with a norm (nothing of it splits along K, so few rows ask for small tiles).
-// 0: 128 x 128, 1: 128 x 64, 2: 64 x 64, two workgroups on a CU for 0 and 2
+// 0: 128 x 128, 1: 128 x 64, 2: 64 x 64, 3: 96 x 64, 4: 32 x 64; two workgroups on a CU for 0, 2 and 4.
+// Ms a prompt of Qwen3-0.6B with 1, 2, 3, 4: 450 rows - / 1.91 / 2.00 / 1.74, 600 2.28 / 2.10 / 2.15 / 2.15, 800 2.35 / 2.24 / 2.29 / 2.31, 1100 2.77 / 2.81 / 2.67 / 3.03,
+// 1531 3.07 / 3.07 / 2.99 / 3.31, 1800 3.43 / 3.63 / 3.66 / 3.99.
 static int gemmp_resid_tile(int M, int N, int K, int* cost) {
-    constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 450, 29, 640}, {128, 64, 14, 400, 0, 0}, {64, 64, 11, 300, 16, 400}};
+    constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 450, 29, 640}, {128, 64, 14, 400, 0, 0}, {64, 64, 11, 300, 16, 400}, {96, 64, 13, 350, 0, 0}, {32, 64, 8, 250, 13, 350}};
     int best = 0;
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < 5; ++i) {
         const long long n = (long long)ceil_div(M, t[i].bm) * ceil_div(N, t[i].bn), stages = K / 32;
         const long long one = stages * t[i].one + t[i].one_fixed, two = stages * t[i].two + t[i].two_fixed;
         const long long c = t[i].two ? n / 512 * two + (n % 512 > 256 ? two : n % 512 > 0 ? one : 0) : ceil_div(n, 256LL) * one;
@@ -1420,6 +1515,8 @@ pgk_status gemm128s_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void
         const int t = gemmp_resid_tile(M, N, K, &cost);
         if (t == 1) return gemmp_launch<8, 4, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
         if (t == 2) return gemmp_launch<8, 2, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        if (t == 3) return gemmp_launch<8, 3, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
+        if (t == 4) return gemmp_launch<8, 1, 2>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
         return gemmp_launch<8, 4, 4>(A, W, nullptr, C, M, N, K, kps, hd, pk, none, ni, no, st);
     }
     if (mode == 3) {
