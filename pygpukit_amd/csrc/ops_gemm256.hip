@@ -449,14 +449,12 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     wait_two_younger();
     __builtin_amdgcn_s_barrier();
     if (late) __builtin_amdgcn_s_barrier();                  // waves 4-7 start one phase behind
-#define G2S_STEP(S, BUF, L)                                                                                   \
+#define G2S_STEP(S, BUF)                                                                                     \
     {   /* phase A */                                                                                        \
         const char* As = g2_smem + a_cur + a_base + (((BUF) & 1) ? a_off1 : a_off0);                           \
         const char* Ws = g2_smem + (BUF) * HALF + w_base + w_off;                                        \
-        if (L) {                                                                                             \
-            _Pragma("unroll") for (int i = 0; i < 8; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 2048); \
-            _Pragma("unroll") for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const uint4*>(Ws + j * 1024); \
-        }                                                                                                    \
+        _Pragma("unroll") for (int i = 0; i < 8; ++i) fa[i] = *reinterpret_cast<const uint4*>(As + i * 2048); \
+        _Pragma("unroll") for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const uint4*>(Ws + j * 1024); \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
         if (((BUF) & 1) == 0) {                                                                              \
             const int a_new = a_cur >= 2 * HALF ? a_cur - 2 * HALF : a_cur + 4 * HALF;                       \
@@ -469,32 +467,23 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
         __builtin_amdgcn_s_barrier();                                                                        \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
         /* phase B */                                                                                        \
-        if (L) {                                                                                             \
         __builtin_amdgcn_s_setprio(1);                                                                       \
         _Pragma("unroll") for (int i = 0; i < 8; ++i)                                                        \
             _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                   \
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_g, ROWS ? fb[j] : fa[i]),     \
                                                                     __builtin_bit_cast(bf16x8_g, ROWS ? fa[i] : fb[j]), acc[i][j], 0, 0, 0); \
         __builtin_amdgcn_s_setprio(0);                                                                       \
-        }                                                                                                    \
         __builtin_amdgcn_sched_barrier(0);                                                                   \
         if (!late) wait_two_younger();                                                                       \
         __builtin_amdgcn_s_barrier();                                                                        \
     }
-#define G2S_LOOP(L)                                                                                          \
-    {                                                                                                        \
-        int s = 0;                                                                                           \
-        for (; s + 4 <= nh; s += 4) {                                                                        \
-            G2S_STEP(s, 0, L) G2S_STEP(s + 1, 1, L) G2S_STEP(s + 2, 2, L) G2S_STEP(s + 3, 3, L)               \
-        }                                                                                                    \
-        if (s < nh) {   /* K % 64 == 0: an even number of stages, so two remain at most */                   \
-            G2S_STEP(s, 0, L) G2S_STEP(s + 1, 1, L)                                                          \
-        }                                                                                                    \
+    int s = 0;
+    for (; s + 4 <= nh; s += 4) {
+        G2S_STEP(s, 0) G2S_STEP(s + 1, 1) G2S_STEP(s + 2, 2) G2S_STEP(s + 3, 3)
     }
-    // waves 4-7 of a last tile of at most 128 rows have none to multiply (SwiGLU of 300 rows, N = 14336, K = 4096: 94.6 us with them, 91.3 without)
-    if (EPI != 1 && late && m0 + 128 >= M) G2S_LOOP(false)
-    else G2S_LOOP(true)
-#undef G2S_LOOP
+    if (s < nh) {   // K % 64 == 0: an even number of stages, so two remain at most
+        G2S_STEP(s, 0) G2S_STEP(s + 1, 1)
+    }
 #undef G2S_STEP
     if (!late) __builtin_amdgcn_s_barrier();                 // match the extra barrier of waves 4-7
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // retire the phantom DMAs before the LDS is given back
