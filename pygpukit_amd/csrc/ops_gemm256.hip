@@ -69,8 +69,9 @@ __device__ __forceinline__ void g2_tile_of(int id, int nwg, int ntm, int ntn, in
 // ---- bf16 C tiles in LDS, for the epilogues.  Kernels with such a tile multiply W fragments by A fragments, so a lane of a 16 x 16 product holds four consecutive columns of
 // one row (row lane & 15, columns 4 (lane >> 4) .. + 4) and puts them down in one 8-byte instruction, where four rows of a column took four of 2 bytes.
 // 16-byte chunks are XOR-ed by the row so that the 16 rows of an instruction meet different banks; whole rows are read back.
-//   us a launch, the other way and this: 1531 rows, K = 1024: SwiGLU (192 x 192) 23.5 / 23.0, QKV heads (192 x 128) 20.0 / 19.5; 4096 rows, K = 4096: SwiGLU, N = 14336 714 /
-// 708, QKV stored from registers (N = 6144) 177 / 172.  fp32 tiles (16 bytes for four of 4) lost as much: += of N = 4096, K = 4096 107 / 113.
+//   us a launch, the other way and this: 1531 rows, K = 1024: SwiGLU (192 x 192) 23.5 / 23.0, QKV heads (192 x 128) 20.0 / 19.5; 256 x 192 tiles stored from registers, 4096
+// rows, K = 4096, N = 6144 177 / 172.  Not for fp32 tiles (16 bytes for four of 4; += of N = 4096, K = 4096 107 / 113), nor for the 256-row tiles that finish SwiGLU and
+// heads: there it gained 0.3..0.8 % where rows are many and lost 5 % where most of a last tile is copies of one row (N = 28672, K = 4096: 4096 rows 714 / 708, 300 rows 90 / 94.6).
 template <int ROWB> __device__ __forceinline__ int ct_off(int row, int byte) {
     static_assert(ROWB % 128 == 0, "chunks are exchanged in groups of 8, or of 16");
     const int sw = ROWB % 256 == 0 ? row & 15 : (row >> 1) & 7;
@@ -88,7 +89,7 @@ __device__ __forceinline__ uint2 ct_bf16(const f32x4_g& v) { return make_uint2(p
 // store 16 bytes of bf16, or (QOUT) 8 e4m3 codes with the row's scale for this 128-column block (absmax / 448 over the 16
 // lanes, quantize_fp8_rows' contract): exactly the fp8 x fp8 down projection's A operand.  Saves the [M][2 I] bf16 round
 // trip through HBM (Llama-3-8B shape, S = 4096: 235 MB written + read back = ~75 us of a 1.4 ms layer) and a launch.
-template <bool QOUT, int TN = 4, bool ROWS = false>   // ROWS: a lane holds columns of a row (ct_off), otherwise rows of a column; TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
+template <bool QOUT, int TN = 4>   // TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
 __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&acc)[8][TN], int tid, int m0, int tn, int M, int I,
                                                    void* outv, float* out_scales) {
     static_assert(TN == 4 || !QOUT, "the e4m3 epilogue needs whole 128-column scale blocks");
@@ -98,25 +99,19 @@ __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&a
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            if constexpr (ROWS) {
-                *reinterpret_cast<uint2*>(smem + ct_off<ROWB>(wr * 128 + i * 16 + l15, (wc * WN + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
-            } else {
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
-                    *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
-                }
+            for (int r = 0; r < 4; ++r) {
+                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
+                *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
             }
-        }
-    auto at = [&](int row, int byte) { return smem + (ROWS ? ct_off<ROWB>(row, byte) : row * ROWB + (byte ^ (((row >> 2) & 3) << 5))); };
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < 256 * CH / G2_THREADS; ++it) {
-        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH;
+        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH, sw = ((row >> 2) & 3) << 5;
         Vec<bf16> g, u;
-        g.raw = *reinterpret_cast<const uint4*>(at(row, c * 16));
-        u.raw = *reinterpret_cast<const uint4*>(at(row, ACT * 2 + c * 16));
+        g.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((c * 16) ^ sw));
+        u.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((ACT * 2 + c * 16) ^ sw));
         float gf[8], uf[8];
         g.to_float(gf);
         u.to_float(uf);
@@ -189,7 +184,6 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
 // ---- QKV-heads epilogue (EPI 3 of the fp8 kernel, 5 of the bf16 one): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
 // g2_swiglu_epilogue), a tile = 256 token rows x two head slots, 16 consecutive lanes take one (row, head) and finish it
 // (HeadRows: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
-template <bool ROWS = false>
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -200,25 +194,20 @@ __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g 
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if constexpr (ROWS) {
-                *reinterpret_cast<uint2*>(smem + ct_off<512>(wr * 128 + i * 16 + l15, (wc * 64 + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
-            } else {
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
-                    *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
-                }
+            for (int r = 0; r < 4; ++r) {
+                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
+                *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
             }
-        }
     hr.angles(c, 2 * tn, hd);
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         hr.finish(c, 2 * tn + h, m0 + r0, 32, M, hd, qkv, N, [&](int i, float (&x)[8]) {
-            const int row = i * 32 + r0, byte = h * 256 + c * 16;
+            const int row = i * 32 + r0, sw = ((row >> 2) & 3) << 5;
             Vec<bf16> raw;
-            raw.raw = *reinterpret_cast<const uint4*>(smem + (ROWS ? ct_off<512>(row, byte) : row * 512 + (byte ^ (((row >> 2) & 3) << 5))));
+            raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((h * 256 + c * 16) ^ sw));
             raw.to_float(x);
         });
 }
@@ -367,7 +356,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
     static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
-    constexpr bool ROWS = EPI != 1;                          // a lane holds columns of a row: ct_off
+    constexpr bool ROWS = EPI == 0 || EPI == 3 || EPI == 4;  // a lane holds columns of a row (ct_off says what that costs the others)
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
     const int late = __builtin_amdgcn_readfirstlane(wr);     // wave-uniform by construction: scalar branches around barriers
@@ -497,18 +486,22 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float f = inv[wr * 128 + i * 16 + l15];
+                f32x4_g f;
+                if constexpr (ROWS) {
+                    const float one = inv[wr * 128 + i * 16 + l15];
+                    f = f32x4_g{one, one, one, one};
+                } else f = *reinterpret_cast<const f32x4_g*>(inv + wr * 128 + i * 16 + q * 4);
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] *= f;
             }
         }
     }
     if constexpr (EPI == 2) {
-        g2_swiglu_epilogue<false, TN, true>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
+        g2_swiglu_epilogue<false, TN>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
         return;
     }
     if constexpr (EPI == 5) {
-        g2_qkv_heads_epilogue<true>(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
+        g2_qkv_heads_epilogue(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
         return;
     }
     if constexpr (EPI == 1 && TN == 4) {
