@@ -2041,8 +2041,8 @@ static pgk_status decode_step_impl(Engine* e, int batch, hipStream_t st, int* la
         pgk_status r;
         // the MFMA projections cost the same for 3 as for 16 sequences (~1.0-1.2 ms per step on Qwen3-0.6B); the GEMV
         // kernels exist for M = 1, 2, 4, 8 only, so 3 / 5 / 6 / 7 sequences would take two or three weight passes there
-        // (measured: 7 sequences 2.46 ms against 1.05).  GEMV stays for exactly 1, 2 and 4 (0.70 / 0.93 / 0.82 ms).
-        const bool mfma_ok = e->batched_mfma && (rem >= e->batched_min || (e->batched_min == 5 && rem == 3));
+        // (measured: 7 sequences 2.46 ms against 1.05).  GEMV stays for exactly 1 and 2, and for 4 where batched_four does not hold.
+        const bool mfma_ok = e->batched_mfma && (rem >= e->batched_min || (e->batched_min == 5 && (rem == 3 || (rem == 4 && e->batched_four))));
         if (mfma_ok) {
             const int m = rem > e->batched_max ? e->batched_max : rem;
             if (m > 16 && e->packed_decode) r = decode_chunk_packed(e, b0, m, rem == m, st, launches, short_ctx);
@@ -2611,6 +2611,11 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
                         (size_t)I * 8 <= 156 * 1024 && wide_aligned(e) && !gemv_only;
         const bool all_fixed = fixed(NQ, H) && fixed(H, QD) && fixed(I, H) && fixed(H, I);
         if (ok) e->wide = 0xE8 | (H >= 1536 || !all_fixed ? 0x10 : 0) | (H >= 1536 && !all_fixed ? 0x06 : 0);
+        // 4 sequences on the register kernels of engine_batched.hip.h, which round where the GEMV kernels of four rows do (Qwen3-0.6B, us a step at contexts to 300 and of
+        // 1500: 776 -> 693, 909 -> 824).  Not e4m3 weights, which those scale in fp32 and these round to bf16, nor K below 1024, which take the kernels by way of an LDS image
+        // (H = 512, 8 layers: 176 against 256).
+        auto deep = [](int K) { return K == 1024 || K == 2048 || K == 3072 || K == 4096; };
+        e->batched_four = !f8 && !(e->wide >> 4 & 1) && deep(H) && deep(I) && deep(QD);
     }
     if (e->wide) A((void**)&e->wide_act, wide_pieces_elems(c.intermediate_size, 7) * 2, &e->ws_bytes);
     A((void**)&e->amax_val, (size_t)B * e->lm_cap * 4, &e->ws_bytes);
