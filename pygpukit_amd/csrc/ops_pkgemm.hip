@@ -34,7 +34,6 @@ typedef float f32x4_p __attribute__((ext_vector_type(4)));
 constexpr int PK_THREADS = 256;
 constexpr int PK_MT = 2;           // m-tiles per workgroup
 constexpr int PK_MB = PK_MT * 16;  // rows per m-block
-constexpr int PK_RING = 16;        // k-steps of weights in flight per n-tile
 
 __device__ __forceinline__ void pk_dma16(const void* src, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
@@ -106,10 +105,14 @@ __device__ unsigned long long g_pk_stamps[6][512][8];
 #define PK_STAMP(i) do { } while (0)
 #endif
 
+// PK_RING = k-steps of weights in flight per n-tile: a wave's whole run of 32 where it has one n-tile of K = 1024, else 16 (two n-tiles with 32 each leave a wave 256
+// registers and were slower: QKV of 93 rows 9.3 -> 9.7 us).  A step of 64 sequences 1149 -> 1141 us, with the arguments preloaded 1107; of 24 1028 -> 1019 -> 981.
 // MT = m-tiles per workgroup: 2 (32-row m-blocks) for prompts, 1 (16 rows) for M <= 96 - decode batches, short prompts - where
 // 32-row blocks would leave CUs without a workgroup.
-template <int NTW, int EPI, int MT>
-__global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
+template <int NTW, int EPI, int MT, int PK_RING>
+__global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(const bf16* a_, const bf16* wp_, const float* ss_in_, int lda_, int M_, int K_, int ksteps_, int nblk_, int mblk_, int splits_,
+                                                             int tile_b_off_, PkArgs g) {
+    // what the load-issue phase needs, in the arguments that arrive preloaded in SGPRs (fused_gemv_kernel, engine.hip)
     constexpr int PK_MT = MT, PK_MB = 16 * MT;
     extern __shared__ __attribute__((aligned(16))) char a_lds[];   // [PK_MB][ksteps * 32] bf16, chunk-swizzled rows
     __shared__ float ssred[4][PK_MB];
@@ -121,21 +124,21 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
     // bytes in its L2.  The grid is padded to whole groups; the padding workgroups leave at once.
     int cb, mb, sp;
     {
-        const int per = 8 * g.mblk * g.splits;
+        const int per = 8 * mblk_ * splits_;
         const int grp = blockIdx.x / per, r = blockIdx.x - grp * per;
         cb = grp * 8 + (r & 7);
         int rest = r >> 3;
-        mb = rest % g.mblk;
-        sp = rest / g.mblk;
-        if (cb >= g.nblk) return;
+        mb = rest % mblk_;
+        sp = rest / mblk_;
+        if (cb >= nblk_) return;
     }
     const int m0 = mb * PK_MB;
-    const int ks0 = sp * g.ksteps, KS = g.ksteps, ksn = g.K / 32;
+    const int ks0 = sp * ksteps_, KS = ksteps_, ksn = K_ / 32;
     const int rb = KS * 64;                                   // bytes per LDS row
-    const int tile_a = cb * g.tiles_per_cb + wid;
+    const int tile_a = cb * (EPI == PK_EPI_QKV ? 8 : 4) + wid;
     const bf16* wrun[NTW];
-    wrun[0] = g.wp + ((size_t)tile_a * ksn + ks0) * 512 + lane * 8;
-    if constexpr (NTW == 2) wrun[1] = g.wp + ((size_t)(tile_a + g.tile_b_off) * ksn + ks0) * 512 + lane * 8;
+    wrun[0] = wp_ + ((size_t)tile_a * ksn + ks0) * 512 + lane * 8;
+    if constexpr (NTW == 2) wrun[1] = wp_ + ((size_t)(tile_a + tile_b_off_) * ksn + ks0) * 512 + lane * 8;
 
     // head epilogue: the m-block's RoPE rows (32 positions x 64 floats, cos and sin) go to LDS by 16 DMA instructions and
     // the gammas are requested first of all (first in = first out).  (Per-lane loads of the 16 entries a lane needs were
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
             constexpr int IPT = PK_MB / 4;                    // instructions per table: 4 rows each
             for (int j = wid; j < 2 * IPT; j += 4) {           // instruction j: table j / IPT, rows 4 (j % IPT) + q, 16 bytes per lane
                 const int row = 4 * (j % IPT) + q;
-                const int pos = min(g.start_pos + min(m0 + row, g.M - 1), g.max_seq - 1);
+                const int pos = min(g.start_pos + min(m0 + row, M_ - 1), g.max_seq - 1);
                 pk_dma16(((j / IPT) ? g.rope_sin : g.rope_cos) + (size_t)pos * 64 + 4 * l15, r0 + j * 1024);
             }
         }
@@ -167,15 +170,15 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
     // rows that arrive un-normalised (pkgemm_resid_nt): 1 / rms of this m-block's rows from the producer's partial sums,
     // 8 threads per row; visible to everyone after the barrier that follows the DMA wait
     __shared__ float inv_lds[PK_MB];
-    const bool scaled = g.ss_in != nullptr;
+    const bool scaled = ss_in_ != nullptr;
     // The row statistics are requested here and reduced only after this wave's DMAs and weight ring are issued (reducing on
     // the spot held those back by an L2 round trip).  Unconditional load, valid dummy address when there is nothing to scale:
     // under a branch the compiler completes the loaded values before the join - the same wait.
     float4 ssu, ssv;
     {
         const int row = threadIdx.x >> 3, sub = threadIdx.x & 7;
-        const float* sp = scaled ? g.ss_in + (size_t)min(m0 + min(row, PK_MB - 1), g.M - 1) * PK_SS_LD + 8 * sub   // a row's PK_SS_LD floats: 8 per thread
-                                 : reinterpret_cast<const float*>(g.wp) + 8 * sub;
+        const float* sp = scaled ? ss_in_ + (size_t)min(m0 + min(row, PK_MB - 1), M_ - 1) * PK_SS_LD + 8 * sub   // a row's PK_SS_LD floats: 8 per thread
+                                 : reinterpret_cast<const float*>(wp_) + 8 * sub;
         ssu = *reinterpret_cast<const float4*>(sp);
         ssv = *reinterpret_cast<const float4*>(sp + 4);
     }
@@ -186,12 +189,12 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
         const uint32_t lds0 = pk_lds_addr(a_lds);
         const int ndma = PK_MB * rb / 1024, gpr = KS >> 2;
         const uint32_t magic = (65536u + gpr - 1) / gpr;
-        const bf16* abase = g.a + (size_t)ks0 * 32;
+        const bf16* abase = a_ + (size_t)ks0 * 32;
         for (int j = wid; j < ndma; j += 4) {
             const int grp = 4 * j + q;
             const int row = (int)(((uint32_t)grp * magic) >> 16), gi = grp - row * gpr;
             const int c = gi * 16 + ((l15 ^ row) & 15);
-            pk_dma16(abase + (size_t)min(m0 + row, g.M - 1) * g.lda + c * 8, lds0 + j * 1024);
+            pk_dma16(abase + (size_t)min(m0 + row, M_ - 1) * lda_ + c * 8, lds0 + j * 1024);
         }
     }
     // weight ring: exactly NTW * PK_RING loads behind the DMAs (clamped k-step: the explicit wait below counts them)
@@ -207,11 +210,10 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) ssum += (8 * sub + i < g.ss_n) ? p8[i] : 0.f;
         ssum = group8_sum(ssum);
-        if (sub == 0 && row < PK_MB) inv_lds[row] = 1.0f / sqrtf(ssum / (float)g.K + g.ss_eps);
+        if (sub == 0 && row < PK_MB) inv_lds[row] = 1.0f / sqrtf(ssum / (float)K_ + g.ss_eps);
     }
     PK_STAMP(1);
-    if constexpr (NTW == 2) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");   // in-order return: every DMA has landed
-    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING < 63 ? NTW * PK_RING : 63) : "memory");   // in-order return: every DMA has landed
     __syncthreads();
     PK_STAMP(2);
 
@@ -289,20 +291,20 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
     if constexpr (EPI == PK_EPI_BF16 || EPI == PK_EPI_XIELU || EPI == PK_EPI_GELU || EPI == PK_EPI_SLAB || EPI == PK_EPI_ACCUM) {
 #pragma unroll
         for (int t = 0; t < NTW; ++t) {
-            const int n = (tile_a + t * g.tile_b_off) * 16 + l15;
+            const int n = (tile_a + t * tile_b_off_) * 16 + l15;
             if constexpr (EPI == PK_EPI_ACCUM) {
                 float* c = reinterpret_cast<float*>(g.c);
                 float old[PK_MT][4];
 #pragma unroll
                 for (int mt = 0; mt < PK_MT; ++mt)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) old[mt][r] = c[(size_t)min(m0 + mt * 16 + 4 * q + r, g.M - 1) * g.ldc + n];
+                    for (int r = 0; r < 4; ++r) old[mt][r] = c[(size_t)min(m0 + mt * 16 + 4 * q + r, M_ - 1) * g.ldc + n];
 #pragma unroll
                 for (int mt = 0; mt < PK_MT; ++mt)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int m = m0 + mt * 16 + 4 * q + r;
-                        if (m < g.M) c[(size_t)m * g.ldc + n] = old[mt][r] + acc[t][mt][r];
+                        if (m < M_) c[(size_t)m * g.ldc + n] = old[mt][r] + acc[t][mt][r];
                     }
             } else {
 #pragma unroll
@@ -310,11 +312,11 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int m = m0 + mt * 16 + 4 * q + r;
-                        if (m < g.M) {
+                        if (m < M_) {
                             if constexpr (EPI == PK_EPI_BF16) reinterpret_cast<bf16*>(g.c)[(size_t)m * g.ldc + n] = from_f<bf16>(acc[t][mt][r]);
                             else if constexpr (EPI == PK_EPI_XIELU) reinterpret_cast<bf16*>(g.c)[(size_t)m * g.ldc + n] = from_f<bf16>(xielu<false>(acc[t][mt][r], g.act_pos, g.act_neg));
                             else if constexpr (EPI == PK_EPI_GELU) reinterpret_cast<bf16*>(g.c)[(size_t)m * g.ldc + n] = from_f<bf16>(gelu_erf(acc[t][mt][r]));
-                            else (reinterpret_cast<float*>(g.c) + (size_t)sp * g.M * g.ldc)[(size_t)m * g.ldc + n] = acc[t][mt][r];
+                            else (reinterpret_cast<float*>(g.c) + (size_t)sp * M_ * g.ldc)[(size_t)m * g.ldc + n] = acc[t][mt][r];
                         }
                     }
             }
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + mt * 16 + 4 * q + r;
                 const float gf = to_f(from_f<bf16>(acc[0][mt][r])), uf = to_f(from_f<bf16>(acc[1][mt][r]));
-                if (m < g.M) c[(size_t)m * g.ldc + n] = from_f<bf16>(gf / (1.0f + __expf(-gf)) * uf);
+                if (m < M_) c[(size_t)m * g.ldc + n] = from_f<bf16>(gf / (1.0f + __expf(-gf)) * uf);
             }
     } else {
         // one head of 128: lane holds dims d = 16 wid + l15 (tile 0) and d + 64 (tile 1) of rows m
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(PkArgs g) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + mt * 16 + 4 * q + r;
-                if (m >= g.M) continue;
+                if (m >= M_) continue;
                 if (is_q) {
                     bf16* dst = reinterpret_cast<bf16*>(g.c) + (size_t)m * g.ldc + (size_t)cb * 128;
                     dst[d] = from_f<bf16>(x0[mt][r]);
@@ -427,8 +429,8 @@ struct PkResidArgs {
     float* ss_out;
 };
 
-template <int MB, int NTW>
-__global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(PkResidArgs g) {
+template <int MB, int NTW, int PK_RING>
+__global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(const bf16* a_, const bf16* wp_, float* h_, const bf16* gamma_next_, int lda_, int M_, int N_, int K_, int mblk_, PkResidArgs g) {
     constexpr int MT = MB / 16, NC = 16 * NTW;
     constexpr int EPT = MB * NC / PK_THREADS;                       // output elements per thread (1 or 2)
     static_assert(MB * NC == 512 || MB * NC == 256, "one workgroup owns 32 x 16, 16 x 32 or 16 x 16 outputs");
@@ -438,14 +440,14 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(PkResidArgs g)
     const int l15 = lane & 15, q = lane >> 4;
     int cb, mb;
     {
-        const int per = 8 * g.mblk;
+        const int per = 8 * mblk_;
         const int grp = blockIdx.x / per, r = blockIdx.x - grp * per;
         cb = grp * 8 + (r & 7);
         mb = r >> 3;
-        if (cb >= g.nblk) return;
+        if (cb >= N_ / NC) return;
     }
     const int m0 = mb * MB, n0 = cb * NC;
-    const int KS = g.K / 32, KSW = KS / 4, ksw0 = wid * KSW;       // this wave's k-steps
+    const int KS = K_ / 32, KSW = KS / 4, ksw0 = wid * KSW;       // this wave's k-steps
     const int rb = KS * 64;
     // the residual values of this thread's outputs first: they are needed last, and first in = first out
     float hold[EPT];
@@ -454,13 +456,13 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(PkResidArgs g)
     for (int i = 0; i < EPT; ++i) {
         const int e = threadIdx.x + PK_THREADS * i;
         em[i] = e / NC; en[i] = e % NC;
-        hold[i] = g.h[(size_t)min(m0 + em[i], g.M - 1) * g.N + n0 + en[i]];
+        hold[i] = h_[(size_t)min(m0 + em[i], M_ - 1) * N_ + n0 + en[i]];
     }
     // (unconditional loads, converted where they are used: under a branch the compiler waits for them right here - two
     // serialised L2 round trips in front of every DMA of the kernel in the first version)
     uint16_t gnb[EPT];
     {
-        const bf16* gsafe = g.gamma_next ? g.gamma_next + n0 : g.a;
+        const bf16* gsafe = gamma_next_ ? gamma_next_ + n0 : a_;
 #pragma unroll
         for (int i = 0; i < EPT; ++i) gnb[i] = gsafe[en[i]].bits;
     }
@@ -472,20 +474,19 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(PkResidArgs g)
             const int grp = 4 * j + q;
             const int row = (int)(((uint32_t)grp * magic) >> 16), gi = grp - row * gpr;
             const int c = gi * 16 + ((l15 ^ row) & 15);
-            pk_dma16(g.a + (size_t)min(m0 + row, g.M - 1) * g.lda + c * 8, lds0 + j * 1024);
+            pk_dma16(a_ + (size_t)min(m0 + row, M_ - 1) * lda_ + c * 8, lds0 + j * 1024);
         }
     }
     const int ksn = KS;
     const bf16* wrun[NTW];
 #pragma unroll
-    for (int t = 0; t < NTW; ++t) wrun[t] = g.wp + ((size_t)(cb * NTW + t) * ksn + ksw0) * 512 + lane * 8;
+    for (int t = 0; t < NTW; ++t) wrun[t] = wp_ + ((size_t)(cb * NTW + t) * ksn + ksw0) * 512 + lane * 8;
     uint4 wr[NTW][PK_RING];
 #pragma unroll
     for (int s = 0; s < PK_RING; ++s)
 #pragma unroll
         for (int t = 0; t < NTW; ++t) wr[t][s] = *reinterpret_cast<const uint4*>(wrun[t] + (size_t)min(s, KSW - 1) * 512);
-    if constexpr (NTW == 2) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING < 63 ? NTW * PK_RING : 63) : "memory");
     __syncthreads();
 
     f32x4_p acc[NTW][MT];
@@ -556,10 +557,10 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(PkResidArgs g)
         const int idx = ((((n >> 4) * MT + (m >> 4)) * 64) + 16 * ((m & 15) >> 2) + (n & 15)) * 4 + (m & 3);
         float v = hold[i];
         v += (kp[idx] + kp[idx + NTW * MT * 256]) + (kp[idx + 2 * NTW * MT * 256] + kp[idx + 3 * NTW * MT * 256]);
-        const bool ok = m0 + m < g.M;
-        if (ok) g.h[(size_t)(m0 + m) * g.N + n0 + n] = v;
-        if (g.gamma_next) {
-            if (ok) g.xpre[(size_t)(m0 + m) * g.N + n0 + n] = from_f<bf16>(v * bf16_bits_to_f(gnb[i]));
+        const bool ok = m0 + m < M_;
+        if (ok) h_[(size_t)(m0 + m) * N_ + n0 + n] = v;
+        if (gamma_next_) {
+            if (ok) g.xpre[(size_t)(m0 + m) * N_ + n0 + n] = from_f<bf16>(v * bf16_bits_to_f(gnb[i]));
             const float sq = group_sum<NC>(v * v);                 // the NC threads of a row are consecutive lanes
             if (n == 0 && ok) g.ss_out[(size_t)(m0 + m) * PK_SS_LD + cb] = sq;
         }
@@ -583,17 +584,18 @@ pgk_status pkgemm_resid_nt(const bf16* a, int lda, const void* wp, float* h, int
     if (ss_n) *ss_n = g.nblk;
     const size_t lds = (size_t)mb * (K / 32) * 64;
     const int grid = ceil_div(g.nblk, 8) * 8 * g.mblk;
-#define PGK_PKR_LAUNCH(MBV, NTWV)                                                                                  \
+#define PGK_PKR_LAUNCH(MBV, NTWV, RINGV)                                                                                  \
     {                                                                                                              \
         static bool attr = false;                                                                                  \
         if (lds > 48 * 1024 && !attr) {                                                                            \
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_resid_kernel<MBV, NTWV>),       \
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_resid_kernel<MBV, NTWV, RINGV>),       \
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));     \
             attr = true;                                                                                           \
         }                                                                                                          \
-        pkgemm_resid_kernel<MBV, NTWV><<<grid, PK_THREADS, lds, st>>>(g);                                          \
+        pkgemm_resid_kernel<MBV, NTWV, RINGV><<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.h, g.gamma_next, g.lda, g.M, g.N, g.K, g.mblk, g);                                          \
     }
-    if (small) PGK_PKR_LAUNCH(16, 1) else if (wide) PGK_PKR_LAUNCH(32, 1) else PGK_PKR_LAUNCH(16, 2)
+    const bool deep = K / 128 == 24;      // all 24 k-steps of a wave's quarter in flight
+    if (small && deep) PGK_PKR_LAUNCH(16, 1, 24) else if (small) PGK_PKR_LAUNCH(16, 1, 16) else if (wide && deep) PGK_PKR_LAUNCH(32, 1, 24) else if (wide) PGK_PKR_LAUNCH(32, 1, 16) else PGK_PKR_LAUNCH(16, 2, 16)
 #undef PGK_PKR_LAUNCH
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
@@ -650,18 +652,20 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
     const size_t lds = (size_t)16 * mt * g.ksteps * 64;
     PGK_REQUIRE(lds <= 128 * 1024, "pkgemm: K per workgroup %d too long for the LDS activation block", g.ksteps * 32);
     const int grid = ceil_div(g.nblk, 8) * 8 * g.mblk * splits;     // whole groups of 8 n-blocks (see the id mapping in the kernel)
-#define PGK_PK_LAUNCH2(NTWV, EPIV, MTV)                                                                            \
+#define PGK_PK_LAUNCH3(NTWV, EPIV, MTV, RINGV)                                                                            \
     {                                                                                                              \
         static size_t attr = 0;                                                                                    \
         if (lds > 48 * 1024 && lds > attr) {                                                                       \
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_kernel<NTWV, EPIV, MTV>),       \
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_kernel<NTWV, EPIV, MTV, RINGV>),       \
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));     \
             attr = 128 * 1024;                                                                                     \
         }                                                                                                          \
-        pkgemm_kernel<NTWV, EPIV, MTV><<<grid, PK_THREADS, lds, st>>>(g);                                          \
+        pkgemm_kernel<NTWV, EPIV, MTV, RINGV><<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.ss_in, g.lda, g.M, g.K, g.ksteps, g.nblk, g.mblk, g.splits, g.tile_b_off, g);                                          \
     }
+#define PGK_PK_LAUNCH2(NTWV, EPIV, MTV)                                                                           \
+    if (NTWV == 1 && g.ksteps == 32) PGK_PK_LAUNCH3(NTWV, EPIV, MTV, 32) else PGK_PK_LAUNCH3(NTWV, EPIV, MTV, 16)
 #define PGK_PK_LAUNCH(NTWV, EPIV)                                                                                  \
-    if (mt == 1) PGK_PK_LAUNCH2(NTWV, EPIV, 1) else PGK_PK_LAUNCH2(NTWV, EPIV, 2)
+    if (mt == 1) { PGK_PK_LAUNCH2(NTWV, EPIV, 1) } else { PGK_PK_LAUNCH2(NTWV, EPIV, 2) }
     switch (epi) {
         case PK_EPI_BF16: PGK_PK_LAUNCH(1, PK_EPI_BF16) break;
         case PK_EPI_XIELU: PGK_PK_LAUNCH(1, PK_EPI_XIELU) break;
@@ -672,6 +676,7 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
         case PK_EPI_QKV: PGK_PK_LAUNCH(2, PK_EPI_QKV) break;
         default: return set_error(PGK_ERR_INVALID, "pkgemm: unknown epilogue %d", epi);
     }
+#undef PGK_PK_LAUNCH3
 #undef PGK_PK_LAUNCH2
 #undef PGK_PK_LAUNCH
     PGK_CHECK_HIP(hipGetLastError());
