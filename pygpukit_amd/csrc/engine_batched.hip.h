@@ -295,11 +295,13 @@ __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl
         }
     };
     const int em = tid >> 4, en = tid & 15;
-    float res0 = 0.f;                                      // of the first group
-    if constexpr (EPI == EPI_RESID) res0 = a.res[(size_t)min(em, M - 1) * a.ld_out + min((int)blockIdx.x * RPG + en, N - 1)];
+    float res0 = 0.f;                                      // of the first group; behind the weights, since its address waits for the arguments that are not preloaded
+    auto load_res = [&]() {
+        if constexpr (EPI == EPI_RESID) res0 = a.res[(size_t)min(em, M - 1) * a.ld_out + min((int)blockIdx.x * RPG + en, N - 1)];
+    };
 
     // ---- activation fragments of this wave's K quarter ----
-    // Issue order = arrival order: rows, gamma and residual (L2) are requested BEFORE the weight stream (HBM), so the RMSNorm
+    // Issue order = arrival order: rows and gamma (L2) are requested BEFORE the weight stream (HBM), so the RMSNorm
     // statistic, its barrier and the bf16 conversion run while the weights are still in flight (the other way round the
     // prologue started when the last weight byte had landed - the batch-1 kernels' lesson).
     uint4 af[S];
@@ -342,6 +344,7 @@ __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl
         }
         __builtin_amdgcn_sched_barrier(0);
         load_w(blockIdx.x * RPG);
+        load_res();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
@@ -400,6 +403,7 @@ __global__ __launch_bounds__(256) void batched_reg_kernel(unsigned long long* tl
             for (int i = 0; i < MR / 2; ++i) r[c][i] = *reinterpret_cast<const u32x4*>(src + (size_t)min(2 * i + (lane >> 5), M - 1) * K + 256 * c);
         __builtin_amdgcn_sched_barrier(0);
         load_w(blockIdx.x * RPG);
+        load_res();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {

@@ -1012,11 +1012,12 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
     }
 }
+// The arguments up to `packed` are what the first DMA waits for: 13 dwords, preloaded into SGPRs (engine.hip, fused_gemv_kernel).
 // (up to 128 x 128: two workgroups a CU, at most 80 KiB of LDS and 128 registers each - but for 128 x 64, whose ring of six takes 88 KiB; the larger ones have a CU to
 // themselves)
 template <int EPI, int WM, int WN>
-__global__ __launch_bounds__(GP_THREADS, WM * WN <= 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
-                                                                       int M, int N, int K, int ntm, int ntn, int kps, QkvHeadArgs hd, int packed, ActArgs xa, NormIn ni, NormOut no, BestOut bo) {
+__global__ __launch_bounds__(GP_THREADS, WM * WN <= 16 ? 4 : 2) void gemmp_bf16_kernel(const bf16* A, const bf16* W, void* Cv, int M, int N, int K, int ntm, int ntn, int kps, int packed,
+                                                                       const bf16* bias, QkvHeadArgs hd, ActArgs xa, NormIn ni, NormOut no, BestOut bo) {
     gemmp_body<EPI, false, WM, WN>(A, W, bias, Cv, M, N, K, ntm, ntn, kps, hd, packed, xa, GroupArgs{}, ni, no, bo);
 }
 template <int EPI>
@@ -1418,7 +1419,7 @@ static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, v
         attr_done = true;
     }
     const int ntm = ceil_div(M, 32 * WM), ntn = EPI == 4 ? ceil_div(N, 16 * WN) : ceil_div(N, 32 * WN);      // SwiGLU: N = I act columns, half a tile's
-    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, kps, hd, packed, xa, ni, no, bo);
+    gemmp_bf16_kernel<EPI, WM, WN><<<dim3(ntm * ntn, ceil_div(K, kps)), GP_THREADS, LDS, st>>>(A, W, C, M, N, K, ntm, ntn, kps, packed, bias, hd, xa, ni, no, bo);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
