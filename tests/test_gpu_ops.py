@@ -800,6 +800,14 @@ def test_sdpa_runs_of_any_count(cfg):
     test_sdpa_few_rows_over_a_long_context("bfloat16", cfg)
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(16, 8, 1531, 1531, 128), (8, 4, 900, 900, 128), (1, 1, 1024, 1024, 64), (2, 1, 2560, 2560, 128), (4, 2, 384, 3585, 64), (1, 1, 200, 4296, 128),
+                                 (1, 1, 100, 4000, 128)])
+def test_sdpa_merges_of_two_to_sixteen_runs(dt, cfg):
+    """2, 3 (fp32 rows), 4 (fp32), 11, 14, 16 and 15 (fp32) runs on a card of 256 CUs: every size of flash_merge_kernel, full and with runs to spare."""
+    test_sdpa_few_rows_over_a_long_context(dt, cfg)
+
+
 @pytest.mark.parametrize("ql", [42, 200])
 def test_sdpa_scratch_belongs_to_the_stream_the_call_names(ql):
     """A call on an explicit stream, other than the current one: its partial rows are not handed to the current stream while the kernels that
