@@ -193,28 +193,26 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(const T* q, const T*
 typedef short sa_v4s __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int sa_voff(int row, int ch) { return row * 256 + ((ch ^ (((row & 3) << 2) | ((row >> 2) & 3))) << 4); }
 
+// Some 2 us of work behind a launch, all of it waiting: what the loads need is 13 dwords, preloaded into SGPRs (lens: q_len << 16 | kv_len), the head of
+// the keys is a grid axis instead of a division, the queries come by LDS-DMA too (as registers their wait is the compiler's, who does not count the
+// DMAs, and it would be for everything), and the scores start when the keys are there, with the values still on their way.  Qwen3-0.6B, whole model, us,
+// before and after: 33 rows 1018 / 1000, 93 1112 / 1100, 128 1147 / 1136.
 template <int NW>
-__global__ __launch_bounds__(64 * NW) void attn_short_kernel(const bf16* q, const bf16* k, const bf16* v, bf16* out, int hq, int hkv,
-                                                             int q_len, int kv_len, float scale, AttnStrides sd, const bf16* gate = nullptr,
-                                                             long long gs = 0) {      // gate: see attn_short_gated
+__global__ __launch_bounds__(64 * NW) void attn_short_kernel(const bf16* q, const bf16* k, const bf16* v, long long qh_s, long long kh_s, int qs, int ks_s, int lens, int rep,
+                                                             bf16* out, float scale, long long oh, long long os, const bf16* gate, long long gs) {   // gate: see attn_short_gated
     constexpr int D = 128, NT = 8;
     __shared__ __attribute__((aligned(16))) char k_lds[128 * 256];
     __shared__ __attribute__((aligned(16))) char v_lds[128 * 256];
+    __shared__ __attribute__((aligned(16))) char q_lds[NW][16 * 256];
+    const int q_len = lens >> 16, kv_len = lens & 0xFFFF;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, q4 = lane >> 4;
-    const int head = blockIdx.y, kvh = head / (hq / hkv);
+    const int kvh = blockIdx.z, head = kvh * rep + blockIdx.y;
     const int qb0 = blockIdx.x * (16 * NW), q0 = qb0 + wid * 16;
     const int causal_off = kv_len - q_len;
-    const bf16* qh = q + (size_t)head * sd.qh;
-    const bf16* kh = k + (size_t)kvh * sd.kh;
-    const bf16* vh = v + (size_t)kvh * sd.kh;
-    // query fragments first (the B operand of S^T): row l15 of this wave's tile, dims 32 ks + 8 q4 .. + 8
-    uint4 qf[4];
+    const bf16* qh = q + (size_t)head * qh_s;
+    const bf16* kh = k + (size_t)kvh * kh_s;
+    const bf16* vh = v + (size_t)kvh * kh_s;
     const int qrow = q0 + l15;
-    {
-        const bf16* qp = qh + (size_t)min(qrow, q_len - 1) * sd.qs + 8 * q4;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) qf[ks] = *reinterpret_cast<const uint4*>(qp + 32 * ks);
-    }
     // positions this workgroup can see, in whole 32-position steps (rows past kv_len come from a clamped address and are masked).
     // Staging is LDS-DMA: one instruction moves 4 rows x 256 bytes, lane i -> row 4 j + (i >> 4), chunk POSITION i & 15, and
     // the swizzle of each image is applied on the source side (both are XORs of the chunk index: involutions).  A loop of
@@ -228,18 +226,33 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const bf16* q, cons
         auto dma = [](const void* src, uint32_t lds_addr) {
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
         };
+        const uint32_t q0_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)&q_lds[wid][0];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {                      // this wave's 16 query rows
+            const int r = 4 * j + q4;
+            dma(qh + (long long)min(q0 + r, q_len - 1) * qs + ((l15 ^ r) << 3), q0_lds + j * 1024);
+        }
         const int ninst = nstep * 8;                       // 4 rows each
         for (int j = wid; j < ninst; j += NW) {
             const int r = 4 * j + q4;
-            dma(kh + (size_t)min(r, kv_len - 1) * sd.ks + ((l15 ^ (r & 15)) << 3), k0 + j * 1024);
+            dma(kh + (long long)min(r, kv_len - 1) * ks_s + ((l15 ^ (r & 15)) << 3), k0 + j * 1024);
         }
         for (int j = wid; j < ninst; j += NW) {
             const int r = 4 * j + q4;
-            dma(vh + (size_t)min(r, kv_len - 1) * sd.ks + ((l15 ^ (((r & 3) << 2) | ((r >> 2) & 3))) << 3), v0 + j * 1024);
+            dma(vh + (long long)min(r, kv_len - 1) * ks_s + ((l15 ^ (((r & 3) << 2) | ((r >> 2) & 3))) << 3), v0 + j * 1024);
         }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's DMAs (and its query fragments); the barrier makes the images everyone's
-    __syncthreads();
+    // this wave's queries and keys: all but the values' 8 nstep / NW instructions; the barrier makes the keys everyone's
+    static_assert(8 % NW == 0, "the same number of instructions to every wave");
+    if (nstep == 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(32 / NW) : "memory");
+    else if (nstep == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(24 / NW) : "memory");
+    else if (nstep == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(16 / NW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 / NW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    uint4 qf[4];                                           // the B operand of S^T: row l15 of this wave's tile, dims 32 ks + 8 q4 .. + 8
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[ks] = *reinterpret_cast<const uint4*>(&q_lds[wid][0] + tD_off<D>(l15, ks * 4 + q4));
     // this wave's own horizon (wave-uniform): tiles of 16 positions it needs
     const int my_need = min(kv_len, causal_off + min(q0 + 16, q_len));
     const int my_steps = (my_need + 31) >> 5;
@@ -282,6 +295,9 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const bf16* q, cons
     }
     ls += __shfl_xor(ls, 16, 64);
     ls += __shfl_xor(ls, 32, 64);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the values
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     // O^T[d][q] += V^T[d][kv] P^T[kv][q] over steps of 32 positions; lane (l15, q4) of the A operand supplies the address of
     // row (l15 >> 2) of its 16-lane group's 4 x 16 block, columns 4 (l15 & 3) .. + 4
     f32x4_t o[D / 16];
@@ -306,7 +322,7 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const bf16* q, cons
     if (qrow < q_len) {
         float inv = ls > 0.f ? 1.f / ls : 0.f;
         if (gate) inv /= 1.0f + __expf(-to_f(gate[(long long)qrow * gs + head]));
-        bf16* op = out + (size_t)head * sd.oh + (size_t)qrow * sd.os + 4 * q4;
+        bf16* op = out + (size_t)head * oh + (size_t)qrow * os + 4 * q4;
 #pragma unroll
         for (int i = 0; i < D / 16; ++i) {
             uint2 w;
@@ -409,15 +425,24 @@ static pgk_status launch_prefill(const T* q, const T* k, const T* v, T* out, int
     return PGK_OK;
 }
 
+static bool attn_short_ok(int hq, int hkv, const AttnStrides& sd) {       // what goes to the kernel in 32 bits
+    return sd.qs == (int)sd.qs && sd.ks == (int)sd.ks && hq % hkv == 0;
+}
+static pgk_status launch_attn_short(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, float scale, const AttnStrides& sd,
+                                    const void* gate, long long gs, hipStream_t st) {
+    attn_short_kernel<2><<<dim3(ceil_div(q_len, 32), hq / hkv, hkv), 128, 0, st>>>((const bf16*)q, (const bf16*)k, (const bf16*)v, sd.qh, sd.kh, (int)sd.qs, (int)sd.ks,
+                                                                                 q_len << 16 | kv_len, hq / hkv, (bf16*)out, scale, sd.oh, sd.os, (const bf16*)gate, gs);
+    PGK_CHECK_HIP(hipGetLastError());
+    return PGK_OK;
+}
+
 // attn_short_kernel with a gate per (query row, head): the head's output row times sigmoid(gate[row * gs + head]) (null: none)
 pgk_status attn_short_gated(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, float scale, const WindowStrides& w,
                             const void* gate, long long gs, hipStream_t st) {
     PGK_REQUIRE(kv_len <= 128 && kv_len >= q_len && w.kh == w.vh && w.ks == w.vs, "attn_short_gated: q_len=%d kv_len=%d", q_len, kv_len);
     const AttnStrides sd{w.qh, w.qs, w.kh, w.ks, w.oh, w.os};
-    attn_short_kernel<2><<<dim3(ceil_div(q_len, 32), hq), 128, 0, st>>>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv, q_len, kv_len, scale, sd,
-                                                                      (const bf16*)gate, gs);
-    PGK_CHECK_HIP(hipGetLastError());
-    return PGK_OK;
+    PGK_REQUIRE(attn_short_ok(hq, hkv, sd), "attn_short_gated: %d heads over %d, rows %lld and %lld apart", hq, hkv, w.qs, w.ks);
+    return launch_attn_short(q, k, v, out, hq, hkv, q_len, kv_len, scale, sd, gate, gs, st);
 }
 
 pgk_status flash_prefill(const void* q, const void* k, const void* v, void* out, int hq, int hkv, int q_len, int kv_len, int d,
@@ -458,12 +483,7 @@ static pgk_status sdpa_dispatch(const void* q, const void* k, const void* v, voi
                                  std::is_same<T, f16>::value ? 1 : 0, st);
         if constexpr (std::is_same<T, bf16>::value) {
             // the whole context in one tile (attn_short_kernel)
-            if (gen2_ok && d == 128 && kv_len <= 128) {
-                attn_short_kernel<2><<<dim3(ceil_div(q_len, 32), hq), 128, 0, st>>>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, hq, hkv,
-                                                                                  q_len, kv_len, scale, sd);
-                PGK_CHECK_HIP(hipGetLastError());
-                return PGK_OK;
-            }
+            if (gen2_ok && d == 128 && kv_len <= 128 && attn_short_ok(hq, hkv, sd)) return launch_attn_short(q, k, v, out, hq, hkv, q_len, kv_len, scale, sd, nullptr, 0, st);
         }
         if (mfma_ok) {
             if (d == 128) return launch_prefill<T, 128>((const T*)q, (const T*)k, (const T*)v, (T*)out, hq, hkv, q_len, kv_len, scale, sd, st);

@@ -303,7 +303,8 @@ pgk_status window_attention(const void* q, const void* k, const void* v, void* o
                        sd.qs % 8 == 0 && sd.qh % 8 == 0 && sd.ks % 8 == 0 && sd.kh % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 7u) == 0 && sd.os % 4 == 0 && sd.oh % 4 == 0 &&
                        (!gate.gc || (gate.gc == 1 && gate.gs % 4 == 0 && gate.gh % 4 == 0 && (reinterpret_cast<uintptr_t>(gate.p) & 7u) == 0));
     // the whole context in one tile and inside every query's window
-    if (flash && dk == 128 && kv_len <= 128 && window >= kv_len && !slopes && !gate.gc && (!gate.p || gate.gh == 1)) return attn_short_gated(q, k, v, out, hq, hkv, q_len, kv_len, scale, sd, gate.p, gate.gs, st);
+    if (flash && dk == 128 && kv_len <= 128 && window >= kv_len && !slopes && !gate.gc && (!gate.p || gate.gh == 1) && sd.qs == (int)sd.qs && sd.ks == (int)sd.ks)
+        return attn_short_gated(q, k, v, out, hq, hkv, q_len, kv_len, scale, sd, gate.p, gate.gs, st);
     if (flash) return flash_window(q, k, v, out, hq, hkv, q_len, kv_len, dk, scale, window, gate, slopes, sd.qh, sd.qs, sd.kh, sd.ks, sd.oh, sd.os, st);
     const size_t lds = ((size_t)dk + 4 * (size_t)dv + 4 * 64 + 8) * 4;
     PGK_REQUIRE(lds <= 64 * 1024, "window_attention: head widths %d / %d do not fit LDS", dk, dv);
