@@ -70,8 +70,8 @@ __device__ __forceinline__ void g2_tile_of(int id, int nwg, int ntm, int ntn, in
 // one row (row lane & 15, columns 4 (lane >> 4) .. + 4) and puts them down in one 8-byte instruction, where four rows of a column took four of 2 bytes.
 // 16-byte chunks are XOR-ed by the row so that the 16 rows of an instruction meet different banks; whole rows are read back.
 //   us a launch, the other way and this: 1531 rows, K = 1024: SwiGLU (192 x 192) 23.5 / 23.0, QKV heads (192 x 128) 20.0 / 19.5; 256 x 192 tiles stored from registers, 4096
-// rows, K = 4096, N = 6144 177 / 172.  Not for fp32 tiles (16 bytes for four of 4; += of N = 4096, K = 4096 107 / 113), nor for the 256-row tiles that finish SwiGLU and
-// heads: there it gained 0.3..0.8 % where rows are many and lost 5 % where most of a last tile is copies of one row (N = 28672, K = 4096: 4096 rows 714 / 708, 300 rows 90 / 94.6).
+// rows, K = 4096, N = 6144 177 / 172.  Not for fp32 tiles (16 bytes for four of 4; += of N = 4096, K = 4096 107 / 113); and in the 256-row tiles that finish SwiGLU and
+// heads where few of their rows are padding (gemm256_rows).
 template <int ROWB> __device__ __forceinline__ int ct_off(int row, int byte) {
     static_assert(ROWB % 128 == 0, "chunks are exchanged in groups of 8, or of 16");
     const int sw = ROWB % 256 == 0 ? row & 15 : (row >> 1) & 7;
@@ -89,7 +89,7 @@ __device__ __forceinline__ uint2 ct_bf16(const f32x4_g& v) { return make_uint2(p
 // store 16 bytes of bf16, or (QOUT) 8 e4m3 codes with the row's scale for this 128-column block (absmax / 448 over the 16
 // lanes, quantize_fp8_rows' contract): exactly the fp8 x fp8 down projection's A operand.  Saves the [M][2 I] bf16 round
 // trip through HBM (Llama-3-8B shape, S = 4096: 235 MB written + read back = ~75 us of a 1.4 ms layer) and a launch.
-template <bool QOUT, int TN = 4>   // TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
+template <bool QOUT, int TN = 4, bool ROWS = false>   // ROWS: a lane holds columns of a row (ct_off), otherwise rows of a column; TN = n-fragments per wave column: 4 = 128 act columns per tile; 3 = 96 (bf16 output only)
 __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&acc)[8][TN], int tid, int m0, int tn, int M, int I,
                                                    void* outv, float* out_scales) {
     static_assert(TN == 4 || !QOUT, "the e4m3 epilogue needs whole 128-column scale blocks");
@@ -99,19 +99,25 @@ __device__ __forceinline__ void g2_swiglu_epilogue(char* smem, const f32x4_g (&a
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<uint2*>(smem + ct_off<ROWB>(wr * 128 + i * 16 + l15, (wc * WN + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
-                *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
+                for (int r = 0; r < 4; ++r) {
+                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * WN + j * 16 + l15) * 2;
+                    *reinterpret_cast<bf16*>(smem + row * ROWB + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);   // (row >> 2) & 3 == q; the XOR stays inside a 128-byte group
+                }
             }
+        }
+    auto at = [&](int row, int byte) { return smem + (ROWS ? ct_off<ROWB>(row, byte) : row * ROWB + (byte ^ (((row >> 2) & 3) << 5))); };
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < 256 * CH / G2_THREADS; ++it) {
-        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH, sw = ((row >> 2) & 3) << 5;
+        const int item = it * G2_THREADS + tid, row = item / CH, c = item % CH;
         Vec<bf16> g, u;
-        g.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((c * 16) ^ sw));
-        u.raw = *reinterpret_cast<const uint4*>(smem + row * ROWB + ((ACT * 2 + c * 16) ^ sw));
+        g.raw = *reinterpret_cast<const uint4*>(at(row, c * 16));
+        u.raw = *reinterpret_cast<const uint4*>(at(row, ACT * 2 + c * 16));
         float gf[8], uf[8];
         g.to_float(gf);
         u.to_float(uf);
@@ -184,6 +190,7 @@ __device__ __forceinline__ void g2_accum_epilogue(char* smem, const f32x4_g (&ac
 // ---- QKV-heads epilogue (EPI 3 of the fp8 kernel, 5 of the bf16 one): the accumulators go to LDS as the bf16 tile the plain kernel would have stored (the layout of
 // g2_swiglu_epilogue), a tile = 256 token rows x two head slots, 16 consecutive lanes take one (row, head) and finish it
 // (HeadRows: per-head RMSNorm, RoPE, q -> qkv buffer, k / v -> cache): bit-identical to GEMM + qknorm_rope_kvwrite_kernel.
+template <bool ROWS = false>
 __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g (&acc)[8][4], int tid, int m0, int tn, int M, int N, bf16* qkv,
                                                       const QkvHeadArgs& hd) {
     const int lane = tid & 63, wid = tid >> 6, wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
@@ -194,20 +201,25 @@ __device__ __forceinline__ void g2_qkv_heads_epilogue(char* smem, const f32x4_g 
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<uint2*>(smem + ct_off<512>(wr * 128 + i * 16 + l15, (wc * 64 + j * 16 + q * 4) * 2)) = ct_bf16(acc[i][j]);
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
-                *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
+                for (int r = 0; r < 4; ++r) {
+                    const int row = wr * 128 + i * 16 + q * 4 + r, colb = (wc * 64 + j * 16 + l15) * 2;
+                    *reinterpret_cast<bf16*>(smem + row * 512 + (colb ^ (q << 5))) = from_f<bf16>(acc[i][j][r]);
+                }
             }
+        }
     hr.angles(c, 2 * tn, hd);
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         hr.finish(c, 2 * tn + h, m0 + r0, 32, M, hd, qkv, N, [&](int i, float (&x)[8]) {
-            const int row = i * 32 + r0, sw = ((row >> 2) & 3) << 5;
+            const int row = i * 32 + r0, byte = h * 256 + c * 16;
             Vec<bf16> raw;
-            raw.raw = *reinterpret_cast<const uint4*>(smem + row * 512 + ((h * 256 + c * 16) ^ sw));
+            raw.raw = *reinterpret_cast<const uint4*>(smem + (ROWS ? ct_off<512>(row, byte) : row * 512 + (byte ^ (((row >> 2) & 3) << 5))));
             raw.to_float(x);
         });
 }
@@ -350,13 +362,12 @@ constexpr size_t G2S_LDS = (G2S_ARING + 4) * (size_t)256 * 64;
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store;
 // 5: QKV heads (QkvHeadArgs; a tile holds two head slots, N % 256 == 0).  Qwen3-0.6B, 3365 rows: 38 us and 14 of the separate pass -> 38.
 // EPI 0, 2, 5: rows scaled by NormIn where given.
-template <int EPI, int TN = 4>
+template <int EPI, int TN = 4, bool ROWS = EPI == 0 || EPI == 3 || EPI == 4>   // ROWS: a lane holds columns of a row (ct_off, gemm256_rows)
 __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                                                     int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa, QkvHeadArgs hd, NormIn ni) {
     static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: G2S_ARING slots of 16 KiB | W: 4 stages of 16 KiB
     constexpr int HALF = 256 * 64, BN = TN * 64, WN = TN * 16;
-    constexpr bool ROWS = EPI == 0 || EPI == 3 || EPI == 4;  // a lane holds columns of a row (ct_off says what that costs the others)
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int wr = wid >> 2, wc = wid & 3, q = lane >> 4, l15 = lane & 15;
     const int late = __builtin_amdgcn_readfirstlane(wr);     // wave-uniform by construction: scalar branches around barriers
@@ -497,11 +508,11 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
         }
     }
     if constexpr (EPI == 2) {
-        g2_swiglu_epilogue<false, TN>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
+        g2_swiglu_epilogue<false, TN, ROWS>(g2_smem, acc, tid, m0, tn, M, N, Cv, nullptr);
         return;
     }
     if constexpr (EPI == 5) {
-        g2_qkv_heads_epilogue(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
+        g2_qkv_heads_epilogue<ROWS>(g2_smem, acc, tid, m0, tn, M, N, reinterpret_cast<bf16*>(Cv), hd);
         return;
     }
     if constexpr (EPI == 1 && TN == 4) {
@@ -1319,17 +1330,24 @@ static bool gemm256_narrow(int M, int N) {
     return N % 192 == 0 && 0.75 * ceil_div(ntm * (N / 192), 256) < (double)ceil_div(ntm * ceil_div(N, G2_BN), 256) - 0.01;
 }
 
+// Of the kernels that finish SwiGLU or heads, the one whose lanes hold columns of a row (ct_off)
+// where at most a tenth of the tiles' rows is padding, copies of the last row: they gain 0.3..1.8 % of a prompt there (ms, other way and this: Qwen3-0.6B, 3100 rows 6.03 / 5.91, 3500 6.49 / 6.38,
+// 4096 7.27 / 7.20; Llama-3-8B shape, e4m3, 4096 49.9 / 49.7, bf16, 1500 and 2850 even), and lose where it is much: 300 rows, N = 28672, K = 4096, 90 us / 94.6.
+static bool gemm256_rows(int M) { return 10LL * ((long long)ceil_div(M, G2_BM) * G2_BM - M) <= M; }
+
 // QKV projection finished head by head: where whole 256-column tiles are what gemm256_bf16_nt would take
 bool gemm256_bf16_qkv_heads_ok(int M, int N, int K) { return K % 64 == 0 && K >= 64 && N % 256 == 0 && !gemm256_narrow(M, N); }
 pgk_status gemm256_bf16_qkv_heads_nt(const bf16* A, const bf16* W, bf16* qkv, int M, int N, int K, const QkvHeadArgs& hd, hipStream_t st, bool packed, const NormIn& ni) {
     PGK_REQUIRE(gemm256_bf16_qkv_heads_ok(M, N, K) && N == (hd.hq + 2 * hd.hkv) * 128, "gemm256 heads: N=%d K=%d (%d + 2 x %d heads)", N, K, hd.hq, hd.hkv);
     static bool attr_done = false;
     if (!attr_done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<5>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)G2S_LDS));
+        for (auto* kfn : {&gemm256s_bf16_kernel<5>, &gemm256s_bf16_kernel<5, 4, true>})
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)G2S_LDS));
         attr_done = true;
     }
     const int ntm = ceil_div(M, G2_BM), ntn = N / G2_BN;
-    gemm256s_bf16_kernel<5><<<ntm * ntn, G2_THREADS, G2S_LDS, st>>>(A, W, nullptr, qkv, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, hd, ni);
+    auto kfn = gemm256_rows(M) ? &gemm256s_bf16_kernel<5, 4, true> : &gemm256s_bf16_kernel<5>;
+    kfn<<<ntm * ntn, G2_THREADS, G2S_LDS, st>>>(A, W, nullptr, qkv, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, hd, ni);
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
 }
@@ -1393,17 +1411,20 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
     constexpr size_t LDS = G2S_LDS;
     static bool attr_done = false;
     if (!attr_done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<2, 3>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
+        for (auto* kfn : {&gemm256s_bf16_kernel<2>, &gemm256s_bf16_kernel<2, 3>, &gemm256s_bf16_kernel<2, 4, true>, &gemm256s_bf16_kernel<2, 3, true>})
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
         attr_done = true;
     }
+    const bool rows = gemm256_rows(M);
     const int ntm = ceil_div(M, G2_BM), ntn = I / 128;
     // 96 act columns per tile (192-column B tiles) when that fills the rounds of the chip better: Qwen3-0.6B at S = 2048 is
     // 8 x 24 = 192 tiles of 128 (three quarters of the CUs, one round) or 8 x 32 = 256 tiles of 96 (all of them)
     if (I % 96 == 0 && 0.75 * ceil_div(ntm * (I / 96), 256) < (double)ceil_div(ntm * ntn, 256) - 0.01) {
-        gemm256s_bf16_kernel<2, 3><<<ntm * (I / 96), G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, I / 96, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
+        auto kfn = rows ? &gemm256s_bf16_kernel<2, 3, true> : &gemm256s_bf16_kernel<2, 3>;
+        kfn<<<ntm * (I / 96), G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, I / 96, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
     } else {
-        gemm256s_bf16_kernel<2><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
+        auto kfn = rows ? &gemm256s_bf16_kernel<2, 4, true> : &gemm256s_bf16_kernel<2>;
+        kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, act, M, I, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
     }
     PGK_CHECK_HIP(hipGetLastError());
     return PGK_OK;
