@@ -362,7 +362,7 @@ constexpr size_t G2S_LDS = (G2S_ARING + 4) * (size_t)256 * 64;
 // EPI 0: bf16 C store (+bias); 1: fp32 C +=; 2: SwiGLU (W = fused gate / up rows, N = I act columns, C = bf16 act [M][I]); 3: xIELU, 4: gelu, bf16 store;
 // 5: QKV heads (QkvHeadArgs; a tile holds two head slots, N % 256 == 0).  Qwen3-0.6B, 3365 rows: 38 us and 14 of the separate pass -> 38.
 // EPI 0, 2, 5: rows scaled by NormIn where given.
-template <int EPI, int TN = 4, bool ROWS = EPI == 0 || EPI == 3 || EPI == 4>   // ROWS: a lane holds columns of a row (ct_off, gemm256_rows)
+template <int EPI, int TN = 4, bool ROWS = false>   // ROWS: a lane holds columns of a row (ct_off; gemm256_rows, gemm256_rows_store)
 __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                                                     int M, int N, int K, int ntm, int ntn, int packed, ActArgs xa, QkvHeadArgs hd, NormIn ni) {
     static_assert(TN == 4 || (TN == 3 && EPI != 1 && EPI != 5), "192-column tiles: no +=, no heads");
@@ -521,32 +521,38 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
             return;
         }
     }
-    if constexpr (!ROWS) {                                   // N % 4 != 0
+    if constexpr (!ROWS) {                                   // EPI 1: N % 4 != 0
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int col = n0 + wc * WN + j * 16 + l15;
             if (col >= N) continue;
+            float b = 0.f;
+            if constexpr (EPI == 0) b = bias ? to_f(bias[col]) : 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = m0 + wr * 128 + i * 16 + q * 4 + r;
-                    if (row < M) reinterpret_cast<float*>(Cv)[(size_t)row * N + col] += acc[i][j][r];
+                    if (row >= M) continue;
+                    if constexpr (EPI == 0) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(acc[i][j][r] + b);
+                    else if constexpr (EPI == 3) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(xielu<false>(acc[i][j][r], xa.pos, xa.neg));
+                    else if constexpr (EPI == 4) reinterpret_cast<bf16*>(Cv)[(size_t)row * N + col] = from_f<bf16>(gelu_erf(acc[i][j][r]));
+                    else reinterpret_cast<float*>(Cv)[(size_t)row * N + col] += acc[i][j][r];
                 }
         }
         return;
     }
-    // four columns of a row to a lane: one 8-byte store where every row is aligned to it
-    const bool whole = (N & 3) == 0 && ((uintptr_t)Cv & 7) == 0;
+    // four columns of a row to a lane: one 8-byte store (gemm256_rows_store: every row is aligned to it)
     bf16* C = reinterpret_cast<bf16*>(Cv);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int col = n0 + wc * WN + j * 16 + q * 4;
+        if (col >= N) continue;
         float b[4] = {0.f, 0.f, 0.f, 0.f};
         if constexpr (EPI == 0) {
             if (bias) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) b[r] = to_f(bias[min(col + r, N - 1)]);
+                for (int r = 0; r < 4; ++r) b[r] = to_f(bias[col + r]);
             }
         }
 #pragma unroll
@@ -560,13 +566,7 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
                 else if constexpr (EPI == 3) v[r] = xielu<false>(v[r], xa.pos, xa.neg);
                 else if constexpr (EPI == 4) v[r] = gelu_erf(v[r]);
             }
-            if (whole) {
-                if (col < N) *reinterpret_cast<uint2*>(C + (size_t)row * N + col) = ct_bf16(v);
-                continue;
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (col + r < N) C[(size_t)row * N + col + r] = from_f<bf16>(v[r]);
+            *reinterpret_cast<uint2*>(C + (size_t)row * N + col) = ct_bf16(v);
         }
     }
 }
@@ -1334,6 +1334,11 @@ static bool gemm256_narrow(int M, int N) {
 // where at most a tenth of the tiles' rows is padding, copies of the last row: they gain 0.3..1.8 % of a prompt there (ms, other way and this: Qwen3-0.6B, 3100 rows 6.03 / 5.91, 3500 6.49 / 6.38,
 // 4096 7.27 / 7.20; Llama-3-8B shape, e4m3, 4096 49.9 / 49.7, bf16, 1500 and 2850 even), and lose where it is much: 300 rows, N = 28672, K = 4096, 90 us / 94.6.
 static bool gemm256_rows(int M) { return 10LL * ((long long)ceil_div(M, G2_BM) * G2_BM - M) <= M; }
+// Of the kernels that store from registers likewise, and only where a lane's four columns are one 8-byte store: stored one by one they are 16 rows to an instruction instead of 4.
+// Us of pgk_gemm_nt, by columns / by rows: 4096 rows, N = K = 4096, C four bytes off a line 116 / 123, N = 4097 174 / 196, 3000 rows, N = 50257, K = 1024 395 / 484;
+// whole and aligned, 4096 rows, N = 4100 173 / 167, 3000 rows, N = 50256, K = 1024 377 / 346, 512 rows, N = 32768, K = 1024 40.8 / 36.8; padding: 300 rows, N = 28672, K = 4096
+// 90 / 99, 600 171 / 178, 257 rows, N = 32768, K = 1024 31.4 / 35, 1100 rows, N = 12288, K = 4096 even.
+static bool gemm256_rows_store(int M, int N, const void* C) { return gemm256_rows(M) && N % 4 == 0 && ((uintptr_t)C & 7) == 0; }
 
 // QKV projection finished head by head: where whole 256-column tiles are what gemm256_bf16_nt would take
 bool gemm256_bf16_qkv_heads_ok(int M, int N, int K) { return K % 64 == 0 && K >= 64 && N % 256 == 0 && !gemm256_narrow(M, N); }
@@ -1369,33 +1374,29 @@ pgk_status gemm256_bf16_nt(const bf16* A, const bf16* W, const bf16* bias, void*
     if (packed || act || ni.ss || !e || atoi(e) != 0) {
         static bool attr_s = false;
         if (!attr_s) {
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
+            for (auto* kfn : {&gemm256s_bf16_kernel<0>, &gemm256s_bf16_kernel<0, 4, true>, &gemm256s_bf16_kernel<0, 3>, &gemm256s_bf16_kernel<0, 3, true>, &gemm256s_bf16_kernel<1>})
+                PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
             attr_s = true;
         }
-        const int ntn3 = N / 192;
-        const bool narrow = !accum_f32 && gemm256_narrow(M, N);
-        if (narrow) {
-            static bool attr_n = false;
-            if (!attr_n) {
-                PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm256s_bf16_kernel<0, 3>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-                attr_n = true;
-            }
-            if (act) {
-                auto kfn = act->gelu ? &gemm256s_bf16_kernel<4, 3> : &gemm256s_bf16_kernel<3, 3>;
-                static bool attr_x[2] = {false, false};
-                if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-                attr_x[act->gelu] = true;
-                kfn<<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn3, packed ? 1 : 0, *act, QkvHeadArgs{}, NormIn{});
-            } else gemm256s_bf16_kernel<0, 3><<<ntm * ntn3, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn3, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
-        } else if (act) {
-            auto kfn = act->gelu ? &gemm256s_bf16_kernel<4> : &gemm256s_bf16_kernel<3>;
-            static bool attr_x[2] = {false, false};
-            if (!attr_x[act->gelu]) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
-            attr_x[act->gelu] = true;
-            kfn<<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, *act, QkvHeadArgs{}, NormIn{});
+        const bool narrow = !accum_f32 && gemm256_narrow(M, N), rows = gemm256_rows_store(M, N, C);
+        const int nt = narrow ? N / 192 : ntn;
+        if (act) {
+            auto pick = [&](auto epi) {
+                constexpr int E = decltype(epi)::value;
+                if (narrow) return rows ? &gemm256s_bf16_kernel<E, 3, true> : &gemm256s_bf16_kernel<E, 3>;
+                return rows ? &gemm256s_bf16_kernel<E, 4, true> : &gemm256s_bf16_kernel<E>;
+            };
+            auto kfn = act->gelu ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 3>{});
+            static bool attr_x[2][2][2] = {};
+            bool& done = attr_x[act->gelu][narrow][rows];
+            if (!done) PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
+            done = true;
+            kfn<<<ntm * nt, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, nt, packed ? 1 : 0, *act, QkvHeadArgs{}, NormIn{});
         } else if (accum_f32) gemm256s_bf16_kernel<1><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, nullptr, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, NormIn{});
-        else gemm256s_bf16_kernel<0><<<ntm * ntn, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, ntn, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
+        else {
+            auto kfn = narrow ? (rows ? &gemm256s_bf16_kernel<0, 3, true> : &gemm256s_bf16_kernel<0, 3>) : rows ? &gemm256s_bf16_kernel<0, 4, true> : &gemm256s_bf16_kernel<0>;
+            kfn<<<ntm * nt, G2_THREADS, LDS, st>>>(A, W, bias, C, M, N, K, ntm, nt, packed ? 1 : 0, ActArgs{}, QkvHeadArgs{}, ni);
+        }
         PGK_CHECK_HIP(hipGetLastError());
         return PGK_OK;
     }

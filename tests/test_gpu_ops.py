@@ -537,7 +537,8 @@ def test_gemm256_exact_integers(N, monkeypatch):
 
 @pytest.mark.parametrize("M,N", [(300, 260), (257, 263), (256, 774), (129, 130), (300, 577)])
 def test_gemm256_stores_of_four_columns_exact_integers(M, N, monkeypatch):
-    """The 256-tile kernels store four columns of a row at once where N % 4 == 0 and single ones elsewhere, with a bias, at the ends of rows and of tiles."""
+    """The stores of the 256-tile kernels, with a bias, at the ends of rows and of tiles: four columns of a row at once (256 rows, N % 4 == 0 or not: see the test below) and
+    single ones."""
     rng = np.random.default_rng(M + N)
     K = 64
     a = rng.integers(-3, 4, (M, K)).astype(np.float32)
@@ -545,6 +546,26 @@ def test_gemm256_stores_of_four_columns_exact_integers(M, N, monkeypatch):
     bias = rng.integers(-8, 9, N).astype(np.float32)
     monkeypatch.setenv("PGK_GEMM256", "1")
     np.testing.assert_array_equal(host(ops.matmul_nt(dev(a, "bfloat16"), dev(w, "bfloat16"), dev(bias, "bfloat16"))), O.bf16_round(a @ w.T + bias))
+
+
+@pytest.mark.parametrize("M", [232, 233, 465, 466])
+@pytest.mark.parametrize("N", [260, 262, 576])
+@pytest.mark.parametrize("off", [0, 2, 4])
+def test_gemm256_stores_by_rows_only_where_they_are_whole(M, N, off, monkeypatch):
+    """Four columns to a store where rows are 8-byte aligned (N % 4 == 0, C not off elements away) and at most a tenth of the tiles' rows is padding (232 | 233, 465 | 466); single
+    columns otherwise.  With a bias, exact integers, and nothing written beside C."""
+    from pygpukit_amd import _hip
+
+    rng = np.random.default_rng(M + N + off)
+    K = 64
+    a, w, b = (rng.integers(-3, 4, s).astype(np.float32) for s in ((M, K), (N, K), (N,)))
+    ad, wd, bd = dev(a, "bfloat16"), dev(w, "bfloat16"), dev(b, "bfloat16")
+    out = dev(np.full(M * N + 8, -77, np.float32), "bfloat16")
+    monkeypatch.setenv("PGK_GEMM256", "1")
+    _hip.call("pgk_gemm_nt", ad.data_ptr(), wd.data_ptr(), bd.data_ptr(), out.data_ptr() + 2 * off, M, N, K, 3, None)
+    got = host(out)
+    np.testing.assert_array_equal(got[off:off + M * N].reshape(M, N), O.bf16_round(a @ w.T + b))
+    assert (got[:off] == -77).all() and (got[off + M * N:] == -77).all()
 
 
 @pytest.mark.parametrize("tile", ["0", "1"])
