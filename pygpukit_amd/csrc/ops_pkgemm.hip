@@ -32,6 +32,7 @@ typedef __bf16 bf16x8_p __attribute__((ext_vector_type(8)));
 typedef float f32x4_p __attribute__((ext_vector_type(4)));
 
 constexpr int PK_THREADS = 256;
+template <int V> using pk_int = std::integral_constant<int, V>;
 constexpr int PK_MT = 2;           // m-tiles per workgroup
 constexpr int PK_MB = PK_MT * 16;  // rows per m-block
 
@@ -113,6 +114,7 @@ template <int NTW, int EPI, int MT, int PK_RING>
 __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(const bf16* a_, const bf16* wp_, const float* ss_in_, int lda_, int M_, int K_, int ksteps_, int nblk_, int mblk_, int splits_,
                                                              int tile_b_off_, PkArgs g) {
     // what the load-issue phase needs, in the arguments that arrive preloaded in SGPRs (fused_gemv_kernel, engine.hip)
+    static_assert(NTW * PK_RING <= 63, "what s_waitcnt can count");
     constexpr int PK_MT = MT, PK_MB = 16 * MT;
     extern __shared__ __attribute__((aligned(16))) char a_lds[];   // [PK_MB][ksteps * 32] bf16, chunk-swizzled rows
     __shared__ float ssred[4][PK_MB];
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_kernel(const bf16* a_, cons
         if (sub == 0 && row < PK_MB) inv_lds[row] = 1.0f / sqrtf(ssum / (float)K_ + g.ss_eps);
     }
     PK_STAMP(1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING < 63 ? NTW * PK_RING : 63) : "memory");   // in-order return: every DMA has landed
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING) : "memory");   // in-order return: every DMA has landed
     __syncthreads();
     PK_STAMP(2);
 
@@ -486,7 +488,7 @@ __global__ __launch_bounds__(PK_THREADS) void pkgemm_resid_kernel(const bf16* a_
     for (int s = 0; s < PK_RING; ++s)
 #pragma unroll
         for (int t = 0; t < NTW; ++t) wr[t][s] = *reinterpret_cast<const uint4*>(wrun[t] + (size_t)min(s, KSW - 1) * 512);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING < 63 ? NTW * PK_RING : 63) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTW * PK_RING) : "memory");
     __syncthreads();
 
     f32x4_p acc[NTW][MT];
@@ -584,21 +586,21 @@ pgk_status pkgemm_resid_nt(const bf16* a, int lda, const void* wp, float* h, int
     if (ss_n) *ss_n = g.nblk;
     const size_t lds = (size_t)mb * (K / 32) * 64;
     const int grid = ceil_div(g.nblk, 8) * 8 * g.mblk;
-#define PGK_PKR_LAUNCH(MBV, NTWV, RINGV)                                                                                  \
-    {                                                                                                              \
-        static bool attr = false;                                                                                  \
-        if (lds > 48 * 1024 && !attr) {                                                                            \
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_resid_kernel<MBV, NTWV, RINGV>),       \
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));     \
-            attr = true;                                                                                           \
-        }                                                                                                          \
-        pkgemm_resid_kernel<MBV, NTWV, RINGV><<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.h, g.gamma_next, g.lda, g.M, g.N, g.K, g.mblk, g);                                          \
-    }
-    const bool deep = K / 128 == 24;      // all 24 k-steps of a wave's quarter in flight
-    if (small && deep) PGK_PKR_LAUNCH(16, 1, 24) else if (small) PGK_PKR_LAUNCH(16, 1, 16) else if (wide && deep) PGK_PKR_LAUNCH(32, 1, 24) else if (wide) PGK_PKR_LAUNCH(32, 1, 16) else PGK_PKR_LAUNCH(16, 2, 16)
-#undef PGK_PKR_LAUNCH
-    PGK_CHECK_HIP(hipGetLastError());
-    return PGK_OK;
+    auto launch = [&](auto rows, auto tiles, auto ring) -> pgk_status {
+        auto kfn = &pkgemm_resid_kernel<decltype(rows)::value, decltype(tiles)::value, decltype(ring)::value>;
+        static bool attr = false;
+        if (lds > 48 * 1024 && !attr) {
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));
+            attr = true;
+        }
+        kfn<<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.h, g.gamma_next, g.lda, g.M, g.N, g.K, g.mblk, g);
+        PGK_CHECK_HIP(hipGetLastError());
+        return PGK_OK;
+    };
+    if (wide) return launch(pk_int<32>{}, pk_int<1>{}, pk_int<16>{});         // at most 16 k-steps to a wave
+    if (!small) return launch(pk_int<16>{}, pk_int<2>{}, pk_int<16>{});
+    if (K / 128 == 24) return launch(pk_int<16>{}, pk_int<1>{}, pk_int<24>{});      // all 24 k-steps of a wave's quarter in flight
+    return launch(pk_int<16>{}, pk_int<1>{}, pk_int<16>{});
 }
 
 // K splits for the N = hidden projections: enough workgroups to cover the chip, and a K range per workgroup whose
@@ -630,7 +632,6 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
     g.ksteps = K / splits / 32;
     g.splits = splits;
     // (m-tile count chosen below, once the n-block count of the epilogue is known)
-    g.tiles_per_cb = 4;
     g.tile_b_off = 0;
     if (epi == PK_EPI_SWIGLU) {
         PGK_REQUIRE(N % 128 == 0, "pkgemm: SwiGLU needs 2 I = %d weight rows with I a multiple of 64", N);
@@ -639,7 +640,6 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
     } else if (epi == PK_EPI_QKV) {
         PGK_REQUIRE(head && N == (g.hq + 2 * g.hkv) * 128, "pkgemm: head epilogue needs head_dim 128 (N=%d)", N);
         g.nblk = N / 128;
-        g.tiles_per_cb = 8;
         g.tile_b_off = 4;
     } else {
         g.nblk = N / 64;
@@ -652,35 +652,29 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
     const size_t lds = (size_t)16 * mt * g.ksteps * 64;
     PGK_REQUIRE(lds <= 128 * 1024, "pkgemm: K per workgroup %d too long for the LDS activation block", g.ksteps * 32);
     const int grid = ceil_div(g.nblk, 8) * 8 * g.mblk * splits;     // whole groups of 8 n-blocks (see the id mapping in the kernel)
-#define PGK_PK_LAUNCH3(NTWV, EPIV, MTV, RINGV)                                                                            \
-    {                                                                                                              \
-        static size_t attr = 0;                                                                                    \
-        if (lds > 48 * 1024 && lds > attr) {                                                                       \
-            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pkgemm_kernel<NTWV, EPIV, MTV, RINGV>),       \
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));     \
-            attr = 128 * 1024;                                                                                     \
-        }                                                                                                          \
-        pkgemm_kernel<NTWV, EPIV, MTV, RINGV><<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.ss_in, g.lda, g.M, g.K, g.ksteps, g.nblk, g.mblk, g.splits, g.tile_b_off, g);                                          \
-    }
-#define PGK_PK_LAUNCH2(NTWV, EPIV, MTV)                                                                           \
-    if (NTWV == 1 && g.ksteps == 32) PGK_PK_LAUNCH3(NTWV, EPIV, MTV, 32) else PGK_PK_LAUNCH3(NTWV, EPIV, MTV, 16)
-#define PGK_PK_LAUNCH(NTWV, EPIV)                                                                                  \
-    if (mt == 1) { PGK_PK_LAUNCH2(NTWV, EPIV, 1) } else { PGK_PK_LAUNCH2(NTWV, EPIV, 2) }
+    auto launch = [&](auto ntw, auto epilogue, auto mtiles, auto ring) -> pgk_status {
+        auto kfn = &pkgemm_kernel<decltype(ntw)::value, decltype(epilogue)::value, decltype(mtiles)::value, decltype(ring)::value>;
+        static bool attr = false;
+        if (lds > 48 * 1024 && !attr) {
+            PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(128 * 1024)));
+            attr = true;
+        }
+        kfn<<<grid, PK_THREADS, lds, st>>>(g.a, g.wp, g.ss_in, g.lda, g.M, g.K, g.ksteps, g.nblk, g.mblk, g.splits, g.tile_b_off, g);
+        PGK_CHECK_HIP(hipGetLastError());
+        return PGK_OK;
+    };
+    auto rows = [&](auto ntw, auto epilogue, auto ring) { return mt == 1 ? launch(ntw, epilogue, pk_int<1>{}, ring) : launch(ntw, epilogue, pk_int<2>{}, ring); };
+    auto one = [&](auto epilogue) { return g.ksteps == 32 ? rows(pk_int<1>{}, epilogue, pk_int<32>{}) : rows(pk_int<1>{}, epilogue, pk_int<16>{}); };
     switch (epi) {
-        case PK_EPI_BF16: PGK_PK_LAUNCH(1, PK_EPI_BF16) break;
-        case PK_EPI_XIELU: PGK_PK_LAUNCH(1, PK_EPI_XIELU) break;
-        case PK_EPI_GELU: PGK_PK_LAUNCH(1, PK_EPI_GELU) break;
-        case PK_EPI_SLAB: PGK_PK_LAUNCH(1, PK_EPI_SLAB) break;
-        case PK_EPI_ACCUM: PGK_PK_LAUNCH(1, PK_EPI_ACCUM) break;
-        case PK_EPI_SWIGLU: PGK_PK_LAUNCH(2, PK_EPI_SWIGLU) break;
-        case PK_EPI_QKV: PGK_PK_LAUNCH(2, PK_EPI_QKV) break;
-        default: return set_error(PGK_ERR_INVALID, "pkgemm: unknown epilogue %d", epi);
+        case PK_EPI_BF16: return one(pk_int<PK_EPI_BF16>{});
+        case PK_EPI_XIELU: return one(pk_int<PK_EPI_XIELU>{});
+        case PK_EPI_GELU: return one(pk_int<PK_EPI_GELU>{});
+        case PK_EPI_SLAB: return one(pk_int<PK_EPI_SLAB>{});
+        case PK_EPI_ACCUM: return one(pk_int<PK_EPI_ACCUM>{});
+        case PK_EPI_SWIGLU: return rows(pk_int<2>{}, pk_int<PK_EPI_SWIGLU>{}, pk_int<16>{});
+        case PK_EPI_QKV: return rows(pk_int<2>{}, pk_int<PK_EPI_QKV>{}, pk_int<16>{});
     }
-#undef PGK_PK_LAUNCH3
-#undef PGK_PK_LAUNCH2
-#undef PGK_PK_LAUNCH
-    PGK_CHECK_HIP(hipGetLastError());
-    return PGK_OK;
+    return set_error(PGK_ERR_INVALID, "pkgemm: unknown epilogue %d", epi);
 }
 
 }  // namespace pgk

@@ -15,7 +15,6 @@ struct PkArgs {
     int M, N, K;
     int ksteps;            // k-steps (32 k) per K split; multiple of 4
     int nblk, mblk, splits;
-    int tiles_per_cb;      // n-tiles between consecutive n-blocks (4; 8 for the head epilogue)
     int tile_b_off;        // NTW == 2: the wave's second n-tile is this many tiles after its first
     void* c;
     int ldc;
