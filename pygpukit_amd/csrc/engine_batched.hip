@@ -70,7 +70,9 @@ static pgk_status batched_proj_t(int pro, int epi, const FusedArgs& a, int M, hi
             case EPI_STORE: return launch_batched_tiled<WT, EPI_STORE>(a, M, st);
             case EPI_RESID: return launch_batched_tiled<WT, EPI_RESID>(a, M, st);
             case EPI_SWIGLU: return launch_batched_tiled<WT, EPI_SWIGLU>(a, M, st);
-            case EPI_LOGITS: return launch_batched_tiled<WT, EPI_LOGITS>(a, M, st, nblk);
+            case EPI_LOGITS:                       // (the lm_head is bf16 whatever the layers are)
+                if constexpr (!std::is_same<WT, fp8e4m3>::value) return launch_batched_tiled<WT, EPI_LOGITS>(a, M, st, nblk);
+                break;
         }
         return set_error(PGK_ERR_INVALID, "batched_proj: epilogue %d", epi);
     }
@@ -78,7 +80,7 @@ static pgk_status batched_proj_t(int pro, int epi, const FusedArgs& a, int M, hi
         switch (epi) {
             case EPI_STORE: return launch_batched<WT, PRO_NORM, EPI_STORE>(a, M, st);
             case EPI_SWIGLU: return launch_batched<WT, PRO_NORM, EPI_SWIGLU>(a, M, st);
-            case EPI_LOGITS:                       // (the lm_head is bf16 whatever the layers are)
+            case EPI_LOGITS:
                 if constexpr (!std::is_same<WT, fp8e4m3>::value) return launch_batched<WT, PRO_NORM, EPI_LOGITS>(a, M, st, nblk);
                 break;
         }

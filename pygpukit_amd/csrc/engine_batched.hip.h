@@ -6,49 +6,24 @@
 // v_mfma_f32_16x16x32_bf16 and 16 weight rows are its B operand, loaded straight from HBM in fragment shape
 // (lane l: W[n0 + (l&15)][k + 8*(l>>4) ..+8], the layout of ops_wsgemm.hip): one MFMA replaces those 32 instructions and
 // the cost of a projection no longer depends on M.
-//   workgroup = 4 waves = 16 output rows (SWIGLU: 16 gate rows and their 16 up rows); the waves split K four ways
-//   (every lane's weight loads - K/128 of them - are issued before the prologue touches the activations), partial
+//   workgroup = 4 waves = 16 output rows (SWIGLU: 16 gate rows and their 16 up rows); the waves split K four ways, partial
 //   16x16 tiles are summed through LDS; prologue = RMSNorm (or plain copy) of the M rows into an LDS image laid out
 //   [k/8][MP] x 16 B so that an A-fragment read is 64 consecutive 16-byte slots; epilogues as in engine.hip
 //   (store / residual add / SiLU(g)*u / logits + per-workgroup argmax partials, lowest index on ties).
 // fp8 weights: 8 codes per lane per step, widened to bf16 with the block scale in registers (as ops_wsgemm.hip).
 
-// MP: activation rows held in LDS (8 or 16).  S: 32-k steps per wave preloaded into registers (K = 128 S when it is one of
-// the instantiated 8 / 16 / 24; any further steps stream through a plain loop).
-template <class WT, int PRO, int EPI, int MP, int S>
+// Any K = 128 steps that the register-fragment kernels below do not take, up to what the image holds.  MP: activation rows held in LDS (8 or 16).
+template <class WT, int PRO, int EPI, int MP>
 __global__ __launch_bounds__(256) void batched_mfma_kernel(unsigned long long* tl, FusedArgs a, int M, int steps /* K / 128 per wave */, int nblk_logits) {
     const TLStamp tls(tl);
     constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value;
     constexpr int NT = (EPI == EPI_SWIGLU) ? 2 : 1;       // weight row groups per workgroup
-    constexpr int MAXS = S > 0 ? S : 1;
     extern __shared__ __attribute__((aligned(16))) char smem[];   // x image [K/8][MP] x 16 B | partial tiles
     __shared__ float s_ss[4][16];
     const int K = a.K, N = a.N;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, q = lane >> 4, l15 = lane & 15;
     const int ngroups = (N + 15) >> 4;                     // 16-row groups; a workgroup takes groups blockIdx.x, + gridDim.x, ...
     const int kw0 = wid * steps * 32;                      // first k of this wave
-    uint4 wv[NT][MAXS];
-    float wsc[NT][MAXS];
-    auto load_w = [&](int n0) {
-        const int nrow = min(n0 + l15, N - 1);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const size_t row = (size_t)(t == 0 ? nrow : N + nrow);
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const int k = kw0 + s * 32 + 8 * q;
-                if constexpr (FP8) {
-                    const uint2 v = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(a.w) + row * K + k);
-                    wv[t][s] = make_uint4(v.x, v.y, 0, 0);
-                    wsc[t][s] = to_f(a.wscale[(row >> 7) * (size_t)(K >> 7) + (k >> 7)]);
-                } else {
-                    wv[t][s] = load_nt16(reinterpret_cast<const bf16*>(a.w) + row * K + k);
-                }
-            }
-        }
-    };
-    // ---- weight loads of the first group's K quarter, all issued before the prologue touches the activations ----
-    load_w(blockIdx.x * 16);
     const int em = tid >> 4, en = tid & 15;                // epilogue element of this thread: (row em, column n0 + en)
 
     // ---- prologue: M rows -> bf16 LDS image, chunk c (8 k) of row m at (c * MP + m) * 16 ----
@@ -121,36 +96,16 @@ __global__ __launch_bounds__(256) void batched_mfma_kernel(unsigned long long* t
     // ---- body: one 16-row group per trip; the LDS image of the activations stays, the partial tiles have their own area ----
     float* red = reinterpret_cast<float*>(smem + (size_t)nchunk * MP * 16);   // [NT][4 waves][16 m][16 n]
     const int am = l15 & (MP - 1);
-    auto bfrag = [&](int t, int s) -> uint4 {
-        if constexpr (FP8) {
-            const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].x, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].x, true);
-            const f32x2 c2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].y, false), c3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[t][s].y, true);
-            const float sc = wsc[t][s];
-            return make_uint4(pack_bf16x2(c0.x * sc, c0.y * sc), pack_bf16x2(c1.x * sc, c1.y * sc), pack_bf16x2(c2.x * sc, c2.y * sc),
-                              pack_bf16x2(c3.x * sc, c3.y * sc));
-        } else {
-            return wv[t][s];
-        }
-    };
     float bv = -INFINITY;          // EPI_LOGITS: best of this thread's elements over the workgroup's groups
     int bi = 0x7FFFFFFF;
     for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
         const int n0 = g * 16;
-        if (g != (int)blockIdx.x) load_w(n0);
         float resv = 0.f;
         if constexpr (EPI == EPI_RESID) resv = a.res[(size_t)min(em, M - 1) * a.ld_out + min(n0 + en, N - 1)];
         f32x4_b acc[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = f32x4_b{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const int kc = (kw0 >> 3) + s * 4 + q;
-            const uint4 af = *reinterpret_cast<const uint4*>(smem + ((size_t)kc * MP + am) * 16);
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_b, af), __builtin_bit_cast(bf16x8_b, bfrag(t, s)), acc[t], 0, 0, 0);
-        }
-        for (int s = S; s < steps; ++s) {          // steps beyond the preloaded ones stream through a plain loop
+        for (int s = 0; s < steps; ++s) {
             const int k = kw0 + s * 32 + 8 * q;
             const uint4 af = *reinterpret_cast<const uint4*>(smem + ((size_t)((k >> 3)) * MP + am) * 16);
             const int nrow = min(n0 + l15, N - 1);
@@ -758,15 +713,15 @@ static pgk_status launch_batched_reg(const FusedArgs& a, int M, hipStream_t st, 
     }
 }
 
-template <class WT, int PRO, int EPI, int MP, int S>
-static pgk_status launch_batched_s(const FusedArgs& a, int M, int steps, int grid, size_t lds, hipStream_t st, int nblk_logits) {
+template <class WT, int PRO, int EPI, int MP>
+static pgk_status launch_batched_image(const FusedArgs& a, int M, int steps, int grid, size_t lds, hipStream_t st, int nblk_logits) {
     static bool done = false;
     if (lds > 48 * 1024 && !done) {
-        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&batched_mfma_kernel<WT, PRO, EPI, MP, S>),
+        PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&batched_mfma_kernel<WT, PRO, EPI, MP>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048));
         done = true;
     }
-    PGK_CHECK_HIP(launch_k(batched_mfma_kernel<WT, PRO, EPI, MP, S>, dim3(grid), dim3(256), lds, st, a, M, steps, nblk_logits));
+    PGK_CHECK_HIP(launch_k(batched_mfma_kernel<WT, PRO, EPI, MP>, dim3(grid), dim3(256), lds, st, a, M, steps, nblk_logits));
     return PGK_OK;
 }
 
@@ -786,8 +741,6 @@ static pgk_status launch_batched(const FusedArgs& a, int M, hipStream_t st, int 
     const int mp = M <= 8 ? 8 : 16;
     const size_t lds = (size_t)(a.K / 8) * mp * 16 + (size_t)NT * 4 * 256 * 4;
     PGK_REQUIRE(lds <= 158 * 1024, "batched decode projection: K=%d does not fit the LDS image", a.K);
-#define PGK_BS(MPV, SV) return launch_batched_s<WT, PRO, EPI, MPV, SV>(a, M, steps, grid, lds, st, nblk_logits);
-    if (mp == 8) PGK_BS(8, 0)
-    PGK_BS(16, 0)
-#undef PGK_BS
+    if (mp == 8) return launch_batched_image<WT, PRO, EPI, 8>(a, M, steps, grid, lds, st, nblk_logits);
+    return launch_batched_image<WT, PRO, EPI, 16>(a, M, steps, grid, lds, st, nblk_logits);
 }
