@@ -106,8 +106,12 @@ __device__ unsigned long long g_pk_stamps[6][512][8];
 #define PK_STAMP(i) do { } while (0)
 #endif
 
-// PK_RING = k-steps of weights in flight per n-tile: a wave's whole run of 32 where it has one n-tile of K = 1024, else 16 (two n-tiles with 32 each leave a wave 256
-// registers and were slower: QKV of 93 rows 9.3 -> 9.7 us).  A step of 64 sequences 1149 -> 1141 us, with the arguments preloaded 1107; of 24 1028 -> 1019 -> 981.
+// PK_RING = k-steps of weights in flight per n-tile: 32 where a wave has one n-tile and whole rings make up its run, else 16 (two n-tiles with 32 each leave a wave 256
+// registers and were slower: QKV of 93 rows 9.3 -> 9.7 us).  Us a step of 64 sequences, K = 1024 1149 -> 1141, with the arguments preloaded 1107, of 24 1028 -> 1019 -> 981; K = 2048,
+// 8 layers 469 -> 450 and 432 -> 423.  Not where a part of a ring is left over, whose requests repeat the last k-step: prompts of 48 and 120 rows with K = 640, 1280 and 1792 showed no
+// gain beyond their spread of 3 %.
+// pkgemm_resid_kernel likewise, 24 or 32 for the quarter of K that a wave has: K = 3072 as above, K = 4096, 8 layers, us a step of 24 sequences 355 -> 349, of 64 389 -> 384; quarters of 20
+// and 28 in rings of 24 and 32 no gain either.
 // MT = m-tiles per workgroup: 2 (32-row m-blocks) for prompts, 1 (16 rows) for M <= 96 - decode batches, short prompts - where
 // 32-row blocks would leave CUs without a workgroup.
 template <int NTW, int EPI, int MT, int PK_RING>
@@ -599,7 +603,9 @@ pgk_status pkgemm_resid_nt(const bf16* a, int lda, const void* wp, float* h, int
     };
     if (wide) return launch(pk_int<32>{}, pk_int<1>{}, pk_int<16>{});         // at most 16 k-steps to a wave
     if (!small) return launch(pk_int<16>{}, pk_int<2>{}, pk_int<16>{});
-    if (K / 128 == 24) return launch(pk_int<16>{}, pk_int<1>{}, pk_int<24>{});      // all 24 k-steps of a wave's quarter in flight
+    // a wave's whole quarter of K in flight (pkgemm_kernel)
+    if (K == 24 * 128) return launch(pk_int<16>{}, pk_int<1>{}, pk_int<24>{});
+    if (K == 32 * 128) return launch(pk_int<16>{}, pk_int<1>{}, pk_int<32>{});
     return launch(pk_int<16>{}, pk_int<1>{}, pk_int<16>{});
 }
 
@@ -664,7 +670,7 @@ pgk_status pkgemm_nt(const bf16* a, int lda, const void* wp, void* c, int ldc, i
         return PGK_OK;
     };
     auto rows = [&](auto ntw, auto epilogue, auto ring) { return mt == 1 ? launch(ntw, epilogue, pk_int<1>{}, ring) : launch(ntw, epilogue, pk_int<2>{}, ring); };
-    auto one = [&](auto epilogue) { return g.ksteps == 32 ? rows(pk_int<1>{}, epilogue, pk_int<32>{}) : rows(pk_int<1>{}, epilogue, pk_int<16>{}); };
+    auto one = [&](auto epilogue) { return g.ksteps % 32 == 0 ? rows(pk_int<1>{}, epilogue, pk_int<32>{}) : rows(pk_int<1>{}, epilogue, pk_int<16>{}); };
     switch (epi) {
         case PK_EPI_BF16: return one(pk_int<PK_EPI_BF16>{});
         case PK_EPI_XIELU: return one(pk_int<PK_EPI_XIELU>{});
