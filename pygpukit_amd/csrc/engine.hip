@@ -2039,9 +2039,9 @@ static pgk_status decode_step_impl(Engine* e, int batch, hipStream_t st, int* la
     while (b0 < batch) {
         const int rem = batch - b0;
         pgk_status r;
-        // the MFMA projections cost the same for 3 as for 16 sequences (~1.0-1.2 ms per step on Qwen3-0.6B); the GEMV
+        // the MFMA projections cost little more for 16 sequences than for 3 (0.69-0.84 ms per step on Qwen3-0.6B at contexts to 300); the GEMV
         // kernels exist for M = 1, 2, 4, 8 only, so 3 / 5 / 6 / 7 sequences would take two or three weight passes there
-        // (measured: 7 sequences 2.46 ms against 1.05).  GEMV stays for exactly 1 and 2, and for 4 where batched_four does not hold.
+        // (7 sequences 2.46 ms).  GEMV stays for exactly 1 and 2, and for 4 where batched_four does not hold.
         const bool mfma_ok = e->batched_mfma && (rem >= e->batched_min || (e->batched_min == 5 && (rem == 3 || (rem == 4 && e->batched_four))));
         if (mfma_ok) {
             const int m = rem > e->batched_max ? e->batched_max : rem;
@@ -2127,9 +2127,10 @@ static pgk_status dense_prefill_rows(Engine* e, int n_seqs, const int32_t* h_slo
     const int g_so = hidden_splits(QD), g_sd = hidden_splits(I), g_sq = gsplit ? engine_gemm_qkv_splits(n, NQKV, H, D == 128) : 1;
     // RMSNorm without a pass of its own: o_proj and down_proj leave x = bf16(h gamma) and h's sums of squares, gate_up and QKV scale their rows
     // (Qwen3-0.6B, 1531 rows: a layer 124 -> 115 us, 3365 rows 193 -> 181; ms a prompt, a pass of its own / carried on tiles of 32 rows: 140 rows 1.53 / 1.48, 200
-    // 1.60 / 1.52, 450 1.85 / 1.73; on tiles of 64 rows 450 took 1.91).  engine_gemm_resid_pays says which products.  Below 512 rows wide models gain nothing by
-    // it (H = 4096, I = 14336, 140, 200 and 450 rows: 1.00x), and narrow ones keep the pass all the same (H = 512, 300 rows 0.38 / 0.34): there the two families of tiles
-    // are held to one another's sums, which a rounding in another place exceeds.
+    // 1.60 / 1.52, 450 1.85 / 1.73; on tiles of 64 rows 450 took 1.91; H = 1280, 1536 and 2048, 129..511 rows 1.02..1.14x).  engine_gemm_resid_pays says which products.
+    // Below 512 rows other widths keep the pass.  Wide ones would gain little (140, 300 and 450 rows: H = 2304 and 3072 1.00..1.03x, 2560 and 4096 1.00..1.02x but for one point, 300 rows of
+    // H = I = 4096 1.09x; Llama-3-8B shape 1.00x), narrow ones 1.13..1.20x (H = 512 and 768); but at H = 512 and 2176 the tests hold two families of tiles to one another's sums, which a
+    // rounding in another place exceeds.
     const bool carry = (n >= 512 || (H >= 1024 && H <= 2048)) && !ws && !staged && (c.weight_format == 0 || pkd) && engine_gemm_carry_ok(n, NQKV, H) && engine_gemm_carry_ok(n, 2 * I, H);
     const bool carry_o = carry && engine_gemm_resid_pays(n, H, QD, g_so), carry_d = carry && g_sq == 1 && engine_gemm_resid_pays(n, H, I, g_sd);
     const bool use_slabs = ws || g_so > 1 || g_sd > 1 || g_sq > 1;
@@ -2613,7 +2614,7 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
         if (ok) e->wide = 0xE8 | (H >= 1536 || !all_fixed ? 0x10 : 0) | (H >= 1536 && !all_fixed ? 0x06 : 0);
         // 4 sequences on the register kernels of engine_batched.hip.h, which round where the GEMV kernels of four rows do (Qwen3-0.6B, us a step at contexts to 300 and of
         // 1500: 776 -> 693, 909 -> 824).  Not e4m3 weights, which those scale in fp32 and these round to bf16, nor K below 1024, which take the kernels by way of an LDS image
-        // (H = 512, 8 layers: 176 against 256).
+        // (H = 512, 8 layers: 176 against 256).  Nor where ops_wide.hip takes four: with it on, H = 1024 alone is left.
         auto deep = [](int K) { return K == 1024 || K == 2048 || K == 3072 || K == 4096; };
         e->batched_four = !f8 && !(e->wide >> 4 & 1) && deep(H) && deep(I) && deep(QD);
     }

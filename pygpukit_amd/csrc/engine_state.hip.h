@@ -140,8 +140,8 @@ struct Engine {
     const bf16 *embed, *lm_head, *final_norm;
     std::vector<pgk_layer_weights_t> layers;
     int nsplit = 1, lm_blocks = 1, lm_cap = 1, log_cap = 4096;
-    bool batched_four = false;  // ... and chunks of 4
     bool batched_mfma = true;   // chunks of 3 and 5..16 sequences use engine_batched.hip.h (PGK_BATCHED_MFMA=0: GEMV kernels only, no ops_wide.hip either, =2: from 3 up)
+    bool batched_four = false;  // ... and chunks of 4
     int batched_min = 5, batched_max = 64;   // PGK_BATCHED_MAX=16: chunks of at most 16 sequences (one weight pass per chunk), the A/B switch of the tiled kernels
     int cu_count = 256;
     int wide = 0;               // bit M: M sequences decode on ops_wide.hip

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(const T* q, const T*
 typedef short sa_v4s __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int sa_voff(int row, int ch) { return row * 256 + ((ch ^ (((row & 3) << 2) | ((row >> 2) & 3))) << 4); }
 
-// Some 2 us of work behind a launch, all of it waiting: what the loads need is 13 dwords, preloaded into SGPRs (lens: q_len << 16 | kv_len), the head of
+// Some 2 us of work behind a launch, all of it waiting: what the loads need is 14 dwords, preloaded into SGPRs (lens: q_len << 16 | kv_len), the head of
 // the keys is a grid axis instead of a division, the queries come by LDS-DMA too (as registers their wait is the compiler's, who does not count the
 // DMAs, and it would be for everything), and the scores start when the keys are there, with the values still on their way.  Qwen3-0.6B, whole model, us,
 // before and after: 33 rows 1018 / 1000, 93 1112 / 1100, 128 1147 / 1136.
