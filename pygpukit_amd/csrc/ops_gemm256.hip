@@ -593,23 +593,30 @@ __global__ __launch_bounds__(G2_THREADS) void gemm256s_bf16_kernel(const bf16* A
 constexpr int GP_THREADS = 512;
 // stages of W that the ring holds; A's has two more.  The smaller tiles' stages are shorter, and latency asks for more of them
 constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 || (WM == 2 && WN == 4) ? 4 : 6; }
-// Tiles of 32 rows: a 2 x 2 split would leave a wave 16 rows.  There (gemmp_kg) the waves split K as well: of a pair of stages one wave of two multiplies the first, its
-// partner the second, each for a piece of 32 x 16 WN; one barrier a pair, and the partners trade halves of their sums at the end.
-constexpr bool gemmp_kg(int WM, int WN) { return WM == 1; }
-constexpr int GP_PAIRS = 6;                                  // pairs of stages in that ring: 12 KiB each for 32 x 64, two workgroups a CU
-template <int WM, int WN, bool B16> constexpr size_t gemmp_lds() {
+// Small tiles, whose stages are over before a barrier and the reads behind it are (gemmp_kg): the waves split K as well.  Of a pair of stages one wave of two multiplies the
+// first, its partner the second, each for a piece of 32 WM x 16 WN; one barrier a pair, fewer fragment reads, and the partners trade halves of their sums at the end.  What is left is
+// the rate of the LDS-DMA, 85 to 110 bytes a ns and CU.  Us a launch, the 2 x 2 split / this: K = 2048, N = 1024: 1531 rows, 96 x 64 13.0 / 12.1, 1000 rows, 64 x 64 10.4 / 9.1; K = 3072
+// 17.5 / 16.3 and 13.6 / 12.1; K = 1024, N = 6144, 93 rows, 64 x 64 5.9 / 5.3.  (64 x 128 has no registers for it: twice the time.)
+constexpr bool gemmp_kg(int EPI, int WM, int WN) { return WM == 1 || (EPI == 8 && WN == 2 && WM <= 3); }
+constexpr int gemmp_pairs(int WM, int WN) { return WM == 1 ? 6 : WM == 2 ? 5 : 4; }      // pairs of stages in that ring: at most 80 KiB, two workgroups a CU
+template <int EPI, int WM, int WN> constexpr size_t gemmp_lds() {
+    constexpr bool B16 = EPI == 3 || EPI == 4;
     const size_t RW = gemmp_ring(WM, WN), tile = (size_t)(32 * WM) * (32 * WN) * (B16 ? 2 : 4);
-    const size_t ring = gemmp_kg(WM, WN) ? GP_PAIRS * (size_t)(32 * (WM + WN) * 128) : (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64);
-    const size_t least = gemmp_kg(WM, WN) ? tile + 1024 + WM * WN * 4096 : tile;
+    const size_t ring = gemmp_kg(EPI, WM, WN) ? gemmp_pairs(WM, WN) * (size_t)(32 * (WM + WN) * 128) : (RW + 2) * (size_t)(32 * WM * 64) + RW * (size_t)(32 * WN * 64);
+    const size_t least = gemmp_kg(EPI, WM, WN) ? tile + 1024 + WM * WN * 4096 : tile;
     return ring > least ? ring : least;
 }
 struct BestOut { float* val; int* idx; };                    // [M][tiles of columns]
+// s_waitcnt's counts are immediates, so the ends of the rings, where a step less is in flight each time, are unrolled over T = 0, 1, ...
+template <int N> __device__ __forceinline__ void gp_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+template <class F, int... T> __device__ __forceinline__ void gp_steps(std::integer_sequence<int, T...>, F f) { (f(std::integral_constant<int, T>{}), ...); }
 template <int EPI, bool GRP, int WM, int WN>
 __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const bf16* bias, void* Cv,
                                            int M, int N, int K, int ntm, int ntn, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa, const GroupArgs& ga, const NormIn& ni, const NormOut& no, const BestOut& bo) {
     extern __shared__ __attribute__((aligned(16))) char g2_smem[];   // A: RA slots of AH bytes | W: RW stages of WH
     constexpr int BM = 32 * WM, BN = 32 * WN, RW = gemmp_ring(WM, WN), RA = RW + 2, AH = BM * 64, WH = BN * 64, NA = WM, NW = WN / 2;   // NA, NW: DMA instructions of a wave for a pair of A's / a stage of W's
-    constexpr bool KG = gemmp_kg(WM, WN);
+    constexpr bool KG = gemmp_kg(EPI, WM, WN);
+    constexpr int GP_PAIRS = gemmp_pairs(WM, WN);
     constexpr bool B16 = EPI == 3 || EPI == 4, ROWS = B16, SCALED = !GRP && (EPI == 0 || EPI == 3 || EPI == 4), PARTS = SCALED && EPI == 4 && BM == 64;   // PARTS: may come as ni.ld says
     static_assert(!SCALED || BM <= 256, "a row for each of the waves that multiply");
     static_assert(WN % 2 == 0 && (EPI != 3 || WN == 4), "W's pieces divide by four waves; a head is 128 columns");
@@ -634,6 +641,14 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     float mine = 0.f;                                        // 1 / rms of row tid (ni.ld: of tid / 4)
     const int part = (wid >> 1) & 1, kg = wid & 1;           // KG: which columns, which stage of a pair; behind the trade rows 16 WM kg .. of those columns
     const int wr = KG ? kg : part, wc = KG ? part : kg, q = lane >> 4, l15 = lane & 15;
+    // EPI 1, 8: this thread's words of the residual stream, requested behind the last DMA and the last product
+    constexpr int OLD = EPI == 1 || EPI == 8 ? BM * (BN / 4) / GP_THREADS : 0;
+    float4 old[OLD > 0 ? OLD : 1];
+    auto residual = [&]() {
+#pragma unroll
+        for (int it = 0; it < OLD; ++it)
+            old[it] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(Cv) + (size_t)min(m0 + (it * GP_THREADS + tid) / (BN / 4), M - 1) * N + min(n0 + tid % (BN / 4) * 4, N - 4));
+    };
     if (wid >= 4) {
         const int pw = __builtin_amdgcn_readfirstlane(wid & 3);
         auto a_row = [&](int r) -> int {
@@ -656,7 +671,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
             else w_src[i] = W + (size_t)min(row + (lane >> 2), wlast) * K + kbeg + ((lane & 3) ^ ((lane >> 4) & 2)) * 8;
         }
         const uint32_t lds0 = g2_lds_addr(g2_smem);
-        // past the end of K the last stage is read again (never consumed): the counts below stay constant
+        // a product of few stages fills the ring with its last one (never consumed)
         auto stage_a = [&](int h, int at) {                  // `at`: byte offset of the ring's slot
             const int k = min(h, nh - 2) * 32;
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + at + pw * NA * 1024);
@@ -671,7 +686,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         };
         if constexpr (KG) {
             constexpr int PB = 2 * (AH + WH), EACH = NA + 2 * NW;     // bytes and DMA instructions of a pair
-            auto stage_pair = [&](int p, int at) {           // past the end of K the last pair is read again
+            auto stage_pair = [&](int p, int at) {
                 const int h = min(2 * p, nh - 2);
                 const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + at);
 #pragma unroll
@@ -683,43 +698,72 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
             };
 #pragma unroll
             for (int p = 0; p < GP_PAIRS; ++p) stage_pair(p, p * PB);
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((GP_PAIRS - 1) * EACH) : "memory");      // pair 0
+            gp_wait<(GP_PAIRS - 1) * EACH>();                // pair 0
             __builtin_amdgcn_s_barrier();
-            int at = 0;
-            for (int p = 0; 2 * p < nh; ++p) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((GP_PAIRS - 2) * EACH) : "memory");  // pair p + 1; pair p is in registers behind the barrier
+            const int np = nh / 2;
+            int at = 0, p = 0;
+            for (; p + GP_PAIRS < np; ++p) {
+                gp_wait<(GP_PAIRS - 2) * EACH>();            // pair p + 1; pair p is in registers behind the barrier
                 __builtin_amdgcn_s_barrier();
                 stage_pair(p + GP_PAIRS, at);
                 at = at == (GP_PAIRS - 1) * PB ? 0 : at + PB;
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // retire the phantom DMAs: the ring becomes the C tile
-            __builtin_amdgcn_s_barrier();
+            residual();
+            if (np >= GP_PAIRS) {
+                gp_steps(std::make_integer_sequence<int, GP_PAIRS>{}, [&](auto t) {
+                    constexpr int LEFT = GP_PAIRS - 2 - decltype(t)::value;
+                    if constexpr (LEFT >= 0) gp_wait<LEFT * EACH + OLD>();
+                    __builtin_amdgcn_s_barrier();
+                });
+            } else {
+                gp_wait<OLD>();
+                for (; p < np; ++p) __builtin_amdgcn_s_barrier();
+            }
+            __builtin_amdgcn_s_barrier();                    // the ring becomes the C tile
             __builtin_amdgcn_s_barrier();                    // the partners' trade
         } else {
         // between W of a stage and the wait for it: W of RW - 2 stages and their A
-        auto wait_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RW - 2) * NW + (RW - 2) / 2 * NA) : "memory"); };
+        constexpr int YOUNGER = (RW - 2) * NW + (RW - 2) / 2 * NA;
         stage_a(0, 0);
 #pragma unroll
         for (int t = 0; t < RW; ++t) {
             if (t & 1) stage_a(t + 1, (t + 1) * AH);
             stage_w(t, t);
         }
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RW - 1) * NW + RW / 2 * NA) : "memory");   // stage 0
+        gp_wait<(RW - 1) * NW + RW / 2 * NA>();              // stage 0
         __builtin_amdgcn_s_barrier();
-        int at = 0, buf = 0;
-        for (int s = 0; s < nh; s += 2) {
-            wait_landed();                                   // stage s + 1
+        if (nh >= RW + 2) {
+            int at = 0, buf = 0, s = 0;
+            for (; s + RW + 2 < nh; s += 2) {
+                gp_wait<YOUNGER>();                          // stage s + 1
+                __builtin_amdgcn_s_barrier();
+                stage_w(s + RW, buf);
+                gp_wait<YOUNGER>();
+                __builtin_amdgcn_s_barrier();
+                stage_a(s + RA, at);
+                stage_w(s + RW + 1, buf + 1);
+                at = at == (RA - 2) * AH ? 0 : at + 2 * AH;
+                buf = buf == RW - 2 ? 0 : buf + 2;
+            }
+            gp_wait<YOUNGER>();
             __builtin_amdgcn_s_barrier();
             stage_w(s + RW, buf);
-            wait_landed();
+            gp_wait<YOUNGER>();
             __builtin_amdgcn_s_barrier();
-            stage_a(s + RA, at);
             stage_w(s + RW + 1, buf + 1);
-            at = at == (RA - 2) * AH ? 0 : at + 2 * AH;
-            buf = buf == RW - 2 ? 0 : buf + 2;
+            residual();
+            // the last RW stages: nothing is left to request.  (Requests for the last stage once more, which kept the counts constant, were waited for at the end.)
+            gp_steps(std::make_integer_sequence<int, RW>{}, [&](auto t) {
+                constexpr int LEFT = RW - 2 - decltype(t)::value, PAIRS = LEFT > 0 ? (LEFT + 1) / 2 - 1 : 0;      // stages requested behind the one waited for; their A
+                if constexpr (LEFT >= 0) gp_wait<LEFT * NW + PAIRS * NA + OLD>();
+                __builtin_amdgcn_s_barrier();
+            });
+        } else {
+            residual();
+            gp_wait<OLD>();
+            for (int s = 0; s < nh; ++s) __builtin_amdgcn_s_barrier();
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // retire the phantom DMAs: the stages become the C tile
-        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();                        // the stages become the C tile
         }
     } else {
         if constexpr (PARTS) {
@@ -781,6 +825,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
                 step(fa[1], fb[1], fa[0], fb[0]);
             }
             if (s < nh) step(fa[0], fb[0], fa[1], fb[1]);
+            residual();
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the reads past the last pair
             __builtin_amdgcn_s_barrier();
             // the lower rows of the piece to kg = 1, the upper ones to kg = 0; behind the C tile, which a faster wave may be writing
@@ -851,6 +896,7 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
         }
 #undef GP_STEP
 #undef GP_MFMA
+        residual();
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads past the last stage, before the stages become the C tile
         __builtin_amdgcn_s_barrier();
         }
@@ -901,17 +947,12 @@ __device__ __forceinline__ void gemmp_body(const bf16* A, const bf16* W, const b
     if constexpr (EPI == 3) hr.angles((tid & 15), tn, hd);
     auto tile4 = [&](int row, int byte) { return *reinterpret_cast<const float4*>(g2_smem + row * ROWB + (byte ^ (((row >> 2) & 3) << 6))); };
     if constexpr (EPI == 1 || EPI == 8) {
-        constexpr int IT = BM * (BN / 4) / GP_THREADS;
         const int c = tid % (BN / 4), gcol = n0 + c * 4;     // a thread's columns are the same in all its rows
-        float4 old[IT];
         uint2 gamma = make_uint2(0, 0);
         if constexpr (EPI == 8) gamma = *reinterpret_cast<const uint2*>(no.gamma + min(gcol, N - 4));
-#pragma unroll
-        for (int it = 0; it < IT; ++it)
-            old[it] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(Cv) + (size_t)min(m0 + (it * GP_THREADS + tid) / (BN / 4), M - 1) * N + min(gcol, N - 4));
         __syncthreads();
 #pragma unroll
-        for (int it = 0; it < IT; ++it) {
+        for (int it = 0; it < OLD; ++it) {
             const int row = (it * GP_THREADS + tid) / (BN / 4), grow = m0 + row;
             float4 v = tile4(row, c * 16);
             const bool live = grow < M && gcol < N;
@@ -1435,7 +1476,7 @@ pgk_status gemm256_bf16_swiglu_nt(const bf16* A, const bf16* W, bf16* act, int M
 template <int EPI, int WM, int WN>
 static pgk_status gemmp_launch(const bf16* A, const bf16* W, const bf16* bias, void* C, int M, int N, int K, int kps, const QkvHeadArgs& hd, int packed, const ActArgs& xa,
                                const NormIn& ni, const NormOut& no, hipStream_t st, const BestOut& bo = BestOut{}) {
-    constexpr size_t LDS = gemmp_lds<WM, WN, EPI == 3 || EPI == 4>();
+    constexpr size_t LDS = gemmp_lds<EPI, WM, WN>();
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemmp_bf16_kernel<EPI, WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
@@ -1564,7 +1605,7 @@ pgk_status gemm_few_logits_nt(const bf16* A, const bf16* wp, float* logits, floa
 
 template <int EPI>
 static pgk_status gemmp_grouped_launch(const bf16* A, const bf16* W, bf16* C, const GroupArgs& g, int max_tiles, int ntn, int N, int K, hipStream_t st) {
-    constexpr size_t LDS = gemmp_lds<4, 4, EPI == 4>();
+    constexpr size_t LDS = gemmp_lds<EPI, 4, 4>();
     static bool attr_done = false;
     if (!attr_done) {
         PGK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemmp_grouped_kernel<EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS));
