@@ -582,8 +582,8 @@ __device__ __forceinline__ void fold_new_token(const NewToken<D, G>& t, DecodeSt
     st.update(s, t.vn);
 }
 
-// split path: grid (nsplit, Hkv, batch)
-template <int D, int G, bool DIRECT>
+// split path: grid (nsplit, Hkv, batch).  U1: groups of 4 waves x PPW rows that a slice asks for at once
+template <int D, int G, bool DIRECT, int U1 = 8>
 __global__ __launch_bounds__(256) void attn_decode_kernel(unsigned long long* tl, AttnArgs a) {
     const TLStamp tls(tl);
     constexpr int LPR = D / 8, PPW = 64 / LPR, RS = D + 2;
@@ -638,14 +638,14 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(unsigned long long* tl
     // no address depends on the context length, so the new token's q/k/v and the slice's first 128 K/V rows are requested
     // before the position is even known (clamped addresses; masked later).  Before, the walk started one scalar and one
     // vector round trip later (position -> slice bounds -> addresses).  Slices beyond the context write empty records.
-    constexpr int U1 = 8;
     const int chunk = decode_chunk_len(a.span, a.nsplit, 4 * PPW);
     const int c0 = (int)blockIdx.x * chunk;
     NewTokenRaw<G> raw;
     new_token_load<D, G>(a, b, kvh, lane, raw);
     __builtin_amdgcn_sched_barrier(0);
     KVBatch<U1> kb0;
-    kv_issue<D, U1, 4>(kb0, a.kcache + head_off, a.vcache + head_off, c0 + wid * PPW, a.max_seq - 1, lane);
+    // (rows behind the slice are the next one's: its last row again, not theirs from another L2.  The last slice has no such end)
+    kv_issue<D, U1, 4>(kb0, a.kcache + head_off, a.vcache + head_off, c0 + wid * PPW, min((int)blockIdx.x == a.nsplit - 1 ? a.max_seq : c0 + chunk, a.max_seq) - 1, lane);
     __builtin_amdgcn_sched_barrier(0);
     const int pos = load_uniform_i32(a.positions + b);   // scalar path (pgk_device.hip.h): not queued behind the vector loads in flight
     const int ctx = min(pos + 1, a.max_seq);
@@ -834,8 +834,9 @@ __device__ __forceinline__ int am_voff(int row, int ch) { return row * 256 + ((c
 
 // OPROJ = false: the whole-context BATCH attention (one workgroup per (sequence, kv head), grid (Hkv, 1, batch)): the same
 // kernel without the W_o slice - the normalised heads leave as bf16 (attn_direct16) or fp32 (attn_direct) rows.
+// The position comes first, by way of the preloaded arguments, and no row behind it is asked for (the last one again: 192 rows whatever the context took a CU as long as 192 do).
 template <int G, bool OPROJ = true>
-__global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long* tl, AttnArgs a) {
+__global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long* tl, const bf16* kcache_, const bf16* vcache_, const int32_t* positions_, int max_seq_, int hkv_, AttnArgs a) {
     const TLStamp tls(tl);
     typedef __bf16 am_bf16x8 __attribute__((ext_vector_type(8)));
     typedef float am_f32x4 __attribute__((ext_vector_type(4)));
@@ -849,15 +850,17 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
     __shared__ __attribute__((aligned(16))) float attn[GD];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, q4 = lane >> 4;
-    const int kvh = blockIdx.x % a.hkv, rb = blockIdx.x / a.hkv, b = blockIdx.z;   // kv head fastest: XCD-aware (attn_oproj_kernel)
+    const int kvh = blockIdx.x % hkv_, rb = blockIdx.x / hkv_, b = blockIdx.z;   // kv head fastest: XCD-aware (attn_oproj_kernel)
     const int r0 = rb * a.rows_per_block;
     const int lr = threadIdx.x % LPW, rip = threadIdx.x / LPW;
     const int npass = a.rows_per_block / RPP;
     const bf16* wbase = a.w_o + (size_t)kvh * GD + lr * 8;
     const int ldw = a.hq * D;
-    const size_t head_off = (((size_t)b * a.hkv + kvh) * a.max_seq) * D;
-    const bf16* kc = a.kcache + head_off;
-    const bf16* vc = a.vcache + head_off;
+    const size_t head_off = (((size_t)b * hkv_ + kvh) * max_seq_) * D;
+    const bf16* kc = kcache_ + head_off;
+    const bf16* vc = vcache_ + head_off;
+    const int pos = load_uniform_i32(positions_ + b);
+    const int c1 = min(pos, max_seq_), last_row = max(c1 - 1, 0);        // cached positions [0, c1)
 
     // Issue order = arrival order, and every wait on it is written out here: the new token's inputs, the cache chunk and
     // nothing else go through LDS-DMA issued as inline asm, so the compiler neither counts them nor - as it does for the
@@ -897,13 +900,13 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
 #pragma unroll
         for (int i = 0; i < AM_CHUNK / 4 / NWV; ++i) {
             const int j = wid + NWV * i;
-            const int rl = 4 * j + q4, rg = min(c0 + rl, a.max_seq - 1);
+            const int rl = 4 * j + q4, rg = min(c0 + rl, last_row);
             dma(kc + (size_t)rg * D + ((l15 ^ (rl & 15)) << 3), lds_u32(k_lds) + j * 1024);
         }
 #pragma unroll
         for (int i = 0; i < AM_CHUNK / 4 / NWV; ++i) {
             const int j = wid + NWV * i;
-            const int rl = 4 * j + q4, rg = min(c0 + rl, a.max_seq - 1);
+            const int rl = 4 * j + q4, rg = min(c0 + rl, last_row);
             dma(vc + (size_t)rg * D + ((l15 ^ (((rl & 3) << 2) | ((rl >> 2) & 3))) << 3), lds_u32(v_lds) + j * 1024);
         }
     };
@@ -912,7 +915,6 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
 #pragma unroll
     for (int p = 0; p < PRE; ++p) pre[p] = load_nt16(wbase + (size_t)(r0 + min(p, npass - 1) * RPP + rip) * ldw);
     __builtin_amdgcn_sched_barrier(0);
-    const int pos = load_uniform_i32(a.positions + b);
     tls.phase(0);
     // in-order return: once at most the operations issued after them are outstanding, this wave's copy of the new token's inputs is in its slot
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (AM_CHUNK / 4 / NWV) + PRE) : "memory");
@@ -968,7 +970,6 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
     }
     tls.phase(1);
     uint4 qf[4];
-    const int c1 = min(pos, a.max_seq);                 // cached positions [0, c1)
     float m_run = -INFINITY, l_run = 0.f;                // of head l15 (lanes l15 >= G carry dummies)
     am_f32x4 o[D / 16];
 #pragma unroll
@@ -997,7 +998,7 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
                 Vec<bf16> kb, vb2;
                 kb.raw = k_sh[lane]; vb2.raw = v_sh[lane];
                 kb.to_float(kn); vb2.to_float(vn);
-                const bool live = pos < a.max_seq;
+                const bool live = pos < max_seq_;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     Vec<bf16> qb;
@@ -1153,7 +1154,7 @@ __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long lon
     static_assert(LPW <= 64 && 256 % LPW == 0, "row slice must fit a wave");
     __shared__ float w_s[G][64];
     __shared__ float inv_l[G];
-    __shared__ __attribute__((aligned(16))) float attn[GD];
+    __shared__ __attribute__((aligned(16))) float part_s[1024], attn[GD];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kvh = blockIdx.x % a.hkv, rb = blockIdx.x / a.hkv, b = blockIdx.z;
     const int r0 = rb * a.rows_per_block;
@@ -1171,18 +1172,18 @@ __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long lon
         m = hrecs[((size_t)wid * a.nsplit + sc) * RS];
         l = hrecs[((size_t)wid * a.nsplit + sc) * RS + 1];
     }
-    // ... and the records' value words of this thread's output element(s): up to 32 slices per element straight into
-    // registers, BEFORE the W_o stream and before the barrier below.  (They used to be read after the barrier, eight at a
-    // time: three to four dependent L2 round trips on the critical path of every layer at context 2048.)
-    constexpr int EPT = (GD + 255) / 256, RPRE = 32;
-    float rv[EPT][RPRE];
+    // ... and the records' values, four to a lane, BEFORE the W_o stream and before the barrier below: 40 slices' in one round trip.  The slices are dealt to groups of
+    // LPS threads, whose sums meet in LDS.  (A word of every slice to a thread was 32 instructions a wave for 32 slices, where this is 8, and a round trip of its own for the 33rd.)
+    constexpr int LPS = GD / 4, NG = 256 / LPS, U = (40 + NG - 1) / NG;
+    struct __attribute__((packed, aligned(8))) Four { float v[4]; };      // (a record's values start 8 bytes off a 16-byte line)
+    const int e4 = (int)threadIdx.x % LPS, grp = (int)threadIdx.x / LPS, g4 = e4 * 4 / D;
+    const float* vals = hrecs + (size_t)g4 * a.nsplit * RS + 2 + e4 * 4 % D;
+    Four rv[U];
+    auto values = [&](int s0) {
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-        const int e = min((int)threadIdx.x + 256 * i, GD - 1), g = e / D, d = e % D;
-        const float* recs = hrecs + (size_t)g * a.nsplit * RS + 2 + d;
-#pragma unroll
-        for (int u = 0; u < RPRE; ++u) rv[i][u] = recs[(size_t)min(u, a.nsplit - 1) * RS];
-    }
+        for (int u = 0; u < U; ++u) rv[u] = *reinterpret_cast<const Four*>(vals + (size_t)min(s0 + u * NG + grp, a.nsplit - 1) * RS);
+    };
+    values(0);
     __builtin_amdgcn_sched_barrier(0);
     uint4 pre[PRE];
     float psc[PRE];
@@ -1204,18 +1205,26 @@ __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long lon
     }
     __syncthreads();
     tls.phase(1);
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0;;) {
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-        const int e = (int)threadIdx.x + 256 * i;
-        if (e < GD) {
-            const int g = e / D, d = e % D;
-            const float* recs = hrecs + (size_t)g * a.nsplit * RS;
-            float o = 0.f;
+        for (int u = 0; u < U; ++u) {
+            const int sl = s0 + u * NG + grp;
+            const float w = sl < a.nsplit ? w_s[g4][min(sl, 63)] : 0.f;
 #pragma unroll
-            for (int u = 0; u < RPRE; ++u) o = fmaf(u < a.nsplit ? w_s[g][u] : 0.f, rv[i][u], o);   // same order as attn_merge_kernel
-            for (int s2 = RPRE; s2 < a.nsplit; ++s2) o = fmaf(w_s[g][s2], recs[(size_t)s2 * RS + 2 + d], o);
-            attn[e] = o * inv_l[g];
+            for (int i = 0; i < 4; ++i) sum[i] = sl < a.nsplit ? fmaf(w, rv[u].v[i], sum[i]) : sum[i];
         }
+        s0 += U * NG;
+        if (s0 >= a.nsplit) break;
+        values(s0);
+    }
+    *reinterpret_cast<float4*>(part_s + grp * GD + e4 * 4) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    __syncthreads();
+    for (int e = threadIdx.x; e < GD; e += 256) {
+        float o = 0.f;
+#pragma unroll
+        for (int n = 0; n < NG; ++n) o += part_s[n * GD + e];
+        attn[e] = o * inv_l[e / D];
     }
     __syncthreads();
     tls.phase(2);
@@ -1535,7 +1544,7 @@ static hipError_t launch_attn_mfma(dim3 grid, hipStream_t st, const AttnArgs& a)
         if (he != hipSuccess) return he;
         attr = true;
     }
-    return launch_k(attn_oproj_mfma_kernel<G, OPROJ>, grid, dim3(256), lds, st, a);
+    return launch_k(attn_oproj_mfma_kernel<G, OPROJ>, grid, dim3(256), lds, st, (const bf16*)a.kcache, (const bf16*)a.vcache, a.positions, a.max_seq, a.hkv, a);
 }
 
 // Slices per sequence of m sequences' split attention on attn_stream_kernel, or 0 where that kernel does not take them (launch_attn says where).  At
@@ -1628,6 +1637,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         if (!one) PGK_CHECK_HIP(merge());
         return PGK_OK;
     }
+    const bool few = decode_chunk_len(span, ns, 4 * (64 / (D / 8))) <= 6 * 4 * (64 / (D / 8));      // slices short of what eight groups ask for
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
     a.g_total = G;
@@ -1652,6 +1662,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         else if (fused) he = launch_k(attn_oproj_kernel<D, GG>, grid, dim3(256), 0, st, a);         \
         else if (direct && D == 128 && e->attn_mfma && m * (int)c.num_kv_heads <= e->cu_count) he = launch_attn_mfma<GG, false>(dim3(c.num_kv_heads, 1, m), st, a); \
         else if (direct) he = launch_k(attn_decode_kernel<D, GG, true>, grid, dim3(256), 0, st, a); \
+        else if (few) he = launch_k(attn_decode_kernel<D, GG, false, 6>, grid, dim3(256), 0, st, a); \
         else he = launch_k(attn_decode_kernel<D, GG, false>, grid, dim3(256), 0, st, a);            \
         break;
     switch (G) {
