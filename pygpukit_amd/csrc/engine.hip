@@ -1637,7 +1637,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         if (!one) PGK_CHECK_HIP(merge());
         return PGK_OK;
     }
-    const bool few = decode_chunk_len(span, ns, 4 * (64 / (D / 8))) <= 6 * 4 * (64 / (D / 8));      // slices short of what eight groups ask for
+    const int groups = decode_chunk_len(span, ns, 4 * (64 / (D / 8))) / (4 * (64 / (D / 8)));      // of a slice
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
     a.g_total = G;
@@ -1662,7 +1662,8 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         else if (fused) he = launch_k(attn_oproj_kernel<D, GG>, grid, dim3(256), 0, st, a);         \
         else if (direct && D == 128 && e->attn_mfma && m * (int)c.num_kv_heads <= e->cu_count) he = launch_attn_mfma<GG, false>(dim3(c.num_kv_heads, 1, m), st, a); \
         else if (direct) he = launch_k(attn_decode_kernel<D, GG, true>, grid, dim3(256), 0, st, a); \
-        else if (few) he = launch_k(attn_decode_kernel<D, GG, false, 6>, grid, dim3(256), 0, st, a); \
+        else if (groups <= 4) he = launch_k(attn_decode_kernel<D, GG, false, 4>, grid, dim3(256), 0, st, a); \
+        else if (groups <= 6) he = launch_k(attn_decode_kernel<D, GG, false, 6>, grid, dim3(256), 0, st, a); \
         else he = launch_k(attn_decode_kernel<D, GG, false>, grid, dim3(256), 0, st, a);            \
         break;
     switch (G) {
