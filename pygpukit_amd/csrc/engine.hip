@@ -1568,12 +1568,29 @@ static int stream_slices(const Engine* e, int m) {
     return chunk ? ceil_div(attn_span(e), chunk) : 0;
 }
 
+// KV slices per (sequence, kv head): as many as fit ONE wave of workgroups over the chip (a 257th workgroup waits
+// for a free CU and adds a tail: 33 slices x 8 heads measured 5 % slower than 32 at context 2048), never more than
+// the workspace was sized for (e->nsplit: ~64 positions per slice at the full cache length)
+// (batches stream enough KV bytes to want two workgroups per CU: measured 22.1 vs 24.6 us at 8 x 2048 positions)
+// Slices are cut by absolute position in whole position-group steps: only as many as the step's context tier needs
+// (the tier, not the cache length: with slices of a 4096-row cache a context of 400 kept 3 of 27 slices busy - 0.671 ms per
+// step against 0.623 on a 1024-row cache)
+static int attn_slices(const Engine* e, int m, int D, int* slice = nullptr) {
+    const int span = attn_span(e);
+    int ns = e->cu_count * (m >= 4 ? 2 : 1) / ((int)e->cfg.num_kv_heads * m);
+    const int ns_cap = ceil_div(span, 64) < e->nsplit ? ceil_div(span, 64) : e->nsplit;     // ~64 positions per slice at least, by the TIER (not the cache: a tier slices alike on every cache)
+    ns = ns < 1 ? 1 : (ns > ns_cap ? ns_cap : ns);
+    const int len = decode_chunk_len(span, ns, 4 * (64 / (D / 8)));
+    if (slice) *slice = len;
+    return ceil_div(span, len);
+}
+
 // `fused`: attention + o_proj partials in one kernel (one sequence at short context); `direct`: one workgroup per
 // (sequence, kv head) walks the whole (short) context and writes the normalised output - no merge launch; otherwise
-// split-KV slices, then `merged` (merge + o_proj partials in one launch) or the merge kernel.
+// split-KV slices, then `merged` (merge + o_proj partials in one launch), nothing (`records`: the consumer merges) or the merge kernel.
 template <int D>
 static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, bool direct, hipStream_t st, bool direct_bf16 = false,
-                              bool merged = false) {
+                              bool merged = false, bool records = false) {
     const auto& c = e->cfg;
     const auto& L = e->layers[layer];
     const int G = c.num_heads / c.num_kv_heads;
@@ -1592,17 +1609,8 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
     a.span = span;
     a.scale = 1.0f / sqrtf((float)D);
     a.part = e->part + (size_t)b0 * c.num_heads * e->nsplit * (D + 2);
-    // KV slices per (sequence, kv head): as many as fit ONE wave of workgroups over the chip (a 257th workgroup waits
-    // for a free CU and adds a tail: 33 slices x 8 heads measured 5 % slower than 32 at context 2048), never more than
-    // the workspace was sized for (e->nsplit: ~64 positions per slice at the full cache length)
-    // (batches stream enough KV bytes to want two workgroups per CU: measured 22.1 vs 24.6 us at 8 x 2048 positions)
-    int ns = e->cu_count * (m >= 4 ? 2 : 1) / (c.num_kv_heads * m);
-    const int ns_cap = ceil_div(span, 64) < e->nsplit ? ceil_div(span, 64) : e->nsplit;     // ~64 positions per slice at least, by the TIER (not the cache: a tier slices alike on every cache)
-    ns = ns < 1 ? 1 : (ns > ns_cap ? ns_cap : ns);
-    // slices are cut by absolute position in whole position-group steps: launch only as many as the step's context tier needs
-    // (the tier, not the cache length: with slices of a 4096-row cache a context of 400 kept 3 of 27 slices busy - 0.671 ms per
-    // step against 0.623 on a 1024-row cache)
-    a.nsplit = ceil_div(span, decode_chunk_len(span, ns, 4 * (64 / (D / 8))));
+    int slice;
+    a.nsplit = attn_slices(e, m, D, &slice);
     a.w_o = (const bf16*)L.w_o; a.w_o_scale = (const bf16*)L.s_o; a.H = c.hidden_size; a.rows_per_block = e->oproj_rows;
     a.opart = e->opart ? e->opart + (size_t)b0 * c.num_kv_heads * c.hidden_size : nullptr;
     // split-KV records -> attention rows, in the type that `direct` would leave
@@ -1637,7 +1645,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         if (!one) PGK_CHECK_HIP(merge());
         return PGK_OK;
     }
-    const int groups = decode_chunk_len(span, ns, 4 * (64 / (D / 8))) / (4 * (64 / (D / 8)));      // of a slice
+    const int groups = slice / (4 * (64 / (D / 8)));            // of a slice
     dim3 grid = fused ? dim3((c.hidden_size / e->oproj_rows) * c.num_kv_heads, 1, m) : dim3(a.nsplit, c.num_kv_heads, m);
     hipError_t he = hipSuccess;
     a.g_total = G;
@@ -1688,7 +1696,7 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         switch (G) { PGK_MO(1) PGK_MO(2) PGK_MO(4) default: break; }
 #undef PGK_MO
         PGK_CHECK_HIP(he);
-    } else if (!fused && !direct) {
+    } else if (!fused && !direct && !records) {
         PGK_CHECK_HIP(merge());
     }
     return PGK_OK;
@@ -1983,6 +1991,11 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
     const int H = c.hidden_size, I = c.intermediate_size, D = c.head_dim, QD = c.num_heads * D, NQKV = e->qkv_dim();
     float* h = e->h + (size_t)b0 * H;
     const bool direct = short_ctx && !(fp8 && M == 1);   // (one sequence on e4m3 weights has always merged split-KV records, whose error is a fifth smaller)
+    // One sequence: o_proj merges the split-KV records on their way in and leaves a partial vector per 2048 columns, gate_up adds those to its input, of which its first workgroup
+    // leaves the sum for down_proj to add to: two residual rows in turn, no launch for the merge
+    const int slices = M == 1 && !direct ? attn_slices(e, 1, D) : 0;
+    const bool merged = slices && wide_merge_ok(QD, D, slices);
+    float *other = e->h2 + (size_t)b0 * H, *parts = e->opart + (size_t)b0 * std::max((int)c.num_kv_heads, wide_merge_parts(QD)) * H;
     for (int l = 0; l < c.num_layers; ++l) {
         const auto& L = e->layers[l];
         FusedArgs a{};
@@ -1992,25 +2005,34 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
         a.out = e->qkv + (size_t)b0 * NQKV; a.ld_out = NQKV;
         if (pgk_status r = wide_proj(fp8, WIDE_NORM, EPI_STORE, a, nullptr, M, e->cu_count, nullptr, st)) return r;
         mark(KC_ATTN);
-        if (D == 128) { if (pgk_status r = launch_attn<128>(e, l, b0, M, false, direct, st)) return r; }
-        else { if (pgk_status r = launch_attn<64>(e, l, b0, M, false, direct, st)) return r; }
+        if (D == 128) { if (pgk_status r = launch_attn<128>(e, l, b0, M, false, direct, st, false, false, merged)) return r; }
+        else { if (pgk_status r = launch_attn<64>(e, l, b0, M, false, direct, st, false, false, merged)) return r; }
         mark(KC_OPROJ);
         a = FusedArgs{};
         a.w = L.w_o; a.wscale = (const bf16*)L.s_o; a.N = H; a.K = QD;
-        a.xin = e->attnv + (size_t)b0 * QD;
-        a.out = h; a.ld_out = H;
-        if (pgk_status r = wide_proj(fp8, WIDE_PLAIN, EPI_RESID, a, nullptr, M, e->cu_count, nullptr, st)) return r;
+        if (merged) {
+            a.part = e->part + (size_t)b0 * c.num_heads * e->nsplit * (D + 2); a.nsplit = slices; a.ld_out = D; a.out = parts;
+            if (pgk_status r = wide_proj(fp8, WIDE_MERGE, EPI_STORE, a, nullptr, M, e->cu_count, nullptr, st)) return r;
+        } else {
+            a.xin = e->attnv + (size_t)b0 * QD;
+            a.out = h; a.ld_out = H;
+            if (pgk_status r = wide_proj(fp8, WIDE_PLAIN, EPI_RESID, a, nullptr, M, e->cu_count, nullptr, st)) return r;
+        }
         mark(KC_GATEUP);
         a = FusedArgs{};
         a.w = L.w_gate_up; a.wscale = (const bf16*)L.s_gate_up; a.N = I; a.K = H;
         a.h = h; a.gamma = (const bf16*)L.mlp_norm; a.eps = c.norm_eps;
-        if (pgk_status r = wide_proj(fp8, WIDE_NORM, EPI_SWIGLU, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
+        if (merged) {
+            a.part = parts; a.nsplit = wide_merge_parts(QD); a.h_out = other;
+            std::swap(h, other);
+        }
+        if (pgk_status r = wide_proj(fp8, merged ? WIDE_NORM_SUM : WIDE_NORM, EPI_SWIGLU, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
         mark(KC_DOWN);
         a = FusedArgs{};
         a.w = L.w_down; a.wscale = (const bf16*)L.s_down; a.N = H; a.K = I;
         a.out = h; a.ld_out = H;
         if (pgk_status r = wide_proj(fp8, WIDE_PIECES, EPI_RESID, a, e->wide_act, M, e->cu_count, nullptr, st)) return r;
-        *launches += 4 + (direct || stream_slices(e, M) == 1 ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads, M);
+        *launches += 4 + (direct || merged || stream_slices(e, M) == 1 ? 0 : 1) + gqa_chunks(c.num_heads / c.num_kv_heads, M);
     }
     mark(KC_LMHEAD);
     FusedArgs a{};
@@ -2028,7 +2050,7 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
         *launches += 1;
     }
     PGK_CHECK_HIP(launch_k(finalize_kernel<bf16>, dim3(M), dim3(256), 0, st, a.amax_val, a.amax_idx, nblk, e->tokens + b0, e->positions + b0, e->token_log + b0, e->step_counter,
-                                       e->cfg.max_batch, e->log_cap, e->embed, h, H, last ? 1 : 0, b0 == 0 ? e->clk_log : nullptr,
+                                       e->cfg.max_batch, e->log_cap, e->embed, e->h + (size_t)b0 * H, H, last ? 1 : 0, b0 == 0 ? e->clk_log : nullptr,
                                        e->rope_cos, e->rope_sin, e->cur_cos + (size_t)b0 * (D / 2), e->cur_sin + (size_t)b0 * (D / 2),
                                        D / 2, c.max_seq_len, M, sampled, (const bf16*)nullptr, H));
     *launches += 2;
@@ -2585,7 +2607,7 @@ pgk_status pgk_engine_create(const pgk_model_config_t* cfg, const void* embed, c
     A((void**)&e->h2, (size_t)B * H * 4, &e->ws_bytes);
     A((void**)&e->qkv, (size_t)B * e->qkv_dim() * 4, &e->ws_bytes);
     A((void**)&e->part, (size_t)B * c.num_heads * e->nsplit * (D + 2) * 4, &e->ws_bytes);
-    A((void**)&e->opart, (size_t)B * c.num_kv_heads * H * 4, &e->ws_bytes);
+    A((void**)&e->opart, (size_t)B * std::max((int)c.num_kv_heads, wide_merge_parts(c.num_heads * D)) * H * 4, &e->ws_bytes);
     A((void**)&e->act16, (size_t)B * c.intermediate_size * 2, &e->ws_bytes);
     A((void**)&e->attnv16, (size_t)B * c.num_heads * c.head_dim * 2, &e->ws_bytes);
     A((void**)&e->x16, (size_t)B * H * 2, &e->ws_bytes);

@@ -25,6 +25,8 @@
 // than one.)
 // i.e. 6.2 TB/s on gate/up and 6.4 on lm_head.  One step: 5.34 -> 3.05 ms, 15.3 -> 3.43 ms, 4.68 -> 2.10 ms (context 700, 1100, 700).
 
+#include <algorithm>
+
 #include "wide.hip.h"
 
 namespace pgk {
@@ -48,6 +50,9 @@ struct WideArgs {
     bf16* pieces_out;
     float* amax_val;
     int* amax_idx;
+    const float* part;       // WIDE_NORM_SUM: [parts][K]; WIDE_MERGE: [K / ld_out heads][parts][2 + ld_out]
+    int parts;
+    float* h_out;
 };
 
 __device__ __forceinline__ f32x4_w mfma_w(const uint4& a, const uint4& b, f32x4_w c) {
@@ -79,13 +84,14 @@ template <bool FP8> __device__ __forceinline__ void piece_of(int k, int& blk, in
     j = k & 7;
 }
 
-// CH: chunks of 256 weight bytes per row and wave (0: run time, WIDE_PIECES only); MT: sequence slots.
+// CH: chunks of 256 weight bytes per row and wave (0: run time, WIDE_PIECES only); MT: sequence slots; NP: WIDE_NORM_SUM's partial vectors, WIDE_MERGE's slices, requested at once.
 // rows: output rows (SWIGLU: pairs) of a workgroup, a multiple of 8.
-template <class WT, int SRC, int EPI, int CH, int MT>
+template <class WT, int SRC, int EPI, int CH, int MT, int NP = 1>
 __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl, const void* w_, const bf16* wscale_, const float* x_, const bf16* gamma_, int N, int rows, int M,
                                                           int K, WideArgs a) {
     const TLStamp tls(tl);
-    constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value, REG = SRC != WIDE_PIECES;
+    constexpr bool FP8 = std::is_same<WT, fp8e4m3>::value, REG = SRC != WIDE_PIECES, SUM = SRC == WIDE_NORM_SUM, MERGE = SRC == WIDE_MERGE, NORM = SRC == WIDE_NORM || SUM;
+    static_assert(MT == 1 || !(SUM || MERGE), "partial vectors and records of one sequence");
     constexpr int KCH = 256 / sizeof(WT), STEPS = KCH / 32;      // k and matrix steps of a chunk
     constexpr int NS = 3, SS = MT < 8 ? 4 : 8;                   // pieces; operand rows s * SS + m
     // The third pieces of eight rows are an operand of their own: rows m those of an even step, rows 8 + m those of the step after it, and only
@@ -102,7 +108,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     const int r0 = blockIdx.x * rows, nr = min(rows, N - r0);
     constexpr int PER = EPI == EPI_SWIGLU ? 8 : 16;              // outputs of a tile
     const int T = (nr + PER - 1) / PER;
-    const int nch = K / KCH;
+    const int kb = MERGE ? (int)blockIdx.y * WIDE_RUN : 0, KL = MERGE ? min(WIDE_RUN, K - kb) : K;      // this workgroup's columns
+    const int nch = KL / KCH;
     constexpr int CHW = CH > 0 ? CH : 1;
     const int cw = REG ? CH : (nch + WD_WAVES - 1) / WD_WAVES;
     const int c0 = wid * cw;
@@ -114,13 +121,36 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     constexpr int XI = REG ? SL / 256 : 1;
     float4 xv[REG ? MT : 1][XI];
     uint2 gv[XI];
-    if constexpr (REG) {
+    if constexpr (REG && !MERGE) {
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             const int k = min(c0 * KCH + i * 256 + lane * 4, K - 4);
-            if constexpr (SRC == WIDE_NORM) gv[i] = *reinterpret_cast<const uint2*>(gamma_ + k);
+            if constexpr (NORM) gv[i] = *reinterpret_cast<const uint2*>(gamma_ + k);
 #pragma unroll
             for (int m = 0; m < MT; ++m) xv[m][i] = *reinterpret_cast<const float4*>(x_ + (size_t)min(m, M - 1) * K + k);
+        }
+    }
+    float4 pv[SUM || MERGE ? NP : 1][XI];
+    if constexpr (SUM) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int i = 0; i < XI; ++i) pv[p][i] = *reinterpret_cast<const float4*>(a.part + (size_t)min(p, a.parts - 1) * K + min(c0 * KCH + i * 256 + lane * 4, K - 4));
+    }
+    // Records of the wave's heads: values four to a lane, (m, l) of slice `lane` to a lane
+    constexpr int HPW = MERGE ? 4 : 1;                           // 64-column quarters of the slice; D = 128: of two heads
+    float2 ml[HPW];
+    struct __attribute__((packed, aligned(8))) Four { float v[4]; };      // (a record's values start 8 bytes off a 16-byte line)
+    if constexpr (MERGE) {
+        static_assert(!MERGE || XI == 1, "a wave's slice is 256 columns");
+        const int D = a.ld_out, rs = D + 2, k = min(kb + c0 * KCH + lane * 4, K - 4), first = min(kb + c0 * KCH, K - 256);
+#pragma unroll
+        for (int h = 0; h < HPW; ++h) ml[h] = *reinterpret_cast<const float2*>(a.part + ((size_t)((first + 64 * h) / D) * a.parts + min(lane, a.parts - 1)) * rs);
+        const float* rec = a.part + (size_t)(k / D) * a.parts * rs + 2 + k % D;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const Four f = *reinterpret_cast<const Four*>(rec + (size_t)min(p, a.parts - 1) * rs);
+            pv[p][0] = make_float4(f.v[0], f.v[1], f.v[2], f.v[3]);
         }
     }
     const int en = threadIdx.x & (PER - 1), em = (threadIdx.x / PER) & 7, et = threadIdx.x / (PER * 8);
@@ -148,12 +178,12 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
         const int row[2] = {half_row(lt, 0), half_row(lt, 1)};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const char* base = reinterpret_cast<const char*>(w_) + ((size_t)(row[i >> 1] + (i & 1) * 4) * K * sizeof(WT) + (size_t)ch * 256);
+            const char* base = reinterpret_cast<const char*>(w_) + ((size_t)(row[i >> 1] + (i & 1) * 4) * K * sizeof(WT) + (size_t)kb * sizeof(WT) + (size_t)ch * 256);
             rb[u][i] = load_nt16(base + w_lane);
         }
         if constexpr (FP8) {                                     // both scales of the chunk in one word; the halves of a tile may lie in different blocks
-            sc0[u] = *(scalar_u32)(wscale_ + (size_t)(row[0] >> 7) * (K >> 7) + ch * 2);
-            sc1[u] = *(scalar_u32)(wscale_ + (size_t)(row[1] >> 7) * (K >> 7) + ch * 2);
+            sc0[u] = *(scalar_u32)(wscale_ + (size_t)(row[0] >> 7) * (K >> 7) + (kb >> 7) + ch * 2);
+            sc1[u] = *(scalar_u32)(wscale_ + (size_t)(row[1] >> 7) * (K >> 7) + (kb >> 7) + ch * 2);
         }
         if constexpr (REG) { if (++lj == ncw) { lj = 0; ++lt; } }
     };
@@ -177,6 +207,45 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     // ---- activations -> pieces -> operands in registers ----
     uint4 A[REG ? CH * STEPS : 1];
     char* third = scratch + 8192;                                // [8 sequences][RS], behind the weights' chunks
+    if constexpr (SUM) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            if (p < a.parts) {
+#pragma unroll
+                for (int i = 0; i < XI; ++i) { xv[0][i].x += pv[p][i].x; xv[0][i].y += pv[p][i].y; xv[0][i].z += pv[p][i].z; xv[0][i].w += pv[p][i].w; }
+            }
+        if (blockIdx.x == 0) {
+#pragma unroll
+            for (int i = 0; i < XI; ++i)
+                if (const int k = c0 * KCH + i * 256 + lane * 4; k < K) *reinterpret_cast<float4*>(a.h_out + k) = xv[0][i];
+        }
+    }
+    if constexpr (MERGE) {                                       // the arithmetic of attn_merge_kernel, slice after slice
+        float w[HPW], inv[HPW];
+#pragma unroll
+        for (int h = 0; h < HPW; ++h) {
+            const float m = lane < a.parts ? ml[h].x : -INFINITY, l = lane < a.parts ? ml[h].y : 0.f, mx = wave_max(m);
+            w[h] = m == -INFINITY ? 0.f : __expf(m - mx);
+            const float tot = wave_sum(w[h] * l);
+            inv[h] = tot > 0.f ? 1.0f / tot : 0.f;
+        }
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+        const int h = lane >> 4;                                 // 64 columns are 16 lanes
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            float ws = 0.f;
+#pragma unroll
+            for (int x = 0; x < HPW; ++x) {
+                const float wx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[x]), p));
+                ws = h == x ? wx : ws;
+            }
+            if (p < a.parts) { o.x = fmaf(ws, pv[p][0].x, o.x); o.y = fmaf(ws, pv[p][0].y, o.y); o.z = fmaf(ws, pv[p][0].z, o.z); o.w = fmaf(ws, pv[p][0].w, o.w); }
+        }
+        float one = inv[0];
+#pragma unroll
+        for (int x = 1; x < HPW; ++x) one = h == x ? inv[x] : one;
+        xv[0][0] = make_float4(o.x * one, o.y * one, o.z * one, o.w * one);
+    }
     if constexpr (REG) {
         uint2 p3[TWO ? MT : 1][XI];
 #pragma unroll
@@ -186,8 +255,8 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
 #pragma unroll
             for (int i = 0; i < XI; ++i) {
                 float v[4] = {xv[m][i].x, xv[m][i].y, xv[m][i].z, xv[m][i].w};
-                if (c0 * KCH + i * 256 + lane * 4 >= K) v[0] = v[1] = v[2] = v[3] = 0.f;
-                if constexpr (SRC == WIDE_NORM) {
+                if (c0 * KCH + i * 256 + lane * 4 >= KL) v[0] = v[1] = v[2] = v[3] = 0.f;
+                if constexpr (NORM) {
                     const float g[4] = {__uint_as_float(gv[i].x << 16), __uint_as_float(gv[i].x & 0xFFFF0000u), __uint_as_float(gv[i].y << 16), __uint_as_float(gv[i].y & 0xFFFF0000u)};
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { ss = fmaf(v[e], v[e], ss); v[e] *= g[e]; }
@@ -202,7 +271,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
                     for (int e = 0; e < 4; ++e) v[e] = s == 0 ? rest(v[e], p[e]) : v[e] - p[e];
                 }
             }
-            if constexpr (SRC == WIDE_NORM) {
+            if constexpr (NORM) {
                 ss = wave_sum(ss);
                 if (lane == 0) s_ss[wid][m] = ss;
             }
@@ -246,7 +315,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     auto reduce = [&](int nt) {                                  // tiles [base_t, base_t + nt): sum the waves, epilogue
         __syncthreads();
         float inv = 1.f;
-        if constexpr (SRC == WIDE_NORM) {
+        if constexpr (NORM) {
             float t = 0.f;
 #pragma unroll
             for (int w = 0; w < WD_WAVES; ++w) t += s_ss[w][em < MT ? em : 0];
@@ -275,7 +344,7 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
                     float* o = a.out + (size_t)em * a.ld_out + n;
                     *o = (base_t + tt == et ? resv : *o) + y;
                 } else {
-                    a.out[(size_t)em * a.ld_out + n] = y;
+                    a.out[MERGE ? (size_t)blockIdx.y * N + n : (size_t)em * a.ld_out + n] = y;
                     if constexpr (EPI == EPI_LOGITS) { if (y > best_v) { best_v = y; best_i = n; } }
                 }
             }
@@ -374,24 +443,25 @@ __global__ __launch_bounds__(WD_THREADS) void wide_kernel(unsigned long long* tl
     tls.end();
 }
 
-template <class WT, int SRC, int EPI, int CH, int MT>
+template <class WT, int SRC, int EPI, int CH, int MT, int NP = 1>
 pgk_status launch_wide(const FusedArgs& a, bf16* pieces, int M, int cu_count, int* n_blk, hipStream_t st) {
     constexpr int KCH = 256 / sizeof(WT);
     constexpr int RS = CH * KCH * 2 + 16;
     constexpr int SCRATCH = wide_scratch(SRC != WIDE_PIECES ? RS : 0, MT);
     constexpr int LDS = WD_WAVES * SCRATCH + WD_TILES * WD_RED * 4;
     static_assert(LDS + 512 <= 160 * 1024, "wide_kernel: LDS");
-    auto kfn = &wide_kernel<WT, SRC, EPI, CH, MT>;
+    auto kfn = &wide_kernel<WT, SRC, EPI, CH, MT, NP>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     PGK_CHECK_HIP(attr);
     // one workgroup per CU while its tiles fit one reduction; the vocabulary is reduced in groups
-    int rows = ceil_div(ceil_div(a.N, cu_count), 8) * 8;
+    const int runs = SRC == WIDE_MERGE ? wide_merge_parts(a.K) : 1;
+    int rows = ceil_div(ceil_div(a.N, std::max(cu_count / runs, 1)), 8) * 8;
     constexpr int MOST = WD_TILES * (EPI == EPI_SWIGLU ? 8 : 16);
     if (EPI != EPI_LOGITS && rows > MOST) rows = ceil_div(ceil_div(a.N, ceil_div(rows, MOST) * cu_count), 8) * 8;
     const int grid = ceil_div(a.N, rows);
     if (n_blk) *n_blk = grid;
-    WideArgs wa{a.eps, a.out, a.ld_out, pieces, pieces, a.amax_val, a.amax_idx};
-    PGK_CHECK_HIP(launch_k(kfn, dim3(grid), dim3(WD_THREADS), LDS, st, a.w, a.wscale, SRC == WIDE_NORM ? a.h : a.xin, a.gamma, a.N, rows, M, a.K, wa));
+    WideArgs wa{a.eps, a.out, a.ld_out, pieces, pieces, a.amax_val, a.amax_idx, a.part, a.nsplit, a.h_out};
+    PGK_CHECK_HIP(launch_k(kfn, dim3(grid, runs), dim3(WD_THREADS), LDS, st, a.w, a.wscale, SRC == WIDE_NORM || SRC == WIDE_NORM_SUM ? a.h : a.xin, a.gamma, a.N, rows, M, a.K, wa));
     return PGK_OK;
 }
 
@@ -416,6 +486,16 @@ template <class WT>
 pgk_status launch_wide_e(int src, int epi, const FusedArgs& a, bf16* pieces, int M, int cu_count, int* n_blk, hipStream_t st) {
     if (src == WIDE_NORM && epi == EPI_STORE) return launch_wide_k<WT, WIDE_NORM, EPI_STORE>(a, pieces, M, cu_count, n_blk, st);
     if (src == WIDE_NORM && epi == EPI_SWIGLU) return launch_wide_k<WT, WIDE_NORM, EPI_SWIGLU>(a, pieces, M, cu_count, n_blk, st);
+    constexpr int F = std::is_same<WT, fp8e4m3>::value ? 2 : 1;          // a slice of 256 k per wave, or of 512
+    if (src == WIDE_NORM_SUM && epi == EPI_SWIGLU && M == 1) {
+        PGK_REQUIRE(a.nsplit >= 1 && a.nsplit <= 2 && a.part && a.h_out && a.h_out != a.h, "wide_proj: %d partial vectors", a.nsplit);
+        if (a.K <= 2048) return launch_wide<WT, WIDE_NORM_SUM, EPI_SWIGLU, 2 / F, 1, 2>(a, pieces, M, cu_count, n_blk, st);
+        return launch_wide<WT, WIDE_NORM_SUM, EPI_SWIGLU, 4 / F, 1, 2>(a, pieces, M, cu_count, n_blk, st);
+    }
+    if (src == WIDE_MERGE && epi == EPI_STORE && M == 1) {
+        PGK_REQUIRE(a.nsplit >= 1 && wide_merge_ok(a.K, a.ld_out, a.nsplit) && a.part, "wide_proj: %d slices of heads of %d", a.nsplit, a.ld_out);
+        return launch_wide<WT, WIDE_MERGE, EPI_STORE, 2 / F, 1, WIDE_SLICES>(a, pieces, M, cu_count, n_blk, st);
+    }
     if (src == WIDE_PLAIN && epi == EPI_RESID) return launch_wide_k<WT, WIDE_PLAIN, EPI_RESID>(a, pieces, M, cu_count, n_blk, st);
     if (src == WIDE_PIECES && epi == EPI_RESID) return launch_wide_k<WT, WIDE_PIECES, EPI_RESID>(a, pieces, M, cu_count, n_blk, st);
     if constexpr (std::is_same<WT, bf16>::value) {
