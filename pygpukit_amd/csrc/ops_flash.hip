@@ -78,6 +78,7 @@ struct FlashMany {
 // NORMALISED partial output (type T) and its (m, l) per row, and flash_merge_kernel combines them.
 struct FlashSplit {
     int nsplit;
+    int run;        // > 0: KV tiles of a run, as many runs as a query tile's tiles make (at most nsplit)
     float* ml;      // [nsplit][Hq][q_len][2]  (m in the exp2 domain, l)
     void* o;        // [nsplit][q_len][Hq][D] of T, or of fp32 (`wide`: up to 128 query rows, and several sequences in one launch)
     bool wide;
@@ -117,6 +118,13 @@ template <class T, int N> __device__ __forceinline__ void flash_gate_cols(const 
     }
 }
 
+// KV tiles and runs of query tile qt where runs hold `run` tiles
+__host__ __device__ inline int flash_tiles(int qt, int q_len, int kv_len) {
+    const int last = qt * FL_BQ + FL_BQ < q_len ? qt * FL_BQ + FL_BQ : q_len, end = kv_len - q_len + last;
+    return ((end < kv_len ? end : kv_len) + FL_BKV - 1) / FL_BKV;
+}
+__host__ __device__ inline int flash_runs(int qt, int q_len, int kv_len, int run) { return (flash_tiles(qt, q_len, kv_len) + run - 1) / run; }
+
 template <class T, int D, bool WIN = false, bool BIAS = false, int SIDES = 1>
 __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
                                                               int q_len, int kv_len, float scale_log2e, FlashStrides sd,
@@ -137,7 +145,7 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     const int kvh = id % hkv, rest = id / hkv;
     const int head = kvh * rep + rest % rep;
     const int rest2 = rest / rep;
-    int split, qt, row0 = 0, rows = q_len;
+    int split, qt, row0 = 0, rows = q_len, nsplit = sp.nsplit;
     if (many.items) {
         const FlashItem it = many.items[rest2 / sp.nsplit];
         split = rest2 % sp.nsplit;
@@ -151,6 +159,10 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
         out += (long long)row0 * sd.os;
         k += (st >> 16) * many.slot_stride;
         v += (st >> 16) * many.slot_stride;
+    } else if (!WIN && sp.run > 0) {
+        qt = (q_len + FL_BQ - 1) / FL_BQ - 1;
+        split = rest2;
+        for (nsplit = flash_runs(qt, q_len, kv_len, sp.run); split >= nsplit; nsplit = flash_runs(--qt, q_len, kv_len, sp.run)) split -= nsplit;
     } else {
         // heavy tiles first - and, when the launch is one round of two workgroups per CU (KV split), the second half of the ids in
         // ASCENDING weight: a CU's two residents are then a heavy and a light run (ids i and i + grid / 2 sit on the same CU when
@@ -181,7 +193,7 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     // this workgroup's run of KV tiles [t0, t1)
     const int first_kv = WIN ? causal_off + qt * FL_BQ - win.window + 1 : 0;
     const int tb = WIN && first_kv > 0 ? first_kv / FL_BKV : 0;            // tiles before it are outside every row's window
-    int t0 = tb + (int)((long long)(nt_all - tb) * split / sp.nsplit), t1 = tb + (int)((long long)(nt_all - tb) * (split + 1) / sp.nsplit);
+    int t0 = tb + (int)((long long)(nt_all - tb) * split / nsplit), t1 = tb + (int)((long long)(nt_all - tb) * (split + 1) / nsplit);
     int last = t1;                                  // where the loop ends; both sides pass as many barriers
     if constexpr (SIDES == 2) {
         const int half = (t1 - t0 + 1) / 2;
@@ -414,9 +426,9 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
     float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const int qrow = qw0 + ql;
-    if constexpr (WIN) { if (sp.nsplit == 1) inv *= flash_gate<T>(win, min(qrow, q_len - 1), head); }
+    if constexpr (WIN) { if (nsplit == 1) inv *= flash_gate<T>(win, min(qrow, q_len - 1), head); }
     if constexpr (std::is_same<T, bf16>::value && D == 128) {
-        if (sp.q8 != nullptr && sp.nsplit == 1) {       // workgroup-uniform
+        if (sp.q8 != nullptr && nsplit == 1) {       // workgroup-uniform
             // the lane's 64 dims (the partner lane ^ 32 holds the other 64), rounded to bf16 as the plain store would
             float amax = 0.f;
 #pragma unroll
@@ -442,19 +454,19 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
         }
     }
     if (qrow < q_len) {
-        float* wrow = sp.nsplit > 1 && sp.wide ? reinterpret_cast<float*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D : nullptr;
-        T* orow = sp.nsplit > 1 ? reinterpret_cast<T*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D
+        float* wrow = nsplit > 1 && sp.wide ? reinterpret_cast<float*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D : nullptr;
+        T* orow = nsplit > 1 ? reinterpret_cast<T*>(sp.o) + (((size_t)split * rows + row0 + qrow) * hq + head) * D
                                 : out + (size_t)head * sd.oh + (size_t)qrow * sd.os;
 #pragma unroll
         for (int i = 0; i < DT; ++i)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 float y[4] = {o[i][4 * g] * inv, o[i][4 * g + 1] * inv, o[i][4 * g + 2] * inv, o[i][4 * g + 3] * inv};
-                if constexpr (WIN) { if (win.gate.gc && sp.nsplit == 1) flash_gate_cols<T, 4>(win, qrow, head, i * 32 + 8 * g + 4 * h, y); }
+                if constexpr (WIN) { if (win.gate.gc && nsplit == 1) flash_gate_cols<T, 4>(win, qrow, head, i * 32 + 8 * g + 4 * h, y); }
                 if (wrow) *reinterpret_cast<float4*>(wrow + i * 32 + 8 * g + 4 * h) = make_float4(y[0], y[1], y[2], y[3]);
                 else *reinterpret_cast<uint2*>(orow + i * 32 + 8 * g + 4 * h) = make_uint2(pack16x2<T>(y[0], y[1]), pack16x2<T>(y[2], y[3]));
             }
-        if (sp.nsplit > 1 && h == 0) {
+        if (nsplit > 1 && h == 0) {
             float* ml = sp.ml + (((size_t)split * hq + head) * rows + row0 + qrow) * 2;
             ml[0] = m_run;
             ml[1] = l_tot;
@@ -469,11 +481,15 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
 // 100 at 2000 1450 / 1410, 1000 at 3000 3123 / 3090.
 template <class T, class P, int D, int RUNS>   // P: type of the partial rows
 __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const P* po, T* out, int hq, int q_len, int nsplit, long long oh, long long os,
-                                                          uint8_t* q8 = nullptr, float* q8s = nullptr, FlashWindow win = FlashWindow{}) {
+                                                          uint8_t* q8 = nullptr, float* q8s = nullptr, FlashWindow win = FlashWindow{}, int run = 0, int kv_len = 0) {
     constexpr int CPR = D / 8, RECS = RUNS == 8 ? 16 : RUNS;
     const uint32_t gid = blockIdx.x * 256u + threadIdx.x, rowi = gid / CPR;      // several runs: at most two workgroups of 128 rows to a CU (flash_plan)
     if (rowi >= (uint32_t)q_len * hq) return;          // the 16 lanes of a (row, head) stay together
     const int c = (int)(gid % CPR), qrow = (int)(rowi / (uint32_t)hq), head = (int)(rowi % (uint32_t)hq);
+    if (run > 0) {
+        nsplit = flash_runs(qrow / FL_BQ, q_len, kv_len, run);
+        if (nsplit == 1) return;                       // the run has left the row itself
+    }
     uint4 v[RUNS][sizeof(P) / 2];
     float2 r[RECS];
     auto rows = [&](int s0) {
@@ -554,7 +570,7 @@ static int flash_cus() {
 //  * Few workgroups (short of 5/8 of the CUs, 1200 positions and more): as many runs as two to a CU hold, of at least 2.5 KV tiles - more where many rows make the merge's
 //    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 23.3 / 15.9, 5000 56.3 / 26.3; 4 heads, 2048
 //    30.3 / 25.8; 8 heads, 2048 33.5 / 29.3.
-//  * Up to a workgroup per CU: two runs, of which a heavy and a light one share a CU.  16 heads, 1531 rows 31.5 (two sides 34.2), 1800 36.9 (39.0).
+//  * Up to a workgroup per CU (and no runs of flash_run_tiles): two runs, of which a heavy and a light one share a CU.  16 heads, 1531 rows 31.5 (two sides 34.2), 1800 36.9 (39.0).
 //  * Shorter contexts, at most a workgroup to four CUs: three or four runs whose rows stay fp32.  In 16 bits they were rounded twice: 2.27e-3 of float64 for 700 rows of 4 heads
 //    where two sides leave 2.00e-3 and these 1.98e-3.  1 head, 1024 rows 23.3 (two sides) / 14.6, 8 heads, 900 21.9 / 21.1.
 //  * Otherwise two sides beyond ten KV tiles, up to five workgroups to four CUs: 16 heads, 2300 rows 54.2 (one side) / 47.5; 32 heads, 1100 31.1 / 28.0.  Up to two to a CU only where
@@ -565,7 +581,28 @@ static int flash_cus() {
 // 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
 // (Results that are rounded to e4m3 next, by whichever kernel, ask for one side: the codes magnify a sum's last bit to a sixteenth, and a prompt in one pass and in pieces would
 // no longer agree - 4096 rows of 32 heads at once and as two of 2048, which alone had two sides, were 0.028 apart in the logits, with one side each under 0.01.)
-struct FlashPlan { int runs, sides; bool fp32; };       // fp32: of partial rows
+struct FlashPlan { int runs, sides; bool fp32; int run; };       // fp32: of partial rows; run: FlashSplit
+// KV tiles of a run where every query tile is cut into as many as it takes, so that the heavy ones do not decide: the fewest, four or more, with which a workgroup has a CU to itself (a few of
+// the lightest may share one: two to a CU take 1.8 times as long).  0: the rules below, for shapes that would need runs of more than 16 tiles.  Us with the merge, one launch behind another,
+// equal runs or sides / this: 16 heads, 1200 rows 28.4 / 24.6, 1531 33.3 / 30.2 (between a layer's other kernels 31.0 / 29.9), 1700 36.1 / 34.8; 8 heads, 1600 26.5 / 23.3, 2048 30.6 / 28.4;
+// 4 heads, 1600 22.0 / 18.5, 2048 25.0 / 21.3; 1000 at 250 27.4 / 24.6; 1 head, 5000 rows, which the rules below cut into 12, 25.1 / 25.8.  Under 1200 keys partial rows are fp32 (below).
+// Deeper in a context nearly every row has partial rows, which lose a bit where they are rounded to 16 bits (1 % more error than the equal runs leave) and time where they are not (800 at 700
+// 30.1 / 32.1, 900 at 800 32.2 / 35.5).
+static int flash_run_tiles(int tiles, int hq, int q_len, int kv_len, int most) {
+    const int cus = flash_cus();
+    for (int run = 4; run <= 16; ++run) {
+        long long wgs = 0;
+        int runs = 1, over = 0;                                  // over: the largest run beyond the CUs
+        for (int qt = tiles - 1; qt >= 0; --qt) {
+            const int n = flash_runs(qt, q_len, kv_len, run);
+            runs = std::max(runs, n);
+            wgs += (long long)n * hq;
+            if (wgs > cus) over = std::max(over, ceil_div(flash_tiles(qt, q_len, kv_len), n));
+        }
+        if (runs <= most && (wgs <= cus || (2 * over <= run && 4 * wgs <= 5LL * cus))) return run;
+    }
+    return 0;
+}
 static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
     if (kv_len < 2LL * q_len) {
@@ -576,14 +613,14 @@ static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
         else if (4 * wgs <= cus) n = 8 * wgs <= cus ? std::min(nt / 3, 4) : std::min(nt / 4, 3);
         if (fp32 && n < 3) n = 1;
         n = std::min<long long>(n, most);
-        if (n > 1) return {(int)n, 1, fp32};
-        return {1, nt > 10 && (4 * wgs <= 5 * cus || (wgs <= 2 * cus && !fp32 && 4LL * kv_len <= 5LL * q_len)) ? 2 : 1, false};
+        if (n > 1) return {(int)n, 1, fp32, 0};
+        return {1, nt > 10 && (4 * wgs <= 5 * cus || (wgs <= 2 * cus && !fp32 && 4LL * kv_len <= 5LL * q_len)) ? 2 : 1, false, 0};
     }
     long long n = cus / wgs;
     if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
     if (n > most) n = most;
     if (n > ceil_div(kv_len, FL_BKV) / 4) n = ceil_div(kv_len, FL_BKV) / 4;
-    return {n < 1 ? 1 : (int)n, 1, false};
+    return {n < 1 ? 1 : (int)n, 1, false, 0};
 }
 // with a sliding window: up to four runs over the `span` keys that the heaviest query tile walks, until two workgroups per CU are reached
 static int flash_window_runs(long long wgs, int span) {
@@ -599,16 +636,18 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
                                const FlashMany& many = FlashMany{}, bool one_side = false) {
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-    const FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1, false} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
+    FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1, false, 0} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
+    if (!WIN && !many.items && !one_side && kv_len >= 1200 && 4LL * kv_len <= 5LL * q_len && plan.runs <= 8)
+        if (const int run = flash_run_tiles(tiles, hq, q_len, kv_len, 16)) plan = {flash_runs(tiles - 1, q_len, kv_len, run), 1, false, run};
     int nsplit = plan.runs;
     const bool wide = many.items || q_len <= 128 || plan.fp32;
     // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
     // tiles of the first-generation kernel 61, 31 and 239)
     if (nsplit > 1 && q_len <= 128) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) nsplit = 1;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) nsplit = 1, plan.run = 0;
     }
-    FlashSplit sp{nsplit, nullptr, nullptr, wide, q8, q8s};
+    FlashSplit sp{nsplit, plan.run, nullptr, nullptr, wide, q8, q8s};
     void* ws = nullptr;
     if (nsplit > 1) {
         const size_t po_bytes = (size_t)nsplit * q_len * hq * D * (wide ? 4 : sizeof(T)), ml_bytes = (size_t)nsplit * hq * q_len * 2 * sizeof(float);
@@ -616,7 +655,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
             sp.o = ws;
             sp.ml = (float*)((char*)ws + ((po_bytes + 255) & ~(size_t)255));
         } else {
-            nsplit = sp.nsplit = 1;        // no memory, or a stream whose end the pool cannot see: slower, and right
+            nsplit = sp.nsplit = 1, sp.run = 0;        // no memory, or a stream whose end the pool cannot see: slower, and right
         }
     }
     auto launch = [&](auto sides) -> hipError_t {
@@ -628,7 +667,12 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
             if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS); e != hipSuccess) return e;
             attr_done = true;
         }
-        kernel<<<tiles * hq * nsplit, SIDES * FL_THREADS, LDS, st>>>(q, k, v, out, hq, hkv, q_len, kv_len, scale * 1.4426950408889634f, sd, sp, win, many);
+        int wgs = tiles * nsplit;
+        if (sp.run > 0) {
+            wgs = 0;
+            for (int i = 0; i < tiles; ++i) wgs += flash_runs(i, q_len, kv_len, sp.run);
+        }
+        kernel<<<wgs * hq, SIDES * FL_THREADS, LDS, st>>>(q, k, v, out, hq, hkv, q_len, kv_len, scale * 1.4426950408889634f, sd, sp, win, many);
         return hipGetLastError();
     };
     hipError_t e;
@@ -639,7 +683,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
         const unsigned grid = (unsigned)((work + 255) / 256);
         auto merge = [&](auto* part, auto runs) {
             using P = std::remove_pointer_t<decltype(part)>;
-            flash_merge_kernel<T, P, D, decltype(runs)::value><<<grid, 256, 0, st>>>(sp.ml, (const P*)part, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win);
+            flash_merge_kernel<T, P, D, decltype(runs)::value><<<grid, 256, 0, st>>>(sp.ml, (const P*)part, out, hq, q_len, nsplit, sd.oh, sd.os, q8, q8s, win, sp.run, kv_len);
         };
         auto pick = [&](auto* part) {
             if (nsplit <= 2) merge(part, std::integral_constant<int, 2>{});

@@ -1031,6 +1031,17 @@ def test_sdpa_of_few_workgroups_in_runs(dt, cfg):
         test_sdpa_nan_and_infinite_keys(cfg)
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("cfg", [(16, 8, 1250, 1250, 128), (16, 2, 1531, 1536, 128), (16, 16, 1281, 1281, 64), (8, 8, 2047, 2047, 128), (4, 2, 1600, 1663, 64), (16, 8, 1000, 1250, 128), (12, 2, 1030, 1281, 64)])
+def test_sdpa_in_runs_of_as_many_tiles(dt, cfg):
+    """Query tiles cut into as many runs as their keys take on a card of 256 CUs: 1 to 6, single ones left without a merge, a last query tile of one row and a context
+    before the rows.  The bars of the tests that are called."""
+    test_sdpa_few_rows_over_a_long_context(dt, cfg)
+    test_sdpa_reads_nothing_behind_the_context(dt, cfg)
+    if dt == "bfloat16" and cfg[1] == 2:
+        test_sdpa_nan_and_infinite_keys(cfg)
+
+
 # ----------------------------------------------------------------------------- paged KV cache / continuous batching
 def _paged_setup(rng, num_seqs, hkv, bs, d, ctxs, dt, num_blocks=None):
     max_blocks = max((c + bs - 1) // bs for c in ctxs) + 1
