@@ -53,8 +53,8 @@ struct FlashStrides { long long qh, qs, kh, ks, oh, os; };
 // One wave-instruction of LDS-DMA: 64 lanes x 16 bytes at per-lane byte offsets of a buffer to LDS [lds, +1024), zeros beyond its end.  (Inline asm: for the
 // builtin hipcc waits for the DMA in front of the next LDS read, whichever buffer that reads.  The waits are the explicit ones in the kernel.)
 typedef uint32_t fl_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void fl_dma16(const fl_u32x4& buffer, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buffer), "s"(lds) : "memory", "m0");
+__device__ __forceinline__ void fl_dma16(const fl_u32x4& buffer, uint32_t off, uint32_t lds, int at) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buffer), "s"(lds), "i"(at) : "memory", "m0", "scc");
 }
 __device__ __forceinline__ uint32_t fl_lds_addr(const char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p; }
 
@@ -136,8 +136,6 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     extern __shared__ __attribute__((aligned(16))) char fl_smem[];   // of each side K[2] | V[2]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wid = wave & 3, ql = lane & 31, h = lane >> 5;
     const int side = SIDES == 1 ? 0 : wave >> 2, side_at = side * (2 * K_BYTES + 2 * V_BYTES);
-    auto Ks = [&](int buf) -> char* { return fl_smem + side_at + buf * K_BYTES; };
-    auto Vs = [&](int buf) -> char* { return fl_smem + side_at + 2 * K_BYTES + buf * V_BYTES; };
 
     // workgroup id -> (kv head, query head in its group, query tile, KV run), heavy tiles first
     const int rep = hq / hkv;
@@ -215,18 +213,22 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
         vo[i] = (uint32_t)(r * sd.ks + (ds ^ fl_v_sw<D>(r)) * 8) * 2;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(fl_lds_addr(fl_smem) + side_at + wid * NI * 1024), row_bytes = (uint32_t)(sd.ks * 2);
-    auto tile_of = [&](const T* base, int t) {
-        const uint64_t at = (uint64_t)(uintptr_t)(base + (size_t)t * FL_BKV * sd.ks);
-        const int last = t < t1 ? min(kv_len - t * FL_BKV, FL_BKV) - 1 : -1;     // last row that is there
-        return fl_u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xFFFFu, last < 0 ? 0u : last * row_bytes + 2 * D, 0x00020000u};   // raw, 32-bit words
+    const uint64_t tile_bytes = (uint64_t)sd.ks * (FL_BKV * 2);
+    const int kv_stop = min(kv_len, t1 * FL_BKV);
+    auto bytes_of = [&](int t) { const int n = min(kv_stop - t * FL_BKV, FL_BKV); return n > 0 ? (n - 1) * row_bytes + 2 * D : 0u; };
+    auto tile_at = [&](uint64_t at, uint32_t bytes) { return fl_u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xFFFFu, bytes, 0x00020000u}; };   // raw, 32-bit words
+    uint64_t k_at = (uint64_t)(uintptr_t)kh + t0 * tile_bytes, v_at = (uint64_t)(uintptr_t)vh + t0 * tile_bytes;       // where the next DMA reads
+    auto dma_k = [&](int buf, uint32_t bytes) {
+        const fl_u32x4 tile = tile_at(k_at, bytes);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fl_dma16(tile, ko[i], lds0, buf * K_BYTES + i * 1024);
+        k_at += tile_bytes;
     };
-    auto dma_k = [&](const fl_u32x4& tile, int t, int i) { fl_dma16(tile, ko[i], lds0 + (t & 1) * K_BYTES + i * 1024); };
-    auto dma_v = [&](const fl_u32x4& tile, int t, int i) { fl_dma16(tile, vo[i], lds0 + 2 * K_BYTES + (t & 1) * V_BYTES + i * 1024); };
-    // what iteration t requests, in KS pieces: K of t + 2, V of t + 1
-    static_assert(2 * NI == KS, "a piece of the DMA per k-step");
-    auto dma_next = [&](int t, int piece) {
-        if (piece < NI) dma_k(tile_of(kh, t + 2), t + 2, piece);
-        else dma_v(tile_of(vh, t + 1), t + 1, piece - NI);
+    auto dma_v = [&](int buf, uint32_t bytes) {
+        const fl_u32x4 tile = tile_at(v_at, bytes);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fl_dma16(tile, vo[i], lds0, 2 * K_BYTES + buf * V_BYTES + i * 1024);
+        v_at += tile_bytes;
     };
     // S^T = K . Q^T of one tile: two 32-kv sub-tiles (rows = positions, column = this lane's query)
     const float slope = BIAS ? win.slopes[head] * win.inv_scale : 0.f;
@@ -243,7 +245,10 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
             for (int r = 0; r < 16; ++r) { s0[r] = 0.f; s1[r] = 0.f; }
         }
     };
-    auto k_frag = [&](const char* kb, int half, int ks) { return *reinterpret_cast<const uint4*>(kb + fl_k_off<D>(32 * half + ql, 2 * ks + h)); };
+    const char* ka[KS];                  // of the first buffer and sub-tile
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ka[ks] = fl_smem + side_at + fl_k_off<D>(ql, 2 * ks + h);
+    auto k_frag = [&](int buf, int half, int ks) { return *reinterpret_cast<const uint4*>(ka[ks] + buf * K_BYTES + half * 64 * D); };
     // tiles entirely above this wave's diagonal contribute nothing (wave-uniform)
     auto live = [&](int t) -> bool {
         return t < t1 && t * FL_BKV <= causal_off + qw0 + 31 && (!WIN || t * FL_BKV + FL_BKV - 1 > causal_off + qw0 - win.window);
@@ -254,13 +259,17 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     // and V(t) have landed and S(t) and O(t - 1) have been read.  Attention with merge, us, staged through registers with S(t) in front of its softmax / this: 16
     // heads, 1531 rows 35.4 / 30.6, 384 at 3585 34.0 / 29.0; 32 heads, 4096 rows 180 / 151.  (As two conditional blocks hipcc keeps S(t + 1) and the softmax apart; the
     // DMA a piece behind each k-step, inside the block, spills 74 registers.)
-    f32x16_fl sc0, sc1;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) dma_k(tile_of(kh, t0), t0, i);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) dma_k(tile_of(kh, t0 + 1), t0 + 1, i);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) dma_v(tile_of(vh, t0), t0, i);
+    // A pass of the loop is two tiles: the buffers' places are immediates then, and S(t + 1) is not copied.  V is read a k-step ahead of its products (the first under the last of S), the first of K
+    // above the softmax; the row sums and the next tile's largest scores are taken under the products with V, where only the matrix units had work, and waves there go first (s_setprio): two on a
+    // SIMD otherwise meet in the same phase.  Before / with all of it, us: 16 heads, 1531 rows 29.7 / 27.7, 384 at 3585 30.2 / 27.8, 400 13.4 / 11.9, 2500 52.2 / 45.2; 32 heads, 1000 rows 26.4 / 23.9,
+    // 3000 99 / 83.6, 4096 171 / 143 (of it s_setprio 88.6 / 83.6 and 155 / 143).  A tile was 270 vector instructions beside 32 matrix instructions, of which two waves overlapped a tenth.
+    // (As a lambda called for both tiles the windows' kernels spill 70 registers.)
+    constexpr bool AHEAD = !WIN;         // V, sums and scores: windows have no registers for it
+    f32x16_fl sc[2][2];                  // S of a pass's two tiles
+    dma_k(0, bytes_of(t0));
+    uint32_t v_bytes = bytes_of(t0 + 1);
+    dma_k(1, v_bytes);
+    dma_v(0, bytes_of(t0));
     // Q^T fragments (B operand): lane = query column, k = d
     {
         const T* qrow = qh + (size_t)min(qw0 + ql, q_len - 1) * sd.qs + 8 * h;
@@ -273,12 +282,12 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    s_init(t0, sc0, sc1);
+    s_init(t0, sc[0][0], sc[0][1]);
     if (live(t0)) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            sc0 = mfma32<T>(k_frag(Ks(t0 & 1), 0, ks), qf[ks], sc0);
-            sc1 = mfma32<T>(k_frag(Ks(t0 & 1), 1, ks), qf[ks], sc1);
+            sc[0][0] = mfma32<T>(k_frag(0, 0, ks), qf[ks], sc[0][0]);
+            sc[0][1] = mfma32<T>(k_frag(0, 1, ks), qf[ks], sc[0][1]);
         }
     }
     // V^T fragments: lane l gets dim 32 i + (l & 31) of rows 16 s + 8 u + 4 h .. + 3.  A 16-lane group's transposing read covers 4 rows x 16
@@ -287,21 +296,53 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     typedef short fl_v4s __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) fl_v4s* fl_lds_v4;
     const int tr = (lane & 15) >> 2, tc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), t8 = 8 * (lane & 1);
-    for (int t = t0; t < last; ++t) {
-        const int buf = t & 1, kv0 = t * FL_BKV;
+    const char* va[DT][2];
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) va[i][u] = fl_smem + side_at + 2 * K_BYTES + fl_v_off<D>(8 * u + 4 * h + tr, 4 * i + tc) + t8;
+    auto v_frag = [&](int buf, int i, int u, int s) {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][u] + buf * V_BYTES + s * 32 * D)));
+    };
+    // this lane's largest score, in two chains.  (This file is built with -fno-honor-nans: without it every operand of a max is first canonicalised with a v_max_f32 x, x, x of
+    // its own.)
+    auto largest = [&](const f32x16_fl& a, const f32x16_fl& b) -> float {
+        float x = -INFINITY, y = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            x = fmaxf(fmaxf(x, a[r]), a[r + 1]);
+            y = fmaxf(fmaxf(y, b[r]), b[r + 1]);
+        }
+        return fmaxf(x, y);
+    };
+    // ... and the row's (the other half of it is in lane ^ 32), in the log2 domain: -inf stays -inf (scale > 0)
+    auto scaled = [&](float x) -> float {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * scale_log2e;
+    };
+    float top = -INFINITY;               // of S(t), before a mask
+    if constexpr (AHEAD) top = scaled(largest(sc[0][0], sc[0][1]));
+    // tile t: sc0 | sc1 are S(t), sn0 | sn1 become S(t + 1); V(t) is in buffer buf, K(t + 1) in the other
+    for (int t2 = t0; t2 < last; t2 += 2)
+#pragma unroll
+    for (int buf = 0; buf < 2; ++buf) {
+        const int t = t2 + buf, kv0 = t * FL_BKV;
+        if (buf && t == last) break;
+        f32x16_fl &sc0 = sc[buf][0], &sc1 = sc[buf][1], &sn0 = sc[buf ^ 1][0], &sn1 = sc[buf ^ 1][1];
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // this wave's share of K(t + 1) and V(t)
         __syncthreads();                                                 // ... everyone's; and everyone has read K(t) and V(t - 1)
-#pragma unroll
-        for (int i = 0; i < KS; ++i) dma_next(t, i);
-        if (live(t)) {
-            f32x16_fl sn0, sn1;                                          // S(t + 1); behind the last tile of what K's other buffer holds, and unused
-            const char* kn = Ks(buf ^ 1);
+        const uint32_t k_bytes = bytes_of(t + 2);
+        dma_k(buf, k_bytes);
+        dma_v(buf ^ 1, v_bytes);
+        v_bytes = k_bytes;
+        if (live(t)) {                                                   // (behind the last tile, S(t + 1) is of what K's other buffer holds, and unused)
+            uint4 k0 = k_frag(buf ^ 1, 0, 0), k1 = k_frag(buf ^ 1, 1, 0);
             // ---- mask, online softmax (this lane: query qw0 + ql, kv rows (r&3) + 8(r>>2) + 4h of each sub-tile) ----
             const bool need_mask = kv0 + FL_BKV - 1 > causal_off + qw0 || kv0 + FL_BKV > kv_len ||
                                    (WIN && kv0 <= causal_off + qw0 + 31 - win.window);   // wave-uniform
             const int lim = min(causal_off + qw0 + ql, kv_len - 1) - kv0 - 4 * h;                  // local kv row <= lim is visible
             const int low = WIN ? causal_off + qw0 + ql - win.window + 1 - kv0 - 4 * h : 0;       // ... and >= low with a window
-            float mx = -INFINITY;
+            float mx = top;
             if (need_mask) {   // diagonal / ragged tiles only: a real wave-uniform branch, not 32 predicated selects per tile
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
@@ -310,15 +351,7 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
                     sc1[r] = 32 + kvl <= lim && (!WIN || 32 + kvl >= low) ? sc1[r] : -INFINITY;
                 }
             }
-            // (this file is built with -fno-honor-nans: without it every operand of a max is first canonicalised with a
-            // v_max_f32 x, x, x of its own - 60 instructions for these 32 values instead of 16 v_max3_f32)
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(fmaxf(sc0[r], sc1[r]), fmaxf(sc0[r + 1], sc1[r + 1])), mx);
-            {   // with the other half of the rows, lane ^ 32
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-                mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-            }
-            mx *= scale_log2e;                                           // -inf stays -inf (scale > 0)
+            if (!AHEAD || need_mask) mx = scaled(largest(sc0, sc1));
             // Deferred rescale: the reference point of a row only moves when its maximum grew by more than 6 (log2
             // domain), so probabilities stay <= 64 (exact in fp32 sums, fine in 16-bit P) and on most tiles - for the whole
             // wave - alpha is exactly 1 and the 64-multiply rescale of O is skipped.
@@ -332,61 +365,74 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
             }
-            float ls = 0.f;
+            uint4 vf[2][DT];                                             // V, a k-step ahead of its products
+            auto load_v = [&](int s) {
+#pragma unroll
+                for (int i = 0; i < DT; ++i) {
+                    const uint2 lo = v_frag(buf, i, 0, s), hi = v_frag(buf, i, 1, s);
+                    vf[s & 1][i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                }
+            };
+            float ls0 = 0.f, ls1 = 0.f, tx = -INFINITY, ty = -INFINITY;
             uint32_t pw0[8], pw1[8];                                     // P, packed
             s_init(t + 1, sn0, sn1);
-            uint4 ka = k_frag(kn, 0, 0), kb2 = k_frag(kn, 1, 0);
             __builtin_amdgcn_sched_barrier(0);
             constexpr int PER = 16 / KS;                                 // rows of S(t) per k-step of S(t + 1)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                const uint4 na = k_frag(kn, 0, ks + 1 < KS ? ks + 1 : ks), nb = k_frag(kn, 1, ks + 1 < KS ? ks + 1 : ks);
-                sn0 = mfma32<T>(ka, qf[ks], sn0);
+                const uint4 n0 = k_frag(buf ^ 1, 0, ks + 1 < KS ? ks + 1 : ks), n1 = k_frag(buf ^ 1, 1, ks + 1 < KS ? ks + 1 : ks);
+                if (AHEAD && ks == KS - 1) load_v(0);
+                sn0 = mfma32<T>(k0, qf[ks], sn0);
 #pragma unroll
                 for (int r = ks * PER; r < (ks + 1) * PER; ++r) {
                     sc0[r] = __builtin_amdgcn_exp2f(fmaf(sc0[r], scale_log2e, -m_use));
                     sc1[r] = __builtin_amdgcn_exp2f(fmaf(sc1[r], scale_log2e, -m_use));
-                    ls += sc0[r] + sc1[r];
-                    if (r == ks * PER + PER / 2 - 1) sn1 = mfma32<T>(kb2, qf[ks], sn1);
+                    if (!AHEAD) ls0 += sc0[r], ls1 += sc1[r];
+                    if (r == ks * PER + PER / 2 - 1) sn1 = mfma32<T>(k1, qf[ks], sn1);
                 }
 #pragma unroll
                 for (int r = ks * PER; r < (ks + 1) * PER; r += 2) {
                     pw0[r / 2] = pack16x2<T>(sc0[r], sc0[r + 1]);
                     pw1[r / 2] = pack16x2<T>(sc1[r], sc1[r + 1]);
                 }
-                ka = na;
-                kb2 = nb;
+                k0 = n0;
+                k1 = n1;
                 __builtin_amdgcn_sched_barrier(0);
             }
-            l_run = l_run * alpha + ls;
             m_run = m_new;
             // ---- O^T += V^T . P^T : 4 k-steps of 16 kv ----
-            const char* vb = Vs(buf);
-            const char* va[DT][2];
-#pragma unroll
-            for (int i = 0; i < DT; ++i)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) va[i][u] = vb + fl_v_off<D>(8 * u + 4 * h + tr, 4 * i + tc) + t8;
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const uint32_t* w = s < 2 ? pw0 + 4 * s : pw1 + 4 * (s - 2);
                 const uint4 pb = make_uint4(w[0], w[1], w[2], w[3]);
+                if (!AHEAD) load_v(s);
+                else if (s < 3) load_v(s + 1);
+                if (AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < DT; ++i) {
-                    const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][0] + s * 32 * D)));
-                    const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][1] + s * 32 * D)));
-                    o[i] = mfma32<T>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb, o[i]);
+                for (int i = 0; i < DT; ++i) o[i] = mfma32<T>(vf[s & 1][i], pb, o[i]);
+                // the matrix units have work: the sums, and the next tile's largest score
+#pragma unroll
+                for (int r = 4 * s; AHEAD && r < 4 * s + 4; ++r) ls0 += sc0[r], ls1 += sc1[r];
+                if (AHEAD && (s == 1 || s == 2)) {
+#pragma unroll
+                    for (int r = 8 * (s - 1); r < 8 * s; r += 2) {
+                        tx = fmaxf(fmaxf(tx, sn0[r]), sn0[r + 1]);
+                        ty = fmaxf(fmaxf(ty, sn1[r]), sn1[r + 1]);
+                    }
                 }
+                if (AHEAD && s == 3) top = scaled(fmaxf(tx, ty));
+                if (AHEAD) __builtin_amdgcn_sched_barrier(0);
             }
-            sc0 = sn0;
-            sc1 = sn1;
+            __builtin_amdgcn_s_setprio(0);
+            l_run = l_run * alpha + (ls0 + ls1);
         } else {
             if (WIN && live(t + 1)) {                                    // left of this wave's windows: the next tile's scores alone
-                s_init(t + 1, sc0, sc1);
+                s_init(t + 1, sn0, sn1);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
-                    sc0 = mfma32<T>(k_frag(Ks(buf ^ 1), 0, ks), qf[ks], sc0);
-                    sc1 = mfma32<T>(k_frag(Ks(buf ^ 1), 1, ks), qf[ks], sc1);
+                    sn0 = mfma32<T>(k_frag(buf ^ 1, 0, ks), qf[ks], sn0);
+                    sn1 = mfma32<T>(k_frag(buf ^ 1, 1, ks), qf[ks], sn1);
                 }
             }
         }
