@@ -635,7 +635,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(unsigned long long* tl
         return;
     }
     // Slices are cut by ABSOLUTE position (slice s = cache rows [s * chunk, (s + 1) * chunk), chunk from the step's context tier a.span <= cache length):
-    // no address depends on the context length, so the new token's q/k/v and the slice's first 128 K/V rows are requested
+    // no address depends on the context length, so the new token's q/k/v and the slice's first K/V rows are requested
     // before the position is even known (clamped addresses; masked later).  Before, the walk started one scalar and one
     // vector round trip later (position -> slice bounds -> addresses).  Slices beyond the context write empty records.
     const int chunk = decode_chunk_len(a.span, a.nsplit, 4 * PPW);
@@ -1984,7 +1984,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
 
 // Wide models, 1..7 sequences: the projections of ops_wide.hip (fp32 activations throughout, one pass over the weights for all sequences).
 // Attention leaves fp32 rows; o_proj and down_proj add to the residual stream themselves: 5 launches per layer, one more where split-KV
-// records are merged.
+// records are merged by a launch of their own (not wide_merge_ok).
 static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStream_t st, int* launches, bool short_ctx) {
     const auto& c = e->cfg;
     const bool fp8 = c.weight_format != 0;

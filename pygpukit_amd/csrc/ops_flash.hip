@@ -262,7 +262,7 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     // A pass of the loop is two tiles: the buffers' places are immediates then, and S(t + 1) is not copied.  V is read a k-step ahead of its products (the first under the last of S), the first of K
     // above the softmax; the row sums and the next tile's largest scores are taken under the products with V, where only the matrix units had work, and waves there go first (s_setprio): two on a
     // SIMD otherwise meet in the same phase.  Before / with all of it, us: 16 heads, 1531 rows 29.7 / 27.7, 384 at 3585 30.2 / 27.8, 400 13.4 / 11.9, 2500 52.2 / 45.2; 32 heads, 1000 rows 26.4 / 23.9,
-    // 3000 99 / 83.6, 4096 171 / 143 (of it s_setprio 88.6 / 83.6 and 155 / 143).  A tile was 270 vector instructions beside 32 matrix instructions, of which two waves overlapped a tenth.
+    // 4096 171 / 143 (of it s_setprio 155 / 143; 3000 rows 88.6 / 83.6).  A tile was 270 vector instructions beside 32 matrix instructions, of which two waves overlapped a tenth.
     // (As a lambda called for both tiles the windows' kernels spill 70 registers.)
     constexpr bool AHEAD = !WIN;         // V, sums and scores: windows have no registers for it
     f32x16_fl sc[2][2];                  // S of a pass's two tiles
@@ -611,8 +611,8 @@ static int flash_cus() {
 }
 
 // KV runs per query tile and sides of a workgroup (1 or 2: half a run's tiles each).
-// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile, 1.47 us a KV tile for a workgroup that has its
-// CU to itself; two sides take 1.1, and merge in LDS.
+// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile; two sides take three quarters of
+// one workgroup's time, and merge in LDS.  (The times below, but for flash_run_tiles', are of a loop that took 1.47 us a KV tile; it is a tenth faster now.)
 //  * Few workgroups (short of 5/8 of the CUs, 1200 positions and more): as many runs as two to a CU hold, of at least 2.5 KV tiles - more where many rows make the merge's
 //    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 23.3 / 15.9, 5000 56.3 / 26.3; 4 heads, 2048
 //    30.3 / 25.8; 8 heads, 2048 33.5 / 29.3.

@@ -17,13 +17,13 @@
 // Measured on the Llama-3-8B shape, us per launch (before: the GEMV kernels; bf16 with 6 sequences took two launches, of 4 and of 2):
 //                 bytes (bf16)   bf16, 1 sequence   bf16, 6 sequences   e4m3, 1 sequence
 //     qkv              50 MB       19.4 -> 11.1         65.2 -> 12.3       19.1 ->  8.6
-//     o_proj           34 MB       (merged)  8.3        (merged)  8.9      (merged) 5.8
+//     o_proj           34 MB       (merged)  8.3        (merged)  8.9      (merged) 5.8   (7.5 with the merge of split attention's records, a launch of 5 before)
 //     gate/up         235 MB       82.7 -> 37.5        193.4 -> 38.1       67.2 -> 23.3
 //     down            117 MB       37.9 -> 20.0        107.9 -> 27.2       39.5 -> 12.9
 //     lm_head        1051 MB      171.2 -> 162.8       371.0 -> 169        (bf16)
 // (5..7 sequences: with two pieces, 16 bits, 12, 8.6, 37.7, 24.6 and 169; the pieces of down's input, read by every workgroup, are what six cost more
 // than one.)
-// i.e. 6.2 TB/s on gate/up and 6.4 on lm_head.  One step: 5.34 -> 3.05 ms, 15.3 -> 3.43 ms, 4.68 -> 2.10 ms (context 700, 1100, 700).
+// i.e. 6.2 TB/s on gate/up and 6.4 on lm_head.  One step: 5.34 -> 3.05 ms, 15.3 -> 3.43 ms, 4.68 -> 2.04 ms (context 700, 1100, 700).
 
 #include <algorithm>
 
