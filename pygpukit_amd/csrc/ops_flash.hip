@@ -630,10 +630,10 @@ static int flash_cus() {
 struct FlashPlan { int runs, sides; bool fp32; int run; };       // fp32: of partial rows; run: FlashSplit
 // KV tiles of a run where every query tile is cut into as many as it takes, so that the heavy ones do not decide: the fewest, four or more, with which a workgroup has a CU to itself (a few of
 // the lightest may share one: two to a CU take 1.8 times as long).  0: the rules below, for shapes that would need runs of more than 16 tiles.  Us with the merge, one launch behind another,
-// equal runs or sides / this: 16 heads, 1200 rows 28.4 / 24.6, 1531 33.3 / 30.2 (between a layer's other kernels 31.0 / 29.9), 1700 36.1 / 34.8; 8 heads, 1600 26.5 / 23.3, 2048 30.6 / 28.4;
+// equal runs / this: 16 heads, 1200 rows 28.4 / 24.6, 1531 33.3 / 30.2 (between a layer's other kernels 31.0 / 29.9), 1700 36.1 / 34.8; 8 heads, 1600 26.5 / 23.3, 2048 30.6 / 28.4;
 // 4 heads, 1600 22.0 / 18.5, 2048 25.0 / 21.3; 1000 at 250 27.4 / 24.6; 1 head, 5000 rows, which the rules below cut into 12, 25.1 / 25.8.  Under 1200 keys partial rows are fp32 (below).
 // Deeper in a context nearly every row has partial rows, which lose a bit where they are rounded to 16 bits (1 % more error than the equal runs leave) and time where they are not (800 at 700
-// 30.1 / 32.1, 900 at 800 32.2 / 35.5).
+// 30.1 / 32.1, 900 at 800 32.2 / 35.5).  Only where the rules below cut into runs as well: a call that needs no scratch memory, as under capture, goes on needing none.
 static int flash_run_tiles(int tiles, int hq, int q_len, int kv_len, int most) {
     const int cus = flash_cus();
     for (int run = 4; run <= 16; ++run) {
@@ -683,7 +683,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
     FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1, false, 0} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
-    if (!WIN && !many.items && !one_side && kv_len >= 1200 && 4LL * kv_len <= 5LL * q_len && plan.runs <= 8)
+    if (!WIN && !many.items && !one_side && kv_len >= 1200 && 4LL * kv_len <= 5LL * q_len && plan.runs > 1 && plan.runs <= 8)
         if (const int run = flash_run_tiles(tiles, hq, q_len, kv_len, 16)) plan = {flash_runs(tiles - 1, q_len, kv_len, run), 1, false, run};
     int nsplit = plan.runs;
     const bool wide = many.items || q_len <= 128 || plan.fp32;
