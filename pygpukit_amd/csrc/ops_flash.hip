@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "flash.hip.h"
+#include "flash_plan.h"
 #include "latent.hip.h"
 #include "pgk_device.hip.h"
 #include "pgk_internal.h"
@@ -58,7 +59,8 @@ __device__ __forceinline__ void fl_dma16(const fl_u32x4& buffer, uint32_t off, u
 }
 __device__ __forceinline__ uint32_t fl_lds_addr(const char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p; }
 
-constexpr int FL_BQ = FLASH_ITEM_ROWS, FL_BKV = 64, FL_THREADS = 256;
+constexpr int FL_THREADS = 256;
+static_assert(FL_BQ == FLASH_ITEM_ROWS, "a listed query tile is one of the kernel's");
 
 // K image: [64 kv][D] 16-bit, 16-byte chunk c (0..D/8-1) of row r at r*2D + ((c ^ (r & (D/8-1))) << 4)
 template <int D> __device__ __forceinline__ int fl_k_off(int r, int c) { return r * (2 * D) + ((c ^ (r & (D / 8 - 1))) << 4); }
@@ -117,13 +119,6 @@ template <class T, int N> __device__ __forceinline__ void flash_gate_cols(const 
         y[j] /= 1.0f + __expf(-to_f(__builtin_bit_cast(T, half)));
     }
 }
-
-// KV tiles and runs of query tile qt where runs hold `run` tiles
-__host__ __device__ inline int flash_tiles(int qt, int q_len, int kv_len) {
-    const int last = qt * FL_BQ + FL_BQ < q_len ? qt * FL_BQ + FL_BQ : q_len, end = kv_len - q_len + last;
-    return ((end < kv_len ? end : kv_len) + FL_BKV - 1) / FL_BKV;
-}
-__host__ __device__ inline int flash_runs(int qt, int q_len, int kv_len, int run) { return (flash_tiles(qt, q_len, kv_len) + run - 1) / run; }
 
 template <class T, int D, bool WIN = false, bool BIAS = false, int SIDES = 1>
 __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
@@ -610,100 +605,30 @@ static int flash_cus() {
     return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 ? cus : 256;
 }
 
-// KV runs per query tile and sides of a workgroup (1 or 2: half a run's tiles each).
-// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile; two sides take three quarters of
-// one workgroup's time, and merge in LDS.  (The times below, but for flash_run_tiles', are of a loop that took 1.47 us a KV tile; it is a tenth faster now.)
-//  * Few workgroups (short of 5/8 of the CUs, 1200 positions and more): as many runs as two to a CU hold, of at least 2.5 KV tiles - more where many rows make the merge's
-//    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 23.3 / 15.9, 5000 56.3 / 26.3; 4 heads, 2048
-//    30.3 / 25.8; 8 heads, 2048 33.5 / 29.3.
-//  * Up to a workgroup per CU (and no runs of flash_run_tiles): two runs, of which a heavy and a light one share a CU.  16 heads, 1531 rows 31.5 (two sides 34.2), 1800 36.9 (39.0).
-//  * Shorter contexts, at most a workgroup to four CUs: three or four runs whose rows stay fp32.  In 16 bits they were rounded twice: 2.27e-3 of float64 for 700 rows of 4 heads
-//    where two sides leave 2.00e-3 and these 1.98e-3.  1 head, 1024 rows 23.3 (two sides) / 14.6, 8 heads, 900 21.9 / 21.1.
-//  * Otherwise two sides beyond ten KV tiles, up to five workgroups to four CUs: 16 heads, 2300 rows 54.2 (one side) / 47.5; 32 heads, 1100 31.1 / 28.0.  Up to two to a CU only where
-//    nearly all of the context is causal and long: 16 heads, 3000 rows 71.2 / 60.0; but 64 heads, 900 rows 26.8 / 34.1, 32 heads, 1300 at 650 47.1 / 52.6.  Beyond, two workgroups
-//    of their own time per CU do more (one barrier makes the sides wait for each other).
-// Longer contexts: as many runs as one round of workgroups holds, at least four KV tiles each: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and
-// that many still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
-// 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
-// (Results that are rounded to e4m3 next, by whichever kernel, ask for one side: the codes magnify a sum's last bit to a sixteenth, and a prompt in one pass and in pieces would
-// no longer agree - 4096 rows of 32 heads at once and as two of 2048, which alone had two sides, were 0.028 apart in the logits, with one side each under 0.01.)
-struct FlashPlan { int runs, sides; bool fp32; int run; };       // fp32: of partial rows; run: FlashSplit
-// KV tiles of a run where every query tile is cut into as many as it takes, so that the heavy ones do not decide: the fewest, four or more, with which a workgroup has a CU to itself (a few of
-// the lightest may share one: two to a CU take 1.8 times as long).  0: the rules below, for shapes that would need runs of more than 16 tiles.  Us with the merge, one launch behind another,
-// equal runs / this: 16 heads, 1200 rows 28.4 / 24.6, 1531 33.3 / 30.2 (between a layer's other kernels 31.0 / 29.9), 1700 36.1 / 34.8; 8 heads, 1600 26.5 / 23.3, 2048 30.6 / 28.4;
-// 4 heads, 1600 22.0 / 18.5, 2048 25.0 / 21.3; 1000 at 250 27.4 / 24.6; 1 head, 5000 rows, which the rules below cut into 12, 25.1 / 25.8.  Under 1200 keys partial rows are fp32 (below).
-// Deeper in a context nearly every row has partial rows, which lose a bit where they are rounded to 16 bits (1 % more error than the equal runs leave) and time where they are not (800 at 700
-// 30.1 / 32.1, 900 at 800 32.2 / 35.5).  Only where the rules below cut into runs as well: a call that needs no scratch memory, as under capture, goes on needing none.
-static int flash_run_tiles(int tiles, int hq, int q_len, int kv_len, int most) {
-    const int cus = flash_cus();
-    for (int run = 4; run <= 16; ++run) {
-        long long wgs = 0;
-        int runs = 1, over = 0;                                  // over: the largest run beyond the CUs
-        for (int qt = tiles - 1; qt >= 0; --qt) {
-            const int n = flash_runs(qt, q_len, kv_len, run);
-            runs = std::max(runs, n);
-            wgs += (long long)n * hq;
-            if (wgs > cus) over = std::max(over, ceil_div(flash_tiles(qt, q_len, kv_len), n));
-        }
-        if (runs <= most && (wgs <= cus || (2 * over <= run && 4 * wgs <= 5LL * cus))) return run;
-    }
-    return 0;
-}
-static FlashPlan flash_plan(long long wgs, int q_len, int kv_len, int most) {
-    const int cus = flash_cus();
-    if (kv_len < 2LL * q_len) {
-        const int nt = ceil_div(kv_len, FL_BKV);
-        const bool fp32 = kv_len < 1200;
-        long long n = 1;
-        if (!fp32) n = 8 * wgs <= 5 * cus ? std::min({8 * wgs > cus ? 12LL : 8LL, 2 * cus / wgs, nt * 40 / (100 + wgs * 256 / cus)}) : wgs <= cus ? 2 : 1;
-        else if (4 * wgs <= cus) n = 8 * wgs <= cus ? std::min(nt / 3, 4) : std::min(nt / 4, 3);
-        if (fp32 && n < 3) n = 1;
-        n = std::min<long long>(n, most);
-        if (n > 1) return {(int)n, 1, fp32, 0};
-        return {1, nt > 10 && (4 * wgs <= 5 * cus || (wgs <= 2 * cus && !fp32 && 4LL * kv_len <= 5LL * q_len)) ? 2 : 1, false, 0};
-    }
-    long long n = cus / wgs;
-    if (n < 4 || kv_len < 4LL * q_len) n = 2 * cus / wgs;
-    if (n > most) n = most;
-    if (n > ceil_div(kv_len, FL_BKV) / 4) n = ceil_div(kv_len, FL_BKV) / 4;
-    return {n < 1 ? 1 : (int)n, 1, false, 0};
-}
-// with a sliding window: up to four runs over the `span` keys that the heaviest query tile walks, until two workgroups per CU are reached
-static int flash_window_runs(long long wgs, int span) {
-    int n = 1;
-    while (n < 4 && wgs * n < 2LL * flash_cus() && ceil_div(span, FL_BKV) >= 4 * (n * 2)) n *= 2;
-    return n;
-}
-
 // q_len: query rows of all sequences where `many` lists several (kv_len: the longest context among them)
 template <class T, int D, bool WIN = false, bool BIAS = false>
 static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int hq, int hkv, int q_len, int kv_len, float scale,
                                const FlashStrides& sd, hipStream_t st, uint8_t* q8 = nullptr, float* q8s = nullptr, const FlashWindow& win = FlashWindow{},
                                const FlashMany& many = FlashMany{}, bool one_side = false) {
-    const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ);
+    const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ), cus = flash_cus();
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
-    FlashPlan plan = WIN ? FlashPlan{flash_window_runs((long long)tiles * hq, span), 1, false, 0} : flash_plan((long long)tiles * hq, q_len, kv_len, 16);
-    if (!WIN && !many.items && !one_side && kv_len >= 1200 && 4LL * kv_len <= 5LL * q_len && plan.runs > 1 && plan.runs <= 8)
-        if (const int run = flash_run_tiles(tiles, hq, q_len, kv_len, 16)) plan = {flash_runs(tiles - 1, q_len, kv_len, run), 1, false, run};
-    int nsplit = plan.runs;
+    const FlashPlan even = WIN ? FlashPlan{flash_window_runs(cus, (long long)tiles * hq, span), 1, false, 0} : flash_even_plan(cus, (long long)tiles * hq, q_len, kv_len, 16);
+    FlashPlan plan = WIN || many.items || one_side ? even : flash_plan(cus, even, hq, q_len, kv_len, 16);
     const bool wide = many.items || q_len <= 128 || plan.fp32;
     // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
     // tiles of the first-generation kernel 61, 31 and 239)
-    if (nsplit > 1 && q_len <= 128) {
+    if (plan.runs > 1 && q_len <= 128) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) nsplit = 1, plan.run = 0;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) plan.runs = 1;
     }
-    FlashSplit sp{nsplit, plan.run, nullptr, nullptr, wide, q8, q8s};
     void* ws = nullptr;
-    if (nsplit > 1) {
-        const size_t po_bytes = (size_t)nsplit * q_len * hq * D * (wide ? 4 : sizeof(T)), ml_bytes = (size_t)nsplit * hq * q_len * 2 * sizeof(float);
-        if (pool_malloc_on(&ws, po_bytes + ml_bytes + 256, st) == PGK_OK) {
-            sp.o = ws;
-            sp.ml = (float*)((char*)ws + ((po_bytes + 255) & ~(size_t)255));
-        } else {
-            nsplit = sp.nsplit = 1, sp.run = 0;        // no memory, or a stream whose end the pool cannot see: slower, and right
-        }
-    }
+    size_t ml_at = 0;
+    plan = flash_granted(plan, even, [&](int runs) {      // no memory, or a stream whose end the pool cannot see: slower, and right
+        ml_at = ((size_t)runs * q_len * hq * D * (wide ? 4 : sizeof(T)) + 255) & ~(size_t)255;
+        return pool_malloc_on(&ws, ml_at + (size_t)runs * hq * q_len * 2 * sizeof(float), st) == PGK_OK;
+    });
+    const int nsplit = plan.runs;
+    const FlashSplit sp{nsplit, plan.run, nsplit > 1 ? (float*)((char*)ws + ml_at) : nullptr, ws, wide, q8, q8s};
     auto launch = [&](auto sides) -> hipError_t {
         constexpr int SIDES = decltype(sides)::value;
         constexpr size_t LDS = SIDES * 4 * (size_t)(64 * D * 2);
