@@ -82,9 +82,12 @@ inline int flash_run_tiles(int cus, int hq, int q_len, int kv_len, int most) {
     }
     return 0;
 }
-// `even`: flash_even_plan's
-inline FlashPlan flash_plan(int cus, const FlashPlan& even, int hq, int q_len, int kv_len, int most) {
+// `even`: flash_even_plan's, which stays where it has few workgroups: its runs are shorter than four tiles there, or few of the CUs work.  Us, even / runs of as many tiles, at 7/16 of the CUs in workgroups
+// and fewer: head dim 128, 1 head, 1200 rows 12.6 / 13.6, 1400 13.0 / 13.7, 1600 13.5 / 13.9, 2 heads, 1000 at 240 13.5 / 14.1; beyond, 1 head, 3300 18.7 / 17.9, 3 heads, 1400 16.7 / 15.2.  Head dim 64, whose partial rows
+// cost half, at 3/4 and fewer: 1 head, 1200 9.6 / 10.6, 2700 12.1 / 12.9, 2 heads, 1400 10.6 / 11.0; beyond, 3 heads, 1400 11.7 / 11.5, 4 heads, 1400 12.5 / 11.8.
+inline FlashPlan flash_plan(int cus, const FlashPlan& even, int hq, int q_len, int kv_len, int d, int most) {
     if (kv_len < 1200 || 4LL * kv_len > 5LL * q_len || even.runs == 1 || even.runs > 8) return even;
+    if (16LL * even.runs * fl_ceil_div(q_len, FL_BQ) * hq <= (d == 64 ? 12 : 7) * cus) return even;
     const int run = flash_run_tiles(cus, hq, q_len, kv_len, most);
     return run ? FlashPlan{flash_runs(fl_ceil_div(q_len, FL_BQ) - 1, q_len, kv_len, run), 1, false, run} : even;
 }

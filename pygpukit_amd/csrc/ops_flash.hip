@@ -613,7 +613,7 @@ static pgk_status flash_launch(const T* q, const T* k, const T* v, T* out, int h
     const int tiles = many.items ? many.n_items : ceil_div(q_len, FL_BQ), cus = flash_cus();
     const int span = WIN && (long long)win.window + FL_BQ < kv_len ? win.window + FL_BQ : kv_len;    // keys the heaviest query tile walks
     const FlashPlan even = WIN ? FlashPlan{flash_window_runs(cus, (long long)tiles * hq, span), 1, false, 0} : flash_even_plan(cus, (long long)tiles * hq, q_len, kv_len, 16);
-    FlashPlan plan = WIN || many.items || one_side ? even : flash_plan(cus, even, hq, q_len, kv_len, 16);
+    FlashPlan plan = WIN || many.items || one_side ? even : flash_plan(cus, even, hq, q_len, kv_len, D, 16);
     const bool wide = many.items || q_len <= 128 || plan.fp32;
     // Up to 128 rows need no scratch memory to be captured: one run (16 heads, us: 64 rows of 1000 31, 128 of 400 19, 100 of 4000 101; on the 64-row
     // tiles of the first-generation kernel 61, 31 and 239)
