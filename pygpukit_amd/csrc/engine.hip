@@ -1984,7 +1984,7 @@ static pgk_status decode_chunk_packed(Engine* e, int b0, int M, bool last, hipSt
 
 // Wide models, 1..7 sequences: the projections of ops_wide.hip (fp32 activations throughout, one pass over the weights for all sequences).
 // Attention leaves fp32 rows; o_proj and down_proj add to the residual stream themselves: 5 launches per layer, one more where split-KV
-// records are merged by a launch of their own (not wide_merge_ok).
+// records are merged by a launch of their own (not wide_merge_ok, wide_merge_pays).
 static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStream_t st, int* launches, bool short_ctx) {
     const auto& c = e->cfg;
     const bool fp8 = c.weight_format != 0;
@@ -1994,7 +1994,7 @@ static pgk_status decode_chunk_wide(Engine* e, int b0, int M, bool last, hipStre
     // One sequence: o_proj merges the split-KV records on their way in and leaves a partial vector per 2048 columns, gate_up adds those to its input, of which its first workgroup
     // leaves the sum for down_proj to add to: two residual rows in turn, no launch for the merge
     const int slices = M == 1 && !direct ? attn_slices(e, 1, D) : 0;
-    const bool merged = slices && wide_merge_ok(QD, D, slices);
+    const bool merged = slices && wide_merge_ok(QD, D, slices) && wide_merge_pays(fp8, H, QD, e->cu_count);
     float *other = e->h2 + (size_t)b0 * H, *parts = e->opart + (size_t)b0 * std::max((int)c.num_kv_heads, wide_merge_parts(QD)) * H;
     for (int l = 0; l < c.num_layers; ++l) {
         const auto& L = e->layers[l];

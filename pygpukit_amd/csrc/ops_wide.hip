@@ -455,7 +455,7 @@ pgk_status launch_wide(const FusedArgs& a, bf16* pieces, int M, int cu_count, in
     PGK_CHECK_HIP(attr);
     // one workgroup per CU while its tiles fit one reduction; the vocabulary is reduced in groups
     const int runs = SRC == WIDE_MERGE ? wide_merge_parts(a.K) : 1;
-    int rows = ceil_div(ceil_div(a.N, std::max(cu_count / runs, 1)), 8) * 8;
+    int rows = wide_rows(a.N, cu_count, runs);
     constexpr int MOST = WD_TILES * (EPI == EPI_SWIGLU ? 8 : 16);
     if (EPI != EPI_LOGITS && rows > MOST) rows = ceil_div(ceil_div(a.N, ceil_div(rows, MOST) * cu_count), 8) * 8;
     const int grid = ceil_div(a.N, rows);
