@@ -8,6 +8,8 @@ import subprocess
 
 import pytest
 
+from tests import flash_cuts
+
 CSRC = os.path.join(os.path.dirname(__file__), "..", "pygpukit_amd", "csrc")
 SHIM = """
 #include "flash_plan.h"
@@ -60,3 +62,11 @@ def test_few_workgroups_keep_the_even_cut(cut, hq, q_len, kv_len, d, even, run):
     got = cut(hq, q_len, kv_len, d)
     assert (got["even"], got["run"]) == (even, run), got
     assert (16 * even * -(-q_len // 128) * hq <= (12 if d == 64 else 7) * 256) == (run == 0)
+
+
+@pytest.mark.parametrize("cuts", ["SIDES", "ANY_COUNT", "MERGES", "FEW_WORKGROUPS", "EQUAL_TILES"])
+def test_shapes_the_kernels_are_tested_with_are_cut_as_listed(cut, cuts):
+    """Each of the GPU tests' shapes takes the route that it stands for."""
+    for (hq, _, q_len, kv_len, d), want in getattr(flash_cuts, cuts).items():
+        got = cut(hq, q_len, kv_len, d)
+        assert (got["runs"], got["run"], got["sides"]) == want, (hq, q_len, kv_len, d, got)

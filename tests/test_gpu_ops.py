@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import cpu_ref as O
+from tests import flash_cuts
 from tests.conftest import load_golden, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -815,15 +816,14 @@ def test_sdpa_nan_and_infinite_keys(cfg):
         assert rel_err(got[~lost], ref[~lost]) < 2.0**-8
 
 
-@pytest.mark.parametrize("cfg", [(32, 8, 600, 1500, 128), (16, 8, 384, 3585, 128), (12, 4, 300, 1900, 128), (18, 6, 257, 1300, 64), (33, 3, 100, 3000, 128)])
+@pytest.mark.parametrize("cfg", flash_cuts.ANY_COUNT)
 def test_sdpa_runs_of_any_count(cfg):
     """3, 5, 7, 4 and 7 runs on a card of 256 CUs: an uneven cut of the KV tiles, a merge whose last four runs are not all there."""
     test_sdpa_few_rows_over_a_long_context("bfloat16", cfg)
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("cfg", [(16, 8, 1531, 1531, 128), (8, 4, 900, 900, 128), (1, 1, 1024, 1024, 64), (2, 1, 2560, 2560, 128), (4, 2, 384, 3585, 64), (1, 1, 200, 4296, 128),
-                                 (1, 1, 100, 4000, 128)])
+@pytest.mark.parametrize("cfg", flash_cuts.MERGES)
 def test_sdpa_merges_of_two_to_sixteen_runs(dt, cfg):
     """2, 3 (fp32 rows), 4 (fp32), 11, 14, 16 and 15 (fp32) runs on a card of 256 CUs: every size of flash_merge_kernel, full and with runs to spare."""
     test_sdpa_few_rows_over_a_long_context(dt, cfg)
@@ -1009,7 +1009,7 @@ def test_sdpa_reads_nothing_behind_the_context(dt, cfg):
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("cfg", [(16, 1, 641, 641, 128), (12, 2, 699, 705, 64), (20, 2, 500, 768, 128), (12, 1, 700, 1199, 128), (33, 3, 1281, 1281, 128)])
+@pytest.mark.parametrize("cfg", flash_cuts.SIDES)
 def test_sdpa_with_the_tiles_of_a_run_shared_by_two_sides(dt, cfg):
     """72 to 96 workgroups, and more than there are CUs: 11 and 12 KV tiles in the heaviest query tile and 2 in the lightest, a context before the rows.  The bars of the
     tests that are called."""
@@ -1020,11 +1020,10 @@ def test_sdpa_with_the_tiles_of_a_run_shared_by_two_sides(dt, cfg):
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("cfg", [(2, 1, 575, 576, 64), (2, 1, 641, 641, 128), (4, 2, 699, 705, 64), (2, 2, 500, 768, 128), (8, 1, 513, 769, 128), (1, 1, 700, 1199, 128), (1, 1, 700, 1200, 64),
-                                 (1, 1, 2049, 2049, 64), (2, 1, 2500, 2501, 128), (9, 3, 1800, 1806, 64), (10, 2, 2000, 2006, 128)])
+@pytest.mark.parametrize("cfg", flash_cuts.FEW_WORKGROUPS)
 def test_sdpa_of_few_workgroups_in_runs(dt, cfg):
-    """Prompts of few heads on a card of 256 CUs: 3, 3, 4, 4, 3 and 4 runs of fp32 rows up to 1199 positions, from 1200 on 7, 8, 11, 3 and 3 (2.5 tiles each and more) whose
-    first query tiles leave most runs empty.  The bars of the tests that are called."""
+    """Prompts of few heads on a card of 256 CUs: 3, 3, 4, 4, 3 and 4 runs of fp32 rows up to 1199 positions, from 1200 on 7, 8, 11, 3 and 2 (2.5 tiles each and more) whose
+    first query tiles leave most runs empty, and up to 3 of 11 and of 15 tiles.  The bars of the tests that are called."""
     test_sdpa_few_rows_over_a_long_context(dt, cfg)
     test_sdpa_reads_nothing_behind_the_context(dt, cfg)
     if dt == "bfloat16" and cfg[1] == 2 and cfg[3] - cfg[2] > 5:
@@ -1032,9 +1031,9 @@ def test_sdpa_of_few_workgroups_in_runs(dt, cfg):
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("cfg", [(16, 8, 1250, 1250, 128), (16, 2, 1531, 1536, 128), (16, 16, 1281, 1281, 64), (8, 8, 2047, 2047, 128), (4, 2, 1600, 1663, 64), (16, 8, 1000, 1250, 128), (12, 2, 1030, 1281, 64)])
+@pytest.mark.parametrize("cfg", flash_cuts.EQUAL_TILES)
 def test_sdpa_in_runs_of_as_many_tiles(dt, cfg):
-    """Query tiles cut into as many runs as their keys take on a card of 256 CUs: 1 to 6, single ones left without a merge, a last query tile of one row and a context
+    """Query tiles cut into as many runs as their keys take on a card of 256 CUs: up to 2, 3, 4, 7, 8 and 13, single ones left without a merge, a last query tile of one row and a context
     before the rows.  The bars of the tests that are called."""
     test_sdpa_few_rows_over_a_long_context(dt, cfg)
     test_sdpa_reads_nothing_behind_the_context(dt, cfg)
