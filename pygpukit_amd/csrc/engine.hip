@@ -1137,8 +1137,8 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
     tls.end();
 }
 
-// long-context path, steps 2 + 3 in ONE launch: merge the split-KV records of a kv head's G query heads (the arithmetic
-// of attn_merge_kernel, same order) and multiply the result with this workgroup's slice of W_o.  Grid as attn_oproj_kernel
+// long-context path, steps 2 + 3 in ONE launch: merge the split-KV records of a kv head's G query heads (the weights
+// of attn_merge_kernel; the slices are dealt to groups of threads, whose sums meet in LDS) and multiply the result with this workgroup's slice of W_o.  Grid as attn_oproj_kernel
 // ((H / rows_per_block) * Hkv, kv head fastest: XCD-aware), output the same per-kv-head partial vectors, which the
 // gate/up kernel's PRO_NORM_SUM prologue adds to the residual stream.  Replaces attn_merge_kernel + the o_proj GEMV:
 // one launch and one dependent-kernel gap less per layer (context 2048, w8a16: the pair took 1.95 + 1.3 + 1.74 us of

@@ -20,20 +20,21 @@ constexpr int flash_runs(int qt, int q_len, int kv_len, int run) { return (flash
 struct FlashPlan { int runs, sides; bool fp32; int run; };
 
 // The same number of runs for every query tile, or two sides.
-// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile; two sides take three quarters of
-// one workgroup's time, and merge in LDS.  (The times below, but for flash_run_tiles', are of a loop that took 1.47 us a KV tile; it is a tenth faster now.)
+// Where the causal edge is most of the work (contexts under twice the rows) a launch lasts as long as its heaviest tile; two sides take three quarters to nine tenths of
+// one workgroup's time, and merge in LDS.
 //  * Few workgroups (short of 5/8 of the CUs, 1200 positions and more): as many runs as two to a CU hold, of at least 2.5 KV tiles - more where many rows make the merge's
-//    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 23.3 / 15.9, 5000 56.3 / 26.3; 4 heads, 2048
-//    30.3 / 25.8; 8 heads, 2048 33.5 / 29.3.
-//  * Up to a workgroup per CU (and no runs of flash_run_tiles): two runs, of which a heavy and a light one share a CU.  16 heads, 1531 rows 31.5 (two sides 34.2), 1800 36.9 (39.0).
+//    traffic count -, at most 8, or 12 where 8 would leave part of a round.  Us with two runs / this rule: head dim 128, 1 head, 1531 rows 20.3 / 13.4, 5000 47.3 / 23.4; 4 heads, 2048
+//    26.6 / 24.4.
+//  * Up to a workgroup per CU (and no runs of flash_run_tiles): two runs, of which a heavy and a light one share a CU.  12 heads, 2400 rows 37.7 (two sides 40.8), but 16 heads, 1800 34.5 (33.8).
 //  * Shorter contexts, at most a workgroup to four CUs: three or four runs whose rows stay fp32.  In 16 bits they were rounded twice: 2.27e-3 of float64 for 700 rows of 4 heads
-//    where two sides leave 2.00e-3 and these 1.98e-3.  1 head, 1024 rows 23.3 (two sides) / 14.6, 8 heads, 900 21.9 / 21.1.
-//  * Otherwise two sides beyond ten KV tiles, up to five workgroups to four CUs: 16 heads, 2300 rows 54.2 (one side) / 47.5; 32 heads, 1100 31.1 / 28.0.  Up to two to a CU only where
-//    nearly all of the context is causal and long: 16 heads, 3000 rows 71.2 / 60.0; but 64 heads, 900 rows 26.8 / 34.1, 32 heads, 1300 at 650 47.1 / 52.6.  Beyond, two workgroups
-//    of their own time per CU do more (one barrier makes the sides wait for each other).
+//    where two sides leave 2.00e-3 and these 1.98e-3.  1 head, 1024 rows 20.4 (two sides) / 12.8, 8 heads, 900 19.8 / 19.9.
+//  * Otherwise two sides beyond ten KV tiles, up to five workgroups to four CUs: 16 heads, 2300 rows 46.6 (one side) / 41.4; 24 heads, 1531 34.3 / 31.5; 32 heads, 1100 27.0 / 25.1.  Up to two to a CU only where
+//    nearly all of the context is causal and long: 16 heads, 3000 rows 63.4 / 53.8; but 64 heads, 900 rows 27.8 / 35.2, 32 heads, 1300 of 1950 47.7 / 52.1, 2500 68.6 / 81.6.  Beyond, two workgroups
+//    of their own time per CU do more (one barrier makes the sides wait for each other).  Since the loop takes two tiles a pass the line is late by 3 %: 32 heads, 1600 rows 38.7 / 39.9, 2000 51.4 / 52.8, 28
+//    heads, 1800 43.6 / 45.0.
 // Longer contexts: as many runs as one round of workgroups holds, at least four KV tiles each: of two per CU (the kernel's occupancy), or of one per CU where all runs are alike and
-// that many still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 at 3000 42.6 (2) 38.9 (4); 384 at 3585 29.0 (5)
-// 32.3 (8); 250 at 2000 21.0 (4) 20.8 (8); 32 heads, 600 at 2400 45.8 (2) 41.6 (3).  Two sides there: 384 at 3585 30.2 / 29.5, 600 at 2400 40.8 / 41.6.
+// that many still cut it well.  A second round costs more than the shorter runs save, and every run costs the merge: 16 heads, 1000 of 4000 50.4 (2) 46.1 (4); 384 of 3585 27.3 (5)
+// 29.8 (8); 250 of 2250 20.4 (4) 19.5 (8); 32 heads, 600 of 3000 48.0 (2) 45.3 (3).  Two sides there: 384 of 3585 52.4, 600 of 3000 48.7.
 // (Results that are rounded to e4m3 next, by whichever kernel, ask for one side: the codes magnify a sum's last bit to a sixteenth, and a prompt in one pass and in pieces would
 // no longer agree - 4096 rows of 32 heads at once and as two of 2048, which alone had two sides, were 0.028 apart in the logits, with one side each under 0.01.)
 inline FlashPlan flash_even_plan(int cus, long long wgs, int q_len, int kv_len, int most) {
@@ -63,10 +64,10 @@ inline int flash_window_runs(int cus, long long wgs, int span) {
 
 // KV tiles of a run where every query tile is cut into as many as it takes, so that the heavy ones do not decide: the fewest, four or more, with which a workgroup has a CU to itself (a few of
 // the lightest may share one: two to a CU take 1.8 times as long).  0: flash_even_plan, for shapes that would need runs of more than 16 tiles.  Us with the merge, one launch behind another,
-// equal runs / this: 16 heads, 1200 rows 28.4 / 24.6, 1531 33.3 / 30.2 (between a layer's other kernels 31.0 / 29.9), 1700 36.1 / 34.8; 8 heads, 1600 26.5 / 23.3, 2048 30.6 / 28.4;
-// 4 heads, 1600 22.0 / 18.5, 2048 25.0 / 21.3; 1000 at 250 27.4 / 24.6; 1 head, 5000 rows, which flash_even_plan cuts into 12, 25.1 / 25.8.  Under 1200 keys partial rows are fp32.
-// Deeper in a context nearly every row has partial rows, which lose a bit where they are rounded to 16 bits (1 % more error than the equal runs leave) and time where they are not (800 at 700
-// 30.1 / 32.1, 900 at 800 32.2 / 35.5).  Only where flash_even_plan cuts into runs as well: a call that needs no scratch memory, as under capture, goes on needing none.
+// even runs / this: 16 heads, 1200 rows 26.1 / 22.2, 1400 29.0 / 24.7, 1600 31.6 / 28.4; 8 heads, 1600 24.5 / 21.4, 2000 28.2 / 25.2; 4 heads, 1600 20.9 / 17.2, 2049 24.4 / 20.1.  Up to 16 runs for the heaviest
+// tile: 1 head, 3900 rows 20.0, with at most 8 20.3 (head dim 64 14.7 / 15.3).  Under 1200 keys partial rows are fp32.
+// Deeper in a context nearly every row has partial rows, which lose a bit where they are rounded to 16 bits (1 % more error than the even runs leave) and time where they are not (800 at 700
+// 30.1 / 32.1, 900 at 800 32.2 / 35.5, with the loop of one tile a pass).
 inline int flash_run_tiles(int cus, int hq, int q_len, int kv_len, int most) {
     const int tiles = fl_ceil_div(q_len, FL_BQ);
     for (int run = 4; run <= 16; ++run) {
@@ -82,9 +83,11 @@ inline int flash_run_tiles(int cus, int hq, int q_len, int kv_len, int most) {
     }
     return 0;
 }
-// `even`: flash_even_plan's, which stays where it has few workgroups: its runs are shorter than four tiles there, or few of the CUs work.  Us, even / runs of as many tiles, at 7/16 of the CUs in workgroups
-// and fewer: head dim 128, 1 head, 1200 rows 12.6 / 13.6, 1400 13.0 / 13.7, 1600 13.5 / 13.9, 2 heads, 1000 at 240 13.5 / 14.1; beyond, 1 head, 3300 18.7 / 17.9, 3 heads, 1400 16.7 / 15.2.  Head dim 64, whose partial rows
-// cost half, at 3/4 and fewer: 1 head, 1200 9.6 / 10.6, 2700 12.1 / 12.9, 2 heads, 1400 10.6 / 11.0; beyond, 3 heads, 1400 11.7 / 11.5, 4 heads, 1400 12.5 / 11.8.
+// `even`: flash_even_plan's.  It stays where it is one run: a call that needs no scratch memory, as under capture, goes on needing none.  And where it has few workgroups: its runs are shorter than four tiles
+// there, or few of the CUs work.  Us, even / runs of as many tiles, up to 7/16 of the CUs in workgroups: head dim 128, 1 head, 1200 rows 12.6 / 13.6, 1400 13.0 / 13.7, 1600 13.5 / 13.9, 2 heads, 1000 of 1240
+// 13.5 / 14.1; beyond, 1 head, 3300 18.7 / 17.9, 3 heads, 1400 16.7 / 15.2.  Head dim 64, whose partial rows cost half, up to 3/4: 1 head, 1200 9.6 / 10.6, 2700 12.1 / 12.9, 2 heads, 1400 10.6 / 11.0;
+// beyond, 3 heads, 1400 11.7 / 11.5, 4 heads, 1400 12.5 / 11.8.  More than eight even runs stay for the one head of 5000 rows and more that has them (23.4 / 23.6, 8000 34.3 / 34.1); they cost where few rows
+// have them: 2 heads, 2049 20.9 / 16.4, 3 heads, 2300 23.1 / 19.7, 1 head, 4200 22.8 / 20.6.
 inline FlashPlan flash_plan(int cus, const FlashPlan& even, int hq, int q_len, int kv_len, int d, int most) {
     if (kv_len < 1200 || 4LL * kv_len > 5LL * q_len || even.runs == 1 || even.runs > 8) return even;
     if (16LL * even.runs * fl_ceil_div(q_len, FL_BQ) * hq <= (d == 64 ? 12 : 7) * cus) return even;

@@ -299,8 +299,7 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
     auto v_frag = [&](int buf, int i, int u, int s) {
         return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fl_lds_v4)(va[i][u] + buf * V_BYTES + s * 32 * D)));
     };
-    // this lane's largest score, in two chains.  (This file is built with -fno-honor-nans: without it every operand of a max is first canonicalised with a v_max_f32 x, x, x of
-    // its own.)
+    // this lane's largest score, in two chains of v_max3_f32
     auto largest = [&](const f32x16_fl& a, const f32x16_fl& b) -> float {
         float x = -INFINITY, y = -INFINITY;
 #pragma unroll
@@ -555,7 +554,7 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float* ml, const
         }
 #pragma unroll
         for (int u = 0; u < RUNS; ++u) {
-            // a run that saw no key has l = 0; any other counts, also one whose l is NaN (asked by its bits: no NaN is honoured in this file's comparisons)
+            // a run that saw no key has l = 0; any other counts, also one whose l is NaN
             const bool live = s0 + u < nsplit && __float_as_uint(r[s0 + u].y) != 0u;
             const float w = live ? r[s0 + u].y * __builtin_amdgcn_exp2f(r[s0 + u].x - mstar) : 0.f;
             float f[8];

@@ -596,7 +596,8 @@ constexpr int gemmp_ring(int WM, int WN) { return WM * WN >= 16 || (WM == 2 && W
 // Small tiles, whose stages are over before a barrier and the reads behind it are (gemmp_kg): the waves split K as well.  Of a pair of stages one wave of two multiplies the
 // first, its partner the second, each for a piece of 32 WM x 16 WN; one barrier a pair, fewer fragment reads, and the partners trade halves of their sums at the end.  What is left is
 // the rate of the LDS-DMA, 85 to 110 bytes a ns and CU.  Us a launch, the 2 x 2 split / this: K = 2048, N = 1024: 1531 rows, 96 x 64 13.0 / 12.1, 1000 rows, 64 x 64 10.4 / 9.1; K = 3072
-// 17.5 / 16.3 and 13.6 / 12.1; K = 1024, N = 6144, 93 rows, 64 x 64 5.9 / 5.3.  (64 x 128 has no registers for it: twice the time.)
+// 17.5 / 16.3 and 13.6 / 12.1.  Only in front of the residual epilogue: SwiGLU's on 64 x 64 (K = 1024, N = 6144, 93 rows) took 5.9 / 5.3 alone, but 0.989 and 0.998 times the speed in a prompt of 93 and a step of
+// 64 sequences.  (64 x 128 has no registers for it: twice the time.)
 constexpr bool gemmp_kg(int EPI, int WM, int WN) { return WM == 1 || (EPI == 8 && WN == 2 && WM <= 3); }
 constexpr int gemmp_pairs(int WM, int WN) { return WM == 1 ? 6 : WM == 2 ? 5 : 4; }      // pairs of stages in that ring: at most 80 KiB, two workgroups a CU
 template <int EPI, int WM, int WN> constexpr size_t gemmp_lds() {
@@ -1509,8 +1510,10 @@ static int gemmp_tile(int M, int cols, int K, int splits, int most) {
 
 // The same for a product that ends in the residual epilogue with a norm (nothing of it splits along K, so few rows ask for small tiles).
 // 0: 128 x 128, 1: 128 x 64, 2: 64 x 64, 3: 96 x 64, 4: 32 x 64; two workgroups on a CU for 0, 2 and 4.
-// Ms a prompt of Qwen3-0.6B with 1, 2, 3, 4: 450 rows - / 1.91 / 2.00 / 1.74, 600 2.28 / 2.10 / 2.15 / 2.15, 800 2.35 / 2.24 / 2.29 / 2.31, 1100 2.77 / 2.81 / 2.67 / 3.03,
-// 1531 3.07 / 3.07 / 2.99 / 3.31, 1800 3.43 / 3.63 / 3.66 / 3.99.
+// Ms a prompt of Qwen3-0.6B with 1, 2, 3, 4: 450 rows 1.95 / 1.73 / 1.93 / 1.66, 600 2.20 / 1.98 / 2.07 / 2.08, 800 2.39 / 2.25 / 2.32 / 2.37, 1100 2.80 / 2.84 / 2.77 / 2.91,
+// 1531 3.14 / 3.20 / 3.06 / 3.41, 1800 3.55 / 3.75 / 3.81 / 4.08.
+// The prices of 64 x 64 and 96 x 64 are from before K was split over their waves, and 96 x 64 is priced for one workgroup a CU though two fit.  What they choose is within 0.4 % of the best tile at 14 lengths
+// from 140 to 2600 rows of Qwen3-0.6B and at 8 of widths 1536 to 3072, but for 2100 rows (96 x 64 would take 4.34 ms, 128 x 128 takes 4.39) and width 3072 at 300 and 700 rows (1.28 / 1.29, 1.96 / 2.07).
 static int gemmp_resid_tile(int M, int N, int K, int* cost) {
     constexpr struct { int bm, bn, one, one_fixed, two, two_fixed; } t[] = {{128, 128, 18, 450, 29, 640}, {128, 64, 14, 400, 0, 0}, {64, 64, 11, 300, 16, 400}, {96, 64, 13, 350, 0, 0}, {32, 64, 8, 250, 13, 350}};
     int best = 0;
@@ -1523,7 +1526,7 @@ static int gemmp_resid_tile(int M, int N, int K, int* cost) {
     return best;
 }
 // Whether that epilogue pays against a product in `splits` slabs (or `splits` = 1, fp32 +=) and the norm's pass, which takes 6 us and a launch, less what
-// the scaled rows cost the next product.  Qwen3-0.6B, us with the norm: 1531 rows o 20.7 / 14.5, down 25 / 20; 384 rows 15 / 11, 17.5 / 14.5.
+// the scaled rows cost the next product.  Qwen3-0.6B, us with the norm, before the small tiles split K: 1531 rows o 20.7 / 14.5, down 25 / 20; 384 rows 15 / 11, 17.5 / 14.5.
 bool gemm128s_resid_pays(int M, int N, int K, int splits) {
     if (N % 64 != 0) return false;
     if (splits == 1) return true;
