@@ -121,7 +121,7 @@ template <class T, int N> __device__ __forceinline__ void flash_gate_cols(const 
 }
 
 template <class T, int D, bool WIN = false, bool BIAS = false, int SIDES = 1>
-__global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
+__global__ __launch_bounds__(SIDES * FL_THREADS, D == 64 && WIN ? 3 : 2) void flash_fwd_kernel(const T* q, const T* k, const T* v, T* out, int hq, int hkv,
                                                               int q_len, int kv_len, float scale_log2e, FlashStrides sd,
                                                               FlashSplit sp, FlashWindow win, FlashMany many) {
     constexpr int NC = D / 8;            // 16-byte chunks per K row
@@ -226,10 +226,14 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
         v_at += tile_bytes;
     };
     // S^T = K . Q^T of one tile: two 32-kv sub-tiles (rows = positions, column = this lane's query)
+    // Windows of head dim 64 hold one register for the mask's two ends and the bias (a row that is there sees none behind the context): with three the kernel with slopes takes 189, of which a SIMD holds two
+    // waves and not three.  16 heads, 1500 rows, 1024 positions, us, 189 / 168: 28.1 / 23.7; 32 heads 36.3 / 30.7.  (Head dim 128 holds two anyway and is 0.5 % faster with three.)
+    constexpr bool FEW = WIN && D == 64;
+    const int q_at = FEW ? causal_off + qw0 + ql - 4 * h : 0;
     const float slope = BIAS ? win.slopes[head] * win.inv_scale : 0.f;
     auto s_init = [&](int t, f32x16_fl& s0, f32x16_fl& s1) {
-        if constexpr (BIAS) {            // rows are keys kv0 + (r & 3) + 8 (r >> 2) + 4 h (+ 32), this lane's query is position qpos
-            const float b0 = slope * (float)(t * FL_BKV + 4 * h - (causal_off + qw0 + ql));
+        if constexpr (BIAS) {            // rows are keys kv0 + (r & 3) + 8 (r >> 2) + 4 h (+ 32), this lane's query is position q_at + 4 h
+            const float b0 = slope * (float)(FEW ? t * FL_BKV - q_at : t * FL_BKV + 4 * h - (causal_off + qw0 + ql));
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 s0[r] = fmaf(slope, (float)((r & 3) + 8 * (r >> 2)), b0);
@@ -334,8 +338,8 @@ __global__ __launch_bounds__(SIDES * FL_THREADS, 2) void flash_fwd_kernel(const 
             // ---- mask, online softmax (this lane: query qw0 + ql, kv rows (r&3) + 8(r>>2) + 4h of each sub-tile) ----
             const bool need_mask = kv0 + FL_BKV - 1 > causal_off + qw0 || kv0 + FL_BKV > kv_len ||
                                    (WIN && kv0 <= causal_off + qw0 + 31 - win.window);   // wave-uniform
-            const int lim = min(causal_off + qw0 + ql, kv_len - 1) - kv0 - 4 * h;                  // local kv row <= lim is visible
-            const int low = WIN ? causal_off + qw0 + ql - win.window + 1 - kv0 - 4 * h : 0;       // ... and >= low with a window
+            const int lim = FEW ? q_at - kv0 : min(causal_off + qw0 + ql, kv_len - 1) - kv0 - 4 * h;                    // local kv row <= lim is visible
+            const int low = !WIN ? 0 : FEW ? lim - win.window + 1 : causal_off + qw0 + ql - win.window + 1 - kv0 - 4 * h;       // ... and >= low with a window
             float mx = top;
             if (need_mask) {   // diagonal / ragged tiles only: a real wave-uniform branch, not 32 predicated selects per tile
 #pragma unroll
