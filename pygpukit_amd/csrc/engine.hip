@@ -1143,7 +1143,7 @@ __global__ __launch_bounds__(256) void attn_oproj_mfma_kernel(unsigned long long
 // gate/up kernel's PRO_NORM_SUM prologue adds to the residual stream.  Replaces attn_merge_kernel + the o_proj GEMV:
 // one launch and one dependent-kernel gap less per layer (context 2048, w8a16: the pair took 1.95 + 1.3 + 1.74 us of
 // every 23.8 us layer; profiles/r02_config3_timeline.json).  W_o bf16 or fp8 (16 codes per lane, block scale in registers).
-template <int D, int G, bool FP8>
+template <int D, int G, bool FP8, bool FEW>
 __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long long* tl, AttnArgs a) {
     const TLStamp tls(tl);
     constexpr int RS = D + 2, GD = G * D;
@@ -1172,18 +1172,19 @@ __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long lon
         m = hrecs[((size_t)wid * a.nsplit + sc) * RS];
         l = hrecs[((size_t)wid * a.nsplit + sc) * RS + 1];
     }
-    // ... and the records' values, four to a lane, BEFORE the W_o stream and before the barrier below: 40 slices' in one round trip.  The slices are dealt to groups of
+    // ... and the records' values, four to a lane, BEFORE the W_o stream and before the barrier below: 40 slices' in one round trip, 16 where there are no more (FEW: two sequences of Qwen3-0.6B at 2048 816 ->
+    // 803 us a step, one at 400 613 -> 602).  The slices are dealt to groups of
     // LPS threads, whose sums meet in LDS.  (A word of every slice to a thread was 32 instructions a wave for 32 slices, where this is 8, and a round trip of its own for the 33rd.)
-    constexpr int LPS = GD / 4, NG = 256 / LPS, U = (40 + NG - 1) / NG;
+    // Four heads of 128 take 36 at once and 12 in a later trip, for 128 registers, of which a SIMD holds four waves: with trips of 40 in one loop it was 214 and two, and two sequences of 32 / 8 heads at 1900, whose
+    // 1024 workgroups then wait for one another, 282 us a step of 8 layers where they take 259 now.
+    constexpr int LPS = GD / 4, NG = 256 / LPS, U = ((FEW ? 16 : GD > 256 ? 36 : 40) + NG - 1) / NG, MORE = GD > 256 ? 6 : U;
     struct __attribute__((packed, aligned(8))) Four { float v[4]; };      // (a record's values start 8 bytes off a 16-byte line)
     const int e4 = (int)threadIdx.x % LPS, grp = (int)threadIdx.x / LPS, g4 = e4 * 4 / D;
     const float* vals = hrecs + (size_t)g4 * a.nsplit * RS + 2 + e4 * 4 % D;
+    auto value = [&](int sl) { return *reinterpret_cast<const Four*>(vals + (size_t)min(sl, a.nsplit - 1) * RS); };
     Four rv[U];
-    auto values = [&](int s0) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) rv[u] = *reinterpret_cast<const Four*>(vals + (size_t)min(s0 + u * NG + grp, a.nsplit - 1) * RS);
-    };
-    values(0);
+    for (int u = 0; u < U; ++u) rv[u] = value(u * NG + grp);
     __builtin_amdgcn_sched_barrier(0);
     uint4 pre[PRE];
     float psc[PRE];
@@ -1206,17 +1207,19 @@ __global__ __launch_bounds__(256) void attn_merge_oproj_kernel(unsigned long lon
     __syncthreads();
     tls.phase(1);
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0;;) {
+    auto add = [&](int sl, const Four& v) {
+        const float w = sl < a.nsplit ? w_s[g4][min(sl, 63)] : 0.f;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int sl = s0 + u * NG + grp;
-            const float w = sl < a.nsplit ? w_s[g4][min(sl, 63)] : 0.f;
+        for (int i = 0; i < 4; ++i) sum[i] = sl < a.nsplit ? fmaf(w, v.v[i], sum[i]) : sum[i];
+    };
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[i] = sl < a.nsplit ? fmaf(w, rv[u].v[i], sum[i]) : sum[i];
-        }
-        s0 += U * NG;
-        if (s0 >= a.nsplit) break;
-        values(s0);
+    for (int u = 0; u < U; ++u) add(u * NG + grp, rv[u]);
+    for (int s0 = U * NG; s0 < a.nsplit; s0 += MORE * NG) {
+        Four more[MORE];
+#pragma unroll
+        for (int u = 0; u < MORE; ++u) more[u] = value(s0 + u * NG + grp);
+#pragma unroll
+        for (int u = 0; u < MORE; ++u) add(s0 + u * NG + grp, more[u]);
     }
     *reinterpret_cast<float4*>(part_s + grp * GD + e4 * 4) = make_float4(sum[0], sum[1], sum[2], sum[3]);
     __syncthreads();
@@ -1687,11 +1690,13 @@ static pgk_status launch_attn(Engine* e, int layer, int b0, int m, bool fused, b
         mark(KC_OPROJ);
         a.rows_per_block = e->moproj_rows;
         const dim3 g2((c.hidden_size / e->moproj_rows) * c.num_kv_heads, 1, m);
-        const bool f8 = c.weight_format != 0;
+        const bool f8 = c.weight_format != 0, few = a.nsplit <= 16;
 #define PGK_MO(GG)                                                                                             \
     case GG:                                                                                                   \
-        he = f8 ? launch_k(attn_merge_oproj_kernel<D, GG, true>, g2, dim3(256), 0, st, a)                       \
-                : launch_k(attn_merge_oproj_kernel<D, GG, false>, g2, dim3(256), 0, st, a);                     \
+        he = few ? (f8 ? launch_k(attn_merge_oproj_kernel<D, GG, true, true>, g2, dim3(256), 0, st, a)          \
+                       : launch_k(attn_merge_oproj_kernel<D, GG, false, true>, g2, dim3(256), 0, st, a))        \
+                 : (f8 ? launch_k(attn_merge_oproj_kernel<D, GG, true, false>, g2, dim3(256), 0, st, a)         \
+                       : launch_k(attn_merge_oproj_kernel<D, GG, false, false>, g2, dim3(256), 0, st, a));      \
         break;
         switch (G) { PGK_MO(1) PGK_MO(2) PGK_MO(4) default: break; }
 #undef PGK_MO

@@ -36,3 +36,11 @@ def test_windowed_attention_of_head_dim_64_leaves_room_for_three_workgroups():
     assert len(got) == 2, list(got)                              # without and with slopes
     for n, k in got.items():
         assert k[".vgpr_count"] <= 168 and k[".private_segment_fixed_size"] == 0, (n, k[".vgpr_count"], k[".private_segment_fixed_size"])
+
+
+def test_merge_and_o_proj_of_four_heads_leaves_room_for_four_workgroups():
+    """One wave on every SIMD, whose 512 registers hold four of up to 128: two sequences launch more than two workgroups to a CU."""
+    got = {n: k for n, k in _kernels().items() if "attn_merge_oproj_kernelILi128ELi4E" in n}
+    assert len(got) == 4, list(got)                              # bf16 and e4m3 weights, up to 16 slices and more
+    for n, k in got.items():
+        assert k[".vgpr_count"] <= 128 and k[".private_segment_fixed_size"] == 0, (n, k[".vgpr_count"], k[".private_segment_fixed_size"])
